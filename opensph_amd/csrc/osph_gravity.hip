@@ -16,8 +16,8 @@
 // a node whose opening ball does not overlap the target's box goes to the node list; a leaf whose ball
 // overlaps goes to the particle list; other nodes are opened.  Nodes containing the target are always
 // opened and the target's own pairs are summed separately, as the reference's walk never holds a node
-// together with its ancestors.  The walk runs one lane per target over skip links (no stack); the sums
-// run one wavefront per target, its lanes split between the target's particles and the list entries.
+// together with its ancestors.  One wavefront walks for a group of up to 16 neighbouring targets, up to 64 nodes
+// at a time from a stack in LDS; the sums run one wavefront (or, for few targets, several) per target.
 #include "osph_device.h"
 #include "osph_gpu.h"
 #include "osph_gravity.h"
@@ -29,6 +29,7 @@
 #include <cstring>
 #include <map>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 namespace osph {
@@ -52,20 +53,12 @@ struct NodeMom {
 };
 static_assert(sizeof(NodeMom) == 128, "NodeMom is 128 bytes");
 
-// What the walk reads of an internal node, in one 64-byte record.
-struct WalkNode {
-    double4 geo;  // centre of mass, r_open
-    uint32_t first, count, left, skip;
-    uint32_t pad[4];
-};
-static_assert(sizeof(WalkNode) == 64, "WalkNode is 64 bytes");
-
-// The screened walk's record of an internal node, in FP32: the centre of mass as an offset from the root
-// box's centre and r_open, both divided by the power of two 2^e at or above the root box's extent (so the
-// offsets lie within [-1/2, 1/2]); count's top bit marks r_open == 0.
+// What the walk reads of a node it can visit, in FP32: the centre of mass as an offset from the root box's
+// centre and r_open, both divided by the power of two 2^e at or above the root box's extent (so the
+// offsets lie within [-1/2, 1/2]); count's top bit marks r_open == 0.  Written with the node's moments.
 struct WalkNodeF {
     float4 geo;
-    uint32_t first, count, left, skip;
+    uint32_t first, count, left, right;
 };
 static_assert(sizeof(WalkNodeF) == 32, "WalkNodeF is 32 bytes");
 constexpr uint32_t WALK_ZERO_R = 0x80000000u;
@@ -76,15 +69,14 @@ struct Tree {
     uint32_t* left;    // [n-1]
     uint32_t* right;   // [n-1]
     uint32_t* parent;  // [2n-1]
-    uint32_t* skip;    // [2n-1]: the node after this subtree in depth-first order
+    uint32_t* skip;    // [2n-1]: the node after this subtree in depth-first order (evaluation at points)
     uint32_t* first;   // [n-1]
     uint32_t* count;   // [n-1]
     double4* geo;      // [n-1]: centre of mass, r_open
     double4* lo;       // [n-1]: box
     double4* hi;
     NodeMom* mom;      // [n-1]
-    WalkNode* wn;      // [n-1]
-    WalkNodeF* wnf;    // [n-1], for the screened walk
+    WalkNodeF* wnf;    // [n-1]
     double ctr[3];     // the root box's centre and 2^-e, the scale of wnf
     double invL;
     uint32_t* flag;    // [n-1]: node depths while the moments are built
@@ -229,9 +221,6 @@ __global__ void __launch_bounds__(BLOCK) k_radix_tree(Tree t, const uint64_t* __
     t.right[i] = rc;
     t.first[i] = uint32_t(lo);
     t.count[i] = uint32_t(hi - lo + 1);
-    t.wn[i].first = uint32_t(lo);
-    t.wn[i].count = uint32_t(hi - lo + 1);
-    t.wn[i].left = lc;
     t.parent[lc] = uint32_t(i);
     t.parent[rc] = uint32_t(i);
     if (i == 0) t.parent[0] = END;
@@ -255,7 +244,6 @@ __global__ void __launch_bounds__(BLOCK) k_skip(Tree t) {
         c = p;
     }
     t.skip[id] = next;
-    if (id + 1 < t.n) t.wn[id].skip = next;
 }
 
 struct Moments {
@@ -320,6 +308,18 @@ __device__ void add_shifted(const Moments& m, const double d[3], double q2[5], d
     }
 }
 
+// The walk's record of a node whose centre c and opening radius are known.
+__device__ __forceinline__ void write_walk_record(const Tree& t, uint32_t id, const double c[3], double r_open) {
+    WalkNodeF f;
+    f.geo = make_float4(float((c[0] - t.ctr[0]) * t.invL), float((c[1] - t.ctr[1]) * t.invL),
+                        float((c[2] - t.ctr[2]) * t.invL), float(r_open * t.invL));
+    f.first = t.first[id];
+    f.count = t.count[id] | (r_open == 0.0 ? WALK_ZERO_R : 0u);
+    f.left = t.left[id];
+    f.right = t.right[id];
+    t.wnf[id] = f;
+}
+
 // Node `node` from its two children: box, centre of mass and opening radius (BarnesHut::buildInner,
 // BarnesHut.cpp:433-468), moments by the parallel-axis theorem.
 __device__ void combine(const Tree& t, uint32_t node) {
@@ -351,7 +351,7 @@ __device__ void combine(const Tree& t, uint32_t node) {
         add_shifted(b, db, out.q2, out.q3);
     }
     t.geo[node] = make_double4(c[0], c[1], c[2], r_open);
-    t.wn[node].geo = make_double4(c[0], c[1], c[2], r_open);
+    write_walk_record(t, node, c, r_open);
     t.lo[node] = make_double4(lo[0], lo[1], lo[2], 0.0);
     t.hi[node] = make_double4(hi[0], hi[1], hi[2], 0.0);
     t.mom[node] = out;
@@ -438,7 +438,7 @@ __global__ void __launch_bounds__(BLOCK) k_leaf_moments(Tree t, const uint32_t* 
     }
     if (sub != 0) return;
     t.geo[i] = make_double4(c[0], c[1], c[2], r_open);
-    t.wn[i].geo = make_double4(c[0], c[1], c[2], r_open);
+    write_walk_record(t, i, c, r_open);
     t.lo[i] = make_double4(lo[0], lo[1], lo[2], 0.0);
     t.hi[i] = make_double4(hi[0], hi[1], hi[2], 0.0);
     t.mom[i] = out;
@@ -558,133 +558,6 @@ __device__ __forceinline__ void node_range(const Tree& t, uint32_t id, uint32_t&
     }
 }
 
-// One lane's interaction list, written 8 entries (32 B) at a time.  Entries wait in registers until a
-// group of 8 is complete, so every store writes whole 32-byte sectors: single 4-byte appends to a row
-// per lane left partly written lines in L2, which the node-record reads evicted (measured 7x the list
-// bytes written to HBM at 8M particles).  Entries from the capacity on are counted, not stored (the host
-// grows the lists and walks again); capacities are multiples of 8.
-struct ListBuf8 {
-    uint32_t* row;
-    uint32_t cap, n = 0;
-    uint32_t b0 = 0, b1 = 0, b2 = 0, b3 = 0, b4 = 0, b5 = 0, b6 = 0, b7 = 0;
-    __device__ __forceinline__ ListBuf8(uint32_t* r, uint32_t c) : row(r), cap(c) {}
-    __device__ __forceinline__ void push(uint32_t id) {
-        // shift in: after 8 pushes b0..b7 hold the group in order
-        b0 = b1;
-        b1 = b2;
-        b2 = b3;
-        b3 = b4;
-        b4 = b5;
-        b5 = b6;
-        b6 = b7;
-        b7 = id;
-        ++n;
-        if ((n & 7u) == 0 && n <= cap) {
-            uint4* dst = reinterpret_cast<uint4*>(row + (n - 8));
-            dst[0] = make_uint4(b0, b1, b2, b3);
-            dst[1] = make_uint4(b4, b5, b6, b7);
-        }
-    }
-    // the last n % 8 entries (b8-r .. b7)
-    __device__ __forceinline__ void flush() {
-        const uint32_t r = n & 7u;
-        if (r == 0 || n > cap) return;
-        const uint32_t base = n - r;
-        const uint32_t v[8] = { b0, b1, b2, b3, b4, b5, b6, b7 };
-#pragma unroll
-        for (uint32_t u = 0; u < 8; ++u) {
-            if (u < r) row[base + u] = v[8 - r + u];
-        }
-    }
-};
-
-// Interaction lists of one target per lane (BarnesHut::evalNode, BarnesHut.cpp:212-312, applied to the
-// target leaf's box).  Lists of target q live at nlist[q * cap_n ...] and xlist[q * cap_x ...]; counts
-// beyond the capacity are reported so that the host can grow the lists and walk again.
-__global__ void __launch_bounds__(BLOCK) k_walk(Tree t, const uint32_t* __restrict__ targets, uint32_t ntargets,
-                                                uint32_t* __restrict__ nlist, uint32_t cap_n,
-                                                uint32_t* __restrict__ xlist, uint32_t cap_x,
-                                                uint32_t* __restrict__ ncount, uint32_t* __restrict__ xcount,
-                                                uint32_t* __restrict__ work, uint32_t* need) {
-    // each XCD walks one contiguous range of the (Morton-ordered) targets, so the node records that
-    // neighbouring targets share stay in its L2
-    const uint32_t q = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-    if (q >= ntargets) return;
-    const uint32_t T = targets[q];
-    uint32_t tf, tc;
-    node_range(t, T, tf, tc);
-    double lo[3], hi[3];
-    if (is_particle(t, T)) {
-        const double4 p = t.pos[tf];
-        lo[0] = hi[0] = p.x;
-        lo[1] = hi[1] = p.y;
-        lo[2] = hi[2] = p.z;
-    } else {
-        const double4 a = t.lo[T], b = t.hi[T];
-        lo[0] = a.x;
-        lo[1] = a.y;
-        lo[2] = a.z;
-        hi[0] = b.x;
-        hi[1] = b.y;
-        hi[2] = b.z;
-    }
-    uint32_t xsum = 0;
-    ListBuf8 nl(nlist + size_t(q) * cap_n, cap_n), xl(xlist + size_t(q) * cap_x, cap_x);
-    uint32_t id = 0;  // the root: internal node 0, or particle 0 when n == 1
-    // a depth-first walk visits each of the 2n - 1 nodes at most once
-    for (size_t visits = 0; id != END; ++visits) {
-        if (visits > 2 * size_t(t.n)) {
-            atomicOr(t.error, 2u);
-            break;
-        }
-        if (id == T) {
-            id = t.skip[id];
-            continue;
-        }
-        if (is_particle(t, id)) {
-            // a single-particle leaf has r_open = 0: always summed pair by pair (BarnesHut.cpp:237-243)
-            xl.push(id);
-            ++xsum;
-            id = t.skip[id];
-            continue;
-        }
-        const WalkNode w = t.wn[id];
-        if (w.first <= tf && tf + tc <= w.first + w.count) {  // an ancestor of the target
-            id = w.left;
-            continue;
-        }
-        const bool is_leaf = w.count <= t.leaf;
-        const double4 g = w.geo;
-        if (is_leaf && g.w == 0.0) {
-            xl.push(id);
-            xsum += w.count;
-            id = w.skip;
-        } else if (g.w == 0.0) {
-            // more than leaf_size coincident particles: no opening ball; their expansion is singular
-            // for a target at the same point, so the node is opened down to its leaves
-            id = w.left;
-        } else if (!ball_overlaps_box(g, lo, hi)) {
-            nl.push(id);
-            id = w.skip;
-        } else if (is_leaf) {
-            xl.push(id);
-            xsum += w.count;
-            id = w.skip;
-        } else {
-            id = w.left;
-        }
-    }
-    nl.flush();
-    xl.flush();
-    const uint32_t nn = nl.n, nx = xl.n;
-    ncount[q] = nn;
-    xcount[q] = nx;
-    work[2 * size_t(q)] = tc * nn;                        // particle-node expansions
-    work[2 * size_t(q) + 1] = tc * xsum + tc * (tc - 1);  // particle pairs
-    if (nn > cap_n) atomicMax(&need[0], nn);
-    if (nx > cap_x) atomicMax(&need[1], nx);
-}
-
 // The target's box: its leaf's box, or the particle itself.
 __device__ __forceinline__ void target_box(const Tree& t, uint32_t T, uint32_t tf, double lo[3], double hi[3]) {
     if (is_particle(t, T)) {
@@ -701,122 +574,6 @@ __device__ __forceinline__ void target_box(const Tree& t, uint32_t T, uint32_t t
         hi[1] = b.y;
         hi[2] = b.z;
     }
-}
-
-__global__ void __launch_bounds__(BLOCK) k_walk_records(Tree t) {
-    const uint32_t i = uint32_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i + 1 >= t.n) return;
-    const WalkNode w = t.wn[i];
-    WalkNodeF f;
-    f.geo = make_float4(float((w.geo.x - t.ctr[0]) * t.invL), float((w.geo.y - t.ctr[1]) * t.invL),
-                        float((w.geo.z - t.ctr[2]) * t.invL), float(w.geo.w * t.invL));
-    f.first = w.first;
-    f.count = w.count | (w.geo.w == 0.0 ? WALK_ZERO_R : 0u);
-    f.left = w.left;
-    f.skip = w.skip;
-    t.wnf[i] = f;
-}
-
-// k_walk with the opening test screened in FP32: the same interaction lists, in the same order, from
-// 32-byte node records instead of 64-byte ones.  In units of the root box (offsets within [-1/2, 1/2]),
-// the rounding of the box, the centre and r_open to FP32 moves S = |box - centre|^2 by at most
-// 7 delta sqrt(S) (delta = 2^-24) and the FP32 arithmetic adds a few ulps of Q = r_open^2 + S; where
-// |r_open^2 - S| is within 16 delta sqrt(Q) + 2e-6 Q, the FP64 test of k_walk decides.
-__global__ void __launch_bounds__(BLOCK) k_walk_screened(Tree t, const uint32_t* __restrict__ targets,
-                                                         uint32_t ntargets, uint32_t* __restrict__ nlist,
-                                                         uint32_t cap_n, uint32_t* __restrict__ xlist, uint32_t cap_x,
-                                                         uint32_t* __restrict__ ncount, uint32_t* __restrict__ xcount,
-                                                         uint32_t* __restrict__ work, uint32_t* need) {
-    // each XCD walks one contiguous range of the (Morton-ordered) targets, so the node records that
-    // neighbouring targets share stay in its L2
-    const uint32_t q = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-    if (q >= ntargets) return;
-    const uint32_t T = targets[q];
-    uint32_t tf, tc;
-    node_range(t, T, tf, tc);
-    float lof[3], hif[3];
-    {
-        double lo[3], hi[3];
-        target_box(t, T, tf, lo, hi);
-        for (int k = 0; k < 3; ++k) {
-            lof[k] = float((lo[k] - t.ctr[k]) * t.invL);
-            hif[k] = float((hi[k] - t.ctr[k]) * t.invL);
-        }
-    }
-    uint32_t xsum = 0;
-    ListBuf8 nl(nlist + size_t(q) * cap_n, cap_n), xl(xlist + size_t(q) * cap_x, cap_x);
-    uint32_t id = 0;
-    for (size_t visits = 0; id != END; ++visits) {
-        if (visits > 2 * size_t(t.n)) {
-            atomicOr(t.error, 2u);
-            break;
-        }
-        if (id == T) {
-            id = t.skip[id];
-            continue;
-        }
-        if (is_particle(t, id)) {
-            xl.push(id);
-            ++xsum;
-            id = t.skip[id];
-            continue;
-        }
-        const WalkNodeF w = t.wnf[id];
-        const uint32_t cnt = w.count & ~WALK_ZERO_R;
-        if (w.first <= tf && tf + tc <= w.first + cnt) {  // an ancestor of the target
-            id = w.left;
-            continue;
-        }
-        const bool is_leaf = cnt <= t.leaf;
-        const bool zero_r = (w.count & WALK_ZERO_R) != 0u;
-        if (is_leaf && zero_r) {
-            xl.push(id);
-            xsum += cnt;
-            id = w.skip;
-            continue;
-        }
-        if (zero_r) {
-            id = w.left;
-            continue;
-        }
-        float S = 0.f;
-        {
-            const float c[3] = { w.geo.x, w.geo.y, w.geo.z };
-            for (int k = 0; k < 3; ++k) {
-                const float l = fmaxf(lof[k] - c[k], 0.f), r = fmaxf(c[k] - hif[k], 0.f);
-                S += l * l + r * r;
-            }
-        }
-        const float R2 = w.geo.w * w.geo.w;
-        const float m = R2 - S, Q = R2 + S;
-        bool overlaps;
-        if (fabsf(m) > 1e-6f * __builtin_amdgcn_sqrtf(Q) + 2e-6f * Q) {
-            overlaps = m > 0.f;
-        } else {
-            double lo[3], hi[3];
-            target_box(t, T, tf, lo, hi);
-            overlaps = ball_overlaps_box(t.geo[id], lo, hi);
-        }
-        if (!overlaps) {
-            nl.push(id);
-            id = w.skip;
-        } else if (is_leaf) {
-            xl.push(id);
-            xsum += cnt;
-            id = w.skip;
-        } else {
-            id = w.left;
-        }
-    }
-    nl.flush();
-    xl.flush();
-    const uint32_t nn = nl.n, nx = xl.n;
-    ncount[q] = nn;
-    xcount[q] = nx;
-    work[2 * size_t(q)] = tc * nn;
-    work[2 * size_t(q) + 1] = tc * xsum + tc * (tc - 1);
-    if (nn > cap_n) atomicMax(&need[0], nn);
-    if (nx > cap_x) atomicMax(&need[1], nx);
 }
 
 // ---- evaluation ---------------------------------------------------------------------------------------
@@ -919,220 +676,98 @@ __device__ __forceinline__ void add_multipole(const NodeMom& q, double drx, doub
     a[2] += az;
 }
 
-// Per-wavefront staging area of k_eval: 64 node expansions (SoA) or 64 source particles.
-// Moments of the orders below ORDER take no LDS (one unused row keeps the arrays legal): the stage's size
-// bounds the wavefronts per CU.
+// 1 / sqrt(x) for x > 0: the hardware estimate and one third-order step, y (1 + e/2 + 3 e^2 / 8) with e = 1 - x y^2.
+__device__ __forceinline__ double rsqrt_step(double x) {
+    const double y = __builtin_amdgcn_rsq(x);
+    const double e = fma(-(x * y), y, 1.0);
+    return fma(y * e, fma(e, 0.375, 0.5), y);
+}
+
+// A node as the evaluation reads it: centre and mass, then by order q2 (6 components) and q3 (10 components),
+// in FP64 with the factors -3 and 7.5 of the expansion; whole 16-byte chunks, so that a lane reads it with
+// 16-byte LDS loads.
+template <typename T, int ORDER>
+struct alignas(16) NodeRow {
+    static constexpr int N = ORDER >= 3 ? 20 : (ORDER >= 2 ? 10 : 4);
+    T v[sizeof(T) == 4 && ORDER == 2 ? 12 : N];
+};
+
+// The components of q2 times f2 and q3 times f3 of a node into its row.
+template <typename T, int ORDER>
+__device__ __forceinline__ void row_moments(NodeRow<T, ORDER>& r, const NodeMom& q, double f2, double f3) {
+    if constexpr (ORDER >= 2) {
+        for (int k = 0; k < 5; ++k) r.v[4 + k] = T(q.q2[k] * f2);
+        r.v[9] = -r.v[4] - r.v[7];  // zz
+    }
+    if constexpr (ORDER >= 3) {
+        for (int k = 0; k < 7; ++k) r.v[10 + k] = T(q.q3[k] * f3);
+        r.v[17] = -r.v[10] - r.v[13];  // xzz
+        r.v[18] = -r.v[11] - r.v[15];  // yzz
+        r.v[19] = -r.v[12] - r.v[16];  // zzz
+    }
+}
+
+// q3:dd of a row's octupole, the contraction over two indices with d.
+__device__ __forceinline__ void octupole_dd(const NodeRow<double, 3>& r, double dx, double dy, double dz, double w[3]) {
+    const double xx = dx * dx, yy = dy * dy, zz = dz * dz;
+    const double xy = (dx + dx) * dy, xz = (dx + dx) * dz, yz = (dy + dy) * dz;
+    w[0] = r.v[10] * xx + r.v[13] * yy + r.v[17] * zz + r.v[11] * xy + r.v[12] * xz + r.v[14] * yz;
+    w[1] = r.v[11] * xx + r.v[15] * yy + r.v[18] * zz + r.v[13] * xy + r.v[14] * xz + r.v[16] * yz;
+    w[2] = r.v[12] * xx + r.v[16] * yy + r.v[19] * zz + r.v[14] * xy + r.v[17] * xz + r.v[18] * yz;
+}
+
+// evaluateGravity (core/gravity/Moments.h:318-360) of a staged node at the point (x, y, z), added to a.  With
+// d from the point to the node's centre and il = 1 / |d|:
+//   monopole   il^3 M d
+//   quadrupole 7.5 il^7 (d.q2.d) d - 3 il^5 q2.d
+//   octupole   7.5 il^7 (q3:dd) - 17.5 il^9 (q3:ddd) d
+// The terms along d share one factor and the tensors carry theirs (-3, 7.5) from the staging: 40 FP64
+// instructions for a quadrupole, against about 65 in the order the reference writes them.
 template <int ORDER>
-struct EvalStage {
-    double c[3][64];
-    double M[64];
-    double q2[ORDER >= 2 ? 5 : 1][64];
-    double q3[ORDER >= 3 ? 7 : 1][64];
-    double4 src[64];
-    double sm[64];
-    uint32_t sidx[64];
-};
-
-// Lanes of a target leaf's wavefront: lane = sp * tc + p, for particle p < tc of the leaf and split
-// sp < S = 64 / tc.  Lanes from S * tc on take no entries.  (Splits of a power-of-two width would leave
-// up to half the lanes idle for leaves of 17 particles; a 25-particle leaf limit makes most leaves
-// 9-25 particles.)
-struct LaneSplit {
-    uint32_t S, p, sp;
-    bool used;
-};
-
-__device__ __forceinline__ LaneSplit lane_split(uint32_t lane, uint32_t tc) {
-    LaneSplit l;
-    l.S = __builtin_amdgcn_readfirstlane(64u / tc);
-    l.sp = lane / tc;
-    l.p = lane - l.sp * tc;
-    l.used = l.sp < l.S;
-    return l;
-}
-
-// Sums the splits' partial accelerations into the lanes of split 0: split sp adds split sp + d for
-// d = 1, 2, 4, ... when sp is a multiple of 2d.
-__device__ __forceinline__ void sum_splits(const LaneSplit& l, uint32_t lane, uint32_t tc, double a[3]) {
-    for (uint32_t d = 1; d < l.S; d <<= 1) {
-        const int src = int(min(lane + d * tc, 63u));
-        const bool take = l.used && (l.sp & (2 * d - 1)) == 0 && l.sp + d < l.S;
-        for (int c = 0; c < 3; ++c) {
-            const double v = __shfl(a[c], src, 64);
-            if (take) a[c] += v;
+__device__ __forceinline__ void expand(const NodeRow<double, ORDER>& r, double x, double y, double z, double a[3]) {
+    const double dx = r.v[0] - x, dy = r.v[1] - y, dz = r.v[2] - z;
+    const double il = rsqrt_step(dx * dx + dy * dy + dz * dz);
+    const double inv = il * il, i3 = inv * il;
+    double s = i3 * r.v[3];
+    if constexpr (ORDER >= 2) {
+        const double i5 = i3 * inv;
+        double vx = r.v[4] * dx + r.v[5] * dy + r.v[6] * dz;
+        double vy = r.v[5] * dx + r.v[7] * dy + r.v[8] * dz;
+        double vz = r.v[6] * dx + r.v[8] * dy + r.v[9] * dz;
+        s += (-2.5 * i5) * (inv * (vx * dx + vy * dy + vz * dz));
+        if constexpr (ORDER >= 3) {
+            double w[3];
+            octupole_dd(r, dx, dy, dz, w);
+            s += (-7.0 / 3.0 * i5) * ((inv * inv) * (w[0] * dx + w[1] * dy + w[2] * dz));
+            vx += inv * w[0];
+            vy += inv * w[1];
+            vz += inv * w[2];
         }
+        a[0] += vx * i5;
+        a[1] += vy * i5;
+        a[2] += vz * i5;
     }
+    a[0] += dx * s;
+    a[1] += dy * s;
+    a[2] += dz * s;
 }
 
-// One wavefront per target leaf, its lanes split as lane_split says.  The node list and the source
-// particles (every listed leaf followed by the target leaf itself) are staged 64 at a time in the
-// wavefront's LDS with coalesced loads; split sp then takes every S-th staged entry, and the splits are
-// summed across lanes at the end.  Accelerations are added to the state planes.
-template <int ORDER>
-__global__ void __launch_bounds__(BLOCK) k_eval(Tree t, Planes s, const uint32_t* __restrict__ order,
-                                                const uint32_t* __restrict__ targets, uint32_t ntargets,
-                                                const uint32_t* __restrict__ nlist, uint32_t cap_n,
-                                                const uint32_t* __restrict__ xlist, uint32_t cap_x,
-                                                const uint32_t* __restrict__ ncount,
-                                                const uint32_t* __restrict__ xcount, const double* __restrict__ grads) {
-    __shared__ EvalStage<ORDER> stage[BLOCK / 64];
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    EvalStage<ORDER>& S_ = stage[wave];
-    const uint32_t q = (xcd_block(blockIdx.x, gridDim.x) * (BLOCK / 64)) + wave;
-    if (q >= ntargets) return;  // uniform over the wavefront
-    const uint32_t T = targets[q];
-    uint32_t tf, tc;
-    node_range(t, T, tf, tc);
-    const LaneSplit ls = lane_split(lane, tc);
-    const uint32_t S = ls.S, sp = ls.sp;
-    const bool active = ls.used;
-    const uint32_t j0 = active ? sp : 64u;  // unused lanes take no entries
-    const uint32_t k = tf + ls.p;
-    const double4 me = t.pos[k];
-    double a[3] = { 0.0, 0.0, 0.0 };
-    const uint32_t nn = min(ncount[q], cap_n), nx = min(xcount[q], cap_x);
-    const uint32_t* nl = nlist + size_t(q) * cap_n;
-    const uint32_t* xl = xlist + size_t(q) * cap_x;
-
-    // node list
-    for (uint32_t base = 0; base < nn; base += 64) {
-        const uint32_t cnt = min(64u, nn - base);
-        if (lane < cnt) {
-            const uint32_t id = nl[base + lane];
-            const double4 g = t.geo[id];
-            const NodeMom& mm = t.mom[id];
-            S_.c[0][lane] = g.x;
-            S_.c[1][lane] = g.y;
-            S_.c[2][lane] = g.z;
-            S_.M[lane] = mm.M;
-            if constexpr (ORDER >= 2) {
-                for (int c = 0; c < 5; ++c) S_.q2[c][lane] = mm.q2[c];
-            }
-            if constexpr (ORDER >= 3) {
-                for (int c = 0; c < 7; ++c) S_.q3[c][lane] = mm.q3[c];
-            }
-        }
-        wave_sync();
-        for (uint32_t j = j0; j < cnt; j += S) {
-            NodeMom mm;
-            mm.M = S_.M[j];
-            if constexpr (ORDER >= 2) {
-                for (int c = 0; c < 5; ++c) mm.q2[c] = S_.q2[c][j];
-            }
-            if constexpr (ORDER >= 3) {
-                for (int c = 0; c < 7; ++c) mm.q3[c] = S_.q3[c][j];
-            }
-            add_multipole(mm, me.x - S_.c[0][j], me.y - S_.c[1][j], me.z - S_.c[2][j], ORDER, a);
-        }
-        wave_sync();
-    }
-
-    // source particles: entries e < nx are the listed leaves, entry nx is the target leaf
-    const uint32_t nent = nx + 1;
-    for (uint32_t eb = 0; eb < nent; eb += 64) {
-        // entry eb + lane: its range and the exclusive prefix of the counts
-        uint32_t f = 0, c = 0;
-        const uint32_t e = eb + lane;
-        if (e < nx) {
-            node_range(t, xl[e], f, c);
-        } else if (e == nx) {
-            f = tf;
-            c = tc;
-        }
-        uint32_t incl = c;
-        for (int o = 1; o < 64; o <<= 1) {
-            const uint32_t v = __shfl_up(incl, o, 64);
-            if (lane >= uint32_t(o)) incl += v;
-        }
-        const uint32_t excl = incl - c;
-        const uint32_t total = __shfl(incl, 63, 64);
-        for (uint32_t s0 = 0; s0 < total; s0 += 64) {
-            const uint32_t slot = s0 + lane;
-            const uint32_t cnt = min(64u, total - s0);
-            // the entry holding this slot: the last lane whose exclusive prefix is <= slot (all lanes take
-            // part in the cross-lane reads; only lanes with a slot load)
-            int lo = 0;
-            for (int step = 32; step > 0; step >>= 1) {
-                const uint32_t ex = __shfl(excl, (lo + step) & 63, 64);
-                if (lo + step < 64 && ex <= slot) lo += step;
-            }
-            const uint32_t fe = __shfl(f, lo, 64), xe = __shfl(excl, lo, 64);
-            if (lane < cnt) {
-                const uint32_t src = fe + (slot - xe);
-                S_.src[lane] = t.pos[src];
-                S_.sm[lane] = t.gm[src];
-                S_.sidx[lane] = src;
-            }
-            wave_sync();
-            for (uint32_t j = j0; j < cnt; j += S) {
-                if (S_.sidx[j] == k) continue;
-                const double4 o = S_.src[j];
-                add_pair<false>(grads, o.x - me.x, o.y - me.y, o.z - me.z, 0.5 * (o.w + me.w), S_.sm[j], a);
-            }
-            wave_sync();
-        }
-    }
-    sum_splits(ls, lane, tc, a);
-    if (sp == 0) {
-        const uint32_t i = order[k];
-        s.d[GAX][i] += a[0];
-        s.d[GAY][i] += a[1];
-        s.d[GAZ][i] += a[2];
-    }
-}
-
-// ---- mixed-precision evaluation ---------------------------------------------------------------------
-
-// Largest value over the wavefront (every lane gets it).
-__device__ __forceinline__ float wave_max_f(float v) {
-    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-    return v;
-}
-
-// Powers of two that bring lengths and G m into FP32's comfortable range: lengths are divided by
-// 2^e with the root box extent in [2^(e-1), 2^e), G m by 2^f with the total G m in [2^(f-1), 2^f).
-// Both divisions are exact in FP64; the results are scaled back by 2^(f - 2e).
-struct EvalScale {
-    double invL, invM, back;
-};
-
-// A wave-uniform double kept in scalar registers.
-__device__ __forceinline__ double uniform_d(double v) {
-    const unsigned long long b = (unsigned long long)__double_as_longlong(v);
-    const uint32_t lo = __builtin_amdgcn_readfirstlane(uint32_t(b)), hi = __builtin_amdgcn_readfirstlane(uint32_t(b >> 32));
-    return __longlong_as_double((long long)((unsigned long long)hi << 32 | lo));
-}
-
-__device__ __forceinline__ EvalScale eval_scale(const Tree& t) {
-    EvalScale sc{ 1.0, 1.0, 1.0 };
-    if (t.n < 2) return sc;
-    const double4 lo = t.lo[0], hi = t.hi[0];
-    const double ext = fmax(fmax(hi.x - lo.x, hi.y - lo.y), hi.z - lo.z);
-    int e = 0, f = 0;
-    if (ext > 0.0) (void)frexp(ext, &e);
-    const double M = t.mom[0].M;
-    if (M > 0.0) (void)frexp(M, &f);
-    sc.invL = uniform_d(ldexp(1.0, -e));
-    sc.invM = uniform_d(ldexp(1.0, -f));
-    sc.back = uniform_d(ldexp(1.0, f - 2 * e));
-    return sc;
-}
-
-// The multipole expansion of add_multipole in FP32, written so that no intermediate leaves FP32's range:
-// with d the vector from the target to the node's centre of mass, il = 1/|d|, u = d il and w = il^2,
+// The multipole expansion in FP32, written so that no intermediate leaves FP32's range: with d the vector from
+// the target to the node's centre of mass, il = 1/|d|, u = d il and w = il^2,
 //   monopole   il^3 M d                                  = w M u
 //   quadrupole il^4 (7.5 u (u.q2.u) - 3 q2.u)            = w^2 t2
 //   octupole   il^5 (7.5 (q3:uu) - 17.5 u (q3:uuu))      = w^2 il t3
-// and an approximated node has size < theta |d|, so w |q2| < theta^2 M and w il |q3| < theta^3 M.
+// and an approximated node has size < theta |d|, so w |q2| < theta^2 M and w il |q3| < theta^3 M.  The row holds
+// q2 and q3 themselves, with the components that follow from the vanishing traces.
 template <int ORDER>
-__device__ __forceinline__ void add_multipole_f(float M, const float* q2, const float* q3, float dx, float dy, float dz,
-                                                float a[3]) {
+__device__ __forceinline__ void expand(const NodeRow<float, ORDER>& r, float mx, float my, float mz, float a[3]) {
+    const float dx = r.v[0] - mx, dy = r.v[1] - my, dz = r.v[2] - mz, M = r.v[3];
     const float il = __builtin_amdgcn_rsqf(dx * dx + dy * dy + dz * dz);
     const float w = il * il;
     const float u0 = dx * il, u1 = dy * il, u2 = dz * il;
     float hx = 0.f, hy = 0.f, hz = 0.f;
     if constexpr (ORDER >= 2) {
-        const float xx = q2[0], xy = q2[1], xz = q2[2], yy = q2[3], yz = q2[4], zz = -xx - yy;
+        const float xx = r.v[4], xy = r.v[5], xz = r.v[6], yy = r.v[7], yz = r.v[8], zz = r.v[9];
         const float Q1x = xx * u0 + xy * u1 + xz * u2;
         const float Q1y = xy * u0 + yy * u1 + yz * u2;
         const float Q1z = xz * u0 + yz * u1 + zz * u2;
@@ -1142,8 +777,8 @@ __device__ __forceinline__ void add_multipole_f(float M, const float* q2, const 
         hz = Q0 * u2 - 3.f * Q1z;
     }
     if constexpr (ORDER >= 3) {
-        const float xxx = q3[0], xxy = q3[1], xxz = q3[2], xyy = q3[3], xyz = q3[4], yyy = q3[5], yyz = q3[6];
-        const float xzz = -xxx - xyy, yzz = -xxy - yyy, zzz = -xxz - yyz;
+        const float xxx = r.v[10], xxy = r.v[11], xxz = r.v[12], xyy = r.v[13], xyz = r.v[14], yyy = r.v[15],
+                    yyz = r.v[16], xzz = r.v[17], yzz = r.v[18], zzz = r.v[19];
         const float Q1x = xxx * u0 * u0 + xyy * u1 * u1 + xzz * u2 * u2 + 2.f * (xxy * u0 * u1 + xxz * u0 * u2 + xyz * u1 * u2);
         const float Q1y = xxy * u0 * u0 + yyy * u1 * u1 + yzz * u2 * u2 + 2.f * (xyy * u0 * u1 + xyz * u0 * u2 + yyz * u1 * u2);
         const float Q1z = xxz * u0 * u0 + yyz * u1 * u1 + zzz * u2 * u2 + 2.f * (xyz * u0 * u1 + xzz * u0 * u2 + yzz * u1 * u2);
@@ -1181,46 +816,498 @@ __device__ __forceinline__ void add_pair_f(const double* __restrict__ grads, flo
     a[2] += rz * f;
 }
 
-// Per-wavefront staging area of k_eval_mixed: the FP32 half of EvalStage.
-template <int ORDER>
-struct EvalStageF {
-    float c[3][64];
-    float M[64];
-    float q2[ORDER >= 2 ? 5 : 1][64];
-    float q3[ORDER >= 3 ? 7 : 1][64];
-    float4 src[64];
-    float sm[64];
-    uint32_t sidx[64];
+// Lanes of a wavefront over m particles (or pairs of particles) of a target leaf: lane = sp * m + p, for p < m
+// and split sp < S = 64 / m.  Lanes from S * m on take no entries.  (Splits of a power-of-two width would leave
+// up to half the lanes idle for 17 particles; a 25-particle leaf limit makes most leaves 9-25 particles.)
+struct LaneSplit {
+    uint32_t m, S, p, sp;
+    bool used;
 };
 
-// k_eval with FP32 arithmetic on offsets from the first particle of the target leaf (R), lengths and
-// G m scaled by eval_scale.  A pair separation taken as the difference of two FP32 offsets is off by at
-// most 2^-23 O, with O the largest offset among the batch's sources and the wavefront's targets: pairs
-// closer than O / 8 (where that is more than 1e-6 of the separation) take theirs in FP64 from the
-// source's FP64 position instead.  The lanes, lists, splits and the order of the staged entries are
-// those of k_eval.  Each batch of up to 64 staged entries is summed in FP32 and added to FP64
-// accumulators; the accelerations are scaled back and added to the state planes in FP64.
+__device__ __forceinline__ LaneSplit lane_split(uint32_t lane, uint32_t m) {
+    LaneSplit l;
+    l.m = m;
+    l.S = __builtin_amdgcn_readfirstlane(64u / m);
+    l.sp = lane / m;
+    l.p = lane - l.sp * m;
+    l.used = l.sp < l.S;
+    return l;
+}
+
+// Sums the splits' partial accelerations into the lanes of split 0: split sp adds split sp + d for
+// d = 1, 2, 4, ... when sp is a multiple of 2d.
+__device__ __forceinline__ void sum_splits(const LaneSplit& l, uint32_t lane, double a[3]) {
+    for (uint32_t d = 1; d < l.S; d <<= 1) {
+        const int src = int(min(lane + d * l.m, 63u));
+        const bool take = l.used && (l.sp & (2 * d - 1)) == 0 && l.sp + d < l.S;
+        for (int c = 0; c < 3; ++c) {
+            const double v = __shfl(a[c], src, 64);
+            if (take) a[c] += v;
+        }
+    }
+}
+
+template <int CTRL>
+__device__ __forceinline__ float dpp_max(float v) {
+    const int b = __float_as_int(v);
+    return fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(b, b, CTRL, 0xf, 0xf, false)));
+}
+
+// Largest value over the wavefront, all lanes active (row shifts by 1, 2, 4, 8, then the row broadcasts: the
+// last lane holds it).
+__device__ __forceinline__ float wave_max_f(float v) {
+    v = dpp_max<0x111>(v);
+    v = dpp_max<0x112>(v);
+    v = dpp_max<0x114>(v);
+    v = dpp_max<0x118>(v);
+    v = dpp_max<0x142>(v);
+    v = dpp_max<0x143>(v);
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+}
+
+// Powers of two that bring lengths and G m into FP32's comfortable range: lengths are divided by
+// 2^e with the root box extent in [2^(e-1), 2^e), G m by 2^f with the total G m in [2^(f-1), 2^f).
+// Both divisions are exact in FP64; the results are scaled back by 2^(f - 2e).
+struct EvalScale {
+    double invL, invM, back;
+};
+
+// A wave-uniform double kept in scalar registers.
+__device__ __forceinline__ double uniform_d(double v) {
+    const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane(uint32_t(b)), hi = __builtin_amdgcn_readfirstlane(uint32_t(b >> 32));
+    return __longlong_as_double((long long)((unsigned long long)hi << 32 | lo));
+}
+
+__device__ __forceinline__ EvalScale eval_scale(const Tree& t) {
+    EvalScale sc{ 1.0, 1.0, 1.0 };
+    if (t.n < 2) return sc;
+    const double4 lo = t.lo[0], hi = t.hi[0];
+    const double ext = fmax(fmax(hi.x - lo.x, hi.y - lo.y), hi.z - lo.z);
+    int e = 0, f = 0;
+    if (ext > 0.0) (void)frexp(ext, &e);
+    const double M = t.mom[0].M;
+    if (M > 0.0) (void)frexp(M, &f);
+    sc.invL = uniform_d(ldexp(1.0, -e));
+    sc.invM = uniform_d(ldexp(1.0, -f));
+    sc.back = uniform_d(ldexp(1.0, f - 2 * e));
+    return sc;
+}
+
+// The walk (BarnesHut::evalNode, BarnesHut.cpp:212-312) for groups of up to WALK_GROUP neighbouring targets, whose
+// lists are mostly the same nodes.  The group's list holds, in depth-first order, the nodes that any of its
+// targets takes: .x the node, .y the targets that approximate it (bit g for target g of the group) and, in the
+// high half, those that sum its particles.  A target's own list is the entries with its bit.
+constexpr uint32_t WALK_GROUP = 16;
+// Stack items: a node to be classified for the targets .y, or (WALK_KNOWN) an entry of the list that waits for the
+// nodes before it.  Node ids take 31 bits: the tree of 2^30 particles would fill 600 GB.
+constexpr uint32_t WALK_KNOWN = 0x80000000u;
+// A step takes up to 64 items from the top and puts back at most two more than each; the last WALK_DFS slots are
+// for single-item steps only, whose growth is bounded by the depth of the tree.
+constexpr uint32_t WALK_STACK = 768, WALK_DFS = 256;
+static_assert(WALK_DFS > 2 * (MAX_DEPTH + 1), "a depth-first walk fits the reserve");
+
+struct alignas(16) WalkStage {
+    uint2 stack[WALK_STACK];
+    float4 box_a[WALK_GROUP];  // lo x, y, z and hi x of the targets' boxes in the records' frame
+    float4 box_b[WALK_GROUP];  // hi y, z and the first particle (bits)
+};
+
+// The opening test of target id (first particle f) on node `node` in FP64.
+__device__ __forceinline__ bool overlaps_exact(const Tree& t, uint32_t id, uint32_t f, uint32_t node) {
+    double lo[3], hi[3];
+    target_box(t, id, f, lo, hi);
+    return ball_overlaps_box(t.geo[node], lo, hi);
+}
+
+// One wavefront per group.  Each lane classifies one node for every target of the group: a node that contains
+// the target is opened (or, when it is the target itself, dropped: its own pairs are summed apart); a node
+// without opening ball (coincident particles) is summed when it is a leaf and opened otherwise, as its expansion
+// is singular; a node whose ball does not overlap the target's box is approximated; an overlapping leaf is
+// summed; others are opened.  A step takes the next 64 items in depth-first order, emits those before the first
+// opened node, and puts the others back with each opened node replaced by its children.
+//
+// With one lane per target instead (each lane its own chain of dependent node loads, 36 cache lines per load
+// instruction) the walk of 8M particles took 5.0 ms and of 20k particles 0.78 ms; this walk takes 1.7 ms
+// and 40 us, bound by instruction issue: about 24 instructions per node and target, while the group shares the
+// node's load and the stack's bookkeeping.
+//
+// With `screen` the opening test runs in FP32 on the records: with offsets within [-1/2, 1/2], the rounding of
+// the box, the centre and r_open moves S = |box - centre|^2 by at most 7 delta sqrt(S) (delta = 2^-24) and the
+// FP32 arithmetic adds a few ulps of Q = r_open^2 + S, so that |r_open^2 - S| > 1e-6 sqrt(Q) + 2e-6 Q (16 delta =
+// 9.5e-7) decides.  The band is taken per node as 2e-6 r_open + 8e-6 r_open^2 + 1e-10: for S <= 3 r_open^2 it
+// is at least that, and beyond, |r_open^2 - S| > 1e-10 alone implies it.  Within the band, and without
+// `screen`, the FP64 test decides, so the lists are those of the FP64 test alone.
+__global__ void __launch_bounds__(BLOCK) k_walk(Tree t, const uint32_t* __restrict__ targets, uint32_t ntargets,
+                                                uint32_t group, int screen, uint2* __restrict__ list, uint32_t cap,
+                                                uint32_t* __restrict__ list_count, uint32_t* need) {
+    __shared__ WalkStage stages[BLOCK / 64];
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    WalkStage& S_ = stages[wave];
+    // each XCD takes one contiguous range of the (Morton-ordered) targets, so the nodes that neighbouring
+    // groups share stay in its L2
+    const uint32_t grp = xcd_block(blockIdx.x, gridDim.x) * (BLOCK / 64) + wave;
+    const uint32_t q0 = grp * group;
+    if (q0 >= ntargets) return;  // uniform over the wavefront
+    const uint32_t gc = min(group, ntargets - q0);
+    if (lane < gc) {
+        const uint32_t id = targets[q0 + lane];
+        uint32_t f, c;
+        node_range(t, id, f, c);
+        double lo[3], hi[3];
+        target_box(t, id, f, lo, hi);
+        float b[6];
+        for (int k = 0; k < 3; ++k) {
+            b[k] = float((lo[k] - t.ctr[k]) * t.invL);
+            b[3 + k] = float((hi[k] - t.ctr[k]) * t.invL);
+        }
+        S_.box_a[lane] = make_float4(b[0], b[1], b[2], b[3]);
+        S_.box_b[lane] = make_float4(b[4], b[5], __uint_as_float(f), 0.f);
+    }
+    if (lane == 0) S_.stack[0] = make_uint2(0u, (1u << gc) - 1u);  // the root: internal node 0, or particle 0
+    wave_sync();
+    uint2* out = list + size_t(grp) * cap;
+    const unsigned long long below = (1ull << lane) - 1ull;
+    uint32_t size = 1, cnt = 0;
+    for (uint32_t steps = 0; size > 0; ++steps) {
+        if (steps > 3u * t.n) {  // every step emits, drops or opens the first of its items
+            if (lane == 0) atomicOr(t.error, 2u);
+            break;
+        }
+        const uint32_t room = size + WALK_DFS < WALK_STACK ? (WALK_STACK - WALK_DFS - size) / 2u : 0u;
+        const uint32_t take = min(min(64u, size), max(room, 1u));
+        uint32_t id = 0, left = 0, right = 0, approx = 0, sum = 0, open = 0;
+        if (lane < take) {
+            const uint2 item = S_.stack[size - 1u - lane];
+            id = item.x & ~WALK_KNOWN;
+            const uint32_t active = item.y;
+            if (item.x & WALK_KNOWN) {
+                approx = active & 0xffffu;
+                sum = active >> 16;
+            } else {
+                WalkNodeF w;
+                if (is_particle(t, id)) {
+                    // a single particle has r_open = 0: always summed pair by pair (BarnesHut.cpp:237-243)
+                    w.geo = make_float4(0.f, 0.f, 0.f, 0.f);
+                    w.first = id - (t.n - 1);
+                    w.count = 1u | WALK_ZERO_R;
+                    w.left = w.right = 0u;
+                } else {
+                    w = t.wnf[id];
+                }
+                const uint32_t count = w.count & ~WALK_ZERO_R;
+                const float R2 = w.geo.w * w.geo.w;
+                const float band = 2e-6f * w.geo.w + 8e-6f * R2 + 1e-10f;
+                uint32_t near = 0, unsure = 0, own = 0;
+                for (uint32_t g = 0; g < gc; ++g) {
+                    const float4 a = S_.box_a[g], b = S_.box_b[g];
+                    const float dx = fmaxf(fmaxf(a.x - w.geo.x, w.geo.x - a.w), 0.f);
+                    const float dy = fmaxf(fmaxf(a.y - w.geo.y, w.geo.y - b.x), 0.f);
+                    const float dz = fmaxf(fmaxf(a.z - w.geo.z, w.geo.z - b.y), 0.f);
+                    const float m = R2 - (dx * dx + dy * dy + dz * dz);
+                    const uint32_t bit = 1u << g;
+                    if (m > 0.f) near |= bit;
+                    if (!(fabsf(m) > band)) unsure |= bit;
+                    if (__float_as_uint(b.z) - w.first < count) own |= bit;  // the node contains the target
+                }
+                if (!screen) unsure = ~0u;
+                if (w.count & WALK_ZERO_R) {
+                    near = ~0u;
+                    unsure = 0u;
+                }
+                for (uint32_t u = unsure & active & ~own; u != 0u; u &= u - 1u) {
+                    const uint32_t g = uint32_t(__builtin_ctz(u));
+                    const bool o = overlaps_exact(t, targets[q0 + g], __float_as_uint(S_.box_b[g].z), id);
+                    near = o ? near | (1u << g) : near & ~(1u << g);
+                }
+                near |= own;
+                approx = active & ~near;
+                if (count <= t.leaf) {
+                    sum = active & near & ~own;
+                } else {
+                    open = active & near;
+                }
+                left = w.left;
+                right = w.right;
+            }
+        }
+        const bool entry = (approx | sum) != 0u;
+        const unsigned long long om = __ballot(open != 0u), em = __ballot(entry);
+        // emitted now: the entries up to and with the first opened node (an entry comes before its children)
+        const unsigned long long head = om ? om ^ (om - 1ull) : ~0ull;
+        if (((em & head) >> lane) & 1ull) {
+            const uint32_t at = cnt + __popcll(em & head & below);
+            if (at < cap) out[at] = make_uint2(id, approx | (sum << 16));
+        }
+        cnt += __popcll(em & head);
+        // the others go back in order, the top first
+        const unsigned long long back = em & ~head;
+        size += __popcll(back) + 2u * __popcll(om) - take;
+        uint32_t at = size - 1u - (__popcll(back & below) + 2u * __popcll(om & below));
+        if ((back >> lane) & 1ull) S_.stack[at--] = make_uint2(id | WALK_KNOWN, approx | (sum << 16));
+        if (open) {
+            S_.stack[at] = make_uint2(left, open);
+            S_.stack[at - 1u] = make_uint2(right, open);
+        }
+        wave_sync();
+    }
+    if (lane == 0) {
+        list_count[grp] = cnt;
+        if (cnt > cap) atomicMax(need, cnt);
+    }
+}
+
+// A wavefront's LDS: 64 staged nodes or source particles, and the node ids and particle positions collected so
+// far (fewer than 64 from before, and up to 64 more from one step or one leaf).
+template <typename T, int ORDER>
+struct alignas(16) EvalStage {
+    struct alignas(16) Src {
+        T x, y, z, m;
+    };
+    union {
+        NodeRow<T, ORDER> row[64];
+        struct {
+            Src src[64];
+            T h[64];
+            uint32_t idx[64];
+        };
+    };
+    uint32_t nodes[128];
+    uint32_t parts[128];
+};
+
+// The lists of the groups of targets (k_walk).
+struct WalkLists {
+    const uint2* list;
+    const uint32_t* count;
+    uint32_t cap, group;
+};
+
+// Interaction counts per target (null: not wanted).
+struct EvalCounts {
+    uint32_t *nodes, *leaves, *work;
+};
+
+// The wavefronts' sums of a shared target (mine: 3 doubles per particle in the wavefront's own stage), added in
+// order by the first wavefront to the accelerations of the target's particles.
+template <typename Stage>
+__device__ __forceinline__ void add_shared(const Planes& s, const uint32_t* __restrict__ order, const Stage* stages,
+                                           uint32_t split, uint32_t wave, uint32_t lane, uint32_t tf, uint32_t tc,
+                                           double back) {
+    static_assert(sizeof(Stage) >= 64 * 3 * sizeof(double), "the stage holds a leaf's sums");
+    __syncthreads();
+    if (wave != 0 || lane >= tc) return;
+    double v[3] = { 0.0, 0.0, 0.0 };
+    for (uint32_t w = 0; w < split; ++w) {
+        const double* from = reinterpret_cast<const double*>(stages + w);
+        for (int c = 0; c < 3; ++c) v[c] += from[3 * lane + c];
+    }
+    const uint32_t i = order[tf + lane];
+    s.d[GAX][i] += v[0] * back;
+    s.d[GAY][i] += v[1] * back;
+    s.d[GAZ][i] += v[2] * back;
+}
+
+// The sums of a target's list in FP64, one target per wavefront (split = 1) or per block (split = the block's
+// wavefronts), added to the accelerations in the state planes.  The group's list is scanned 64 entries at a time;
+// the target's nodes and the particles of its leaves are collected in LDS, staged by batches and summed.  With
+// split > 1 every wavefront of the block scans alike and evaluates every split-th batch.
+//
+// A lane holds two particles of the target, p and p + m with m = ceil(tc / 2).  That halves the LDS reads of the
+// staged entries, which take as long as the arithmetic of one, and fills the wavefront better (17 particles: 63
+// lanes of 9 x 7, against 51 of 17 x 3).  A batch is B = S floor(64 / S) entries, so that each of the S splits of
+// the wavefront takes the same number.  One comparison against the batch's largest softening radius sends a pair
+// to the branch that handles softening and the particle itself; the others are Newtonian.
+template <int ORDER>
+__global__ void __launch_bounds__(BLOCK) k_eval(Tree t, Planes s, const uint32_t* __restrict__ order,
+                                                const uint32_t* __restrict__ targets, uint32_t ntargets, WalkLists wl,
+                                                uint32_t split, EvalCounts counts, const double* __restrict__ grads) {
+    using Stage = EvalStage<double, ORDER>;
+    __shared__ Stage stages[BLOCK / 64];
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    Stage& S_ = stages[wave];
+    const uint32_t block = xcd_block(blockIdx.x, gridDim.x);
+    const uint32_t q = split > 1 ? block : block * (BLOCK / 64) + wave;
+    const uint32_t part = split > 1 ? wave : 0u;
+    if (q >= ntargets) return;  // uniform over the wavefront, and over the block when it shares a target
+    uint32_t tf, tc;
+    node_range(t, targets[q], tf, tc);
+    const LaneSplit ls = lane_split(lane, (tc + 1) / 2);
+    const uint32_t S = ls.S, B = __builtin_amdgcn_readfirstlane(S * (64u / S));
+    const uint32_t j0 = ls.used ? ls.sp : 64u;  // unused lanes take no entries
+    const bool two = ls.p + ls.m < tc;
+    const uint32_t k0 = tf + ls.p, k1 = two ? k0 + ls.m : k0;
+    const double4 me0 = t.pos[k0], me1 = t.pos[k1];
+    const float hmax = wave_max_f(ls.used ? fmaxf(float(me0.w), float(me1.w)) * 1.000001f : 0.f);  // rounded up
+    double a0[3] = { 0.0, 0.0, 0.0 }, a1[3] = { 0.0, 0.0, 0.0 };
+    const unsigned long long below = (1ull << lane) - 1ull;
+    const uint32_t grp = q / wl.group, abit = 1u << (q - grp * wl.group), sbit = abit << 16;
+    const uint2* list = wl.list + size_t(grp) * wl.cap;
+    const uint32_t entries = wl.count[grp];
+    uint32_t at = 0, nfill = 0, pfill = 0;     // scanned entries, collected nodes, collected particles
+    uint32_t nbatch = 0, pbatch = 0;           // batches so far
+    uint32_t ncnt = 0, xcnt = 0, xsum = 0;
+    // leaves whose particles are still to be collected: range (ef, ec) in the lanes of `em`; first the target
+    uint32_t ef = tf, ec = tc;
+    unsigned long long em = 1ull;
+    for (;;) {
+        while (em != 0ull && pfill < B) {
+            const int l = __builtin_ctzll(em);
+            em &= em - 1ull;
+            const uint32_t f = __builtin_amdgcn_readlane(ef, l), c = __builtin_amdgcn_readlane(ec, l);
+            if (lane < c) S_.parts[pfill + lane] = f + lane;
+            pfill += c;
+            xsum += c;
+        }
+        wave_sync();
+        if (at < entries && em == 0ull && nfill < B && pfill < B) {
+            const uint2 e = at + lane < entries ? list[at + lane] : make_uint2(0u, 0u);
+            at += 64u;
+            const unsigned long long am = __ballot((e.y & abit) != 0u);
+            em = __ballot((e.y & sbit) != 0u);
+            if (e.y & abit) S_.nodes[nfill + __popcll(am & below)] = e.x;
+            nfill += __popcll(am);
+            if (e.y & sbit) node_range(t, e.x, ef, ec);
+            ncnt += __popcll(am);
+            xcnt += __popcll(em);
+            continue;
+        }
+        if (nfill >= B || (at >= entries && nfill > 0)) {
+            const uint32_t cnt = min(nfill, B);
+            nfill -= cnt;
+            if (nbatch++ % split == part) {
+                if (lane < cnt) {
+                    const uint32_t id = S_.nodes[nfill + lane];
+                    const double4 g = t.geo[id];
+                    const NodeMom& mm = t.mom[id];
+                    NodeRow<double, ORDER> r;
+                    r.v[0] = g.x;
+                    r.v[1] = g.y;
+                    r.v[2] = g.z;
+                    r.v[3] = mm.M;
+                    row_moments<double, ORDER>(r, mm, -3.0, 7.5);
+                    S_.row[lane] = r;
+                }
+                wave_sync();
+                for (uint32_t j = j0; j < cnt; j += S) {
+                    const NodeRow<double, ORDER> r = S_.row[j];
+                    expand<ORDER>(r, me0.x, me0.y, me0.z, a0);
+                    expand<ORDER>(r, me1.x, me1.y, me1.z, a1);
+                }
+                wave_sync();
+            }
+        }
+        const bool last = at >= entries && em == 0ull;
+        if (pfill >= B || (last && pfill > 0)) {
+            const uint32_t cnt = min(pfill, B);
+            pfill -= cnt;
+            if (pbatch++ % split == part) {
+                float reach = 0.f;
+                if (lane < cnt) {
+                    const uint32_t src = S_.parts[pfill + lane];
+                    const double4 o = t.pos[src];
+                    S_.src[lane] = { o.x, o.y, o.z, t.gm[src] };
+                    S_.h[lane] = o.w;
+                    S_.idx[lane] = src;
+                    reach = float(o.w);
+                }
+                wave_sync();
+                // pairs beyond `far` are Newtonian: farther than (h_i + h_j), the support of the softened kernel at
+                // the mean h, for the largest h of the batch and of the targets (0 for point particles)
+                double far = 0.0;
+                if (grads) {
+                    const double r = double(wave_max_f(reach) * 1.000001f + hmax);
+                    far = r * r;
+                }
+                auto pair = [&](uint32_t j, uint32_t k, const typename Stage::Src& o, const double4& me, double* a) {
+                    const double rx = o.x - me.x, ry = o.y - me.y, rz = o.z - me.z;
+                    const double d2 = rx * rx + ry * ry + rz * rz;
+                    if (d2 <= far) {
+                        if (S_.idx[j] != k) add_pair<false>(grads, rx, ry, rz, 0.5 * (S_.h[j] + me.w), o.m, a);
+                    } else {
+                        const double il = rsqrt_step(d2);
+                        const double f = (o.m * il) * (il * il);
+                        a[0] += rx * f;
+                        a[1] += ry * f;
+                        a[2] += rz * f;
+                    }
+                };
+                for (uint32_t j = j0; j < cnt; j += S) {
+                    const typename Stage::Src o = S_.src[j];
+                    pair(j, k0, o, me0, a0);
+                    pair(j, k1, o, me1, a1);
+                }
+                wave_sync();
+            }
+        }
+        if (last && nfill == 0 && pfill == 0) break;
+    }
+    sum_splits(ls, lane, a0);
+    sum_splits(ls, lane, a1);
+    if (counts.nodes && lane == 0 && part == 0) {
+        counts.nodes[q] = ncnt;
+        counts.leaves[q] = xcnt;
+        counts.work[2 * size_t(q)] = tc * ncnt;            // particle-node expansions
+        counts.work[2 * size_t(q) + 1] = tc * (xsum - 1);  // particle pairs (xsum with the target's own)
+    }
+    const bool writes = ls.used && ls.sp == 0;
+    if (split > 1) {
+        double* mine = reinterpret_cast<double*>(&S_);
+        for (int c = 0; c < 3; ++c) {
+            if (writes) mine[3 * ls.p + c] = a0[c];
+            if (writes && two) mine[3 * (ls.p + ls.m) + c] = a1[c];
+        }
+        add_shared(s, order, stages, split, wave, lane, tf, tc, 1.0);
+        return;
+    }
+    if (writes) {
+        const uint32_t i = order[k0];
+        s.d[GAX][i] += a0[0];
+        s.d[GAY][i] += a0[1];
+        s.d[GAZ][i] += a0[2];
+        if (two) {
+            const uint32_t i2 = order[k1];
+            s.d[GAX][i2] += a1[0];
+            s.d[GAY][i2] += a1[1];
+            s.d[GAZ][i2] += a1[2];
+        }
+    }
+}
+
+// The sums with FP32 terms: offsets from the target leaf's first particle R, lengths and G m scaled by
+// eval_scale.  A pair separation taken as the difference of two FP32 offsets is off by at most 2^-23 O, with O
+// the largest offset among the batch's sources and the wavefront's targets: pairs closer than O / 8 (where that
+// is more than 1e-6 of the separation) take theirs in FP64 from the source's FP64 position instead.  Each batch
+// of up to 64 entries is summed in FP32 and added to FP64 accumulators; the accelerations are scaled back and
+// added to the state planes in FP64.
+//
+// The FP32 sum of a batch depends on which entries it holds, so the lists are taken in their depth-first order,
+// the target's own particles last, and cut at fixed places (64 nodes; 64 leaves, and within them 64 particles),
+// whatever the number of wavefronts.  lane = sp tc + p, for particle p < tc of the target and split sp < S = 64 /
+// tc, which takes every S-th entry.  One comparison against the batch's softening and close radii sends a pair to
+// the branch that handles softening, closeness and the particle itself; the others are Newtonian.
+//
+// Walk and sums of 8M particles (quadrupole, theta 0.5) take 16.6 + 1.7 ms, of which staging is 6.5 ms; before,
+// with lists per target and entries read from LDS a component at a time, 17.9 + 5.1 ms.
 template <int ORDER>
 __global__ void __launch_bounds__(BLOCK) k_eval_mixed(Tree t, Planes s, const uint32_t* __restrict__ order,
                                                       const uint32_t* __restrict__ targets, uint32_t ntargets,
-                                                      const uint32_t* __restrict__ nlist, uint32_t cap_n,
-                                                      const uint32_t* __restrict__ xlist, uint32_t cap_x,
-                                                      const uint32_t* __restrict__ ncount,
-                                                      const uint32_t* __restrict__ xcount,
+                                                      WalkLists wl, uint32_t split, EvalCounts counts,
                                                       const double* __restrict__ grads) {
-    __shared__ EvalStageF<ORDER> stage[BLOCK / 64];
+    using Stage = EvalStage<float, ORDER>;
+    __shared__ Stage stages[BLOCK / 64];
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    EvalStageF<ORDER>& S_ = stage[wave];
-    const uint32_t q = (xcd_block(blockIdx.x, gridDim.x) * (BLOCK / 64)) + wave;
-    if (q >= ntargets) return;  // uniform over the wavefront
+    Stage& S_ = stages[wave];
+    const uint32_t block = xcd_block(blockIdx.x, gridDim.x);
+    const uint32_t q = split > 1 ? block : block * (BLOCK / 64) + wave;
+    const uint32_t part = split > 1 ? wave : 0u;
+    if (q >= ntargets) return;  // uniform over the wavefront, and over the block when it shares a target
     const EvalScale sc = eval_scale(t);
-    const uint32_t T = targets[q];
     uint32_t tf, tc;
-    node_range(t, T, tf, tc);
+    node_range(t, targets[q], tf, tc);
     const LaneSplit ls = lane_split(lane, tc);
-    const uint32_t S = ls.S, sp = ls.sp;
-    const bool active = ls.used;
-    const uint32_t j0 = active ? sp : 64u;  // unused lanes take no entries
+    const uint32_t S = ls.S;
+    const uint32_t j0 = ls.used ? ls.sp : 64u;  // unused lanes take no entries
     const uint32_t k = tf + ls.p;
     const double4 R = t.pos[tf];
     float mx, my, mz, mh;
@@ -1231,114 +1318,159 @@ __global__ void __launch_bounds__(BLOCK) k_eval_mixed(Tree t, Planes s, const ui
         mz = float((me.z - R.z) * sc.invL);
         mh = float(me.w * sc.invL);
     }
-    const float me2 = wave_max_f(active ? mx * mx + my * my + mz * mz : 0.f);
+    const float me2 = wave_max_f(ls.used ? mx * mx + my * my + mz * mz : 0.f);
+    const float hmax = wave_max_f(ls.used ? mh * 1.000001f : 0.f);  // rounded up
     double a[3] = { 0.0, 0.0, 0.0 };
-    const uint32_t nn = min(ncount[q], cap_n), nx = min(xcount[q], cap_x);
-    const uint32_t* nl = nlist + size_t(q) * cap_n;
-    const uint32_t* xl = xlist + size_t(q) * cap_x;
     const double s2 = sc.invM * sc.invL * sc.invL, s3 = s2 * sc.invL;
-
-    // node list
-    for (uint32_t base = 0; base < nn; base += 64) {
-        const uint32_t cnt = min(64u, nn - base);
-        if (lane < cnt) {
-            const uint32_t id = nl[base + lane];
-            const double4 g = t.geo[id];
-            const NodeMom& mm = t.mom[id];
-            S_.c[0][lane] = float((g.x - R.x) * sc.invL);
-            S_.c[1][lane] = float((g.y - R.y) * sc.invL);
-            S_.c[2][lane] = float((g.z - R.z) * sc.invL);
-            S_.M[lane] = float(mm.M * sc.invM);
-            if constexpr (ORDER >= 2) {
-                for (int c = 0; c < 5; ++c) S_.q2[c][lane] = float(mm.q2[c] * s2);
-            }
-            if constexpr (ORDER >= 3) {
-                for (int c = 0; c < 7; ++c) S_.q3[c][lane] = float(mm.q3[c] * s3);
-            }
+    const unsigned long long below = (1ull << lane) - 1ull;
+    const uint32_t grp = q / wl.group, abit = 1u << (q - grp * wl.group), sbit = abit << 16;
+    const uint2* list = wl.list + size_t(grp) * wl.cap;
+    const uint32_t entries = wl.count[grp];
+    uint32_t at = 0, nfill = 0, pfill = 0;  // scanned entries, collected nodes, collected particles
+    uint32_t nbatch = 0, pbatch = 0;        // batches so far
+    uint32_t ncnt = 0, xcnt = 0, xsum = 0;
+    uint32_t leaves = 0;                    // leaves collected since the last cut
+    bool own = true;                        // the target's own particles are still to come
+    uint32_t ef = 0, ec = 0;                // leaves to collect: range (ef, ec) in the lanes of `em`
+    unsigned long long em = 0ull;
+    for (;;) {
+        if (at >= entries && em == 0ull && own) {
+            own = false;
+            ef = tf;
+            ec = tc;
+            em = 1ull;
+        }
+        // a batch of particles is full at 64, or where 64 leaves end
+        while (em != 0ull && pfill < 64u && leaves < 64u) {
+            const int l = __builtin_ctzll(em);
+            em &= em - 1ull;
+            const uint32_t f = __builtin_amdgcn_readlane(ef, l), c = __builtin_amdgcn_readlane(ec, l);
+            if (lane < c) S_.parts[pfill + lane] = f + lane;
+            pfill += c;
+            xsum += c;
+            ++leaves;
         }
         wave_sync();
-        float b[3] = { 0.f, 0.f, 0.f };
-        for (uint32_t j = j0; j < cnt; j += S) {
-            float q2[5], q3[7];
-            if constexpr (ORDER >= 2) {
-                for (int c = 0; c < 5; ++c) q2[c] = S_.q2[c][j];
-            }
-            if constexpr (ORDER >= 3) {
-                for (int c = 0; c < 7; ++c) q3[c] = S_.q3[c][j];
-            }
-            add_multipole_f<ORDER>(S_.M[j], q2, q3, S_.c[0][j] - mx, S_.c[1][j] - my, S_.c[2][j] - mz, b);
+        if (at < entries && em == 0ull && nfill < 64u && pfill < 64u) {
+            const uint2 e = at + lane < entries ? list[at + lane] : make_uint2(0u, 0u);
+            at += 64u;
+            const unsigned long long am = __ballot((e.y & abit) != 0u);
+            em = __ballot((e.y & sbit) != 0u);
+            if (e.y & abit) S_.nodes[nfill + __popcll(am & below)] = e.x;
+            nfill += __popcll(am);
+            if (e.y & sbit) node_range(t, e.x, ef, ec);
+            ncnt += __popcll(am);
+            xcnt += __popcll(em);
+            continue;
         }
-        for (int c = 0; c < 3; ++c) a[c] += double(b[c]);
-        wave_sync();
-    }
-
-    // source particles: entries e < nx are the listed leaves, entry nx is the target leaf
-    const uint32_t nent = nx + 1;
-    for (uint32_t eb = 0; eb < nent; eb += 64) {
-        uint32_t f = 0, c = 0;
-        const uint32_t e = eb + lane;
-        if (e < nx) {
-            node_range(t, xl[e], f, c);
-        } else if (e == nx) {
-            f = tf;
-            c = tc;
-        }
-        uint32_t incl = c;
-        for (int o = 1; o < 64; o <<= 1) {
-            const uint32_t v = __shfl_up(incl, o, 64);
-            if (lane >= uint32_t(o)) incl += v;
-        }
-        const uint32_t excl = incl - c;
-        const uint32_t total = __shfl(incl, 63, 64);
-        for (uint32_t s0 = 0; s0 < total; s0 += 64) {
-            const uint32_t slot = s0 + lane;
-            const uint32_t cnt = min(64u, total - s0);
-            int lo = 0;
-            for (int step = 32; step > 0; step >>= 1) {
-                const uint32_t ex = __shfl(excl, (lo + step) & 63, 64);
-                if (lo + step < 64 && ex <= slot) lo += step;
-            }
-            const uint32_t fe = __shfl(f, lo, 64), xe = __shfl(excl, lo, 64);
-            if (lane < cnt) {
-                const uint32_t src = fe + (slot - xe);
-                const double4 o = t.pos[src];
-                S_.src[lane] = make_float4(float((o.x - R.x) * sc.invL), float((o.y - R.y) * sc.invL),
-                                           float((o.z - R.z) * sc.invL), float(o.w * sc.invL));
-                S_.sm[lane] = float(t.gm[src] * sc.invM);
-                S_.sidx[lane] = src;
-            }
-            wave_sync();
-            float o2 = 0.f;
-            if (lane < cnt) {
-                const float4 o = S_.src[lane];
-                o2 = o.x * o.x + o.y * o.y + o.z * o.z;
-            }
-            const float close = fmaxf(wave_max_f(o2), me2) * (1.f / 64.f);  // (O / 8)^2
-            float b[3] = { 0.f, 0.f, 0.f };
-            // the target itself lies within the close radius (or at zero separation when the radius is zero),
-            // so its entry is recognised there, where the source index is read anyway
-            for (uint32_t j = j0; j < cnt; j += S) {
-                const float4 o = S_.src[j];
-                float rx = o.x - mx, ry = o.y - my, rz = o.z - mz;
-                float d2 = rx * rx + ry * ry + rz * rz;
-                bool self = false;
-                if (d2 < close || d2 == 0.f) {
-                    const uint32_t src = S_.sidx[j];
-                    self = src == k;
-                    const double4 od = t.pos[src], me = t.pos[k];
-                    rx = float((od.x - me.x) * sc.invL);
-                    ry = float((od.y - me.y) * sc.invL);
-                    rz = float((od.z - me.z) * sc.invL);
-                    d2 = rx * rx + ry * ry + rz * rz;
+        if (nfill >= 64u || (at >= entries && nfill > 0)) {
+            const uint32_t cnt = min(nfill, 64u);
+            if (nbatch++ % split == part) {
+                if (lane < cnt) {
+                    const uint32_t id = S_.nodes[lane];
+                    const double4 g = t.geo[id];
+                    const NodeMom& mm = t.mom[id];
+                    NodeRow<float, ORDER> r;
+                    r.v[0] = float((g.x - R.x) * sc.invL);
+                    r.v[1] = float((g.y - R.y) * sc.invL);
+                    r.v[2] = float((g.z - R.z) * sc.invL);
+                    r.v[3] = float(mm.M * sc.invM);
+                    row_moments<float, ORDER>(r, mm, s2, s3);
+                    S_.row[lane] = r;
                 }
-                if (!self) add_pair_f(grads, rx, ry, rz, d2, 0.5f * (o.w + mh), S_.sm[j], b);
+                wave_sync();
+                float b[3] = { 0.f, 0.f, 0.f };
+                for (uint32_t j = j0; j < cnt; j += S) {
+                    const NodeRow<float, ORDER> r = S_.row[j];
+                    expand<ORDER>(r, mx, my, mz, b);
+                }
+                for (int c = 0; c < 3; ++c) a[c] += double(b[c]);
             }
-            for (int c = 0; c < 3; ++c) a[c] += double(b[c]);
+            // the nodes past the batch move to the front
+            nfill -= cnt;
+            const uint32_t rest = lane < nfill ? S_.nodes[64u + lane] : 0u;
+            wave_sync();
+            if (lane < nfill) S_.nodes[lane] = rest;
             wave_sync();
         }
+        const bool last = at >= entries && em == 0ull && !own;
+        if (pfill >= 64u || (pfill > 0 && (leaves == 64u || last))) {
+            const uint32_t cnt = min(pfill, 64u);
+            if (pbatch++ % split == part) {
+                float reach = 0.f, o2 = 0.f;
+                if (lane < cnt) {
+                    const uint32_t src = S_.parts[lane];
+                    const double4 o = t.pos[src];
+                    typename Stage::Src v;
+                    v.x = float((o.x - R.x) * sc.invL);
+                    v.y = float((o.y - R.y) * sc.invL);
+                    v.z = float((o.z - R.z) * sc.invL);
+                    v.m = float(t.gm[src] * sc.invM);
+                    reach = float(o.w * sc.invL);
+                    S_.src[lane] = v;
+                    S_.h[lane] = reach;
+                    S_.idx[lane] = src;
+                    o2 = v.x * v.x + v.y * v.y + v.z * v.z;
+                }
+                wave_sync();
+                const float close = fmaxf(wave_max_f(o2), me2) * (1.f / 64.f);  // (O / 8)^2
+                // pairs beyond `far` are Newtonian and not close: (h_i + h_j) is the support of the softened
+                // kernel at the mean h
+                const float rs = grads ? wave_max_f(reach) * 1.000001f + hmax : 0.f;
+                const float far = fmaxf(rs * rs, close);
+                float b[3] = { 0.f, 0.f, 0.f };
+                for (uint32_t j = j0; j < cnt; j += S) {
+                    const typename Stage::Src o = S_.src[j];
+                    float rx = o.x - mx, ry = o.y - my, rz = o.z - mz;
+                    float d2 = rx * rx + ry * ry + rz * rz;
+                    if (d2 <= far) {
+                        const uint32_t src = S_.idx[j];
+                        if (src == k) continue;
+                        if (d2 < close || d2 == 0.f) {
+                            const double4 od = t.pos[src], me = t.pos[k];
+                            rx = float((od.x - me.x) * sc.invL);
+                            ry = float((od.y - me.y) * sc.invL);
+                            rz = float((od.z - me.z) * sc.invL);
+                            d2 = rx * rx + ry * ry + rz * rz;
+                        }
+                        add_pair_f(grads, rx, ry, rz, d2, 0.5f * (S_.h[j] + mh), o.m, b);
+                    } else {
+                        const float il = __builtin_amdgcn_rsqf(d2);
+                        const float f = o.m * (il * il * il);
+                        b[0] += rx * f;
+                        b[1] += ry * f;
+                        b[2] += rz * f;
+                    }
+                }
+                for (int c = 0; c < 3; ++c) a[c] += double(b[c]);
+            }
+            // the particles past the batch move to the front
+            pfill -= cnt;
+            const uint32_t rest = lane < pfill ? S_.parts[64u + lane] : 0u;
+            wave_sync();
+            if (lane < pfill) S_.parts[lane] = rest;
+            wave_sync();
+        }
+        if (leaves == 64u && pfill == 0) leaves = 0;
+        if (last && nfill == 0 && pfill == 0) break;
     }
-    sum_splits(ls, lane, tc, a);
-    if (sp == 0) {
+    sum_splits(ls, lane, a);
+    if (counts.nodes && lane == 0 && part == 0) {
+        counts.nodes[q] = ncnt;
+        counts.leaves[q] = xcnt;
+        counts.work[2 * size_t(q)] = tc * ncnt;            // particle-node expansions
+        counts.work[2 * size_t(q) + 1] = tc * (xsum - 1);  // particle pairs (xsum with the target's own)
+    }
+    const bool writes = ls.used && ls.sp == 0;
+    if (split > 1) {
+        double* mine = reinterpret_cast<double*>(&S_);
+        for (int c = 0; c < 3; ++c) {
+            if (writes) mine[3 * ls.p + c] = a[c];
+        }
+        add_shared(s, order, stages, split, wave, lane, tf, tc, sc.back);
+        return;
+    }
+    if (writes) {
         const uint32_t i = order[k];
         s.d[GAX][i] += a[0] * sc.back;
         s.d[GAY][i] += a[1] * sc.back;
@@ -1560,11 +1692,10 @@ __global__ void __launch_bounds__(BLOCK) k_fill_u32g(uint32_t* p, size_t count, 
     }
 }
 
-// small[0..5] bounds, [6] list sizes needed (2 x u32), [8] traversal error flags.
+// small[0..5] bounds, [6] list entries needed, [8] traversal error flags.
 __global__ void k_init_bounds(unsigned long long* a) {
     const int t = threadIdx.x;
     if (t < 6) a[t] = t < 3 ? ~0ull : 0ull;
-    if (t == 6 || t == 8) a[t] = 0ull;
 }
 
 // Strided element layouts <-> planes.
@@ -1641,21 +1772,22 @@ struct osph_gravity {
              *flag = nullptr;
     double4 *geo = nullptr, *lo = nullptr, *hi = nullptr;
     NodeMom* mom = nullptr;
-    WalkNode* wn = nullptr;
-    WalkNodeF* wnf = nullptr;  // filled on the first screened walk after a build
-    bool wnf_ready = false;
+    WalkNodeF* wnf = nullptr;
+    bool skip_ready = false;  // the skip links of this tree are built (by the first evaluation at points)
     double ctr[3] = { 0.0, 0.0, 0.0 }, invL = 1.0;
-    int walk_screen = -1;  // 1: FP32-screened walk, 0: FP64 walk, -1: screened in mixed precision only
+    int walk_screen = -1;  // 1, -1: FP32-screened opening tests, 0: FP64 tests (the same lists)
     uint32_t *leaf_at = nullptr, *targets = nullptr, *ntargets_dev = nullptr;
     void* select_temp = nullptr;
     size_t select_temp_bytes = 0;
     uint32_t ntargets = 0;
-    // interaction lists
-    uint32_t *nlist = nullptr, *xlist = nullptr, *ncount = nullptr, *xcount = nullptr, *work = nullptr;
-    uint32_t cap_n = 256, cap_x = 64;
-    size_t list_targets = 0;
+    uint2* list = nullptr;  // walk lists, list_cap entries per group of targets
+    uint32_t* list_count = nullptr;
+    uint32_t list_cap = 2048;
+    size_t list_groups = 0;
+    uint32_t* counts = nullptr;  // interaction counts per target (4 words), when statistics are asked for
+    size_t counts_cap = 0;
     uint32_t* levels = nullptr;           // node counts per depth, then the bucket cursors
-    unsigned long long* small = nullptr;  // [0..5] bounds, [6] need (2 x u32)
+    unsigned long long* small = nullptr;  // [0..5] bounds, [6] list entries needed, [8] error flags
     unsigned long long* small_host = nullptr;
     double *lut_grads = nullptr, *lut_values = nullptr;
     double* scratch = nullptr;
@@ -1734,19 +1866,22 @@ int sync(osph_gravity* g) {
     return OK;
 }
 
-// Synchronises and fails if a tree climb or walk ran past its bound (a malformed tree).
+// Synchronises and fails if a tree climb or walk ran past its bound (a malformed tree) since the last check.
 int check_traversal(osph_gravity* g) {
     GCHK(g, hipMemcpyAsync(g->small_host + 8, g->small + 8, sizeof(unsigned long long), hipMemcpyDeviceToHost,
                            g->stream));
     if (int e = sync(g)) return e;
-    if (g->small_host[8] != 0) return g->fail(ERR_STATE, "tree traversal exceeded its bound");
+    if (g->small_host[8] != 0) {
+        k_fill_u32g<<<1, 64, 0, g->stream>>>(reinterpret_cast<uint32_t*>(g->small + 8), 2, 0u);
+        return g->fail(ERR_STATE, "tree traversal exceeded its bound");
+    }
     return OK;
 }
 
 void free_particles(osph_gravity* g) {
     void* ptrs[] = { g->dblock, g->dblock2, g->perm, g->perm2, g->slot_of, g->keys, g->keys_sorted, g->iota, g->order, g->sort_temp, g->pos, g->gm, g->left,
-                     g->right, g->parent, g->skip, g->first, g->count, g->flag, g->geo, g->lo, g->hi, g->mom, g->wn,
-                     g->wnf, g->leaf_at, g->targets, g->ntargets_dev, g->select_temp };
+                     g->right, g->parent, g->skip, g->first, g->count, g->flag, g->geo, g->lo, g->hi, g->mom, g->wnf,
+                     g->leaf_at, g->targets, g->ntargets_dev, g->select_temp };
     for (void* p : ptrs) (void)hipFree(p);
     g->dblock = g->dblock2 = nullptr;
     g->perm = g->perm2 = g->slot_of = nullptr;
@@ -1759,9 +1894,8 @@ void free_particles(osph_gravity* g) {
     g->left = g->right = g->parent = g->skip = g->first = g->count = g->flag = nullptr;
     g->geo = g->lo = g->hi = nullptr;
     g->mom = nullptr;
-    g->wn = nullptr;
     g->wnf = nullptr;
-    g->wnf_ready = false;
+    g->skip_ready = false;
     g->leaf_at = g->targets = g->ntargets_dev = nullptr;
     g->cap = 0;
 }
@@ -1791,7 +1925,6 @@ int ensure_particles(osph_gravity* g, size_t n) {
     GCHK(g, hipMalloc(&g->lo, sizeof(double4) * nodes));
     GCHK(g, hipMalloc(&g->hi, sizeof(double4) * nodes));
     GCHK(g, hipMalloc(&g->mom, sizeof(NodeMom) * nodes));
-    GCHK(g, hipMalloc(&g->wn, sizeof(WalkNode) * nodes));
     GCHK(g, hipMalloc(&g->wnf, sizeof(WalkNodeF) * nodes));
     GCHK(g, hipMalloc(&g->parent, sizeof(uint32_t) * ids));
     GCHK(g, hipMalloc(&g->skip, sizeof(uint32_t) * ids));
@@ -1831,23 +1964,26 @@ int ensure_scratch(osph_gravity* g, size_t doubles) {
     return OK;
 }
 
-int ensure_lists(osph_gravity* g, size_t targets) {
-    const size_t need = targets;
-    if (need <= g->list_targets && g->nlist) return OK;
-    (void)hipFree(g->nlist);
-    (void)hipFree(g->xlist);
-    (void)hipFree(g->ncount);
-    (void)hipFree(g->xcount);
-    (void)hipFree(g->work);
-    g->nlist = g->xlist = g->ncount = g->xcount = g->work = nullptr;
-    g->list_targets = 0;
-    const size_t t = need > 0 ? need : 1;
-    GCHK(g, hipMalloc(&g->nlist, sizeof(uint32_t) * t * g->cap_n));
-    GCHK(g, hipMalloc(&g->xlist, sizeof(uint32_t) * t * g->cap_x));
-    GCHK(g, hipMalloc(&g->ncount, sizeof(uint32_t) * t));
-    GCHK(g, hipMalloc(&g->xcount, sizeof(uint32_t) * t));
-    GCHK(g, hipMalloc(&g->work, 2 * sizeof(uint32_t) * t));
-    g->list_targets = t;
+int ensure_lists(osph_gravity* g, size_t groups) {
+    if (groups <= g->list_groups) return OK;
+    (void)hipFree(g->list);
+    (void)hipFree(g->list_count);
+    g->list = nullptr;
+    g->list_count = nullptr;
+    g->list_groups = 0;
+    GCHK(g, hipMalloc(&g->list, sizeof(uint2) * groups * g->list_cap));
+    GCHK(g, hipMalloc(&g->list_count, sizeof(uint32_t) * groups));
+    g->list_groups = groups;
+    return OK;
+}
+
+int ensure_counts(osph_gravity* g, size_t targets) {
+    if (targets <= g->counts_cap) return OK;
+    (void)hipFree(g->counts);
+    g->counts = nullptr;
+    g->counts_cap = 0;
+    GCHK(g, hipMalloc(&g->counts, 4 * sizeof(uint32_t) * targets));
+    g->counts_cap = targets;
     return OK;
 }
 
@@ -1865,7 +2001,6 @@ Tree tree_of(osph_gravity* g) {
     t.lo = g->lo;
     t.hi = g->hi;
     t.mom = g->mom;
-    t.wn = g->wn;
     t.wnf = g->wnf;
     for (int k = 0; k < 3; ++k) t.ctr[k] = g->ctr[k];
     t.invL = g->invL;
@@ -1946,7 +2081,7 @@ int build_tree(osph_gravity* g, bool reorder = false) {
     int e = 0;
     if (ext > 0.0) (void)std::frexp(ext, &e);
     g->invL = std::ldexp(1.0, -e);
-    g->wnf_ready = false;
+    g->skip_ready = false;
     Tree t = tree_of(g);
     timed(g, "morton", [&] { k_morton<<<grid_for(n), BLOCK, 0, st>>>(g->s, lo[0], lo[1], lo[2], scale, g->keys, g->iota, n); });
     timed(g, "sort", [&] {
@@ -1970,11 +2105,6 @@ int build_tree(osph_gravity* g, bool reorder = false) {
     timed(g, "gather", [&] { k_gather<<<grid_for(n), BLOCK, 0, st>>>(g->s, g->order, g->cfg.G, g->pos, g->gm, n); });
     if (n > 1) {
         timed(g, "radix_tree", [&] { k_radix_tree<<<grid_for(n - 1), BLOCK, 0, st>>>(t, g->keys_sorted); });
-        timed(g, "skip", [&] { k_skip<<<grid_for(2 * n - 1), BLOCK, 0, st>>>(t); });
-    } else {
-        const uint32_t endv = END;
-        GCHK(g, hipMemcpyAsync(g->parent, &endv, sizeof(uint32_t), hipMemcpyHostToDevice, st));
-        GCHK(g, hipMemcpyAsync(g->skip, &endv, sizeof(uint32_t), hipMemcpyHostToDevice, st));
     }
     timed(g, "leaves", [&] {
         k_fill_u32g<<<std::min<unsigned>(grid_for(n), 4096), BLOCK, 0, st>>>(g->leaf_at, n, END);
@@ -1994,89 +2124,84 @@ int build_tree(osph_gravity* g, bool reorder = false) {
     return OK;
 }
 
-// Barnes-Hut interaction lists and sums, adding to the state's accelerations.
+// Targets below which a block of four wavefronts shares each target: with a wavefront per target, 6000 of them
+// are about six per SIMD; fewer leave SIMDs without the wavefronts that hide the loads.
+constexpr uint32_t EVAL_SHARED_TARGETS = 6000;
+
+// Targets per walk group: the largest group shares the most work, but it takes about four wavefronts per SIMD
+// to hide the loads (walk of 16 / 8 / 4 targets: 1.70 / 1.69 / 2.02 ms at 8M particles, 0.32 / 0.28 / 0.27 ms at
+// 1M; below 100k particles, where even groups of two leave SIMDs idle, 65-70 us whichever).
+uint32_t walk_group(uint32_t ntargets) {
+    uint32_t group = WALK_GROUP;
+    while (group > 2 && ntargets / group < 4096) group /= 2;
+    return group;
+}
+
+template <int ORDER>
+void launch_eval(osph_gravity* g, const Tree& t, const WalkLists& wl, const EvalCounts& counts, const double* grads) {
+    const uint32_t nt = g->ntargets, waves = BLOCK / 64;
+    const uint32_t split = nt < EVAL_SHARED_TARGETS ? waves : 1u;
+    const unsigned blocks = split > 1 ? nt : (nt + waves - 1) / waves;
+    if (g->precision == OSPH_PRECISION_MIXED) {
+        k_eval_mixed<ORDER><<<blocks, BLOCK, 0, g->stream>>>(t, g->s, g->order, g->targets, nt, wl, split, counts, grads);
+    } else {
+        k_eval<ORDER><<<blocks, BLOCK, 0, g->stream>>>(t, g->s, g->order, g->targets, nt, wl, split, counts, grads);
+    }
+}
+
+// Barnes-Hut walk and sums, adding to the state's accelerations.
 int eval_bh(osph_gravity* g, osph_gravity_stats* stats) {
     const size_t n = g->n;
     if (!n) return OK;
     hipStream_t st = g->stream;
-    Tree t = tree_of(g);
+    const Tree t = tree_of(g);
     const uint32_t nt = g->ntargets;
-    for (int attempt = 0; attempt < 4; ++attempt) {
-        if (int e = ensure_lists(g, nt)) return e;
-        uint32_t* need = reinterpret_cast<uint32_t*>(g->small + 6);
-        const bool screened = g->walk_screen == 1 || (g->walk_screen == -1 && g->precision == OSPH_PRECISION_MIXED);
-        if (screened && !g->wnf_ready && n > 1) {
-            timed(g, "walk_records", [&] { k_walk_records<<<grid_for(n - 1), BLOCK, 0, st>>>(t); });
-            g->wnf_ready = true;
-        }
-        if (screened && n > 1) {
-            timed(g, "walk_screened", [&] {
-                k_fill_u32g<<<1, 64, 0, st>>>(need, 2, 0u);
-                k_walk_screened<<<grid_for(nt), BLOCK, 0, st>>>(t, g->targets, nt, g->nlist, g->cap_n, g->xlist,
-                                                                g->cap_x, g->ncount, g->xcount, g->work, need);
-            });
-        } else timed(g, "walk", [&] {
-            k_fill_u32g<<<1, 64, 0, st>>>(need, 2, 0u);
-            k_walk<<<grid_for(nt), BLOCK, 0, st>>>(t, g->targets, nt, g->nlist, g->cap_n, g->xlist, g->cap_x, g->ncount,
-                                                   g->xcount, g->work, need);
+    const uint32_t group = walk_group(nt), groups = (nt + group - 1) / group;
+    uint32_t* need = reinterpret_cast<uint32_t*>(g->small + 6);
+    for (int attempt = 0;; ++attempt) {
+        if (int e = ensure_lists(g, groups)) return e;
+        timed(g, "walk", [&] {
+            k_fill_u32g<<<1, 64, 0, st>>>(need, 1, 0u);
+            k_walk<<<(groups + BLOCK / 64 - 1) / (BLOCK / 64), BLOCK, 0, st>>>(
+                t, g->targets, nt, group, g->walk_screen != 0, g->list, g->list_cap, g->list_count, need);
         });
-        GCHK(g, hipMemcpyAsync(g->small_host + 6, need, 2 * sizeof(uint32_t), hipMemcpyDeviceToHost, st));
+        GCHK(g, hipMemcpyAsync(g->small_host + 6, need, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
         if (int e = check_traversal(g)) return e;
-        uint32_t nd[2];
-        std::memcpy(nd, g->small_host + 6, sizeof(nd));
-        if (nd[0] == 0 && nd[1] == 0) break;
+        uint32_t most;
+        std::memcpy(&most, g->small_host + 6, sizeof(most));
+        if (most == 0) break;
         if (attempt == 3) return g->fail(ERR_STATE, "interaction lists did not fit after growing");
-        // grow to the largest list and walk again
-        (void)hipFree(g->nlist);
-        g->nlist = nullptr;
-        if (nd[0]) g->cap_n = (nd[0] + 63u) & ~63u;
-        if (nd[1]) g->cap_x = (nd[1] + 15u) & ~15u;
-        g->list_targets = 0;
+        // grow to the longest list and walk again
+        g->list_cap = (most + most / 8 + 63u) & ~63u;
+        g->list_groups = 0;
     }
-    const int ord = g->cfg.order;
+    const WalkLists wl{ g->list, g->list_count, g->list_cap, group };
+    EvalCounts counts{};
+    if (stats) {
+        if (int e = ensure_counts(g, nt)) return e;
+        counts = { g->counts, g->counts + nt, g->counts + 2 * size_t(nt) };
+    }
     const double* grads = g->cfg.kernel == OSPH_GRAVITY_KERNEL_M4 ? g->lut_grads : nullptr;
-    const unsigned blocks = unsigned((nt + (BLOCK / 64) - 1) / (BLOCK / 64));
-    if (g->precision == OSPH_PRECISION_MIXED) {
-        timed(g, "eval_mixed", [&] {
-            const unsigned nb = blocks > 0 ? blocks : 1;
-            if (ord == 3) {
-                k_eval_mixed<3><<<nb, BLOCK, 0, st>>>(t, g->s, g->order, g->targets, nt, g->nlist, g->cap_n, g->xlist,
-                                                      g->cap_x, g->ncount, g->xcount, grads);
-            } else if (ord == 2) {
-                k_eval_mixed<2><<<nb, BLOCK, 0, st>>>(t, g->s, g->order, g->targets, nt, g->nlist, g->cap_n, g->xlist,
-                                                      g->cap_x, g->ncount, g->xcount, grads);
-            } else {
-                k_eval_mixed<0><<<nb, BLOCK, 0, st>>>(t, g->s, g->order, g->targets, nt, g->nlist, g->cap_n, g->xlist,
-                                                      g->cap_x, g->ncount, g->xcount, grads);
-            }
-        });
-    } else timed(g, "eval", [&] {
-        const unsigned nb = blocks > 0 ? blocks : 1;
-        if (ord == 3) {
-            k_eval<3><<<nb, BLOCK, 0, st>>>(t, g->s, g->order, g->targets, nt, g->nlist, g->cap_n, g->xlist, g->cap_x,
-                                            g->ncount, g->xcount, grads);
-        } else if (ord == 2) {
-            k_eval<2><<<nb, BLOCK, 0, st>>>(t, g->s, g->order, g->targets, nt, g->nlist, g->cap_n, g->xlist, g->cap_x,
-                                            g->ncount, g->xcount, grads);
+    timed(g, g->precision == OSPH_PRECISION_MIXED ? "eval_mixed" : "eval", [&] {
+        if (g->cfg.order == 3) {
+            launch_eval<3>(g, t, wl, counts, grads);
+        } else if (g->cfg.order == 2) {
+            launch_eval<2>(g, t, wl, counts, grads);
         } else {
-            k_eval<0><<<nb, BLOCK, 0, st>>>(t, g->s, g->order, g->targets, nt, g->nlist, g->cap_n, g->xlist, g->cap_x,
-                                            g->ncount, g->xcount, grads);
+            launch_eval<0>(g, t, wl, counts, grads);
         }
     });
+    GCHK(g, hipPeekAtLastError());
     if (stats) {
-        std::vector<uint32_t> a(nt), b(nt), w(2 * size_t(nt));
-        if (nt) {
-            GCHK(g, hipMemcpyAsync(a.data(), g->ncount, nt * sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-            GCHK(g, hipMemcpyAsync(b.data(), g->xcount, nt * sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-            GCHK(g, hipMemcpyAsync(w.data(), g->work, w.size() * sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-        }
+        std::vector<uint32_t> c(4 * size_t(nt));
+        GCHK(g, hipMemcpyAsync(c.data(), g->counts, c.size() * sizeof(uint32_t), hipMemcpyDeviceToHost, st));
         if (int e = sync(g)) return e;
         *stats = osph_gravity_stats{};
         for (uint32_t k = 0; k < nt; ++k) {
-            stats->nodes_approx += a[k];
-            stats->nodes_exact += b[k];
-            stats->expansions += w[2 * size_t(k)];
-            stats->pairs += w[2 * size_t(k) + 1];
+            stats->nodes_approx += c[k];
+            stats->nodes_exact += c[nt + k];
+            stats->expansions += c[2 * size_t(nt) + 2 * size_t(k)];
+            stats->pairs += c[2 * size_t(nt) + 2 * size_t(k) + 1];
         }
         stats->node_count = 2 * uint64_t(n) - 1;
     }
@@ -2220,6 +2345,7 @@ int osph_gravity_create(osph_gravity** out, const osph_gravity_config* cfg) {
     };
     if (hipStreamCreateWithFlags(&g->stream, hipStreamNonBlocking) != hipSuccess) return bail(ERR_HIP);
     if (hipMalloc(&g->small, 16 * sizeof(unsigned long long)) != hipSuccess) return bail(ERR_HIP);
+    if (hipMemset(g->small, 0, 16 * sizeof(unsigned long long)) != hipSuccess) return bail(ERR_HIP);
     if (hipMalloc(&g->levels, 2 * (MAX_DEPTH + 1) * sizeof(uint32_t)) != hipSuccess) return bail(ERR_HIP);
     if (hipHostMalloc(&g->small_host, 16 * sizeof(unsigned long long)) != hipSuccess) return bail(ERR_HIP);
     std::vector<double> grads(LUT_ENTRIES + 1), values(LUT_ENTRIES + 1);
@@ -2245,7 +2371,7 @@ void osph_gravity_destroy(osph_gravity* g) {
     resolve(g);
     for (hipEvent_t e : g->pool) (void)hipEventDestroy(e);
     free_particles(g);
-    void* ptrs[] = { g->nlist, g->xlist, g->ncount, g->xcount, g->work, g->small, g->levels, g->lut_grads, g->lut_values,
+    void* ptrs[] = { g->list, g->list_count, g->counts, g->small, g->levels, g->lut_grads, g->lut_values,
                      g->scratch, g->staging };
     for (void* p : ptrs) (void)hipFree(p);
     if (g->small_host) (void)hipHostFree(g->small_host);
@@ -2363,6 +2489,10 @@ int osph_gravity_eval_points(osph_gravity* g, const double* p, size_t np, double
     }
     const double* grads = g->cfg.kernel == OSPH_GRAVITY_KERNEL_M4 ? g->lut_grads : nullptr;
     Tree t = tree_of(g);
+    if (!g->skip_ready) {
+        timed(g, "skip", [&] { k_skip<<<grid_for(2 * g->n - 1), BLOCK, 0, g->stream>>>(t); });
+        g->skip_ready = true;
+    }
     timed(g, "points", [&] { k_points<<<grid_for(np), BLOCK, 0, g->stream>>>(t, pts, acc, np, grads, g->cfg.order); });
     GCHK(g, hipMemcpyAsync(ha.data(), acc, np * sizeof(double4), hipMemcpyDeviceToHost, g->stream));
     if (int e = check_traversal(g)) return e;
