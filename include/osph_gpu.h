@@ -249,7 +249,8 @@ int osph_adjoint_clear(osph_ctx* ctx);
 /* Launch-shape tuning of the neighbour-list and pair kernels (no reference counterpart: the reference
  * has no device kernels).  Keys: "pairs_block", "lists_block" (64, 128 or 256 threads) and
  * "pairs_lds", "lists_lds" (0..65536 bytes of dynamic LDS per block, which caps resident blocks per CU),
- * "pairs_lanes" (1, 2 or 4 lanes share one particle's neighbour list in the pair kernels, default 1),
+ * "pairs_lanes" (1, the default: one lane per particle in the pair kernels, or a group of lanes when the particles are
+ * too few to fill the GPU; 2 or 4: a group of lanes; the sums are the same, bit for bit),
  * "cell_divisor" (1 to 4: neighbour-grid cells of 2 h_max / divisor, default 3), "lists_screen" (1: FP32-screened
  * neighbour test, 0: FP64 only, -1: screened in mixed precision only), "reorder_period" (the resident state
  * is moved into cell order every this many neighbour searches; 0 never; default 40), "fuse_finalize" (1: the
@@ -264,7 +265,7 @@ int osph_tune(osph_ctx* ctx, const char* key, long long value);
  * was.  One key at a time, in order, the fastest value is kept.  The chosen values are applied and written
  * to chosen[n_keys] (5 for the default space); *best_ms is their time per step; trial_ms[0 ..] (up to
  * trial_cap) the time of every candidate, *n_trials their number.  Every candidate gives the same
- * neighbour sets; the lanes per particle change the order of the pair sums. */
+ * neighbour sets and sums. */
 int osph_autotune(osph_ctx* ctx, double dt, int steps, const char* const* keys, const int* n_values,
                   const long long* values, int n_keys, long long* chosen, double* best_ms, double* trial_ms,
                   int trial_cap, int* n_trials);

@@ -34,6 +34,7 @@ struct BatchPlan {
     std::vector<size_t> sizes;
     Tuning tune{};
     bool mixed = false;
+    int lanes = 1;  // lanes per particle in the pair kernel
     size_t total = 0;
     std::vector<uint32_t> pfirst;  // host copy of the particle table's first[]
     uint32_t* tables = nullptr;
@@ -1322,15 +1323,18 @@ int make_plan(const std::vector<osph_ctx*>& ms, BatchPlan*& out) {
     P->mixed = lead->cfg.precision == OSPH_PRECISION_MIXED;
     // block tables: particles (BLOCK threads), lists (lists_block), pairs (pairs_block, lanes per particle)
     std::vector<uint32_t> host;
-    auto table = [&](int block, int per, BatchBlocks& t, std::vector<uint32_t>& first) {
+    auto table = [&](int block, size_t per, BatchBlocks& t, std::vector<uint32_t>& first) {
         first.assign(count + 1, 0u);
-        for (size_t k = 0; k < count; ++k) first[k + 1] = first[k] + batch_blocks_for(ms[k]->n * size_t(per), block);
+        for (size_t k = 0; k < count; ++k) first[k + 1] = first[k] + batch_blocks_for(ms[k]->n * per, block);
         t.total = first[count];
     };
+    size_t total = 0;
+    for (const osph_ctx* c : ms) total += c->n;
+    P->lanes = pair_lanes(P->tune, total);
     std::vector<uint32_t> pf, lf, qf;
     table(BLOCK, 1, P->pb, pf);
     table(P->tune.lists_block, 1, P->lb, lf);
-    table(P->tune.pairs_block, P->tune.pairs_lanes, P->qb, qf);
+    table(P->tune.pairs_block, size_t(P->lanes), P->qb, qf);
     P->pfirst = pf;
     size_t words = 0;
     for (const auto* f : { &pf, &lf, &qf }) words += f->size() + f->back();
@@ -1477,7 +1481,7 @@ int batch_step(const std::vector<osph_ctx*>& ms, const std::vector<double>& dts,
         batch_permute(l, P->dev, P->pb);
         batch_pack(l, P->dev, P->pb, P->mixed);
         batch_lists(l, P->dev, P->lb, screened, plain);
-        batch_pairs(l, P->dev, P->qb, P->mixed, fuse, lead->lut);
+        batch_pairs(l, P->dev, P->qb, P->mixed, fuse, P->lanes, lead->lut);
         if (!fuse) batch_finalize_correct(l, P->dev, P->pb);
     };
     if (P->tune.batch_graph) {

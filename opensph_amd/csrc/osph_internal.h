@@ -182,7 +182,7 @@ __host__ __device__ inline size_t list_quad(size_t k, uint32_t j, uint32_t quads
 struct Tuning {
     int pairs_block = 256;
     int pairs_lds = 0;
-    int pairs_lanes = 1;  // lanes per particle in the pair kernels (1, 2 or 4)
+    int pairs_lanes = 1;  // 1: one lane per particle in the pair kernels, or a group when they are few; 2, 4: a group
     int lists_block = 256;
     int lists_lds = 0;
     int cell_divisor = 3;  // cells of 2 h_max(class) / divisor
@@ -194,6 +194,27 @@ struct Tuning {
                               // -1 for FP64 only (the mixed step measured 1.246 ms unfused, 1.234 ms fused)
     int batch_graph = 1;      // batched steps replay their stages after the sort as a captured HIP graph
 };
+
+// Lanes per particle in the pair kernels: a group of 16 or of 4 while one lane each leaves the chip waiting for the
+// gathers of a single wavefront per SIMD (also when the tuner asks for more than one).  Fused pair kernel in us with
+// 16 / 4 / 1 lanes, gas (one class) and impact: 2k particles FP64 24 / 50 / 98 and 33 / 66 / 149, mixed 15 / 31 / 48;
+// 21k FP64 57 / 60 / 98 and 74 / 90 / 181, mixed 30 / 31 / 48; 43k FP64 103 / 78 / 100 and 138 / 110 / 183, mixed
+// 47 / 36 / 49; 85k FP64 190 / 145 / 118 and 247 / 170 / 201, mixed 87 / 65 / 59.
+constexpr size_t PAIRS_BELOW_16 = 24576, PAIRS_BELOW_4 = 65536;
+inline int pair_lanes(const Tuning& t, size_t n) {
+    if (n < PAIRS_BELOW_16) return 16;
+    return t.pairs_lanes > 1 || n < PAIRS_BELOW_4 ? 4 : 1;
+}
+
+// Particles below which the list kernel gives each a group of lanes: one lane per particle takes about 80 us
+// however few they are, and 170 us where two smoothing-length classes meet (a lane there walks ~1000 candidates).
+// Measured, groups against single lanes: one class, 85k particles 47 against 80 us (mixed) and 61 against 82 us
+// (FP64), 169k 84 against 84 and 114 against 90; two classes, 170k 85 against 168 and 113 against 171, 340k 162
+// against 177 and 212 against 188.
+constexpr size_t LISTS_SHARED_BELOW = 131072, LISTS_SHARED_BELOW_CLASSES = 262144;
+inline bool lists_shared(const Grid& g, size_t n) {
+    return n < (g.nclass > 1 ? LISTS_SHARED_BELOW_CLASSES : LISTS_SHARED_BELOW);
+}
 
 struct Launch {
     hipStream_t stream;
@@ -366,7 +387,9 @@ void batch_cells(const Launch& l, const BatchMember* M, BatchBlocks pb);
 void batch_permute(const Launch& l, const BatchMember* M, BatchBlocks pb);
 void batch_pack(const Launch& l, const BatchMember* M, BatchBlocks pb, bool mixed);
 void batch_lists(const Launch& l, const BatchMember* M, BatchBlocks lb, bool screened, bool plain);
-void batch_pairs(const Launch& l, const BatchMember* M, BatchBlocks qb, bool mixed, bool fuse, const double* lut);
+// lanes: lanes per particle (the blocks qb are dealt accordingly).
+void batch_pairs(const Launch& l, const BatchMember* M, BatchBlocks qb, bool mixed, bool fuse, int lanes,
+                 const double* lut);
 void batch_finalize_correct(const Launch& l, const BatchMember* M, BatchBlocks pb);
 size_t sort_pairs64_temp_bytes(size_t n, int key_bits);
 hipError_t sort_pairs64(const Launch& l, void* temp, size_t temp_bytes, const uint64_t* keys_in, uint64_t* keys_out,

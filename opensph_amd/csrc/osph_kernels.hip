@@ -621,6 +621,121 @@ __device__ __forceinline__ void neighbor_list_at(const double4* __restrict__ pos
     if (cnt > kmax) atomicOr(overflow, 1u);
 }
 
+// The same list, with the same entries in the same order, from LIST_LANES lanes per particle: each lane takes one
+// row of cells at a time and counts its hits, a prefix sum over the group places them.  One lane per particle
+// walks its ~37 rows one after the other, each row two dependent loads (80 us whatever the particle count, until
+// the particles fill the chip); here the group's rows are in flight together.  The rows are numbered over the
+// rectangle of planes and rows around the particle; those of its corners yield no candidates.
+constexpr uint32_t LIST_LANES = 16;
+template <bool SCREEN>
+__device__ __forceinline__ void neighbor_list_shared_at(const double4* __restrict__ pos,
+                                                        const float4* __restrict__ posf, const Screen& sc,
+                                                        const Grid& g, const uint32_t* __restrict__ first,
+                                                        uint32_t* __restrict__ list, uint32_t* __restrict__ count,
+                                                        uint32_t kmax, uint32_t* overflow, size_t k, uint32_t sub) {
+    const double4 me = pos[k];
+    const float4 mf = SCREEN ? posf[k] : make_float4(0.f, 0.f, 0.f, 0.f);
+    const double p[3] = { me.x, me.y, me.z };
+    uint32_t cnt = 0;
+    auto hits = [&](uint32_t k2) {
+        if (SCREEN) {
+            const float4 o = posf[k2];
+            const float dx = mf.x - o.x, dy = mf.y - o.y, dz = mf.z - o.z;
+            const float d2 = dx * dx + dy * dy + dz * dz;
+            const float hs = mf.w + o.w;
+            const float rr = hs * hs;
+            if (d2 < rr * sc.lo) return k2 != k;
+            if (d2 > rr * sc.hi) return false;
+        }
+        const double4 o = pos[k2];
+        return exact_pair(me.x, me.y, me.z, me.w, o.x, o.y, o.z, o.w) && k2 != k;
+    };
+    auto put = [&](uint32_t at, uint32_t k2) {
+        if (at < kmax) list[4 * list_quad(k, at >> 2, kmax >> 2) + (at & 3u)] = k2;
+    };
+    for (int cls = 0; cls < g.nclass; ++cls) {
+        const GridClass& G = g.c[cls];
+        if (G.empty) continue;
+        const double R = me.w + G.hmax;  // h_i + h_j <= R for every member j
+        double d2b = 0.0;
+        for (int a = 0; a < 3; ++a) {
+            const double t = dmax(G.lo[a] - p[a], p[a] - G.hi[a]);
+            if (t > 0.0) d2b += t * t;
+        }
+        if (d2b > R * R * (1.0 + 1e-6)) continue;
+        // the geometry of neighbor_list_at: FP32 in cell units, R widened by 1e-3 cells
+        const float pcx = float((p[0] - G.lo[0]) * G.inv_cell);
+        const float pcy = float((p[1] - G.lo[1]) * G.inv_cell);
+        const float pcz = float((p[2] - G.lo[2]) * G.inv_cell);
+        const float Rc = float(R * G.inv_cell) * (1.0f + 1e-6f) + 1e-3f;
+        const float R2c = Rc * Rc;
+        const int z0 = max(0, int(floorf(pcz - Rc))), z1 = min(G.dim[2] - 1, int(floorf(pcz + Rc)));
+        const int y0 = max(0, int(floorf(pcy - Rc))), y1 = min(G.dim[1] - 1, int(floorf(pcy + Rc)));
+        const int ny = y1 - y0 + 1, rows = z1 < z0 || ny <= 0 ? 0 : (z1 - z0 + 1) * ny;
+        for (int r0 = 0; r0 < rows; r0 += int(LIST_LANES)) {  // uniform over the group
+            const int r = r0 + int(sub);
+            uint32_t b = 0, e = 0;
+            if (r < rows) {
+                const int dz = r / ny;
+                const int cz = z0 + dz, cy = y0 + (r - dz * ny);
+                const float fz = float(cz), fy = float(cy);
+                const float tz = fmaxf(fmaxf(fz - pcz, pcz - (fz + 1.0f)), 0.0f);
+                const float ty = fmaxf(fmaxf(fy - pcy, pcy - (fy + 1.0f)), 0.0f);
+                const float t2 = R2c - (tz * tz + ty * ty);
+                if (t2 >= 0.0f) {
+                    const float w = __builtin_amdgcn_sqrtf(t2);
+                    const int x0 = max(0, int(floorf(pcx - w)));
+                    const int x1 = min(G.dim[0] - 1, int(floorf(pcx + w)));
+                    if (x0 <= x1) {
+                        const uint32_t row = G.base + ((spread2(uint32_t(cy)) | (spread2(uint32_t(cz)) << 1)) << G.bits);
+                        b = first[row + uint32_t(x0)];
+                        e = first[row + uint32_t(x1) + 1u];
+                    }
+                }
+            }
+            // the hits of the first 64 candidates as a mask; the rest of a longer row is counted here and
+            // tested again when its hits are placed
+            unsigned long long mask = 0ull;
+            uint32_t mine = 0;
+            for (uint32_t k2 = b; k2 < e; ++k2) {
+                if (hits(k2)) {
+                    if (k2 - b < 64u) mask |= 1ull << (k2 - b);
+                    ++mine;
+                }
+            }
+            uint32_t incl = mine;
+            for (uint32_t o = 1; o < LIST_LANES; o <<= 1) {
+                const uint32_t v = __shfl_up(incl, o, int(LIST_LANES));
+                if (sub >= o) incl += v;
+            }
+            uint32_t at = cnt + incl - mine;
+            for (unsigned long long m = mask; m != 0ull; m &= m - 1ull) put(at++, b + uint32_t(__builtin_ctzll(m)));
+            for (uint32_t k2 = b + 64u; k2 < e; ++k2) {
+                if (hits(k2)) put(at++, k2);
+            }
+            cnt += __shfl(incl, int(LIST_LANES) - 1, int(LIST_LANES));
+        }
+    }
+    if (sub == 0) {
+        count[k] = cnt;
+        if (cnt > kmax) atomicOr(overflow, 1u);
+    }
+}
+
+template <bool SCREEN>
+__global__ void __launch_bounds__(BLOCK) k_neighbor_lists_shared(const double4* __restrict__ pos,
+                                                                 const float4* __restrict__ posf, Screen sc, Grid g,
+                                                                 const uint32_t* __restrict__ first,
+                                                                 uint32_t* __restrict__ list,
+                                                                 uint32_t* __restrict__ count, uint32_t kmax,
+                                                                 uint32_t* overflow, size_t n) {
+    const size_t t = size_t(xcd_block(blockIdx.x, gridDim.x)) * blockDim.x + threadIdx.x;
+    const size_t k = t / LIST_LANES;
+    if (k < n) {  // uniform over each group of lanes
+        neighbor_list_shared_at<SCREEN>(pos, posf, sc, g, first, list, count, kmax, overflow, k, uint32_t(t % LIST_LANES));
+    }
+}
+
 template <bool SCREEN>
 __global__ void __launch_bounds__(BLOCK) k_neighbor_lists(const double4* __restrict__ pos,
                                                           const float4* __restrict__ posf, Screen sc, Grid g,
@@ -639,40 +754,6 @@ __device__ __forceinline__ double lut_grad(const double* __restrict__ grads, dou
     const double ratio = fi - double(i1);
     return grads[i1] * (1.0 - ratio) + grads[i1 + 1] * ratio;
 }
-
-// Sum of v over the LPP adjacent lanes that share one particle (LPP = 1, 2 or 4), by DPP quad
-// permutations (lane ^ 1, then lane ^ 2).  Every lane of the group gets the same, order-fixed result:
-// (v0 + v1) + (v2 + v3) on lanes 0 and 1, (v2 + v3) + (v0 + v1) on lanes 2 and 3, equal since FP
-// addition commutes.  All lanes of the wave must be active.
-template <int CTRL>
-__device__ __forceinline__ double dpp_move(double v) {
-    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, false);
-    return __hiloint2double(hi, lo);
-}
-
-template <int LPP>
-__device__ __forceinline__ double group_sum(double v) {
-    static_assert(LPP == 1 || LPP == 2 || LPP == 4, "lanes per particle must be 1, 2 or 4");
-    if constexpr (LPP >= 2) v += dpp_move<0xb1>(v);  // quad_perm [1, 0, 3, 2]
-    if constexpr (LPP >= 4) v += dpp_move<0x4e>(v);  // quad_perm [2, 3, 0, 1]
-    return v;
-}
-
-// Particle handled by this lane and the lane's rank among the LPP lanes of that particle.  Lanes past
-// the end keep running (with an empty list) so that the group sums see every lane active.
-template <int LPP>
-struct PairLane {
-    size_t k;
-    uint32_t sub;
-    bool valid;
-    __device__ __forceinline__ PairLane(size_t t, size_t n) {
-        k = t / LPP;
-        sub = uint32_t(t % LPP);
-        valid = k < n;
-        if (!valid) k = n - 1;
-    }
-};
 
 // The pair sums of particle i that the finalize, the corrector and the criteria use: acceleration, du,
 // velocity divergence and gradient (xx, yy, zz, xy, xz, yz).  The fused pair kernels hand them over in
@@ -714,9 +795,8 @@ struct StageOf {
     static_assert(sizeof(Rec) % 16 == 0, "records are whole 16-byte chunks");
 };
 
-// The neighbour list of one particle, split among its LPP lanes by quads (4 entries, 16 B): lane `sub`
-// takes quads sub, sub + LPP, ..., in order, the next quad loaded one quad ahead.  f(record, entry) runs
-// for each listed entry of the lane.
+// The neighbour list of one particle, on one lane: quads (4 entries, 16 B) in order, the next quad loaded one
+// quad ahead.  f(record, entry) runs for each listed entry.
 //
 // STAGED (1, 2): the records are fetched cooperatively.  In each step the wavefront needs one record per lane;
 // pass i of the CH load passes has lane L fetch chunk c of the record of lane r, (r, c) = divmod(64 i +
@@ -728,31 +808,25 @@ struct StageOf {
 // With STAGED == 2 the next step's loads are issued before the current step's compute.
 // Every lane of the wavefront must call this (lanes without entries load their own record as a
 // stand-in, and run no f).
-template <int LPP, int STAGED, typename Rec, typename F>
+template <int STAGED, typename Rec, typename F>
 __device__ __forceinline__ void for_each_neighbor(const Rec* __restrict__ rec, const uint32_t* __restrict__ list,
-                                                  size_t k, uint32_t quads, uint32_t listed, uint32_t sub,
+                                                  size_t k, uint32_t quads, uint32_t listed,
                                                   uint4* __restrict__ stage, F&& f) {
     using S = StageOf<Rec>;
     const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t nq = (listed + 3u) >> 2;
-    const uint32_t myq = sub < nq ? (nq - sub + LPP - 1) / LPP : 0u;  // quads of this lane
-    uint32_t total = 0;  // entries of this lane
-    if (myq > 0) {
-        const uint32_t tail = listed - 4u * (sub + (myq - 1) * LPP);
-        total = 4u * (myq - 1) + (tail < 4u ? tail : 4u);
-    }
+    const uint32_t myq = (listed + 3u) >> 2, total = listed;
     const uint4* list4 = reinterpret_cast<const uint4*>(list);
     auto row = [&](uint32_t j) { return list4[list_quad(k, j, quads)]; };
     if constexpr (STAGED == 0 || STAGED == 3) {
         if (myq == 0) return;
-        uint4 quad = row(sub);
-        uint4 nquad = myq > 1 ? row(sub + LPP) : quad;
+        uint4 quad = row(0);
+        uint4 nquad = myq > 1 ? row(1) : quad;
         auto entry_of = [&](uint32_t t) -> uint32_t {
             const uint32_t sel = t & 3u;
             if (sel == 0 && t > 0) {
                 quad = nquad;
                 const uint32_t j = (t >> 2) + 1;
-                nquad = j < myq ? row(sub + j * LPP) : quad;
+                nquad = j < myq ? row(j) : quad;
             }
             return sel == 0 ? quad.x : (sel == 1 ? quad.y : (sel == 2 ? quad.z : quad.w));
         };
@@ -778,9 +852,9 @@ __device__ __forceinline__ void for_each_neighbor(const Rec* __restrict__ rec, c
     }
     // (in the staged loops the step index is uniform across the wavefront, so the entry is taken from
     // rotating registers rather than selected by index, which the compiler would place in scratch)
-    const uint4 first = myq > 0 ? row(sub) : make_uint4(0, 0, 0, 0);
+    const uint4 first = myq > 0 ? row(0) : make_uint4(0, 0, 0, 0);
     uint32_t q0 = first.x, q1 = first.y, q2 = first.z, q3 = first.w;  // entries of the current quad, next first
-    uint4 nquad = myq > 1 ? row(sub + LPP) : first;
+    uint4 nquad = myq > 1 ? row(1) : first;
     // the entry of step t for this lane (its own index as a stand-in when it has none); steps in order
     auto entry = [&](uint32_t t) -> uint32_t {
         const bool act = t < total;
@@ -790,7 +864,7 @@ __device__ __forceinline__ void for_each_neighbor(const Rec* __restrict__ rec, c
             q2 = nquad.z;
             q3 = nquad.w;
             const uint32_t j = (t >> 2) + 1;
-            if (j < myq) nquad = row(sub + j * LPP);
+            if (j < myq) nquad = row(j);
         }
         const uint32_t e = act ? q0 : uint32_t(k);
         q0 = q1;
@@ -847,6 +921,217 @@ __device__ __forceinline__ void for_each_neighbor(const Rec* __restrict__ rec, c
     }
 }
 
+// ---- a group of lanes per particle -------------------------------------------------------------------
+// For particles too few to fill the chip with one lane each (pair_lanes), LANES (4 or 16) lanes share a particle: each
+// evaluates the terms of one listed neighbour and puts them into the group's LDS rows; lane l of the group then
+// adds components l, l + LANES, ... of the rows to its accumulators, in list order.  Every sum is the one a single lane makes, bit
+// for bit, so how many lanes a particle gets is a question of speed only.  (With one partial sum per lane the
+// sums would depend on it, and a small member of a large ensemble would have to be stepped with the lanes it gets
+// alone: 10 % slower for members of 5k to 200k particles.)
+// The sums then go through LDS to the first lanes of the block, one particle each, for the stores and the fused
+// finalize: with one active lane per group that part would take as long as the pairs.
+constexpr int PAIR_SUMS = 11;  // ax, ay, az, du, div v, grad v (xx, yy, zz, xy, xz, yz)
+enum PairSum : int { SUM_A = 0, SUM_DU = 3, SUM_DIV = 4, SUM_G = 5 };
+
+// FP64: a component gets up to three products factor * x per neighbour, each one fused multiply-add as on a single
+// lane (pressure, stress and viscosity for the accelerations; one product for the others).
+struct alignas(16) PairTerms64 {
+    double m, mr;       // factors: mass for the accelerations and du, m / rho_i for the velocity gradients
+    double x[11];       // first product of each component
+    double stress[3], visc[3];
+    double pad;
+    __device__ __forceinline__ void clear() {
+        m = mr = 0.0;
+        for (int c = 0; c < 11; ++c) x[c] = 0.0;
+        for (int c = 0; c < 3; ++c) stress[c] = visc[c] = 0.0;
+    }
+    __device__ __forceinline__ void factors(double mj, double mjr) {
+        m = mj;
+        mr = mjr;
+    }
+    __device__ __forceinline__ void divergence(double, double v) { x[SUM_DIV] = v; }
+    __device__ __forceinline__ void pressure(double, double vx, double vy, double vz) {
+        x[0] = -vx;
+        x[1] = -vy;
+        x[2] = -vz;
+    }
+    __device__ __forceinline__ void gradient(double, const double v[6]) {
+        for (int c = 0; c < 6; ++c) x[SUM_G + c] = v[c];
+    }
+    __device__ __forceinline__ void stresses(double, double vx, double vy, double vz) {
+        stress[0] = vx;
+        stress[1] = vy;
+        stress[2] = vz;
+    }
+    __device__ __forceinline__ void viscosity(double, double vx, double vy, double vz, double heat) {
+        visc[0] = -vx;
+        visc[1] = -vy;
+        visc[2] = -vz;
+        x[SUM_DU] = heat;
+    }
+    __device__ __forceinline__ double add_to(double acc, int c) const {
+        const double f = c < SUM_DIV ? m : mr;
+        acc = fma(f, x[c], acc);
+        if (c < 3) {
+            acc = fma(f, stress[c], acc);
+            acc = fma(f, visc[c], acc);
+        }
+        return acc;
+    }
+};
+static_assert(sizeof(PairTerms64) == 160, "PairTerms64 is 160 bytes");
+
+// The sums of one lane's particle in FP64, the same products accumulated in place.
+struct PairAcc64 {
+    double ax = 0.0, ay = 0.0, az = 0.0, du = 0.0, divv = 0.0;
+    double g[6] = { 0.0, 0.0, 0.0, 0.0, 0.0, 0.0 };
+    __device__ __forceinline__ void factors(double, double) {}
+    __device__ __forceinline__ void divergence(double mjr, double v) { divv += mjr * v; }
+    __device__ __forceinline__ void pressure(double mj, double vx, double vy, double vz) {
+        ax -= mj * vx;
+        ay -= mj * vy;
+        az -= mj * vz;
+    }
+    __device__ __forceinline__ void gradient(double mjr, const double v[6]) {
+        for (int c = 0; c < 6; ++c) g[c] += mjr * v[c];
+    }
+    __device__ __forceinline__ void stresses(double mj, double vx, double vy, double vz) {
+        ax += mj * vx;
+        ay += mj * vy;
+        az += mj * vz;
+    }
+    __device__ __forceinline__ void viscosity(double mj, double vx, double vy, double vz, double heat) {
+        ax -= mj * vx;
+        ay -= mj * vy;
+        az -= mj * vz;
+        du += mj * heat;
+    }
+};
+
+// Mixed precision: one FP32 term per component, widened and added in FP64.
+struct alignas(16) PairTermsF {
+    float x[12];
+    __device__ __forceinline__ void clear() {
+        for (int c = 0; c < 12; ++c) x[c] = 0.f;
+    }
+    __device__ __forceinline__ void divergence(float v) { x[SUM_DIV] = v; }
+    __device__ __forceinline__ void gradient(int c, float v) { x[SUM_G + c] = v; }
+    __device__ __forceinline__ void heat(float v) { x[SUM_DU] = v; }
+    __device__ __forceinline__ void force(float vx, float vy, float vz) {
+        x[0] = vx;
+        x[1] = vy;
+        x[2] = vz;
+    }
+    __device__ __forceinline__ double add_to(double acc, int c) const { return acc + double(x[c]); }
+};
+
+// FP64 accumulators of FP32 terms: each term is widened exactly and summed in FP64 (on gfx950 an FP64 add
+// issues at the rate of an unpacked FP32 add, so this costs two instructions per term).
+struct PairAccF {
+    double ax = 0.0, ay = 0.0, az = 0.0, du = 0.0, divv = 0.0;
+    double g[6] = { 0.0, 0.0, 0.0, 0.0, 0.0, 0.0 };
+    __device__ __forceinline__ void divergence(float v) { divv += double(v); }
+    __device__ __forceinline__ void gradient(int c, float v) { g[c] += double(v); }
+    __device__ __forceinline__ void heat(float v) { du += double(v); }
+    __device__ __forceinline__ void force(float vx, float vy, float vz) {
+        ax += double(vx);
+        ay += double(vy);
+        az += double(vz);
+    }
+};
+
+// The sums of particle k by its group of LANES lanes: acc[i] = component sub + i LANES.  rows: the group's LANES rows.
+// Every lane of the wavefront must call this.
+template <int LANES>
+constexpr int GROUP_SUMS = (PAIR_SUMS + LANES - 1) / LANES;
+template <int LANES, typename Terms, typename Rec, typename F>
+__device__ __forceinline__ void sum_shared(const Rec* __restrict__ rec, const uint32_t* __restrict__ list, size_t k,
+                                           uint32_t quads, uint32_t listed, uint32_t sub, Terms* rows,
+                                           double (&acc)[GROUP_SUMS<LANES>], F&& f) {
+    auto entry = [&](uint32_t t) { return t < listed ? list[4 * list_quad(k, t >> 2, quads) + (t & 3u)] : uint32_t(k); };
+    uint32_t e = entry(sub);
+    Rec o = rec[e];
+    for (uint32_t t0 = 0; __any(t0 < listed); t0 += LANES) {
+        // the next record is loaded before the current one's terms
+        const uint32_t en = entry(t0 + LANES + sub);
+        const Rec on = rec[en];
+        Terms v;
+        v.clear();
+        if (t0 + sub < listed) f(o, e, v);
+        rows[sub] = v;
+        wave_sync();
+        const uint32_t cnt = t0 < listed ? min(listed - t0, uint32_t(LANES)) : 0u;
+#pragma unroll
+        for (int i = 0; i < GROUP_SUMS<LANES>; ++i) {
+            const int c = int(sub) + i * LANES;
+            if (c >= PAIR_SUMS) continue;
+            if (cnt == uint32_t(LANES)) {
+#pragma unroll
+                for (int r = 0; r < LANES; ++r) acc[i] = rows[r].add_to(acc[i], c);
+            } else {
+                for (uint32_t r = 0; r < cnt; ++r) acc[i] = rows[r].add_to(acc[i], c);
+            }
+        }
+        wave_sync();
+        o = on;
+        e = en;
+    }
+}
+
+// The groups' sums through LDS to one thread per particle: thread p < blockDim.x / LANES gets those of the block's
+// particle p.
+template <int LANES, typename Acc>
+__device__ __forceinline__ void collect_shared(const double (&acc)[GROUP_SUMS<LANES>], uint32_t sub,
+                                               double (*all)[PAIR_SUMS], Acc& ps) {
+#pragma unroll
+    for (int i = 0; i < GROUP_SUMS<LANES>; ++i) {
+        const int c = int(sub) + i * LANES;
+        if (c < PAIR_SUMS) all[threadIdx.x / LANES][c] = acc[i];
+    }
+    __syncthreads();
+    if (threadIdx.x < blockDim.x / LANES) {
+        const double* v = all[threadIdx.x];
+        ps.ax = v[0];
+        ps.ay = v[1];
+        ps.az = v[2];
+        ps.du = v[SUM_DU];
+        ps.divv = v[SUM_DIV];
+        for (int c = 0; c < 6; ++c) ps.g[c] = v[SUM_G + c];
+    }
+}
+
+// Stores the pair sums of particle order[k] and, FUSED, goes on with its finalize, corrector and criteria.  Every
+// thread of the block must call this (threads without a particle: valid false).
+template <bool FUSED, typename Acc>
+__device__ __forceinline__ void pairs_finish(DevState& s, const Params& prm, const uint32_t* __restrict__ order, size_t k,
+                                             bool valid, uint32_t cnt, const Acc& ps, const FuseArgs& fa) {
+    const bool solid = prm.solid_stress != 0;
+    double cv[4] = { INFINITY, INFINITY, INFINITY, INFINITY };
+    if (valid) {
+        const uint32_t i = order[k];
+        const double ax = prm.add_accel ? ps.ax + s.d[AX][i] : ps.ax;
+        const double ay = prm.add_accel ? ps.ay + s.d[AY][i] : ps.ay;
+        const double az = prm.add_accel ? ps.az + s.d[AZ][i] : ps.az;
+        s.d[AX][i] = ax;
+        s.d[AY][i] = ay;
+        s.d[AZ][i] = az;
+        s.d[DU][i] = ps.du;
+        s.d[DIVV][i] = ps.divv;
+        if (solid) {
+            for (int c = 0; c < 6; ++c) s.d[GXX + c][i] = ps.g[c];
+        }
+        s.u[NCNT][i] = cnt;
+        if (FUSED && !*fa.overflow) {
+            const osph_material m = fa.mats[s.u[MAT][i]];
+            const PairSums sums{ { ax, ay, az }, ps.du, ps.divv, { ps.g[0], ps.g[1], ps.g[2], ps.g[3], ps.g[4], ps.g[5] } };
+            finalize_at(s, m, prm, i, sums);
+            correct_at(s, m, prm, fa.dt, i, sums.a);
+            criteria_values(s, m, prm, i, sums.a, sums.divv, cv);
+        }
+    }
+    if (FUSED && !*fa.overflow) reduce_criteria(cv, fa.mins);
+}
+
 // FP64 pair sums in gather form.  For particle i (sorted position k) and each neighbour j, the kernel
 // gradient of SymmetrizeSmoothingLengths<LutKernel<3>> (Kernel.h:32-36,640-643) at hbar, then the
 // contributions every derivative of the term set makes to particle i:
@@ -857,27 +1142,24 @@ __device__ __forceinline__ void for_each_neighbor(const Rec* __restrict__ rec, c
 //   StandardAV                               av/Standard.h:62-83
 //   NeighborCountTerm                        HelperTerms.h:38-46
 // The accumulated buffers replace the storage buffers (Accumulated::store, Accumulated.cpp:87-100).
-// LPP lanes share one particle: each sums its share of the list, then the partial sums are added across
-// the group (fewer particles in flight per XCD, so their neighbour records stay in its L2).
-template <int LPP, bool FUSED>
+// With LANES > 1, a group of lanes shares one particle (sum_shared).
+template <int LANES, bool FUSED>
 __device__ __forceinline__ void pairs_fp64_body(size_t t, DevState s, const Params& prm,
                                                 const PairRec* __restrict__ rec, const uint32_t* __restrict__ group,
                                                 const uint32_t* __restrict__ order, const uint32_t* __restrict__ list,
                                                 const uint32_t* __restrict__ count, const double* __restrict__ lut,
                                                 uint32_t kmax, size_t n, const FuseArgs& fa) {
-    const PairLane<LPP> ln(t, n);
-    const size_t k = ln.k;
+    const uint32_t sub = uint32_t(t % LANES);
+    size_t k = t / LANES;
+    bool valid = k < n;  // lanes past the end keep running, with an empty list
+    if (!valid) k = n - 1;
     const PairRec me = rec[k];
     const uint32_t gi = group[k];
     const double rhoInv = 1.0 / me.rho;
-    double ax = 0.0, ay = 0.0, az = 0.0, du = 0.0, divv = 0.0;
-    double gxx = 0.0, gyy = 0.0, gzz = 0.0, gxy = 0.0, gxz = 0.0, gyz = 0.0;
-    const uint32_t cnt = ln.valid ? count[k] : 0u;
+    uint32_t cnt = valid ? count[k] : 0u;
     const uint32_t listed = cnt < kmax ? cnt : kmax;
     const bool solid = prm.solid_stress != 0;
-    __shared__ uint4 stage[PAIRS64_STAGE ? (BLOCK / 64) * StageOf<PairRec>::WORDS : 1];
-    uint4* my_stage = PAIRS64_STAGE ? stage + (threadIdx.x >> 6) * StageOf<PairRec>::WORDS : stage;
-    for_each_neighbor<LPP, PAIRS64_STAGE>(rec, list, k, kmax >> 2, listed, ln.sub, my_stage, [&](const PairRec& o, uint32_t k2) {
+    auto term = [&](const PairRec& o, uint32_t k2, auto& sum) {
         const double rx = me.x - o.x, ry = me.y - o.y, rz = me.z - o.z;
         const double hbar = 0.5 * (me.h + o.h);
         const double hInv = 1.0 / hbar;
@@ -889,27 +1171,17 @@ __device__ __forceinline__ void pairs_fp64_body(size_t t, DevState s, const Para
         const double wx = o.vx - me.vx, wy = o.vy - me.vy, wz = o.vz - me.vz;  // v_j - v_i
         const double mj = o.m;
         const double mjr = mj * rhoInv;
-        // velocity divergence
-        divv += mjr * (wx * gx + wy * gy + wz * gz);
-        // pressure gradient
-        {
-            const double coef = me.pr + o.pr;
-            ax -= mj * (coef * gx);
-            ay -= mj * (coef * gy);
-            az -= mj * (coef * gz);
-        }
+        sum.factors(mj, mjr);
+        sum.divergence(mjr, wx * gx + wy * gy + wz * gz);
+        const double coef = me.pr + o.pr;
+        sum.pressure(mj, coef * gx, coef * gy, coef * gz);
         if (solid && gi == group[k2] && gi != NO_GROUP) {
-            gxx += mjr * (wx * gx);
-            gyy += mjr * (wy * gy);
-            gzz += mjr * (wz * gz);
-            gxy += mjr * (0.5 * (wx * gy + wy * gx));
-            gxz += mjr * (0.5 * (wx * gz + wz * gx));
-            gyz += mjr * (0.5 * (wy * gz + wz * gy));
+            const double gv[6] = { wx * gx, wy * gy, wz * gz, 0.5 * (wx * gy + wy * gx), 0.5 * (wx * gz + wz * gx),
+                                   0.5 * (wy * gz + wz * gy) };
+            sum.gradient(mjr, gv);
             const double xx = me.sxx + o.sxx, yy = me.syy + o.syy, xy = me.sxy + o.sxy;
             const double xz = me.sxz + o.sxz, yz = me.syz + o.syz;
-            ax += mj * (xx * gx + xy * gy + xz * gz);
-            ay += mj * (xy * gx + yy * gy + yz * gz);
-            az += mj * (xz * gx + yz * gy + (-xx - yy) * gz);
+            sum.stresses(mj, xx * gx + xy * gy + xz * gz, xy * gx + yy * gy + yz * gz, xz * gx + yz * gy + (-xx - yy) * gz);
         }
         // artificial viscosity, only in convergent flow
         const double dvdr = -(wx * rx + wy * ry + wz * rz);  // (v_i - v_j) . (r_i - r_j)
@@ -918,59 +1190,30 @@ __device__ __forceinline__ void pairs_fp64_body(size_t t, DevState s, const Para
             const double csbar = 0.5 * (me.cs + o.cs);
             const double mu = hbar * dvdr / (d2 + 1.e-2 * (hbar * hbar));
             const double av = (-prm.av_alpha * csbar * mu + prm.av_beta * (mu * mu)) / rhobar;
-            ax -= mj * (av * gx);
-            ay -= mj * (av * gy);
-            az -= mj * (av * gz);
-            du += mj * (0.5 * av * -(wx * gx + wy * gy + wz * gz));
+            sum.viscosity(mj, av * gx, av * gy, av * gz, 0.5 * av * -(wx * gx + wy * gy + wz * gz));
         }
-    });
-    ax = group_sum<LPP>(ax);
-    ay = group_sum<LPP>(ay);
-    az = group_sum<LPP>(az);
-    du = group_sum<LPP>(du);
-    divv = group_sum<LPP>(divv);
-    if (solid) {
-        gxx = group_sum<LPP>(gxx);
-        gyy = group_sum<LPP>(gyy);
-        gzz = group_sum<LPP>(gzz);
-        gxy = group_sum<LPP>(gxy);
-        gxz = group_sum<LPP>(gxz);
-        gyz = group_sum<LPP>(gyz);
+    };
+    PairAcc64 ps;
+    if constexpr (LANES > 1) {
+        __shared__ PairTerms64 rows[BLOCK];
+        __shared__ double all[BLOCK / LANES][PAIR_SUMS];
+        double acc[GROUP_SUMS<LANES>] = {};
+        sum_shared<LANES>(rec, list, k, kmax >> 2, listed, sub, rows + threadIdx.x / LANES * LANES, acc, term);
+        collect_shared<LANES>(acc, sub, all, ps);
+        // from here on thread p of the block goes on with its particle p
+        k = (t - threadIdx.x) / LANES + threadIdx.x;
+        valid = threadIdx.x < blockDim.x / LANES && k < n;
+        if (valid) cnt = count[k];
+    } else {
+        __shared__ uint4 stage[PAIRS64_STAGE ? (BLOCK / 64) * StageOf<PairRec>::WORDS : 1];
+        uint4* my_stage = PAIRS64_STAGE ? stage + (threadIdx.x >> 6) * StageOf<PairRec>::WORDS : stage;
+        for_each_neighbor<PAIRS64_STAGE>(rec, list, k, kmax >> 2, listed, my_stage,
+                                         [&](const PairRec& o, uint32_t k2) { term(o, k2, ps); });
     }
-    double cv[4] = { INFINITY, INFINITY, INFINITY, INFINITY };
-    if (ln.valid && ln.sub == 0) {
-        const uint32_t i = order[k];
-        if (prm.add_accel) {
-            ax += s.d[AX][i];
-            ay += s.d[AY][i];
-            az += s.d[AZ][i];
-        }
-        s.d[AX][i] = ax;
-        s.d[AY][i] = ay;
-        s.d[AZ][i] = az;
-        s.d[DU][i] = du;
-        s.d[DIVV][i] = divv;
-        if (solid) {
-            s.d[GXX][i] = gxx;
-            s.d[GYY][i] = gyy;
-            s.d[GZZ][i] = gzz;
-            s.d[GXY][i] = gxy;
-            s.d[GXZ][i] = gxz;
-            s.d[GYZ][i] = gyz;
-        }
-        s.u[NCNT][i] = cnt;
-        if (FUSED && !*fa.overflow) {
-            const osph_material m = fa.mats[s.u[MAT][i]];
-            const PairSums ps{ { ax, ay, az }, du, divv, { gxx, gyy, gzz, gxy, gxz, gyz } };
-            finalize_at(s, m, prm, i, ps);
-            correct_at(s, m, prm, fa.dt, i, ps.a);
-            criteria_values(s, m, prm, i, ps.a, ps.divv, cv);
-        }
-    }
-    if (FUSED && !*fa.overflow) reduce_criteria(cv, fa.mins);
+    pairs_finish<FUSED>(s, prm, order, k, valid, cnt, ps, fa);
 }
 
-template <int LPP, bool FUSED>
+template <int LANES, bool FUSED>
 __global__ void __launch_bounds__(BLOCK) k_pairs_fp64(DevState s, Params prm, const PairRec* __restrict__ rec,
                                                       const uint32_t* __restrict__ group,
                                                       const uint32_t* __restrict__ order,
@@ -978,8 +1221,8 @@ __global__ void __launch_bounds__(BLOCK) k_pairs_fp64(DevState s, Params prm, co
                                                       const uint32_t* __restrict__ count,
                                                       const double* __restrict__ lut, uint32_t kmax, size_t n,
                                                       FuseArgs fa) {
-    pairs_fp64_body<LPP, FUSED>(size_t(xcd_block(blockIdx.x, gridDim.x)) * blockDim.x + threadIdx.x, s, prm, rec,
-                                group, order, list, count, lut, kmax, n, fa);
+    pairs_fp64_body<LANES, FUSED>(size_t(xcd_block(blockIdx.x, gridDim.x)) * blockDim.x + threadIdx.x, s, prm, rec,
+                                   group, order, list, count, lut, kmax, n, fa);
 }
 
 // ---- mixed precision ---------------------------------------------------------------------------------
@@ -1057,13 +1300,6 @@ __device__ __forceinline__ float m4_grad_f(float q2) {
     return (-0.75f * INV_PI) * (t * t) * __builtin_amdgcn_rcpf(q);
 }
 
-// FP64 accumulator of FP32 terms: each term is widened exactly and summed in FP64 (on gfx950 an FP64 add
-// issues at the rate of an unpacked FP32 add, so this costs two instructions per term).
-struct Acc {
-    double sum = 0.0;
-    __device__ __forceinline__ void add(float v) { sum += double(v); }
-};
-
 // Mixed-precision pair sums: the same terms and gather form as k_pairs_fp64, evaluated in FP32 on the
 // records' fixed-point positions and velocities and accumulated in FP64; results are written in FP64.  A
 // difference of fixed-point coordinates is an exact int32 (each frame spans less than 2^31 steps), rounded
@@ -1071,36 +1307,37 @@ struct Acc {
 // whatever the magnitudes of the absolute values.  Divisions are hardware reciprocals
 // (about 1 ulp) times the numerator.  Groups (SUM_ONLY_UNDAMAGED) compare by the records' 4-bit codes,
 // and through the group array for groups beyond the codes' range.
-template <int LPP, bool FUSED>
+template <int LANES, bool FUSED>
 __device__ __forceinline__ void pairs_mixed_body(size_t t, DevState s, const Params& prm, const Fixed& F,
                                                  const PairRecF* __restrict__ rec, const uint32_t* __restrict__ group,
                                                  const uint32_t* __restrict__ order,
                                                  const uint32_t* __restrict__ list, const uint32_t* __restrict__ count,
                                                  uint32_t kmax, size_t n, const FuseArgs& fa) {
-    const PairLane<LPP> ln(t, n);
-    const size_t k = ln.k;
+    const uint32_t sub = uint32_t(t % LANES);
+    size_t k = t / LANES;
+    bool valid = k < n;  // lanes past the end keep running, with an empty list
+    if (!valid) k = n - 1;
     const PairRecF me = rec[k];
     const uint32_t gi = group[k];
     const uint32_t gci = __float_as_uint(me.cs) & 15u;
     const float csi = __uint_as_float(__float_as_uint(me.cs) & ~15u);
     const float rhoInv = 1.0f / me.rho;
     const float alpha = float(prm.av_alpha), beta = float(prm.av_beta);
-    Acc ax, ay, az, du, divv, gxx, gyy, gzz, gxy, gxz, gyz;
-    const uint32_t cnt = ln.valid ? count[k] : 0u;
+    uint32_t cnt = valid ? count[k] : 0u;
     const uint32_t listed = cnt < kmax ? cnt : kmax;
     const bool solid = prm.solid_stress != 0;
     const bool grouped = solid && gci != GROUP_CODE_NONE;  // stress terms with the particle's own group
-    // the LDS stage exists whenever the gather mode uses it (one uint4 otherwise)
-    __shared__ uint4 stage[PAIRSMX_STAGE ? (BLOCK / 64) * StageOf<PairRecF>::WORDS : 1];
-    uint4* my_stage = PAIRSMX_STAGE ? stage + (threadIdx.x >> 6) * StageOf<PairRecF>::WORDS : stage;
-    for_each_neighbor<LPP, PAIRSMX_STAGE>(rec, list, k, kmax >> 2, listed, ln.sub, my_stage, [&](const PairRecF& o, uint32_t e) {
+    // the fused multiply-adds are written out: which products fuse must not depend on the instance, as the sums
+    // are the same bits with one lane and with a group
+    auto term = [&](const PairRecF& o, uint32_t e, auto& sum) {
+#pragma clang fp contract(off)
         const float rx = float(int32_t(me.x - o.x)) * F.stepf;
         const float ry = float(int32_t(me.y - o.y)) * F.stepf;
         const float rz = float(int32_t(me.z - o.z)) * F.stepf;
         const float hbar = 0.5f * (me.h + o.h);
         const float hInv = __builtin_amdgcn_rcpf(hbar);
         const float hInv2 = hInv * hInv;
-        const float d2 = rx * rx + ry * ry + rz * rz;
+        const float d2 = fmaf(rz, rz, fmaf(rx, rx, ry * ry));
         const float gk = m4_grad_f(d2 * hInv2);
         const float h5g = (hInv2 * hInv2) * hInv * gk;
         const float gx = rx * h5g, gy = ry * h5g, gz = rz * h5g;
@@ -1109,83 +1346,62 @@ __device__ __forceinline__ void pairs_mixed_body(size_t t, DevState s, const Par
         const float wz = float(int32_t(o.vz - me.vz)) * F.vstepf;
         const float mj = o.m;
         const float mjr = mj * rhoInv;
-        const float wg = wx * gx + wy * gy + wz * gz;
-        divv.add(mjr * wg);
+        const float wgx = wx * gx, wgy = wy * gy, wgz = wz * gz;
+        const float wg = wgx + wgy + wgz;
+        sum.divergence(mjr * wg);
         const float coef = me.pr + o.pr;
         float fx = -(coef * gx), fy = -(coef * gy), fz = -(coef * gz);
         bool same = grouped && (__float_as_uint(o.cs) & 15u) == gci;
         if (same && gci == GROUP_CODE_WIDE) same = group[e] == gi;
         if (same) {
-            gxx.add(mjr * (wx * gx));
-            gyy.add(mjr * (wy * gy));
-            gzz.add(mjr * (wz * gz));
-            gxy.add(mjr * (0.5f * (wx * gy + wy * gx)));
-            gxz.add(mjr * (0.5f * (wx * gz + wz * gx)));
-            gyz.add(mjr * (0.5f * (wy * gz + wz * gy)));
+            sum.gradient(0, mjr * wgx);
+            sum.gradient(1, mjr * wgy);
+            sum.gradient(2, mjr * wgz);
+            sum.gradient(3, mjr * (0.5f * fmaf(wx, gy, wy * gx)));
+            sum.gradient(4, mjr * (0.5f * fmaf(wx, gz, wz * gx)));
+            sum.gradient(5, mjr * (0.5f * fmaf(wy, gz, wz * gy)));
             const float xx = me.sxx + o.sxx, yy = me.syy + o.syy, xy = me.sxy + o.sxy;
             const float xz = me.sxz + o.sxz, yz = me.syz + o.syz;
-            fx += xx * gx + xy * gy + xz * gz;
-            fy += xy * gx + yy * gy + yz * gz;
-            fz += xz * gx + yz * gy + (-xx - yy) * gz;
+            fx += fmaf(xz, gz, fmaf(xx, gx, xy * gy));
+            fy += fmaf(yz, gz, fmaf(yy, gy, xy * gx));
+            fz += fmaf(-xx - yy, gz, fmaf(xz, gx, yz * gy));
         }
-        const float dvdr = -(wx * rx + wy * ry + wz * rz);
+        const float dvdr = -fmaf(wz, rz, fmaf(wx, rx, wy * ry));
         if (dvdr < 0.0f) {
             const float rhobar = 0.5f * (me.rho + o.rho);
             const float csbar = 0.5f * (csi + __uint_as_float(__float_as_uint(o.cs) & ~15u));
-            const float mu = hbar * dvdr * __builtin_amdgcn_rcpf(d2 + 1.e-2f * (hbar * hbar));
-            const float av = (-alpha * csbar * mu + beta * (mu * mu)) * __builtin_amdgcn_rcpf(rhobar);
-            fx -= av * gx;
-            fy -= av * gy;
-            fz -= av * gz;
-            du.add(mj * (0.5f * av * -wg));
+            const float mu = hbar * dvdr * __builtin_amdgcn_rcpf(fmaf(1.e-2f, hbar * hbar, d2));
+            const float av = fmaf(beta, mu * mu, -(alpha * csbar * mu)) * __builtin_amdgcn_rcpf(rhobar);
+            fx = fmaf(-av, gx, fx);
+            fy = fmaf(-av, gy, fy);
+            fz = fmaf(-av, gz, fz);
+            sum.heat(mj * (0.5f * av * -wg));
         }
-        ax.add(mj * fx);
-        ay.add(mj * fy);
-        az.add(mj * fz);
-    });
-    const double sax = group_sum<LPP>(ax.sum), say = group_sum<LPP>(ay.sum), saz = group_sum<LPP>(az.sum);
-    const double sdu = group_sum<LPP>(du.sum), sdivv = group_sum<LPP>(divv.sum);
-    double g[6] = { 0.0, 0.0, 0.0, 0.0, 0.0, 0.0 };
-    if (solid) {
-        g[0] = group_sum<LPP>(gxx.sum);
-        g[1] = group_sum<LPP>(gyy.sum);
-        g[2] = group_sum<LPP>(gzz.sum);
-        g[3] = group_sum<LPP>(gxy.sum);
-        g[4] = group_sum<LPP>(gxz.sum);
-        g[5] = group_sum<LPP>(gyz.sum);
+        sum.force(mj * fx, mj * fy, mj * fz);
+    };
+    PairAccF ps;
+    if constexpr (LANES > 1) {
+        __shared__ PairTermsF rows[BLOCK];
+        __shared__ double all[BLOCK / LANES][PAIR_SUMS];
+        double acc[GROUP_SUMS<LANES>] = {};
+        sum_shared<LANES>(rec, list, k, kmax >> 2, listed, sub, rows + threadIdx.x / LANES * LANES, acc, term);
+        collect_shared<LANES>(acc, sub, all, ps);
+        // from here on thread p of the block goes on with its particle p
+        k = (t - threadIdx.x) / LANES + threadIdx.x;
+        valid = threadIdx.x < blockDim.x / LANES && k < n;
+        if (valid) cnt = count[k];
+    } else {
+        // the LDS stage exists whenever the gather mode uses it (one uint4 otherwise)
+        constexpr bool STAGE = PAIRSMX_STAGE == 1 || PAIRSMX_STAGE == 2;
+        __shared__ uint4 stage[STAGE ? (BLOCK / 64) * StageOf<PairRecF>::WORDS : 1];
+        uint4* my_stage = STAGE ? stage + (threadIdx.x >> 6) * StageOf<PairRecF>::WORDS : stage;
+        for_each_neighbor<PAIRSMX_STAGE>(rec, list, k, kmax >> 2, listed, my_stage,
+                                         [&](const PairRecF& o, uint32_t e) { term(o, e, ps); });
     }
-    double cv[4] = { INFINITY, INFINITY, INFINITY, INFINITY };
-    if (ln.valid && ln.sub == 0) {
-        const uint32_t i = order[k];
-        const double fax = prm.add_accel ? sax + s.d[AX][i] : sax;
-        const double fay = prm.add_accel ? say + s.d[AY][i] : say;
-        const double faz = prm.add_accel ? saz + s.d[AZ][i] : saz;
-        s.d[AX][i] = fax;
-        s.d[AY][i] = fay;
-        s.d[AZ][i] = faz;
-        s.d[DU][i] = sdu;
-        s.d[DIVV][i] = sdivv;
-        if (solid) {
-            s.d[GXX][i] = g[0];
-            s.d[GYY][i] = g[1];
-            s.d[GZZ][i] = g[2];
-            s.d[GXY][i] = g[3];
-            s.d[GXZ][i] = g[4];
-            s.d[GYZ][i] = g[5];
-        }
-        s.u[NCNT][i] = cnt;
-        if (FUSED && !*fa.overflow) {
-            const osph_material m = fa.mats[s.u[MAT][i]];
-            const PairSums ps{ { fax, fay, faz }, sdu, sdivv, { g[0], g[1], g[2], g[3], g[4], g[5] } };
-            finalize_at(s, m, prm, i, ps);
-            correct_at(s, m, prm, fa.dt, i, ps.a);
-            criteria_values(s, m, prm, i, ps.a, ps.divv, cv);
-        }
-    }
-    if (FUSED && !*fa.overflow) reduce_criteria(cv, fa.mins);
+    pairs_finish<FUSED>(s, prm, order, k, valid, cnt, ps, fa);
 }
 
-template <int LPP, bool FUSED>
+template <int LANES, bool FUSED>
 __global__ void __launch_bounds__(BLOCK) k_pairs_mixed(DevState s, Params prm, Fixed F,
                                                        const PairRecF* __restrict__ rec,
                                                        const uint32_t* __restrict__ group,
@@ -1193,8 +1409,8 @@ __global__ void __launch_bounds__(BLOCK) k_pairs_mixed(DevState s, Params prm, F
                                                        const uint32_t* __restrict__ list,
                                                        const uint32_t* __restrict__ count, uint32_t kmax, size_t n,
                                                        FuseArgs fa) {
-    pairs_mixed_body<LPP, FUSED>(size_t(xcd_block(blockIdx.x, gridDim.x)) * blockDim.x + threadIdx.x, s, prm, F, rec,
-                                 group, order, list, count, kmax, n, fa);
+    pairs_mixed_body<LANES, FUSED>(size_t(xcd_block(blockIdx.x, gridDim.x)) * blockDim.x + threadIdx.x, s, prm, F, rec,
+                                    group, order, list, count, kmax, n, fa);
 }
 
 // ScalarGradyKippModel::integrate (core/physics/Damage.cpp:128-170) for particle i.
@@ -1830,6 +2046,17 @@ void launch_neighbor_lists(const Launch& l, const double4* pos, const float4* po
                            size_t n) {
     if (!n) return;
     const int b = l.tune.lists_block;
+    if (lists_shared(g, n)) {
+        const unsigned grid = grid_for(n * LIST_LANES, b);
+        if (sc.on) {
+            k_neighbor_lists_shared<true><<<grid, b, size_t(l.tune.lists_lds), l.stream>>>(
+                pos, posf, sc, g, first, list, count, kmax, overflow, n);
+        } else {
+            k_neighbor_lists_shared<false><<<grid, b, size_t(l.tune.lists_lds), l.stream>>>(
+                pos, posf, sc, g, first, list, count, kmax, overflow, n);
+        }
+        return;
+    }
     if (sc.on) {
         k_neighbor_lists<true><<<grid_for(n, b), b, size_t(l.tune.lists_lds), l.stream>>>(
             pos, posf, sc, g, first, list, count, kmax, overflow, n);
@@ -1843,16 +2070,17 @@ void launch_pairs_fp64(const Launch& l, DevState s, Params prm, const PairRec* r
                        const uint32_t* order, const uint32_t* list, const uint32_t* count, const double* lut_grads,
                        uint32_t kmax, size_t n, const FuseArgs* fuse) {
     if (!n) return;
-    const int b = l.tune.pairs_block, lpp = l.tune.pairs_lanes;
-    const unsigned grid = grid_for(n * size_t(lpp), b);
+    const int b = l.tune.pairs_block;
+    const int lanes = pair_lanes(l.tune, n);
+    const unsigned grid = grid_for(n * size_t(lanes), b);
     const size_t lds = size_t(l.tune.pairs_lds);
     const FuseArgs fa = fuse ? *fuse : FuseArgs{};
 #define OSPH_PAIRS64(P, F) \
     k_pairs_fp64<P, F><<<grid, b, lds, l.stream>>>(s, prm, rec, group, order, list, count, lut_grads, kmax, n, fa)
-    if (lpp == 4) {
+    if (lanes == 16) {
+        if (fuse) OSPH_PAIRS64(16, true); else OSPH_PAIRS64(16, false);
+    } else if (lanes == 4) {
         if (fuse) OSPH_PAIRS64(4, true); else OSPH_PAIRS64(4, false);
-    } else if (lpp == 2) {
-        if (fuse) OSPH_PAIRS64(2, true); else OSPH_PAIRS64(2, false);
     } else {
         if (fuse) OSPH_PAIRS64(1, true); else OSPH_PAIRS64(1, false);
     }
@@ -1869,16 +2097,17 @@ void launch_pairs_mixed(const Launch& l, DevState s, Params prm, Fixed fx, const
                         const uint32_t* order, const uint32_t* list, const uint32_t* count, uint32_t kmax, size_t n,
                         const FuseArgs* fuse) {
     if (!n) return;
-    const int b = l.tune.pairs_block, lpp = l.tune.pairs_lanes;
-    const unsigned grid = grid_for(n * size_t(lpp), b);
+    const int b = l.tune.pairs_block;
+    const int lanes = pair_lanes(l.tune, n);
+    const unsigned grid = grid_for(n * size_t(lanes), b);
     const size_t lds = size_t(l.tune.pairs_lds);
     const FuseArgs fa = fuse ? *fuse : FuseArgs{};
 #define OSPH_PAIRSMX(P, F) \
     k_pairs_mixed<P, F><<<grid, b, lds, l.stream>>>(s, prm, fx, rec, group, order, list, count, kmax, n, fa)
-    if (lpp == 4) {
+    if (lanes == 16) {
+        if (fuse) OSPH_PAIRSMX(16, true); else OSPH_PAIRSMX(16, false);
+    } else if (lanes == 4) {
         if (fuse) OSPH_PAIRSMX(4, true); else OSPH_PAIRSMX(4, false);
-    } else if (lpp == 2) {
-        if (fuse) OSPH_PAIRSMX(2, true); else OSPH_PAIRSMX(2, false);
     } else {
         if (fuse) OSPH_PAIRSMX(1, true); else OSPH_PAIRSMX(1, false);
     }
@@ -2061,7 +2290,7 @@ __global__ void __launch_bounds__(BLOCK) kb_lists(const BatchMember* __restrict_
     neighbor_list_at<SCREEN>(a.pos, a.posf, a.screen, a.grid, a.cell_first, a.list, a.count, a.kmax, overflow_of(a), k);
 }
 
-template <bool MIXED, int LPP, bool FUSED>
+template <bool MIXED, int LANES, bool FUSED>
 __global__ void __launch_bounds__(BLOCK) kb_pairs(const BatchMember* __restrict__ M, BatchBlocks qb,
                                                   const double* __restrict__ lut) {
     uint32_t m, bid, nb;
@@ -2069,10 +2298,10 @@ __global__ void __launch_bounds__(BLOCK) kb_pairs(const BatchMember* __restrict_
     const size_t t = size_t(xcd_block(bid, nb)) * blockDim.x + threadIdx.x;
     const FuseArgs fa{ a.mats, a.dt, a.small + SMALL_CRITERIA, overflow_of(a) };
     if constexpr (MIXED) {
-        pairs_mixed_body<LPP, FUSED>(t, a.s2, a.prm, a.fx, static_cast<const PairRecF*>(a.rec), a.group, a.order,
+        pairs_mixed_body<LANES, FUSED>(t, a.s2, a.prm, a.fx, static_cast<const PairRecF*>(a.rec), a.group, a.order,
                                      a.list, a.count, a.kmax, a.n, fa);
     } else {
-        pairs_fp64_body<LPP, FUSED>(t, a.s2, a.prm, static_cast<const PairRec*>(a.rec), a.group, a.order, a.list,
+        pairs_fp64_body<LANES, FUSED>(t, a.s2, a.prm, static_cast<const PairRec*>(a.rec), a.group, a.order, a.list,
                                     a.count, lut, a.kmax, a.n, fa);
     }
 }
@@ -2132,27 +2361,23 @@ void batch_lists(const Launch& l, const BatchMember* M, BatchBlocks lb, bool scr
     if (plain) kb_lists<false><<<lb.total, b, lds, l.stream>>>(M, lb);
 }
 
-void batch_pairs(const Launch& l, const BatchMember* M, BatchBlocks qb, bool mixed, bool fuse, const double* lut) {
-    const int b = l.tune.pairs_block, lpp = l.tune.pairs_lanes;
+void batch_pairs(const Launch& l, const BatchMember* M, BatchBlocks qb, bool mixed, bool fuse, int lanes,
+                 const double* lut) {
+    const int b = l.tune.pairs_block;
     const size_t lds = size_t(l.tune.pairs_lds);
 #define OSPH_BPAIRS(MX, P, F) kb_pairs<MX, P, F><<<qb.total, b, lds, l.stream>>>(M, qb, lut)
-    if (mixed) {
-        if (lpp == 4) {
-            if (fuse) OSPH_BPAIRS(true, 4, true); else OSPH_BPAIRS(true, 4, false);
-        } else if (lpp == 2) {
-            if (fuse) OSPH_BPAIRS(true, 2, true); else OSPH_BPAIRS(true, 2, false);
-        } else {
-            if (fuse) OSPH_BPAIRS(true, 1, true); else OSPH_BPAIRS(true, 1, false);
-        }
-    } else {
-        if (lpp == 4) {
-            if (fuse) OSPH_BPAIRS(false, 4, true); else OSPH_BPAIRS(false, 4, false);
-        } else if (lpp == 2) {
-            if (fuse) OSPH_BPAIRS(false, 2, true); else OSPH_BPAIRS(false, 2, false);
-        } else {
-            if (fuse) OSPH_BPAIRS(false, 1, true); else OSPH_BPAIRS(false, 1, false);
-        }
-    }
+#define OSPH_BPAIRS_OF(P)                                                       \
+    do {                                                                        \
+        if (mixed) {                                                            \
+            if (fuse) OSPH_BPAIRS(true, P, true); else OSPH_BPAIRS(true, P, false);   \
+        } else {                                                                \
+            if (fuse) OSPH_BPAIRS(false, P, true); else OSPH_BPAIRS(false, P, false); \
+        }                                                                       \
+    } while (0)
+    if (lanes == 16) OSPH_BPAIRS_OF(16);
+    else if (lanes == 4) OSPH_BPAIRS_OF(4);
+    else OSPH_BPAIRS_OF(1);
+#undef OSPH_BPAIRS_OF
 #undef OSPH_BPAIRS
 }
 
