@@ -7,9 +7,7 @@ after one untimed step; the starting settings are run once before their timed ru
 on a state size the buffers. The resident state is copied on the device before the first candidate and
 restored after every one, so the tuning leaves the run where it was (the derivative planes included).
 
-Every candidate gives the same neighbour sets. The lane split of the pair kernels changes the order of
-the summation, so the derivatives may differ in the last bits (within the parity tolerances). No
-reference counterpart: the reference has no device kernels.
+Every candidate gives the same neighbour sets and the same sums. No reference counterpart: the reference has no device kernels.
 """
 from __future__ import annotations
 

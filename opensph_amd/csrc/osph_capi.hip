@@ -90,12 +90,13 @@ struct osph_ctx {
     int since_reorder = 0;
 
     // neighbour structures (all sized for cap particles)
-    uint32_t *keys = nullptr, *keys_sorted = nullptr, *iota = nullptr, *order = nullptr;
+    uint32_t *keys_sorted = nullptr, *order = nullptr;  // keys_sorted: batched steps
+    uint2 *where = nullptr, *bucket = nullptr;          // rows of the particles, and their buckets (launch_cell_sort)
     const char* failed_launch = nullptr;  // name of the first timed launch that left a HIP error
-    void* sort_temp = nullptr;
-    size_t sort_temp_bytes = 0;
+    uint32_t *row_count = nullptr, *row_start = nullptr;  // [slot_cap] counts (zero between searches) and their sums
+    size_t slot_cap = 0;
     uint32_t* cell_first = nullptr;  // [cells + 1]: first sorted position of each cell (valid rows only)
-    uint32_t* row_range = nullptr;   // [2 rows]: sorted range of each row of cells
+    uint32_t* row_range = nullptr;   // [2 rows]: sorted range of each row of cells (batched steps)
     size_t row_cap = 0;
     size_t cell_cap = 0;
     PairRec* rec = nullptr;
@@ -218,11 +219,10 @@ void free_state(osph_ctx* c) {
     c->dblock2 = nullptr;
     c->ublock2 = nullptr;
     c->perm = c->perm2 = c->slot_of = nullptr;
-    (void)hipFree(c->keys);
     (void)hipFree(c->keys_sorted);
-    (void)hipFree(c->iota);
+    (void)hipFree(c->where);
+    (void)hipFree(c->bucket);
     (void)hipFree(c->order);
-    (void)hipFree(c->sort_temp);
     (void)hipFree(c->rec);
     (void)hipFree(c->recf);
     (void)hipFree(c->posf);
@@ -231,8 +231,8 @@ void free_state(osph_ctx* c) {
     (void)hipFree(c->count);
     c->dblock = nullptr;
     c->ublock = nullptr;
-    c->keys = c->keys_sorted = c->iota = c->order = nullptr;
-    c->sort_temp = nullptr;
+    c->keys_sorted = c->order = nullptr;
+    c->where = c->bucket = nullptr;
     c->rec = nullptr;
     c->recf = nullptr;
     c->posf = nullptr;
@@ -272,6 +272,22 @@ int ensure_rows(osph_ctx* c, size_t rows) {
     c->row_cap = 0;
     HIPCHK(c, hipMalloc(&c->row_range, 2 * rows * sizeof(uint32_t)));
     c->row_cap = rows;
+    return OSPH_OK;
+}
+
+// The row counts and sums; new counts start at zero, and every search leaves them so.
+int ensure_slots(osph_ctx* c, uint32_t slots) {
+    const size_t need = row_slots(slots);
+    if (need <= c->slot_cap) return OSPH_OK;
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    (void)hipFree(c->row_count);
+    (void)hipFree(c->row_start);
+    c->row_count = c->row_start = nullptr;
+    c->slot_cap = 0;
+    HIPCHK(c, hipMalloc(&c->row_count, need * sizeof(uint32_t)));
+    HIPCHK(c, hipMalloc(&c->row_start, need * sizeof(uint32_t)));
+    launch_clear_u32(Launch{ c->stream }, c->row_count, need, 0u);
+    c->slot_cap = need;
     return OSPH_OK;
 }
 
@@ -544,9 +560,11 @@ int plan_search(osph_ctx* c, const unsigned long long* sh, size_t* rows_out) {
     g.hmin = href;
     g.nclass = last + 1;
     uint32_t base = 0;
+    g.slots = 0;
     for (int cl = 0; cl < g.nclass; ++cl) {
         GridClass& G = g.c[cl];
         G.base = base;
+        G.slot0 = g.slots;
         if (ccount[cl] == 0) {
             G.empty = 1;
             continue;
@@ -575,6 +593,7 @@ int plan_search(osph_ctx* c, const unsigned long long* sh, size_t* rows_out) {
                                   << bits;
         if (uint64_t(base) + rows_end > (uint64_t(1) << 32) - 2) return c->fail(OSPH_ERR_STATE, "cell count exceeds 32 bits");
         base += uint32_t(rows_end);
+        g.slots += uint32_t(rows_end >> bits);
     }
     g.key_bits = 1;
     while (g.key_bits < 32 && (uint64_t(1) << g.key_bits) < uint64_t(base)) ++g.key_bits;
@@ -654,24 +673,9 @@ int search_finish(osph_ctx* c) {
     if (int e = plan_search(c, c->small_host, &rows)) return e;
     const Grid g = c->grid;
 
-    timed(c, "cell_keys", [&] { launch_cell_keys(l, c->s, g, c->keys, c->iota, c->row_range, 2 * rows, n); });
-    const size_t sort_need = sort_pairs_temp_bytes(n, g.key_bits);
-    if (sort_need > c->sort_temp_bytes) {
-        HIPCHK(c, hipStreamSynchronize(c->stream));
-        (void)hipFree(c->sort_temp);
-        c->sort_temp = nullptr;
-        c->sort_temp_bytes = 0;
-        HIPCHK(c, hipMalloc(&c->sort_temp, sort_need));
-        c->sort_temp_bytes = sort_need;
-    }
-    hipError_t sort_err = hipSuccess;
-    timed(c, "sort", [&] {
-        sort_err = sort_pairs(l, c->sort_temp, c->sort_temp_bytes, c->keys, c->keys_sorted, c->iota, c->order, n,
-                              g.key_bits);
-    });
-    HIPCHK(c, sort_err);
-    timed(c, "cell_ranges", [&] {
-        launch_cell_first(l, c->keys_sorted, g, c->row_range, c->cell_first, rows, n);
+    if (int e = ensure_slots(c, g.slots)) return e;
+    timed(c, "cell_sort", [&] {
+        launch_cell_sort(l, c->s, g, c->row_count, c->row_start, c->where, c->bucket, c->order, c->cell_first, rows, n);
     });
     if (reorder_due(c)) {
         // move the state into this search's cell order: the record gather and the pair kernels' writes
@@ -987,6 +991,8 @@ void osph_destroy(osph_ctx* c) {
     free_state(c);
     (void)hipFree(c->cell_first);
     (void)hipFree(c->row_range);
+    (void)hipFree(c->row_count);
+    (void)hipFree(c->row_start);
     (void)hipFree(c->list);
     (void)hipFree(c->staging);
     (void)hipFree(c->scratch);
@@ -1021,9 +1027,9 @@ int osph_resize(osph_ctx* c, size_t n) {
         HIPCHK(c, hipMalloc(&c->perm, sizeof(uint32_t) * cap));
         HIPCHK(c, hipMalloc(&c->perm2, sizeof(uint32_t) * cap));
         HIPCHK(c, hipMalloc(&c->slot_of, sizeof(uint32_t) * cap));
-        HIPCHK(c, hipMalloc(&c->keys, sizeof(uint32_t) * cap));
         HIPCHK(c, hipMalloc(&c->keys_sorted, sizeof(uint32_t) * cap));
-        HIPCHK(c, hipMalloc(&c->iota, sizeof(uint32_t) * cap));
+        HIPCHK(c, hipMalloc(&c->where, sizeof(uint2) * cap));
+        HIPCHK(c, hipMalloc(&c->bucket, sizeof(uint2) * cap));
         HIPCHK(c, hipMalloc(&c->order, sizeof(uint32_t) * cap));
         if (c->cfg.precision == OSPH_PRECISION_MIXED) {
             HIPCHK(c, hipMalloc(&c->recf, sizeof(PairRecF) * cap));
@@ -1037,8 +1043,6 @@ int osph_resize(osph_ctx* c, size_t n) {
         launch_clear_u32(L(c), reinterpret_cast<uint32_t*>(c->posf + cap), 4 * POS_SLACK, 0u);
         HIPCHK(c, hipMalloc(&c->group, sizeof(uint32_t) * cap));
         HIPCHK(c, hipMalloc(&c->count, sizeof(uint32_t) * cap));
-        c->sort_temp_bytes = sort_pairs_temp_bytes(cap, 32);
-        HIPCHK(c, hipMalloc(&c->sort_temp, std::max<size_t>(c->sort_temp_bytes, 256)));
         c->cap = cap;
         for (int k = 0; k < NDPLANES; ++k) c->s.d[k] = c->dblock + size_t(k) * cap;
         for (int k = 0; k < NIPLANES; ++k) c->s.u[k] = c->ublock + size_t(k) * cap;

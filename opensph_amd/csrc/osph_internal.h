@@ -90,6 +90,7 @@ struct GridClass {
     int dim[3];
     int bits;             // 2^bits > every dim: x slots per row, and the width of y and z in the row key
     uint32_t base;        // offset of the class's cells in the cell tables and in the sort keys
+    uint32_t slot0;       // offset of the class's rows (by the Morton code of y, z) in the row arrays
     int empty;
 };
 
@@ -99,6 +100,7 @@ struct GridClass {
 struct Grid {
     int nclass;
     int key_bits;  // bits of the sort key that can be nonzero
+    uint32_t slots;  // rows of all classes, by their Morton codes
     double hmin;
     GridClass c[MAX_CLASSES];
 };
@@ -133,16 +135,6 @@ __host__ __device__ inline uint32_t morton_spread(uint32_t v) {
 
 __host__ __device__ inline uint32_t morton3(uint32_t x, uint32_t y, uint32_t z) {
     return morton_spread(x) | (morton_spread(y) << 1) | (morton_spread(z) << 2);
-}
-
-// The inverse of spread2: the even bits of v, packed.
-__host__ __device__ inline uint32_t compact2(uint32_t v) {
-    v &= 0x55555555u;
-    v = (v | (v >> 1)) & 0x33333333u;
-    v = (v | (v >> 2)) & 0x0f0f0f0fu;
-    v = (v | (v >> 4)) & 0x00ff00ffu;
-    v = (v | (v >> 8)) & 0x0000ffffu;
-    return v;
 }
 
 __host__ __device__ inline uint32_t spread2(uint32_t v) {
@@ -273,15 +265,13 @@ void launch_scatter_planes(const Launch& l, const double* src, int nc, double* c
                            size_t n);
 void launch_gather_planes(const Launch& l, double* dst, int nc, double* const* planes, const uint32_t* slot_of,
                           size_t n);
-// Cell keys and the identity permutation; also clears the first `clear` words of `range` (the row
-// ranges that launch_cell_first fills).
-void launch_cell_keys(const Launch& l, DevState s, Grid g, uint32_t* keys, uint32_t* idx, uint32_t* range,
-                      size_t clear, size_t n);
 void launch_clear_u32(const Launch& l, uint32_t* p, size_t count, uint32_t value);
-// first[cell] = the first sorted position whose cell index is >= cell, for every cell (x, y, z) of a
-// row (y < dim_y, z < dim_z) with x in [0, dim_x]; row_range (2 per row) is scratch.
-void launch_cell_first(const Launch& l, const uint32_t* keys, Grid g, uint32_t* row_range, uint32_t* first,
-                       size_t rows, size_t n);
+// The particles ordered by cell (order[], ties by slot), and first[cell] = the first sorted position whose cell
+// index is >= cell, for every cell (x, y, z) of a row (y < dim_y, z < dim_z) with x in [0, dim_x].  row_count and
+// row_start: row_slots(g.slots) words, the counts zero (and zero again afterwards); where, bucket: n entries.
+size_t row_slots(uint32_t slots);
+void launch_cell_sort(const Launch& l, DevState s, Grid g, uint32_t* row_count, uint32_t* row_start, uint2* where,
+                      uint2* bucket, uint32_t* order, uint32_t* first, size_t rows, size_t n);
 void launch_pack(const Launch& l, DevState s, Params prm, const uint32_t* order, PairRec* rec, double4* pos,
                  float4* posf, Screen sc, uint32_t* group, size_t n);
 // Neighbour lists are row-major: list[k * kmax + c], kmax a multiple of 4.
@@ -328,12 +318,6 @@ void launch_stream_copy(hipStream_t stream, const void* a, void* b, size_t bytes
 // last 12 doubles.
 size_t integrals_scratch_doubles(size_t n);
 void launch_integrals(const Launch& l, DevState s, double* scratch, size_t n);
-// Temporary storage of the radix sort of n pairs by the low key_bits bits (the algorithm, and with it
-// the storage, depends on both).
-size_t sort_pairs_temp_bytes(size_t n, int key_bits);
-hipError_t sort_pairs(const Launch& l, void* temp, size_t temp_bytes, const uint32_t* keys_in, uint32_t* keys_out,
-                      const uint32_t* vals_in, uint32_t* vals_out, size_t n, int key_bits);
-
 // ---- batched stepping: one launch per stage for every member of an ensemble -----------------------------
 // What the kernels of one predictor-corrector step read for one member of a batch (in device memory, one
 // entry per member).  Every batched kernel runs the same per-particle code as the single-run kernel,

@@ -256,15 +256,6 @@ __device__ __forceinline__ uint32_t cell_key_of(const DevState& s, const Grid& g
     return g.c[cls].base + row_key(uint32_t(c[0]), uint32_t(c[1]), uint32_t(c[2]), g.c[cls].bits);
 }
 
-__global__ void __launch_bounds__(BLOCK) k_cell_keys(DevState s, Grid g, uint32_t* keys, uint32_t* idx,
-                                                     uint32_t* range, size_t clear, size_t n) {
-    const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    for (size_t t = i; t < clear; t += size_t(gridDim.x) * blockDim.x) range[t] = 0u;
-    if (i >= n) return;
-    keys[i] = cell_key_of(s, g, i);
-    idx[i] = uint32_t(i);
-}
-
 __global__ void __launch_bounds__(BLOCK) k_fill_u32(uint32_t* p, size_t count, uint32_t value) {
     for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < count; i += size_t(gridDim.x) * blockDim.x) {
         p[i] = value;
@@ -316,71 +307,236 @@ __device__ __forceinline__ void row_range_at(const uint32_t* __restrict__ keys, 
     range[2 * q + 1] = first_at_least(keys, g, row + (1u << G.bits), 0u, n);
 }
 
-// Row number (as row_of numbers them) of a cell key, from its class and the (y, z) of its Morton row key;
-// *cls = the class.
-__device__ __forceinline__ uint32_t row_index_of(const Grid& g, uint32_t key, int* cls) {
-    uint32_t off = 0, q = 0;
-    for (int c = 0; c < g.nclass; ++c) {
-        const GridClass& G = g.c[c];
-        if (G.empty) continue;
-        if (key >= G.base) {
-            const uint32_t m = (key - G.base) >> G.bits;
-            q = off + compact2(m >> 1) * uint32_t(G.dim[1]) + compact2(m);
-            *cls = c;
+// ---- sort by cell and cell table ------------------------------------------------------------------------
+// The order of the particles by cell and the cell table, by rows of cells: a row (slot0(class) + Morton(y, z), the
+// sort key without x) is a bucket, and a row's particles are ordered by (x, particle) on their own.  Four launches
+// -- count, scan, scatter, order -- whatever the particle count, where a radix sort of the keys took 3 passes over
+// them (onesweep, 84 us at 1M particles) or about ten merge launches (below 1M: 120 us at 559k, 40 us at 43k),
+// and two more kernels built the table (30 us at 1M).  Measured here: 12 + 8 + 6 + 14 us at 1M, 20 us in all up to
+// 170k particles (launch latency).
+// The buckets are filled with atomics, in any order; the order within a row does not depend on it.
+
+// Counts the particles of every row: where[i] = (row << 8 | x, rank in the row).  One atomic per row and wavefront.
+__global__ void __launch_bounds__(BLOCK) k_row_count(DevState s, Grid g, uint32_t* __restrict__ row_count,
+                                                     uint2* __restrict__ where, size_t n) {
+    const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    const bool valid = i < n;
+    const uint32_t lane = threadIdx.x & 63u;
+    uint32_t row = 0xffffffffu, x = 0;
+    if (valid) {
+        const int cls = h_class(s.d[H][i], g.hmin, g.nclass);
+        int c[3];
+        cell_of(g.c[cls], s.d[X][i], s.d[Y][i], s.d[Z][i], c);
+        row = g.c[cls].slot0 + (spread2(uint32_t(c[1])) | (spread2(uint32_t(c[2])) << 1));
+        x = uint32_t(c[0]);
+    }
+    // the lanes of one row: its first lane adds their number, each gets its rank among them
+    uint32_t leader = lane, before = 0, total = 0;
+    for (unsigned long long open = __ballot(valid); open != 0ull;) {
+        const int l = __builtin_ctzll(open);
+        const unsigned long long same = __ballot(row == uint32_t(__builtin_amdgcn_readlane(row, l))) & open;
+        if ((same >> lane) & 1ull) {
+            leader = uint32_t(l);
+            before = uint32_t(__popcll(same & ((1ull << lane) - 1ull)));
+            total = uint32_t(__popcll(same));
         }
-        off += uint32_t(G.dim[1]) * uint32_t(G.dim[2]);
+        open &= ~same;
     }
-    return q;
+    uint32_t base = 0;
+    if (valid && leader == lane) base = atomicAdd(&row_count[row], total);
+    base = uint32_t(__shfl(int(base), int(leader), 64));
+    if (valid) where[i] = make_uint2((row << 8) | x, base + before);
 }
 
-// The cell table of the rows that hold particles, in one pass over the sorted keys (rows are contiguous
-// runs of them, cells contiguous runs inside a row).  The thread of sorted position k writes
-// first[cell] = k for the cells after the previous particle's cell (from x = 0 when k starts its row)
-// up to its own, and, when k ends its row, first[cell] = k + 1 for the cells after its own up to the
-// row's spare slot x = dim_x; it also records the row's range of sorted positions.  Rows without
-// particles keep the empty range [0, 0) that k_cell_keys left, and k_empty_rows fills their cells.
-__global__ void __launch_bounds__(BLOCK) k_row_cells(const uint32_t* __restrict__ keys, Grid g,
-                                                     uint32_t* __restrict__ range, uint32_t* __restrict__ first,
-                                                     uint32_t n) {
-    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= n) return;
-    int cls = 0, cp = 0, cn = 0;
-    const uint32_t key = keys[k];
-    const uint32_t q = row_index_of(g, key, &cls);
-    const GridClass& G = g.c[cls];
-    // the cell's x in its row (the class's keys start at G.base, which need not be a multiple of 2^bits)
-    const uint32_t xmask = (1u << G.bits) - 1u;
-    const uint32_t x = (key - G.base) & xmask;
-    const uint32_t rowbase = key - x;
-    uint32_t xlo = 0;
-    if (k > 0) {
-        const uint32_t kp = keys[k - 1];
-        if (row_index_of(g, kp, &cp) == q) xlo = ((kp - G.base) & xmask) + 1u;
+// row_start = exclusive prefix sums of the counts (slots + 1 entries).  Block b sums the counts before its tile of
+// SCAN_TILE itself, and scans its tile: no second pass and no waiting for other blocks (53k slots at the 1M impact:
+// 14 blocks, the last reading 230 KB; one block stepping through all of them took 25 us).
+constexpr uint32_t SCAN_BLOCK = 1024, SCAN_TILE = 4 * SCAN_BLOCK;
+__global__ void __launch_bounds__(SCAN_BLOCK) k_row_scan(const uint32_t* __restrict__ row_count,
+                                                         uint32_t* __restrict__ row_start) {
+    __shared__ uint32_t wave_sum[2][SCAN_BLOCK / 64];
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    // the arrays hold whole tiles, the entries past the last row zero
+    const uint4* in = reinterpret_cast<const uint4*>(row_count);
+    const uint32_t tile = blockIdx.x * SCAN_BLOCK;  // in quads
+    uint32_t prior = 0;
+    for (uint32_t t = threadIdx.x; t < tile; t += SCAN_BLOCK) {
+        const uint4 q = in[t];
+        prior += q.x + q.y + q.z + q.w;
     }
-    if (xlo == 0) range[2 * size_t(q)] = k;
-    for (uint32_t c = xlo; c <= x; ++c) first[rowbase + c] = k;
-    const bool last = k + 1 == n || row_index_of(g, keys[k + 1], &cn) != q;
-    if (last) {
-        range[2 * size_t(q) + 1] = k + 1;
-        for (uint32_t c = x + 1; c <= uint32_t(G.dim[0]); ++c) first[rowbase + c] = k + 1;
+    const uint4 c = in[tile + threadIdx.x];
+    const uint32_t sum = c.x + c.y + c.z + c.w;
+    uint32_t incl = sum;
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t u = uint32_t(__shfl_up(int(incl), o, 64));
+        if (lane >= uint32_t(o)) incl += u;
     }
+    for (int o = 32; o > 0; o >>= 1) prior += uint32_t(__shfl_xor(int(prior), o, 64));
+    if (lane == 63u) {
+        wave_sum[0][wave] = incl;
+        wave_sum[1][wave] = prior;
+    }
+    __syncthreads();
+    uint32_t run = incl - sum;
+    for (uint32_t w = 0; w < SCAN_BLOCK / 64; ++w) run += wave_sum[1][w] + (w < wave ? wave_sum[0][w] : 0u);
+    uint4 o;
+    o.x = run;
+    o.y = o.x + c.x;
+    o.z = o.y + c.y;
+    o.w = o.z + c.z;
+    reinterpret_cast<uint4*>(row_start)[tile + threadIdx.x] = o;
 }
 
-// The cells of the rows without particles (empty range): equal entries, so that every x-run of them
-// reads as an empty range of sorted positions.
-__global__ void __launch_bounds__(BLOCK) k_empty_rows(Grid g, const uint32_t* __restrict__ range,
-                                                      uint32_t* __restrict__ first, size_t rows, int xslots) {
-    const size_t t = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    const size_t q = t / size_t(xslots);
-    const uint32_t x = uint32_t(t % size_t(xslots));
-    if (q >= rows) return;
-    if (range[2 * q] != range[2 * q + 1]) return;
-    int cls;
-    uint32_t cy, cz;
-    if (!row_of(g, q, cls, cy, cz)) return;
+// bucket[row_start + rank] = (particle, x): x in the high word, so that the 64-bit values order by (x, particle).
+// The counts go back to zero for the next search.
+__global__ void __launch_bounds__(BLOCK) k_row_scatter(const uint2* __restrict__ where,
+                                                       const uint32_t* __restrict__ row_start,
+                                                       uint32_t* __restrict__ row_count, uint32_t slots,
+                                                       uint2* __restrict__ bucket, size_t n) {
+    const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    for (size_t t = i; t < slots; t += size_t(gridDim.x) * blockDim.x) row_count[t] = 0u;
+    if (i >= n) return;
+    const uint2 w = where[i];
+    bucket[row_start[w.x >> 8] + w.y] = make_uint2(uint32_t(i), w.x & 255u);
+}
+
+// Ascending sort of v[0..m) by the block: bitonic with every comparator directed upwards (the first step of each
+// merge mirrors), so that the missing partners past m act as largest values.
+__device__ __forceinline__ void block_sort(unsigned long long* v, uint32_t m) {
+    for (uint32_t size = 2; size < 2 * m; size <<= 1) {
+        for (uint32_t step = size; step > 1; step >>= 1) {
+            __syncthreads();
+            const uint32_t half = step >> 1;
+            for (uint32_t p = threadIdx.x; p < m; p += blockDim.x) {
+                const uint32_t q = step == size ? p ^ (size - 1u) : p ^ half;
+                if (q > p && q < m) {
+                    const unsigned long long a = v[p], b = v[q];
+                    if (b < a) {
+                        v[p] = b;
+                        v[q] = a;
+                    }
+                }
+            }
+        }
+    }
+    __syncthreads();
+}
+
+// One wavefront per row (y < dim_y, z < dim_z of every class): its particles ordered by (x, particle) into order[],
+// and first[cell] = the first sorted position whose cell is >= cell, for x in [0, dim_x].  Up to ROW_WAVE
+// particles in LDS: counted by x, placed, and each ranked among those of its own cell (0.6 per cell at the
+// impact).  The block sorts longer rows together, in LDS up to ROW_BLOCK particles (rows of 1M particles' cells
+// hold ~64; far outliers that stretch the grid to its 250 cells make them longer).
+constexpr uint32_t ROW_WAVE = 512, ROW_BLOCK = 2048;
+struct RowStage {
+    uint32_t start[256];      // counts by x, then their exclusive prefix sums
+    uint32_t idx[ROW_WAVE];   // particles placed by cell
+};
+__global__ void __launch_bounds__(BLOCK) k_row_order(Grid g, const uint32_t* __restrict__ row_start,
+                                                     uint2* __restrict__ bucket, uint32_t* __restrict__ order,
+                                                     uint32_t* __restrict__ first, size_t rows) {
+    constexpr int WAVES = BLOCK / 64;
+    union Lds {
+        RowStage stage[WAVES];
+        unsigned long long key[ROW_BLOCK];
+    };
+    __shared__ Lds lds;
+    __shared__ uint32_t long_row[WAVES][4];  // first position, particles, cell base and dim_x of a long row
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63u;
+    const size_t q = size_t(blockIdx.x) * WAVES + wave;
+    int cls = 0;
+    uint32_t cy = 0, cz = 0;
+    const bool valid = q < rows && row_of(g, q, cls, cy, cz);
     const GridClass& G = g.c[cls];
-    if (x > uint32_t(G.dim[0])) return;
-    first[G.base + row_key(x, cy, cz, G.bits)] = 0u;
+    const uint32_t mor = spread2(cy) | (spread2(cz) << 1);
+    const uint32_t dimx = uint32_t(G.dim[0]), cell0 = G.base + (mor << G.bits);
+    uint32_t s0 = 0, cnt = 0;
+    if (valid) {
+        s0 = row_start[G.slot0 + mor];
+        cnt = row_start[G.slot0 + mor + 1u] - s0;
+    }
+    s0 = __builtin_amdgcn_readfirstlane(s0);
+    cnt = __builtin_amdgcn_readfirstlane(cnt);
+    if (lane == 0) long_row[wave][1] = 0u;
+    if (valid && cnt == 0) {
+        for (uint32_t x = lane; x <= dimx; x += 64u) first[cell0 + x] = s0;
+    } else if (valid && cnt <= ROW_WAVE) {
+        RowStage& S = lds.stage[wave];
+        reinterpret_cast<uint4*>(S.start)[lane] = make_uint4(0u, 0u, 0u, 0u);
+        wave_sync();
+        uint2 e[ROW_WAVE / 64];
+        uint32_t rank[ROW_WAVE / 64];
+#pragma unroll
+        for (uint32_t k = 0; k < ROW_WAVE / 64; ++k) {
+            if (64u * k >= cnt) break;
+            if (64u * k + lane < cnt) {
+                e[k] = bucket[s0 + 64u * k + lane];
+                rank[k] = atomicAdd(&S.start[e[k].y], 1u);
+            }
+        }
+        wave_sync();
+        const uint4 c = reinterpret_cast<const uint4*>(S.start)[lane];
+        const uint32_t sum = c.x + c.y + c.z + c.w;
+        uint32_t incl = sum;
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t u = uint32_t(__shfl_up(int(incl), o, 64));
+            if (lane >= uint32_t(o)) incl += u;
+        }
+        uint4 st;
+        st.x = incl - sum;
+        st.y = st.x + c.x;
+        st.z = st.y + c.y;
+        st.w = st.z + c.z;
+        reinterpret_cast<uint4*>(S.start)[lane] = st;
+        wave_sync();
+        for (uint32_t x = lane; x <= dimx; x += 64u) first[cell0 + x] = s0 + S.start[x];
+#pragma unroll
+        for (uint32_t k = 0; k < ROW_WAVE / 64; ++k) {
+            if (64u * k >= cnt) break;
+            if (64u * k + lane < cnt) S.idx[S.start[e[k].y] + rank[k]] = e[k].x;
+        }
+        wave_sync();
+#pragma unroll
+        for (uint32_t k = 0; k < ROW_WAVE / 64; ++k) {
+            if (64u * k >= cnt) break;
+            if (64u * k + lane < cnt) {
+                const uint32_t a = S.start[e[k].y], b = S.start[e[k].y + 1u];  // x <= 250: x + 1 is an entry
+                uint32_t r = a;
+                for (uint32_t j = a; j < b; ++j) r += S.idx[j] < e[k].x ? 1u : 0u;
+                order[s0 + r] = e[k].x;
+            }
+        }
+    } else if (valid && lane == 0) {
+        long_row[wave][0] = s0;
+        long_row[wave][1] = cnt;
+        long_row[wave][2] = cell0;
+        long_row[wave][3] = dimx;
+    }
+    __syncthreads();
+    for (int w = 0; w < WAVES; ++w) {
+        const uint32_t f = long_row[w][0], m = long_row[w][1];
+        if (m == 0) continue;
+        unsigned long long* v = reinterpret_cast<unsigned long long*>(bucket + f);
+        if (m <= ROW_BLOCK) {
+            for (uint32_t p = threadIdx.x; p < m; p += BLOCK) lds.key[p] = v[p];
+            v = lds.key;
+        }
+        block_sort(v, m);
+        for (uint32_t p = threadIdx.x; p < m; p += BLOCK) order[f + p] = uint32_t(v[p]);
+        for (uint32_t x = threadIdx.x; x <= long_row[w][3]; x += BLOCK) {
+            uint32_t lo = 0, hi = m;
+            while (lo < hi) {
+                const uint32_t mid = lo + ((hi - lo) >> 1);
+                if (uint32_t(v[mid] >> 32) < x) {
+                    lo = mid + 1;
+                } else {
+                    hi = mid;
+                }
+            }
+            first[long_row[w][2] + x] = f + lo;
+        }
+        __syncthreads();
+    }
 }
 
 // One thread per cell x in [0, dim_x] of a row: the binary search runs inside the row's own range.
@@ -1989,10 +2145,17 @@ void launch_bounds_reduce(const Launch& l, DevState s, unsigned long long* acc, 
     k_bounds<<<g, BLOCK, 0, l.stream>>>(s, acc, n);
 }
 
-void launch_cell_keys(const Launch& l, DevState s, Grid g, uint32_t* keys, uint32_t* idx, uint32_t* range,
-                      size_t clear, size_t n) {
-    if (!n) return;
-    k_cell_keys<<<grid_for(n), BLOCK, 0, l.stream>>>(s, g, keys, idx, range, clear, n);
+// Whole scan tiles with an entry past the last row.
+size_t row_slots(uint32_t slots) { return (size_t(slots) / SCAN_TILE + 1) * SCAN_TILE; }
+
+void launch_cell_sort(const Launch& l, DevState s, Grid g, uint32_t* row_count, uint32_t* row_start, uint2* where,
+                      uint2* bucket, uint32_t* order, uint32_t* first, size_t rows, size_t n) {
+    // without particles nothing reads the table
+    if (!rows || !n) return;
+    k_row_count<<<grid_for(n), BLOCK, 0, l.stream>>>(s, g, row_count, where, n);
+    k_row_scan<<<unsigned(row_slots(g.slots) / SCAN_TILE), SCAN_BLOCK, 0, l.stream>>>(row_count, row_start);
+    k_row_scatter<<<grid_for(n), BLOCK, 0, l.stream>>>(where, row_start, row_count, g.slots, bucket, n);
+    k_row_order<<<grid_for(rows, BLOCK / 64), BLOCK, 0, l.stream>>>(g, row_start, bucket, order, first, rows);
 }
 
 void launch_clear_u32(const Launch& l, uint32_t* p, size_t count, uint32_t value) {
@@ -2000,18 +2163,6 @@ void launch_clear_u32(const Launch& l, uint32_t* p, size_t count, uint32_t value
     unsigned g = grid_for(count);
     g = g > 4096 ? 4096 : g;
     k_fill_u32<<<g, BLOCK, 0, l.stream>>>(p, count, value);
-}
-
-void launch_cell_first(const Launch& l, const uint32_t* keys, Grid g, uint32_t* row_range, uint32_t* first,
-                       size_t rows, size_t n) {
-    // without particles nothing reads the tables (and the row ranges were not cleared)
-    if (!rows || !n) return;
-    int xslots = 1;
-    for (int c = 0; c < g.nclass; ++c) {
-        if (!g.c[c].empty) xslots = xslots > g.c[c].dim[0] + 1 ? xslots : g.c[c].dim[0] + 1;
-    }
-    k_row_cells<<<grid_for(n), BLOCK, 0, l.stream>>>(keys, g, row_range, first, uint32_t(n));
-    k_empty_rows<<<grid_for(rows * size_t(xslots)), BLOCK, 0, l.stream>>>(g, row_range, first, rows, xslots);
 }
 
 size_t bounds_partials(size_t n) { return size_t(grid_for(n)) * BOUND_VALUES; }
@@ -2398,31 +2549,6 @@ hipError_t sort_pairs64(const Launch& l, void* temp, size_t temp_bytes, const ui
     if (!n) return hipSuccess;
     return rocprim::radix_sort_pairs(temp, temp_bytes, keys_in, keys_out, vals_in, vals_out, n, 0u,
                                      unsigned(key_bits), l.stream);
-}
-
-// Radix sort of the cell keys: rocPRIM's onesweep with launch shapes measured at the 1M impact (24-bit
-// keys): 1024 threads x 4 items per block 84 us per sort, against 119 us for its default of 1024 x 16
-// (65 blocks per pass on 256 CUs); 512 x 8: 95 us, 256 x 8: 124 us.  12-bit digits exceed the LDS.
-constexpr unsigned SORT_BLOCK = 1024, SORT_ITEMS = 4, SORT_BITS = 8;
-using SortConfig = rocprim::radix_sort_config<
-    rocprim::default_config, rocprim::default_config,
-    rocprim::radix_sort_onesweep_config<rocprim::kernel_config<SORT_BLOCK, SORT_ITEMS>,
-                                        rocprim::kernel_config<SORT_BLOCK, SORT_ITEMS>, SORT_BITS,
-                                        rocprim::block_radix_rank_algorithm::match>>;
-
-size_t sort_pairs_temp_bytes(size_t n, int key_bits) {
-    size_t bytes = 0;
-    (void)rocprim::radix_sort_pairs<SortConfig>(nullptr, bytes, (const uint32_t*)nullptr, (uint32_t*)nullptr,
-                                                (const uint32_t*)nullptr, (uint32_t*)nullptr, n, 0u,
-                                                unsigned(key_bits));
-    return bytes;
-}
-
-hipError_t sort_pairs(const Launch& l, void* temp, size_t temp_bytes, const uint32_t* keys_in, uint32_t* keys_out,
-                      const uint32_t* vals_in, uint32_t* vals_out, size_t n, int key_bits) {
-    if (!n) return hipSuccess;
-    return rocprim::radix_sort_pairs<SortConfig>(temp, temp_bytes, keys_in, keys_out, vals_in, vals_out, n, 0u,
-                                                 unsigned(key_bits), l.stream);
 }
 
 }  // namespace osph
