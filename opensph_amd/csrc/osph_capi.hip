@@ -800,20 +800,32 @@ void launch_pair_sums(osph_ctx* c, const FuseArgs* fuse = nullptr) {
 int integrate(osph_ctx* c, osph_stats* stats) {
     const size_t n = c->n;
     Launch l = L(c);
-    if (int e = build_neighbors(c, 1)) return e;
-    if (int e = gravity_eval(c)) return e;
-    launch_pair_sums(c);
-    timed(c, "finalize", [&] { launch_finalize(l, c->s, c->mats_dev, c->prm, n); });
-    if (stats) {
-        std::vector<uint32_t> cnt(n);
-        if (n) HIPCHK(c, hipMemcpyAsync(cnt.data(), c->s.u[NCNT], n * sizeof(uint32_t), hipMemcpyDeviceToHost,
-                                         c->stream));
+    c->neighbors_valid = false;
+    if (n) {
+        if (int e = search_grid(c, 1, 0.0)) return e;
+        if (int e = gravity_eval(c)) return e;
+    }
+    // the whole evaluation is queued before the list overflow flag is read; after an overflow the lists grow and
+    // the lists, the sums and the finalize, which assign everything they write, run again
+    for (int attempt = 0; n; ++attempt) {
+        if (int e = launch_lists(c)) return e;
+        launch_pair_sums(c);
+        timed(c, "finalize", [&] { launch_finalize(l, c->s, c->mats_dev, c->prm, n); });
+        if (stats) timed(c, "count_stats", [&] { launch_count_stats(l, c->s.u[NCNT], c->small + SMALL_COUNTS, n); });
+        HIPCHK(c, hipMemcpyAsync(c->small_host + SMALL_OVERFLOW, c->small + SMALL_OVERFLOW,
+                                 4 * sizeof(unsigned long long), hipMemcpyDeviceToHost, c->stream));
         if (int e = sync_check(c)) return e;
-        stats->neighbors_min = n ? *std::min_element(cnt.begin(), cnt.end()) : 0;
-        stats->neighbors_max = n ? *std::max_element(cnt.begin(), cnt.end()) : 0;
-        double sum = 0.0;
-        for (uint32_t v : cnt) sum += v;
-        stats->neighbors_mean = n ? sum / double(n) : 0.0;
+        if (!overflowed(c)) break;
+        if (attempt == 3) return c->fail(OSPH_ERR_STATE, "neighbour list did not fit after growing");
+        if (int e = grow_lists(c)) return e;
+        launch_clear_u32(l, reinterpret_cast<uint32_t*>(c->small + SMALL_COUNTS), 6, 0u);
+    }
+    c->neighbors_valid = true;
+    if (stats) {
+        const unsigned long long* v = c->small_host + SMALL_COUNTS;
+        stats->neighbors_min = n ? ~uint32_t(v[0]) : 0;
+        stats->neighbors_max = n ? uint32_t(v[1]) : 0;
+        stats->neighbors_mean = n ? double(v[2]) / double(n) : 0.0;
     }
     return OSPH_OK;
 }
@@ -950,6 +962,7 @@ int osph_create(osph_ctx** out, const osph_config* cfg, const osph_material* mat
     *out = nullptr;
     if (cfg->precision != OSPH_PRECISION_FP64 && cfg->precision != OSPH_PRECISION_MIXED) return OSPH_ERR_ARG;
     osph_ctx* c = new osph_ctx();
+    transfer_attach();
     c->cfg = *cfg;
     c->prm = make_params(*cfg);
     c->mats.assign(materials, materials + n_materials);
@@ -1005,6 +1018,7 @@ void osph_destroy(osph_ctx* c) {
     if (c->small_host) (void)hipHostFree(c->small_host);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
+    transfer_detach();
 }
 
 const char* osph_last_error(const osph_ctx* c) {
@@ -1097,11 +1111,14 @@ int osph_get_quantity(osph_ctx* c, int q, int order, void* host, size_t stride) 
     if (n == 0) return OSPH_OK;
     if (!host) return c->fail(OSPH_ERR_ARG, "null host buffer");
     if (int e = ensure_staging(c, n * stride)) return e;
-    if ((n * stride) % 4 == 0) launch_clear_u32(L(c), reinterpret_cast<uint32_t*>(c->staging), n * stride / 4, 0u);
+    const bool gaps = stride != size_t(d.ncomp) * size_t(d.elem);  // bytes of an element that no component fills
+    if (gaps && (n * stride) % 4 == 0) {
+        launch_clear_u32(L(c), reinterpret_cast<uint32_t*>(c->staging), n * stride / 4, 0u);
+    }
     void* src[8];
     plane_ptrs(c, d, src);
     launch_planes_to_stage(L(c), c->staging, stride, d.ncomp, d.off, d.elem, src, c->slot_of, n);
-    HIPCHK(c, hipMemcpyAsync(host, c->staging, n * stride, hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, copy_to_host(c->stream, host, c->staging, n * stride));
     return sync_check(c);
 }
 
@@ -1148,8 +1165,7 @@ int osph_get_pairs(osph_ctx* c, uint32_t* pi, uint32_t* pj, size_t cap, size_t* 
 
 int osph_integrate(osph_ctx* c, osph_stats* stats) {
     if (!c) return OSPH_ERR_ARG;
-    if (int e = integrate(c, stats)) return e;
-    return sync_check(c);
+    return integrate(c, stats);
 }
 
 int osph_integrals(osph_ctx* c, double out[OSPH_INTEGRALS]) {
@@ -2180,7 +2196,7 @@ int osph_adjoint_backward(osph_ctx* c, const double* seed_r, const double* seed_
     auto out = [&](double* host, int nc, double* const* planes) -> int {
         if (!host || !n) return OSPH_OK;
         launch_gather_planes(l, io.p, nc, planes, c->slot_of, n);
-        HIPCHK(c, hipMemcpyAsync(host, io.p, n * nc * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(c, copy_to_host(c->stream, host, io.p, n * nc * sizeof(double)));
         return sync_check(c);
     };
     if (int e = out(grad_r, 3, lp + LRX_)) return e;

@@ -21,6 +21,7 @@
 #include "osph_device.h"
 #include "osph_gpu.h"
 #include "osph_gravity.h"
+#include "osph_transfer.h"
 
 #include <hipcub/hipcub.hpp>
 
@@ -2271,7 +2272,7 @@ int download_vectors(osph_gravity* g, double* host, size_t stride, int plane0, i
     }
     k_stage<<<grid_for(n), BLOCK, 0, g->stream>>>(g->staging, stride, ncomp, g->s, plane0,
                                                   g->identity ? nullptr : g->perm, n);
-    GCHK(g, hipMemcpyAsync(host, g->staging, n * stride, hipMemcpyDeviceToHost, g->stream));
+    GCHK(g, copy_to_host(g->stream, host, g->staging, n * stride));
     return sync(g);
 }
 
@@ -2338,6 +2339,7 @@ int osph_gravity_create(osph_gravity** out, const osph_gravity_config* cfg) {
         if (cfg->leaf_size < 1 || cfg->leaf_size > 64) return ERR_ARG;
     }
     osph_gravity* g = new osph_gravity();
+    transfer_attach();
     g->cfg = *cfg;
     auto bail = [&](int code) {
         osph_gravity_destroy(g);
@@ -2377,6 +2379,7 @@ void osph_gravity_destroy(osph_gravity* g) {
     if (g->small_host) (void)hipHostFree(g->small_host);
     if (g->stream) (void)hipStreamDestroy(g->stream);
     delete g;
+    transfer_detach();
 }
 
 const char* osph_gravity_last_error(const osph_gravity* g) { return g ? g->err.c_str() : "null context"; }

@@ -7,6 +7,7 @@
 #include <cstdint>
 
 #include "osph_gpu.h"
+#include "osph_transfer.h"
 
 namespace osph {
 
@@ -215,11 +216,13 @@ struct Launch {
 
 // Accumulators of one step (64 words of device memory): SMALL_BOUNDS + 0..7 global bounds,
 // SMALL_CRITERIA + 0..3 the criterion minima, SMALL_OVERFLOW the list overflow flag (low 32 bits),
+// SMALL_COUNTS + 0..2 the neighbour count statistics,
 // SMALL_CLASSES + CLASS_STRIDE * c + 0..8 the bounds of class c, SMALL_VEL + 0..5 the velocity bounds
 // (min x, y, z, max x, y, z; mixed precision only).
 constexpr int SMALL_BOUNDS = 0;
 constexpr int SMALL_CRITERIA = 8;
 constexpr int SMALL_OVERFLOW = 12;
+constexpr int SMALL_COUNTS = 13;  // 3 words (launch_count_stats)
 constexpr int SMALL_CLASSES = 16;
 constexpr int CLASS_STRIDE = 10;
 constexpr int SMALL_VEL = 56;
@@ -241,6 +244,10 @@ void launch_advance(const Launch& l, DevState s, const osph_material* mats, Para
 size_t bounds_partials(size_t n);
 // Values of the per-block partial bounds (partials per block).
 size_t bounds_values();
+
+// The smallest and largest neighbour count and their sum into stats[0..2], for osph_stats (stats[0] holds the
+// complement of the smallest; all start at zero).
+void launch_count_stats(const Launch& l, const uint32_t* counts, unsigned long long* stats, size_t n);
 
 // ---- adjoint (osph_adjoint.hip) -----------------------------------------------------------------------
 // Materials whose Tillotson parameters (a, b, A) get a gradient.

@@ -1988,6 +1988,29 @@ __global__ void __launch_bounds__(BLOCK) k_criteria(DevState s, const osph_mater
     reduce_criteria(v, mins);
 }
 
+// Statistics of the neighbour counts (SymmetricSolver.cpp:172-179): a bounded grid, so that few blocks meet in the
+// three words.
+constexpr unsigned STATS_BLOCKS = 128;
+__global__ void __launch_bounds__(BLOCK) k_count_stats(const uint32_t* __restrict__ counts,
+                                                       unsigned long long* __restrict__ stats, size_t n) {
+    unsigned long long inv = 0ull, mx = 0ull, sum = 0ull;
+    for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += size_t(gridDim.x) * blockDim.x) {
+        const uint32_t c = counts[i];
+        const unsigned long long comp = uint32_t(~c);
+        inv = comp > inv ? comp : inv;
+        mx = c > mx ? c : mx;
+        sum += c;
+    }
+    inv = wave_max(inv);
+    mx = wave_max(mx);
+    for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
+    if ((threadIdx.x & 63u) == 0) {
+        atomicMax(&stats[0], inv);
+        atomicMax(&stats[1], mx);
+        atomicAdd(&stats[2], sum);
+    }
+}
+
 struct StageDesc {
     int ncomp;
     int elem;
@@ -2279,6 +2302,12 @@ void launch_finalize_correct(const Launch& l, DevState s, const osph_material* m
                              unsigned long long* mins, const uint32_t* overflow, size_t n) {
     if (!n) return;
     k_finalize_correct<<<grid_for(n), BLOCK, 0, l.stream>>>(s, mats, prm, dt, mins, overflow, n);
+}
+
+void launch_count_stats(const Launch& l, const uint32_t* counts, unsigned long long* stats, size_t n) {
+    if (!n) return;
+    const unsigned g = grid_for(n);
+    k_count_stats<<<g < STATS_BLOCKS ? g : STATS_BLOCKS, BLOCK, 0, l.stream>>>(counts, stats, n);
 }
 
 void launch_criteria(const Launch& l, DevState s, const osph_material* mats, Params prm, unsigned long long* mins,
