@@ -1524,36 +1524,149 @@ __global__ void __launch_bounds__(BLOCK) k_points(Tree t, const double4* __restr
     acc[q] = make_double4(a[0], a[1], a[2], 0.0);
 }
 
-// BruteForceGravity::evalImpl (BruteForceGravity.h:112-131) for targets tg[0..nt): sources in storage
-// order, staged through LDS; the per-target sum runs in source order like the reference's two loops.
-__global__ void __launch_bounds__(BLOCK) k_direct(Planes s, size_t n, const uint32_t* __restrict__ tg, size_t nt,
-                                                  const double* __restrict__ grads, double G, double4* __restrict__ out) {
+// The term of one source in the direct sum, with the bits of add_pair<true> on a sum of zero.  That form takes 1 / h, a
+// square root and three quotients (about 90 instructions).  Most pairs are far outside the softening and of ordinary
+// size, and take a form with the same roundings in about 45: the branch decided on |r|^2 against 4 h^2 with room for
+// every rounding of the quotient it replaces, the square root and the quotients by Goldschmidt's iteration from one
+// reciprocal square root, each corrected by its exact remainder (Markstein 1990).  False where the bounds that keep
+// the remainders exact do not hold (also for NaN); t is then not to be used.
+template <bool M4>
+__device__ __forceinline__ bool far_term(double rx, double ry, double rz, double h, double m, double t[3]) {
 #pragma clang fp contract(off)
-    __shared__ double4 sp[BLOCK];
-    __shared__ double sm[BLOCK];
-    const size_t q = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    const bool active = q < nt;
-    const uint32_t i = active ? tg[q] : 0u;
+    const double d2 = rx * rx + ry * ry + rz * rz;
+    const double least = fmin(fmin(fabs(rx), fabs(ry)), fabs(rz));
+    const double y = __builtin_amdgcn_rsq(d2);
+    double l = d2 * y, u = 0.5 * y;
+    const double e = fma(-u, l, 0.5);
+    l = fma(l, e, l);
+    u = fma(u, e, u);
+    l = fma(fma(-l, l, d2), u, l);
+    l = fma(fma(-l, l, d2), u, l);
+    const double l3 = l * l * l;
+    const double u2 = u + u;
+    double il3 = u2 * u2 * u2;
+    il3 = fma(fma(-l3, il3, 1.0), il3, il3);
+    const double qx = rx * il3, qy = ry * il3, qz = rz * il3;
+    t[0] = m * fma(fma(-l3, qx, rx), il3, qx);
+    t[1] = m * fma(fma(-l3, qy, ry), il3, qy);
+    t[2] = m * fma(fma(-l3, qz, rz), il3, qz);
+    // (bitwise: no branches between the conditions)
+    return bool(int(d2 >= 1.e-100) & int(d2 <= 1.e100) & int(least >= 1.e-140) &
+                int(!M4 || d2 > (4.0 * (1.0 + 1.e-12)) * (h * h)));
+}
+
+// BruteForceGravity::evalImpl (BruteForceGravity.h:112-131) for targets tg[0..nt): sources in storage order, each
+// target's sum in source order like the reference's two loops.  One lane per target left most of the chip idle up to
+// some 100k targets, so DIRECT_WAVES wavefronts share DIRECT_TARGETS targets: each puts the terms of DIRECT_SUB * 4
+// sources of a chunk into LDS, and one lane per target and component adds the chunk in order while the others are at
+// the next one (two buffers, one barrier per chunk; that chain has the higher wave priority).  A term of zero (the
+// target itself, sources past the end) leaves a sum that started at +0 as it is.  Issue-bound, 75 instructions a
+// term; few targets per block keep the last wave of blocks short.  n targets and sources, M4, before -> now:
+// 500 174 -> 13 us, 3000 1039 -> 51, 12345 4245 -> 534, 30000 10355 -> 2472 (364 G terms/s).  32 targets per block:
+// 17, 81, 539, 2413 us; 64: 26, 131, 547, 2508; 8 sources a wavefront per chunk: 735 us at 12345; sources gathered from
+// the planes instead of LDS: 656; the general form for every pair: 612.
+constexpr int DIRECT_TARGETS = 16, DIRECT_WAVES = 8, DIRECT_SUB = 2;
+
+template <bool M4>
+__global__ void __launch_bounds__(DIRECT_WAVES * 64) k_direct(Planes s, size_t n, const uint32_t* __restrict__ tg,
+                                                               size_t nt, const double* __restrict__ grads, double G,
+                                                               double4* __restrict__ out) {
+#pragma clang fp contract(off)
+    constexpr int T = DIRECT_TARGETS, W = DIRECT_WAVES, SUB = DIRECT_SUB;
+    constexpr uint32_t PER = 64 / T;            // sources of a wavefront's instruction
+    constexpr uint32_t CHUNK = W * SUB * PER;   // sources of a chunk
+    constexpr uint32_t PLANES = M4 ? 5 : 4;
+    constexpr uint32_t LOADS = (PLANES * CHUNK + W * 64 - 1) / (W * 64);
+    static_assert(3 * T <= W * 64 && T <= W * 64, "a thread for every target and component");
+    __shared__ double term[2][CHUNK][3 * T];           // 48 KB
+    __shared__ __align__(16) double src[2][CHUNK][6];  // x y z m h
+    const uint32_t q = threadIdx.x % T, k0 = threadIdx.x / 64 * (SUB * PER) + threadIdx.x % 64 / T;
+    const size_t qt = size_t(blockIdx.x) * T + q;
+    const uint32_t i = tg[qt < nt ? qt : nt - 1];
     const double xi = s.d[GX][i], yi = s.d[GY][i], zi = s.d[GZ][i], hi = s.d[GH][i];
-    double a[3] = { 0.0, 0.0, 0.0 };
-    for (size_t base = 0; base < n; base += BLOCK) {
-        const size_t j = base + threadIdx.x;
-        if (j < n) {
-            sp[threadIdx.x] = make_double4(s.d[GX][j], s.d[GY][j], s.d[GZ][j], s.d[GH][j]);
-            sm[threadIdx.x] = s.d[GM][j];
-        }
-        __syncthreads();
-        const size_t cnt = n - base < size_t(BLOCK) ? n - base : size_t(BLOCK);
-        if (active) {
-            for (size_t c = 0; c < cnt; ++c) {
-                if (base + c == i) continue;
-                const double4 o = sp[c];
-                add_pair<true>(grads, o.x - xi, o.y - yi, o.z - zi, 0.5 * (o.w + hi), sm[c], a);
-            }
-        }
-        __syncthreads();
+    // the planes of a source in the order of src, and this thread's elements of a chunk
+    const double* lp[LOADS];
+    uint32_t lk[LOADS];
+    for (uint32_t v = 0; v < LOADS; ++v) {
+        const uint32_t e = threadIdx.x + v * (W * 64), c = e / CHUNK;
+        lp[v] = c == 0 ? s.d[GX] : c == 1 ? s.d[GY] : c == 2 ? s.d[GZ] : c == 3 ? s.d[GM] : s.d[GH];
+        lk[v] = e % CHUNK;
     }
-    if (active) out[q] = make_double4(G * a[0], G * a[1], G * a[2], 0.0);
+    auto fetch = [&](size_t base, double (&r)[LOADS]) {
+        for (uint32_t v = 0; v < LOADS; ++v) {
+            const size_t j = base + lk[v];
+            r[v] = lp[v][j < n ? j : n - 1];
+        }
+    };
+    auto place = [&](int buf, const double (&r)[LOADS]) {
+        for (uint32_t v = 0; v < LOADS; ++v) {
+            const uint32_t e = threadIdx.x + v * (W * 64);
+            if (e < PLANES * CHUNK) src[buf][lk[v]][e / CHUNK] = r[v];
+        }
+    };
+    double a = 0.0, next[LOADS];
+    fetch(0, next);
+    place(0, next);
+    __syncthreads();
+    int buf = 0;
+    for (size_t base = 0; base < n; base += CHUNK, buf ^= 1) {
+        const uint32_t left = uint32_t(n - base < CHUNK ? n - base : CHUNK);
+        const uint32_t self = i - uint32_t(base);
+        fetch(base + CHUNK, next);
+        double rx[SUB], ry[SUB], rz[SUB], h[SUB], m[SUB], t[SUB][3];
+        bool far[SUB];
+#pragma unroll
+        for (int v = 0; v < SUB; ++v) {
+            const double* o = src[buf][k0 + v * PER];
+            rx[v] = o[0] - xi;
+            ry[v] = o[1] - yi;
+            rz[v] = o[2] - zi;
+            m[v] = o[3];
+            if (M4) h[v] = 0.5 * (o[4] + hi);
+        }
+#pragma unroll
+        for (int v = 0; v < SUB; ++v) far[v] = far_term<M4>(rx[v], ry[v], rz[v], M4 ? h[v] : 0.0, m[v], t[v]);
+#pragma unroll
+        for (int v = 0; v < SUB; ++v) {
+            const uint32_t k = k0 + v * PER;
+            if (!far[v] || k >= left || k == self) {
+                for (int c = 0; c < 3; ++c) t[v][c] = 0.0;
+                if (k < left && k != self) {
+                    add_pair<true>(M4 ? grads : nullptr, rx[v], ry[v], rz[v], M4 ? h[v] : 0.0, m[v], t[v]);
+                }
+            }
+            for (int c = 0; c < 3; ++c) term[buf][k][c * T + q] = t[v][c];
+        }
+        place(buf ^ 1, next);
+        __syncthreads();
+        if (threadIdx.x < 3 * T) {
+            __builtin_amdgcn_s_setprio(2);  // the chunk's longest chain
+            constexpr uint32_t B = 16;
+            static_assert(CHUNK % B == 0, "whole batches");
+            double now[B];
+#pragma unroll
+            for (uint32_t k = 0; k < B; ++k) now[k] = term[buf][k][threadIdx.x];
+            for (uint32_t b = B; b < CHUNK; b += B) {
+                double then[B];
+#pragma unroll
+                for (uint32_t k = 0; k < B; ++k) then[k] = term[buf][b + k][threadIdx.x];
+#pragma unroll
+                for (uint32_t k = 0; k < B; ++k) a += now[k];
+#pragma unroll
+                for (uint32_t k = 0; k < B; ++k) now[k] = then[k];
+            }
+#pragma unroll
+            for (uint32_t k = 0; k < B; ++k) a += now[k];
+            __builtin_amdgcn_s_setprio(0);
+        }
+    }
+    // the three components of a target to one lane
+    __syncthreads();
+    if (threadIdx.x < 3 * T) term[0][0][threadIdx.x] = a;
+    __syncthreads();
+    if (threadIdx.x < T && qt < nt) {
+        out[qt] = make_double4(G * term[0][0][q], G * term[0][0][T + q], G * term[0][0][2 * T + q], 0.0);
+    }
 }
 
 // BruteForceGravity::evalEnergy (BruteForceGravity.h:103-115): per-particle sums m_i m_j value.
@@ -2214,7 +2327,9 @@ int eval_direct(osph_gravity* g, const uint32_t* tg_dev, size_t nt, double4* out
     if (!nt) return OK;
     const double* grads = g->cfg.kernel == OSPH_GRAVITY_KERNEL_M4 ? g->lut_grads : nullptr;
     timed(g, "direct", [&] {
-        k_direct<<<grid_for(nt), BLOCK, 0, g->stream>>>(g->s, g->n, tg_dev, nt, grads, g->cfg.G, out);
+        const auto kernel = grads ? k_direct<true> : k_direct<false>;
+        kernel<<<unsigned((nt + DIRECT_TARGETS - 1) / DIRECT_TARGETS), DIRECT_WAVES * 64, 0, g->stream>>>(
+            g->s, g->n, tg_dev, nt, grads, g->cfg.G, out);
     });
     return OK;
 }
