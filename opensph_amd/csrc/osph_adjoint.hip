@@ -186,6 +186,14 @@ struct PairGrad {
     double rho_o, rho_q, p_o, p_q, c_o, c_q;
 };
 
+// What both directions of a pair share: with (o, q) exchanged, r, w and G change sign and the rest is the same to
+// the last bit.
+template <typename T>
+struct PairCommon {
+    T r[3], w[3], G[3], K, Kp, wg, C, Pi, mu, den, rhobar, csbar, hbar;
+    bool conv;
+};
+
 // Gradient of L = la . da + ld ddivv + lh dheat, the pair (owner o, other q) contributions to o's
 // acceleration, velocity divergence and AV heating (the forward k_pairs_fp64 terms without stress):
 //   da = m_q (-(p_o/rho_o^2 + p_q/rho_q^2) - Pi) G,  ddivv = m_q/rho_o w.G,  dheat = -m_q Pi w.G / 2,
@@ -195,65 +203,74 @@ struct PairGrad {
 // velocity difference w are taken in FP64 and rounded once (a close pair's separation is a small
 // difference of large coordinates), and whose results the caller adds to FP64 sums.
 template <typename T>
-__device__ void pair_adjoint(const AdjRec& o, const AdjRec& q, const double* __restrict__ lut, double alpha_d,
-                             double beta_d, PairGrad& out) {
+__device__ __forceinline__ PairCommon<T> pair_common(const AdjRec& o, const AdjRec& q, const double* __restrict__ lut,
+                                                     T alpha, T beta) {
 #pragma clang fp contract(off)
-    const T alpha = T(alpha_d), beta = T(beta_d);
-    const T r[3] = { T(o.x - q.x), T(o.y - q.y), T(o.z - q.z) };
-    const T w[3] = { T(q.vx - o.vx), T(q.vy - o.vy), T(q.vz - o.vz) };
-    const T oh = T(o.h), qh = T(q.h), orho = T(o.rho), qrho = T(q.rho), op = T(o.p), qp = T(q.p);
-    const T hbar = T(0.5) * (oh + qh);
-    const T hInv = T(1) / hbar;
+    PairCommon<T> p;
+    p.r[0] = T(o.x - q.x), p.r[1] = T(o.y - q.y), p.r[2] = T(o.z - q.z);
+    p.w[0] = T(q.vx - o.vx), p.w[1] = T(q.vy - o.vy), p.w[2] = T(q.vz - o.vz);
+    const T orho = T(o.rho), qrho = T(q.rho);
+    p.hbar = T(0.5) * (T(o.h) + T(q.h));
+    const T hInv = T(1) / p.hbar;
     const T hInv2 = hInv * hInv;
-    const T s = r[0] * r[0] + r[1] * r[1] + r[2] * r[2];
+    const T s = p.r[0] * p.r[0] + p.r[1] * p.r[1] + p.r[2] * p.r[2];
     double gd, dgd;
     lut_grad_slope(lut, double(s * hInv2), gd, dgd);
     const T g = T(gd), dg = T(dgd);
     const T h5 = (hInv2 * hInv2) * hInv;
-    const T K = h5 * g, Kp = h5 * dg * hInv2;  // G = K r, dK/ds = Kp
-    const T G[3] = { K * r[0], K * r[1], K * r[2] };
-    const T wg = w[0] * G[0] + w[1] * G[1] + w[2] * G[2];
-    const T dvdr = -(w[0] * r[0] + w[1] * r[1] + w[2] * r[2]);
-    const T Po = op / (orho * orho), Pq = qp / (qrho * qrho);
-    const T mq = T(q.m);
-    T Pi = T(0), mu = T(0), den = T(1), rhobar = T(1), csbar = T(0);
-    const bool conv = dvdr < T(0);
-    if (conv) {
-        rhobar = T(0.5) * (orho + qrho);
-        csbar = T(0.5) * (T(o.cs) + T(q.cs));
-        den = s + T(1.e-2) * (hbar * hbar);
-        mu = hbar * dvdr / den;
-        Pi = (-alpha * csbar * mu + beta * (mu * mu)) / rhobar;
+    p.K = h5 * g, p.Kp = h5 * dg * hInv2;  // G = K r, dK/ds = Kp
+    for (int k = 0; k < 3; ++k) p.G[k] = p.K * p.r[k];
+    p.wg = p.w[0] * p.G[0] + p.w[1] * p.G[1] + p.w[2] * p.G[2];
+    const T dvdr = -(p.w[0] * p.r[0] + p.w[1] * p.r[1] + p.w[2] * p.r[2]);
+    p.Pi = T(0), p.mu = T(0), p.den = T(1), p.rhobar = T(1), p.csbar = T(0);
+    p.conv = dvdr < T(0);
+    if (p.conv) {
+        p.rhobar = T(0.5) * (orho + qrho);
+        p.csbar = T(0.5) * (T(o.cs) + T(q.cs));
+        p.den = s + T(1.e-2) * (p.hbar * p.hbar);
+        p.mu = p.hbar * dvdr / p.den;
+        p.Pi = (-alpha * p.csbar * p.mu + beta * (p.mu * p.mu)) / p.rhobar;
     }
+    p.C = -(T(o.p) / (orho * orho) + T(q.p) / (qrho * qrho)) - p.Pi;
+    return p;
+}
+
+// One direction: sign is +1 for the pair of pair_common and -1 for the exchanged one.
+template <typename T>
+__device__ __forceinline__ void pair_adjoint(const PairCommon<T>& p, const AdjRec& o, const AdjRec& q, T sign, T alpha,
+                                             T beta, PairGrad& out) {
+#pragma clang fp contract(off)
+    T r[3], w[3], G[3];
+    for (int k = 0; k < 3; ++k) r[k] = sign * p.r[k], w[k] = sign * p.w[k], G[k] = sign * p.G[k];
+    const T orho = T(o.rho), qrho = T(q.rho), op = T(o.p), qp = T(q.p), mq = T(q.m);
     const T la[3] = { T(o.lax), T(o.lay), T(o.laz) };
     const T old = T(o.ld), olh = T(o.lh);
     const T A = la[0] * G[0] + la[1] * G[1] + la[2] * G[2];
-    const T C = -(Po + Pq) - Pi;
-    const T gPi = -mq * A - T(0.5) * mq * olh * wg;
+    const T gPi = -mq * A - T(0.5) * mq * olh * p.wg;
     const T gP = -mq * A;
-    const T cw = mq * old / orho - T(0.5) * mq * olh * Pi;  // coefficient of w in dL/dG and of G in dL/dw
+    const T cw = mq * old / orho - T(0.5) * mq * olh * p.Pi;  // coefficient of w in dL/dG and of G in dL/dw
     T gG[3], gw[3];
     for (int k = 0; k < 3; ++k) {
-        gG[k] = mq * C * la[k] + cw * w[k];
+        gG[k] = mq * p.C * la[k] + cw * w[k];
         gw[k] = cw * G[k];
     }
     T gmu = T(0), gc = T(0), grb = T(0), gdvdr = T(0), gs = T(0);
-    if (conv) {
-        gmu = gPi * (-alpha * csbar + T(2) * beta * mu) / rhobar;
-        gc = gPi * (-alpha * mu / rhobar);
-        grb = gPi * (-Pi / rhobar);
-        gdvdr = gmu * hbar / den;
-        gs = gmu * (-mu / den);
+    if (p.conv) {
+        gmu = gPi * (-alpha * p.csbar + T(2) * beta * p.mu) / p.rhobar;
+        gc = gPi * (-alpha * p.mu / p.rhobar);
+        grb = gPi * (-p.Pi / p.rhobar);
+        gdvdr = gmu * p.hbar / p.den;
+        gs = gmu * (-p.mu / p.den);
     }
     const T gGr = gG[0] * r[0] + gG[1] * r[1] + gG[2] * r[2];
     for (int k = 0; k < 3; ++k) {
-        out.gr[k] = double(K * gG[k] + T(2) * Kp * gGr * r[k] + T(2) * gs * r[k] - gdvdr * w[k]);
+        out.gr[k] = double(p.K * gG[k] + T(2) * p.Kp * gGr * r[k] + T(2) * gs * r[k] - gdvdr * w[k]);
         out.gw[k] = double(gw[k] - gdvdr * r[k]);
     }
     const T ro3 = orho * orho * orho, rq3 = qrho * qrho * qrho;
     out.p_o = double(gP / (orho * orho));
     out.p_q = double(gP / (qrho * qrho));
-    out.rho_o = double(-(mq * old / (orho * orho)) * wg - T(2) * op * gP / ro3 + T(0.5) * grb);
+    out.rho_o = double(-(mq * old / (orho * orho)) * p.wg - T(2) * op * gP / ro3 + T(0.5) * grb);
     out.rho_q = double(-T(2) * qp * gP / rq3 + T(0.5) * grb);
     out.c_o = double(T(0.5) * gc);
     out.c_q = double(T(0.5) * gc);
@@ -306,8 +323,13 @@ __global__ void __launch_bounds__(BLOCK) k_adj_seed(DevState s, AdjPlanes ap, co
 }
 
 // F's vector-Jacobian product gathered per particle over its neighbour list: its own pair terms (owner
-// = itself) and the terms each neighbour receives from it (owner = the neighbour).
-template <typename T>
+// = itself) and the terms each neighbour receives from it (owner = the neighbour).  LANES neighbouring lanes
+// share a particle, an entry of the list each in turn, and add their FP64 sums in a fixed order: a
+// lane's chain of 50 dependent pair terms was the time of anything below 40k particles.  One lane and both directions
+// of a pair from the start -> this, FP64 us per step: 2k 187 -> 48, 10k 203 -> 60, 40k 217 -> 115, 100k 343 -> 227, 300k
+// 820 -> 632 (the part from what the directions share: 822 -> 632).  16 lanes: 39, 65, 142, 320, 927 before that;
+// 4 lanes: 72, 79, 148, 300, 822.  Bound by the divides (25 a pair).
+template <typename T, int LANES>
 __global__ void __launch_bounds__(BLOCK) k_adj_pairs(AdjPlanes ap, const AdjRec* __restrict__ rec,
                                                      const uint32_t* __restrict__ order,
                                                      const uint32_t* __restrict__ list,
@@ -315,39 +337,38 @@ __global__ void __launch_bounds__(BLOCK) k_adj_pairs(AdjPlanes ap, const AdjRec*
                                                      const double* __restrict__ lut, double alpha, double beta,
                                                      uint32_t kmax, size_t n) {
 #pragma clang fp contract(off)
-    const size_t k = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (k >= n) return;
+    const size_t at = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    const size_t k = at / LANES;
+    const uint32_t sub = uint32_t(at % LANES);
+    if (k >= n) return;  // whole groups of lanes
     const AdjRec me = rec[k];
-    double gr[3] = { 0.0, 0.0, 0.0 }, gv[3] = { 0.0, 0.0, 0.0 };
-    double grho = 0.0, gp = 0.0, gc = 0.0;
+    double g[9];  // r*, v*, rho*, p, cs
+    for (int q = 0; q < 9; ++q) g[q] = 0.0;
     const uint32_t cnt = count[k];
     const uint32_t listed = cnt < kmax ? cnt : kmax;
-    const uint4* list4 = reinterpret_cast<const uint4*>(list);
-    for (uint32_t c = 0; c < listed; c += 4) {
-        const uint4 qd = list4[list_quad(k, c >> 2, kmax >> 2)];
-        const uint32_t ent[4] = { qd.x, qd.y, qd.z, qd.w };
-        for (uint32_t t = 0; t < 4 && c + t < listed; ++t) {
-            const AdjRec o = rec[ent[t]];
-            PairGrad a, b;
-            pair_adjoint<T>(me, o, lut, alpha, beta, a);  // this particle's own terms
-            pair_adjoint<T>(o, me, lut, alpha, beta, b);  // the neighbour's terms from this particle
-            for (int d = 0; d < 3; ++d) {
-                gr[d] += a.gr[d] - b.gr[d];  // r = r_me - r_o in a, r_o - r_me in b
-                gv[d] += -a.gw[d] + b.gw[d];  // w = v_o - v_me in a, v_me - v_o in b
-            }
-            grho += a.rho_o + b.rho_q;
-            gp += a.p_o + b.p_q;
-            gc += a.c_o + b.c_q;
+    for (uint32_t c = sub; c < listed; c += LANES) {
+        const AdjRec o = rec[list[4 * size_t(list_quad(k, c >> 2, kmax >> 2)) + (c & 3)]];
+        const PairCommon<T> pair = pair_common<T>(me, o, lut, T(alpha), T(beta));
+        PairGrad a, b;
+        pair_adjoint<T>(pair, me, o, T(1), T(alpha), T(beta), a);   // this particle's own terms
+        pair_adjoint<T>(pair, o, me, T(-1), T(alpha), T(beta), b);  // the neighbour's terms from this particle
+        for (int d = 0; d < 3; ++d) {
+            g[GRX + d] += a.gr[d] - b.gr[d];   // r = r_me - r_o in a, r_o - r_me in b
+            g[GVX + d] += -a.gw[d] + b.gw[d];  // w = v_o - v_me in a, v_me - v_o in b
         }
+        g[GRHO] += a.rho_o + b.rho_q;
+        g[GP] += a.p_o + b.p_q;
+        g[GC] += a.c_o + b.c_q;
     }
+    for (int o = LANES / 2; o > 0; o >>= 1) {
+        for (int q = 0; q < 9; ++q) g[q] += __shfl_xor(g[q], o, LANES);
+    }
+    if (sub) return;
     const uint32_t i = order[k];
-    for (int d = 0; d < 3; ++d) {
-        ap.g[GRX + d][i] = gr[d];
-        ap.g[GVX + d][i] = gv[d];
-    }
-    ap.g[GRHO][i] += grho;
-    ap.g[GP][i] += gp;
-    ap.g[GC][i] = gc;
+    for (int q = 0; q < GRHO; ++q) ap.g[q][i] = g[q];
+    ap.g[GRHO][i] += g[GRHO];
+    ap.g[GP][i] += g[GP];
+    ap.g[GC][i] = g[GC];
 }
 
 // The equation of state, prediction and correction adjoints, per slot: the adjoints of X_{n+1} in ap.l
@@ -470,11 +491,9 @@ void launch_adj_step(const Launch& l, DevState s, double* const* lplanes, double
     for (int c = 0; c < 9; ++c) ap.g[c] = gplanes[c];
     AdjRec* r = static_cast<AdjRec*>(rec);
     k_adj_seed<<<grid_for(n), BLOCK, 0, l.stream>>>(s, ap, order, dt, r, n);
-    if (fp32) {
-        k_adj_pairs<float><<<grid_for(n), BLOCK, 0, l.stream>>>(ap, r, order, list, count, lut, alpha, beta, kmax, n);
-    } else {
-        k_adj_pairs<double><<<grid_for(n), BLOCK, 0, l.stream>>>(ap, r, order, list, count, lut, alpha, beta, kmax, n);
-    }
+    constexpr int LANES = 8;
+    const auto pairs = fp32 ? k_adj_pairs<float, LANES> : k_adj_pairs<double, LANES>;
+    pairs<<<grid_for(n * LANES), BLOCK, 0, l.stream>>>(ap, r, order, list, count, lut, alpha, beta, kmax, n);
     const unsigned g = grid_for(n);
     k_adj_finish<<<g, BLOCK, 0, l.stream>>>(s, ap, mats, nmat, dt, part, clamped, n);
     k_adj_theta<<<ADJ_MAX_MATERIALS * 3, BLOCK, 0, l.stream>>>(part, g, theta);
