@@ -42,7 +42,7 @@ struct BatchPlan {
     BatchMember* dev = nullptr;
     BatchMember* host = nullptr;
     unsigned long long* small = nullptr;
-    unsigned long long* small_host = nullptr;
+    Mailbox box;  // host mirror of small
     uint64_t *keys = nullptr, *keys_sorted = nullptr;
     uint32_t *vals = nullptr, *vals_sorted = nullptr;
     void* sort_temp = nullptr;
@@ -63,7 +63,7 @@ struct BatchPlan {
         void* dp[] = { tables, dev, small, keys, keys_sorted, vals, vals_sorted, sort_temp };
         for (void* p : dp) (void)hipFree(p);
         if (host) (void)hipHostFree(host);
-        if (small_host) (void)hipHostFree(small_host);
+        mailbox_destroy(box);
     }
 };
 
@@ -110,7 +110,8 @@ struct osph_ctx {
     uint32_t kmax = 96;
     size_t list_cap = 0;
     unsigned long long* small = nullptr;     // accumulators, layout SMALL_* in osph_internal.h
-    unsigned long long* small_host = nullptr;  // pinned mirror
+    Mailbox box;                              // host mirror of small
+    unsigned long long* small_host = nullptr;  // its words
     double* lut = nullptr;
     float* lutf = nullptr;
     Grid grid{};
@@ -443,6 +444,17 @@ int sync_check(osph_ctx* c) {
     return OSPH_OK;
 }
 
+// Words [first, first + count) of the accumulators to small_host, and the wait for them.
+void post_small(osph_ctx* c, int first, int count) { mailbox_post(c->stream, c->box, first, c->small + first, count); }
+
+int wait_box(osph_ctx* c, Mailbox& box) {
+    if (hipPeekAtLastError() != hipSuccess) return sync_check(c);
+    HIPCHK(c, mailbox_wait(c->stream, box));
+    return OSPH_OK;
+}
+
+int wait_small(osph_ctx* c) { return wait_box(c, c->box); }
+
 // Grid + sort + pack + neighbour lists for the current positions (ISymmetricFinder::build).
 // FP32 screen of the neighbour test.  Coordinates are rounded once to FP32 relative to lo, so each
 // carries an absolute error below eps D (D the largest extent, eps = 2^-24) and a difference below
@@ -472,9 +484,8 @@ int ensure_href(osph_ctx* c) {
     Launch l = L(c);
     timed(c, "init_small", [&] { launch_init_small(l, c->small); });
     timed(c, "bounds", [&] { launch_bounds_reduce(l, c->s, c->small, c->n); });
-    HIPCHK(c, hipMemcpyAsync(c->small_host, c->small, 8 * sizeof(unsigned long long), hipMemcpyDeviceToHost,
-                             c->stream));
-    if (int e = sync_check(c)) return e;
+    post_small(c, 0, 8);
+    if (int e = wait_small(c)) return e;
     const double h0 = decode_ord(c->small_host[7]);
     if (!(h0 > 0.0) || !std::isfinite(h0)) return c->fail(OSPH_ERR_STATE, "smoothing lengths must be positive");
     c->href = h0;
@@ -504,7 +515,6 @@ int search_begin(osph_ctx* c, int mode, double dt) {
     if (int e = ensure_href(c)) return e;
     if (mode == 2) swap_predictions(c);
     const double href = c->href;
-    unsigned long long* cacc = c->small + SMALL_CLASSES;
     const bool vel = c->cfg.precision == OSPH_PRECISION_MIXED;
     if (bounds_partials(n) > c->bounds_part_cap) {
         (void)hipFree(c->bounds_part);
@@ -515,9 +525,7 @@ int search_begin(osph_ctx* c, int mode, double dt) {
     }
     timed(c, mode == 2 ? "advance" : (mode == 1 ? "material_init" : "class_bounds"),
           [&] { launch_advance(l, c->s, c->mats_dev, c->prm, mode, dt, href, c->small, vel, c->bounds_part, n); });
-    HIPCHK(c, hipMemcpyAsync(c->small_host + SMALL_CLASSES, cacc,
-                             (SMALL_VEL + 6 - SMALL_CLASSES) * sizeof(unsigned long long), hipMemcpyDeviceToHost,
-                             c->stream));
+    post_small(c, SMALL_CLASSES, SMALL_VEL + 6 - SMALL_CLASSES);
     return OSPH_OK;
 }
 
@@ -668,7 +676,7 @@ void swap_state(osph_ctx* c, const DevState& dst) {
 int search_finish(osph_ctx* c) {
     const size_t n = c->n;
     Launch l = L(c);
-    if (int e = sync_check(c)) return e;
+    if (int e = wait_small(c)) return e;
     size_t rows = 0;
     if (int e = plan_search(c, c->small_host, &rows)) return e;
     const Grid g = c->grid;
@@ -734,9 +742,8 @@ bool overflowed(const osph_ctx* c) {
 int build_lists(osph_ctx* c) {
     for (int attempt = 0; attempt < 4; ++attempt) {
         if (int e = launch_lists(c)) return e;
-        HIPCHK(c, hipMemcpyAsync(&c->small_host[SMALL_OVERFLOW], overflow_flag(c), sizeof(uint32_t),
-                                 hipMemcpyDeviceToHost, c->stream));
-        if (int e = sync_check(c)) return e;
+        post_small(c, SMALL_OVERFLOW, 1);
+        if (int e = wait_small(c)) return e;
         if (!overflowed(c)) {
             c->neighbors_valid = true;
             return OSPH_OK;
@@ -812,9 +819,8 @@ int integrate(osph_ctx* c, osph_stats* stats) {
         launch_pair_sums(c);
         timed(c, "finalize", [&] { launch_finalize(l, c->s, c->mats_dev, c->prm, n); });
         if (stats) timed(c, "count_stats", [&] { launch_count_stats(l, c->s.u[NCNT], c->small + SMALL_COUNTS, n); });
-        HIPCHK(c, hipMemcpyAsync(c->small_host + SMALL_OVERFLOW, c->small + SMALL_OVERFLOW,
-                                 4 * sizeof(unsigned long long), hipMemcpyDeviceToHost, c->stream));
-        if (int e = sync_check(c)) return e;
+        post_small(c, SMALL_OVERFLOW, 4);
+        if (int e = wait_small(c)) return e;
         if (!overflowed(c)) break;
         if (attempt == 3) return c->fail(OSPH_ERR_STATE, "neighbour list did not fit after growing");
         if (int e = grow_lists(c)) return e;
@@ -977,7 +983,8 @@ int osph_create(osph_ctx** out, const osph_config* cfg, const osph_material* mat
     if (hipMemcpy(c->mats_dev, materials, sizeof(osph_material) * n_materials, hipMemcpyHostToDevice) != hipSuccess)
         return bail(OSPH_ERR_HIP);
     if (hipMalloc(&c->small, SMALL_WORDS * sizeof(unsigned long long)) != hipSuccess) return bail(OSPH_ERR_HIP);
-    if (hipHostMalloc(&c->small_host, SMALL_WORDS * sizeof(unsigned long long)) != hipSuccess) return bail(OSPH_ERR_HIP);
+    if (mailbox_create(c->box, SMALL_WORDS) != hipSuccess) return bail(OSPH_ERR_HIP);
+    c->small_host = c->box.host;
     std::vector<double> values(LUT_ENTRIES + 1), grads(LUT_ENTRIES + 1);
     build_lut(values.data(), grads.data());
     if (hipMalloc(&c->lut, grads.size() * sizeof(double)) != hipSuccess) return bail(OSPH_ERR_HIP);
@@ -1015,7 +1022,7 @@ void osph_destroy(osph_ctx* c) {
     (void)hipFree(c->small);
     (void)hipFree(c->lut);
     (void)hipFree(c->lutf);
-    if (c->small_host) (void)hipHostFree(c->small_host);
+    mailbox_destroy(c->box);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
     transfer_detach();
@@ -1235,9 +1242,8 @@ int osph_timestep(osph_ctx* c, double* dt, int* crit) {
     uint32_t* m32 = reinterpret_cast<uint32_t*>(c->small + SMALL_CRITERIA);
     launch_clear_u32(L(c), m32, 8, 0xffffffffu);
     timed(c, "criteria", [&] { launch_criteria(L(c), c->s, c->mats_dev, c->prm, c->small + SMALL_CRITERIA, c->n); });
-    HIPCHK(c, hipMemcpyAsync(c->small_host + SMALL_CRITERIA, c->small + SMALL_CRITERIA,
-                             4 * sizeof(unsigned long long), hipMemcpyDeviceToHost, c->stream));
-    if (int e = sync_check(c)) return e;
+    post_small(c, SMALL_CRITERIA, 4);
+    if (int e = wait_small(c)) return e;
     select_timestep(c, c->small_host + SMALL_CRITERIA, dt, crit);
     return OSPH_OK;
 }
@@ -1269,9 +1275,7 @@ void launch_second_half(osph_ctx* c, double dt) {
                                     c->n);
         });
     }
-    (void)hipMemcpyAsync(c->small_host + SMALL_CRITERIA, c->small + SMALL_CRITERIA,
-                         (SMALL_OVERFLOW + 1 - SMALL_CRITERIA) * sizeof(unsigned long long), hipMemcpyDeviceToHost,
-                         c->stream);
+    post_small(c, SMALL_CRITERIA, SMALL_OVERFLOW + 1 - SMALL_CRITERIA);
 }
 
 int step_middle(osph_ctx* c, double dt) {
@@ -1290,7 +1294,7 @@ int step_end(osph_ctx* c, double dt, double* next_dt, int* crit) {
         return OSPH_OK;
     }
     for (int attempt = 0; attempt < 4; ++attempt) {
-        if (int e = sync_check(c)) return e;
+        if (int e = wait_small(c)) return e;
         if (!overflowed(c)) {
             c->neighbors_valid = true;
             select_timestep(c, c->small_host + SMALL_CRITERIA, next_dt, crit);
@@ -1382,7 +1386,7 @@ int make_plan(const std::vector<osph_ctx*>& ms, BatchPlan*& out) {
     HIPCHK(lead, hipHostMalloc(&P->host, count * sizeof(BatchMember)));
     std::memset(static_cast<void*>(P->host), 0, count * sizeof(BatchMember));
     HIPCHK(lead, hipMalloc(&P->small, count * SMALL_WORDS * sizeof(unsigned long long)));
-    HIPCHK(lead, hipHostMalloc(&P->small_host, count * SMALL_WORDS * sizeof(unsigned long long)));
+    HIPCHK(lead, mailbox_create(P->box, count * SMALL_WORDS));
     for (osph_ctx* c : ms) {
         P->sizes.push_back(c->n);
         P->total += c->n;
@@ -1443,9 +1447,8 @@ int batch_step(const std::vector<osph_ctx*>& ms, const std::vector<double>& dts,
     // predictions, material initialize and grid bounds of every member; one readback of all bounds
     HIPCHK(lead, hipMemcpyAsync(P->dev, P->host, count * sizeof(BatchMember), hipMemcpyHostToDevice, st));
     batch_advance(l, P->dev, int(count), P->pb, P->mixed);
-    HIPCHK(lead, hipMemcpyAsync(P->small_host, P->small, count * SMALL_WORDS * sizeof(unsigned long long),
-                                hipMemcpyDeviceToHost, st));
-    if (int e = sync_check(lead)) return e;
+    mailbox_post(st, P->box, 0, P->small, count * SMALL_WORDS);
+    if (int e = wait_box(lead, P->box)) return e;
     // each member's grid, screen and fixed-point frames, planned as its own search plans them
     int key_bits = 1;
     bool screened = false, plain = false;
@@ -1454,7 +1457,7 @@ int batch_step(const std::vector<osph_ctx*>& ms, const std::vector<double>& dts,
         osph_ctx* c = ms[k];
         BatchMember& b = P->host[k];
         size_t rows = 0;
-        if (int e = plan_search(c, P->small_host + SMALL_WORDS * k, &rows)) return e;
+        if (int e = plan_search(c, P->box.host + SMALL_WORDS * k, &rows)) return e;
         if (int e = ensure_list(c, list_entries(c->n, c->kmax))) return e;
         int xslots = 1;
         for (int cl = 0; cl < c->grid.nclass; ++cl) {
@@ -1520,13 +1523,12 @@ int batch_step(const std::vector<osph_ctx*>& ms, const std::vector<double>& dts,
     } else {
         rest();
     }
-    HIPCHK(lead, hipMemcpyAsync(P->small_host, P->small, count * SMALL_WORDS * sizeof(unsigned long long),
-                                hipMemcpyDeviceToHost, st));
-    if (int e = sync_check(lead)) return e;
+    mailbox_post(st, P->box, 0, P->small, count * SMALL_WORDS);
+    if (int e = wait_box(lead, P->box)) return e;
     for (size_t k = 0; k < count; ++k) {
         osph_ctx* c = ms[k];
         if (P->host[k].reorder) swap_state(c, P->host[k].s2);
-        const unsigned long long* sh = P->small_host + SMALL_WORDS * k;
+        const unsigned long long* sh = P->box.host + SMALL_WORDS * k;
         uint32_t flag;
         std::memcpy(&flag, &sh[SMALL_OVERFLOW], sizeof(uint32_t));
         if (!flag) {

@@ -10,6 +10,7 @@
 #include "osph_transfer.h"
 
 #include <algorithm>
+#include <chrono>
 #include <cstring>
 #include <mutex>
 #include <system_error>
@@ -112,7 +113,58 @@ hipError_t copy_range(hipStream_t stream, PinnedBuffer& b, unsigned char* host, 
     return err;
 }
 
+__global__ void __launch_bounds__(256) k_post(const unsigned long long* __restrict__ src, size_t count,
+                                              unsigned long long* __restrict__ host, unsigned long long* __restrict__ posts,
+                                              unsigned long long value) {
+    for (size_t k = threadIdx.x; k < count; k += blockDim.x) {
+        __hip_atomic_store(host + k, src[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(posts, value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// Watching the count costs a core its time: past this the thread sleeps in the runtime's wait, which is what a device
+// error ends too.
+constexpr std::chrono::milliseconds WATCH{ 20 };
+
 }  // namespace
+
+hipError_t mailbox_create(Mailbox& box, size_t words) {
+    box = Mailbox{};
+    const hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&box.host), (words + 1) * sizeof(unsigned long long),
+                                       hipHostMallocCoherent | hipHostMallocPortable | hipHostMallocMapped);
+    if (e != hipSuccess) {
+        box.host = nullptr;
+        return e;
+    }
+    box.words = words;
+    std::fill(box.host, box.host + words + 1, 0ull);
+    return hipSuccess;
+}
+
+void mailbox_destroy(Mailbox& box) {
+    if (box.host) (void)hipHostFree(box.host);
+    box = Mailbox{};
+}
+
+MailboxPost mailbox_next(Mailbox& box) { return { box.host, box.host + box.words, ++box.posts }; }
+
+void mailbox_post(hipStream_t stream, Mailbox& box, size_t first, const unsigned long long* dev, size_t count) {
+    k_post<<<1, count > 64 ? 256 : 64, 0, stream>>>(dev, count, box.host + first, box.host + box.words, ++box.posts);
+}
+
+hipError_t mailbox_wait(hipStream_t stream, Mailbox& box) {
+    const auto end = std::chrono::steady_clock::now() + WATCH;
+    while (__atomic_load_n(box.host + box.words, __ATOMIC_ACQUIRE) != box.posts) {
+        for (int k = 0; k < 16; ++k) __builtin_ia32_pause();
+        if (std::chrono::steady_clock::now() < end) continue;
+        if (const hipError_t e = hipStreamSynchronize(stream)) return e;
+        if (__atomic_load_n(box.host + box.words, __ATOMIC_ACQUIRE) == box.posts) break;
+        return hipErrorLaunchFailure;  // the stream is idle and a post is missing
+    }
+    return hipSuccess;
+}
 
 void transfer_attach() {
     PinnedPool& p = pool();
