@@ -902,13 +902,25 @@ __global__ void __launch_bounds__(BLOCK) k_neighbor_lists(const double4* __restr
     if (k < n) neighbor_list_at<SCREEN>(pos, posf, sc, g, first, list, count, kmax, overflow, k);
 }
 
-// LutKernel<3>::gradImpl (core/sph/kernel/Kernel.h:129-144): linear interpolation in q^2.
-__device__ __forceinline__ double lut_grad(const double* __restrict__ grads, double q2) {
-    if (!(q2 < 4.0)) return 0.0;  // outside the support (also catches NaN, which must not become an index)
-    const double fi = double(LUT_ENTRIES / 4) * q2;
+// LutKernel<3>::gradImpl (core/sph/kernel/Kernel.h:129-144), linear interpolation in q^2, in two parts: the table's two
+// entries, and what is made of them.  One 16-byte load at 8-byte alignment fetches both.
+struct LutPair {
+    double a, b, ratio;
+    bool inside;
+    __device__ __forceinline__ double value() const { return inside ? fma(b, ratio, a * (1.0 - ratio)) : 0.0; }
+};
+
+__device__ __forceinline__ LutPair lut_fetch(const double* __restrict__ grads, double q2) {
+    typedef double Two __attribute__((ext_vector_type(2), aligned(8)));
+    LutPair p;
+    p.inside = q2 < 4.0;  // outside the support (also NaN, which must not become an index) the value is 0
+    const double fi = double(LUT_ENTRIES / 4) * (p.inside ? q2 : 0.0);
     const uint32_t i1 = uint32_t(fi);
-    const double ratio = fi - double(i1);
-    return grads[i1] * (1.0 - ratio) + grads[i1 + 1] * ratio;
+    p.ratio = fi - double(i1);
+    const Two v = *reinterpret_cast<const Two*>(grads + i1);
+    p.a = v.x;
+    p.b = v.y;
+    return p;
 }
 
 // The pair sums of particle i that the finalize, the corrector and the criteria use: acceleration, du,
@@ -933,148 +945,98 @@ __device__ void criteria_values(const DevState& s, const osph_material& m, const
 __device__ void reduce_criteria(double v[4], unsigned long long* mins);
 
 
-// How the pair kernels gather neighbour records (for_each_neighbor): 0 directly, 1 through the LDS stage,
-// 2 through the LDS stage with the next step's loads issued before the current step's compute, 3 directly
-// with the next neighbour's record loaded before the current one's terms.  For the 64-B mixed record at
-// the 1M impact, in one A/B on one box: 0.432 ms (0), 0.417 ms (3); the 80-B record it replaced ran at
-// 0.415 ms directly.
-constexpr int PAIRS64_STAGE = 1;
-constexpr int PAIRSMX_STAGE = 3;
-
-// Per-wavefront LDS staging of neighbour records: 64 records of CH 16-byte chunks each, at an odd stride
-// of chunks (CH | 1) so that the lanes' 16-byte reads of their own record spread over all banks.
+// Per-wavefront LDS stage of neighbour records: 64 records of CH 16-byte chunks.  Chunk c of lane r's record lies at
+// place c ^ swizzle(r) of the record, so that 16 consecutive lanes' reads of one chunk fall on all 64 banks.
 template <typename Rec>
 struct StageOf {
     static constexpr uint32_t CH = sizeof(Rec) / 16;
-    static constexpr uint32_t STRIDE = CH | 1u;
-    static constexpr uint32_t WORDS = 64 * STRIDE;  // uint4 per wavefront
-    static_assert(sizeof(Rec) % 16 == 0, "records are whole 16-byte chunks");
+    static constexpr uint32_t WORDS = 64 * CH;  // uint4 per wavefront
+    static_assert(sizeof(Rec) % 16 == 0 && (CH == 4 || CH == 8), "a power of two of 16-byte chunks");
+    static __device__ __forceinline__ uint32_t swizzle(uint32_t r) { return (r / (16u / CH)) % CH; }
 };
 
-// The neighbour list of one particle, on one lane: quads (4 entries, 16 B) in order, the next quad loaded one
-// quad ahead.  f(record, entry) runs for each listed entry.
+// The neighbour lists of a wavefront's particles, one on each lane, entry t of every list at step t: x = early(record,
+// entry) on all lanes, then f(record, entry, x) on those whose list has the entry (the others hold their own record).
+// Every lane of the wavefront must call this.
 //
-// STAGED (1, 2): the records are fetched cooperatively.  In each step the wavefront needs one record per lane;
-// pass i of the CH load passes has lane L fetch chunk c of the record of lane r, (r, c) = divmod(64 i +
-// L, CH), into the wavefront's LDS stage, and each lane then reads its own record back.  Consecutive
-// lanes fetch consecutive chunks of one record, so a load instruction touches ~64 / CH records' cache
-// lines instead of one line per lane: CH times fewer line accesses in the texture path, for a longer
-// dependency chain (shuffle, load, LDS write, LDS read).  It pays for the 128-B FP64 record (1.16 ->
-// 1.06 ms at the impact) and not for the (then 80-B) mixed one (0.45 -> 0.51 ms), which gathers directly.
-// With STAGED == 2 the next step's loads are issued before the current step's compute.
-// Every lane of the wavefront must call this (lanes without entries load their own record as a
-// stand-in, and run no f).
-template <int STAGED, typename Rec, typename F>
+// A lane that loads a whole record by itself touches a cache line of its own in every load instruction, CH times as
+// many as when consecutive lanes fetch the chunks of one record.  So the wavefront fetches the 64 records of a step
+// together, straight into its LDS stage (no registers in between), while the terms of the step before are evaluated;
+// early is where f's own loads go, ahead of the next records'.  The trip count is the wavefront's and the steps of a
+// list quad are written out, so that the accumulators and the quad stay where they are (with a condition on each lane
+// the compiler moved them about, 40 of 180 instructions a step).  Per step at the 1M impact, direct loads or loads
+// staged through registers -> this: mixed 551 -> 488 us, FP64 1035 -> 804, 531k particles FP64 434 -> 378.  Mixed is
+// bound by the issue (139 instructions a step, 75 % of the issue slots), FP64 by the L1 cache (168 accesses and 62
+// line fills a step, 40 % of them the kernel table's).  Buffer loads with 32-bit offsets in place of the global ones:
+// 490 and 777 us, but no record past 4 GB; the table's entries computed instead: 762 us; wavefronts of five to a SIMD
+// for the mixed kernel (96 registers): 496 us.
+template <typename Rec, typename E, typename F>
 __device__ __forceinline__ void for_each_neighbor(const Rec* __restrict__ rec, const uint32_t* __restrict__ list,
-                                                  size_t k, uint32_t quads, uint32_t listed,
-                                                  uint4* __restrict__ stage, F&& f) {
+                                                  size_t k, uint32_t quads, uint32_t listed, uint4* stage, E&& early,
+                                                  F&& f) {
     using S = StageOf<Rec>;
+    constexpr uint32_t CH = S::CH, PER = 64u / CH;  // records per load
     const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t myq = (listed + 3u) >> 2, total = listed;
-    const uint4* list4 = reinterpret_cast<const uint4*>(list);
-    auto row = [&](uint32_t j) { return list4[list_quad(k, j, quads)]; };
-    if constexpr (STAGED == 0 || STAGED == 3) {
-        if (myq == 0) return;
-        uint4 quad = row(0);
-        uint4 nquad = myq > 1 ? row(1) : quad;
-        auto entry_of = [&](uint32_t t) -> uint32_t {
-            const uint32_t sel = t & 3u;
-            if (sel == 0 && t > 0) {
-                quad = nquad;
-                const uint32_t j = (t >> 2) + 1;
-                nquad = j < myq ? row(j) : quad;
-            }
-            return sel == 0 ? quad.x : (sel == 1 ? quad.y : (sel == 2 ? quad.z : quad.w));
-        };
-        if constexpr (STAGED == 0) {
-            for (uint32_t t = 0; t < total; ++t) {
-                const uint32_t e = entry_of(t);
-                const Rec o = rec[e];
-                f(o, e);
-            }
-        } else {
-            // the next neighbour's record is loaded before the current one's terms are evaluated
-            uint32_t e = entry_of(0);
-            Rec o = rec[e];
-            for (uint32_t t = 0; t < total; ++t) {
-                const uint32_t en = t + 1 < total ? entry_of(t + 1) : e;
-                const Rec on = rec[en];
-                f(o, e);
-                o = on;
-                e = en;
-            }
-        }
-        return;
-    }
-    // (in the staged loops the step index is uniform across the wavefront, so the entry is taken from
-    // rotating registers rather than selected by index, which the compiler would place in scratch)
-    const uint4 first = myq > 0 ? row(0) : make_uint4(0, 0, 0, 0);
-    uint32_t q0 = first.x, q1 = first.y, q2 = first.z, q3 = first.w;  // entries of the current quad, next first
-    uint4 nquad = myq > 1 ? row(1) : first;
-    // the entry of step t for this lane (its own index as a stand-in when it has none); steps in order
-    auto entry = [&](uint32_t t) -> uint32_t {
-        const bool act = t < total;
-        if (act && (t & 3u) == 0 && t > 0) {
-            q0 = nquad.x;
-            q1 = nquad.y;
-            q2 = nquad.z;
-            q3 = nquad.w;
-            const uint32_t j = (t >> 2) + 1;
-            if (j < myq) nquad = row(j);
-        }
-        const uint32_t e = act ? q0 : uint32_t(k);
-        q0 = q1;
-        q1 = q2;
-        q2 = q3;
-        return e;
+    uint32_t most = listed;
+    for (int o = 32; o > 0; o >>= 1) most = max(most, uint32_t(__shfl_xor(int(most), o, 64)));
+    most = __builtin_amdgcn_readfirstlane(most);
+    if (most == 0) return;
+    const uint4* my_list = reinterpret_cast<const uint4*>(list) + list_quad(k, 0, quads);
+    const uint32_t last = listed ? (listed - 1) >> 2 : 0u;
+    auto row = [&](uint32_t j) { return my_list[min(j, last) * LIST_TILE]; };
+    // the records this lane fetches chunks of (its own record stands in for entries past its list)
+    struct Fetch {
+        uint32_t at[CH];  // in units of 16 bytes
     };
-    const uint4* src = reinterpret_cast<const uint4*>(rec);
-    // pass i: this lane's chunk of the records of every lane's entry e
-    uint4 v[S::CH];
-    auto fetch = [&](uint32_t e) {
+    auto plan = [&](uint32_t t, uint32_t e) {
+        const int mine = int((t < listed ? e : uint32_t(k)) * CH);
+        Fetch p;
 #pragma unroll
-        for (uint32_t i = 0; i < S::CH; ++i) {
-            const uint32_t q = i * 64u + lane;
-            const uint32_t r = q / S::CH, c = q - r * S::CH;
-            const uint32_t er = uint32_t(__shfl(int(e), int(r), 64));
-            v[i] = src[size_t(er) * S::CH + c];
-        }
+        for (uint32_t i = 0; i < CH; ++i) p.at[i] = uint32_t(__shfl(mine, int(i * PER + lane / CH), 64));
+        return p;
     };
-    auto put = [&]() {
+    auto issue = [&](const Fetch& p) {
 #pragma unroll
-        for (uint32_t i = 0; i < S::CH; ++i) {
-            const uint32_t q = i * 64u + lane;
-            const uint32_t r = q / S::CH, c = q - r * S::CH;
-            stage[r * S::STRIDE + c] = v[i];
+        for (uint32_t i = 0; i < CH; ++i) {
+            const uint32_t c = (lane % CH) ^ S::swizzle(i * PER + lane / CH);
+            const auto* g = reinterpret_cast<const __attribute__((address_space(1))) void*>(
+                (uint64_t(p.at[i]) << 4) + reinterpret_cast<uintptr_t>(reinterpret_cast<const uint4*>(rec) + c));
+            __builtin_amdgcn_global_load_lds(g, (__attribute__((address_space(3))) void*)(stage + i * 64u), 16, 0, 0);
         }
     };
-    uint32_t e = entry(0);
-    if constexpr (STAGED == 2) fetch(e);
-    for (uint32_t t = 0; __any(t < total); ++t) {
-        const bool act = t < total;
-        const uint32_t ecur = e;
-        wave_sync();  // the previous step's reads of the stage come first
-        if constexpr (STAGED == 2) {
-            put();
-            // the next step's loads leave before this step's compute (pipelined)
-            if (__any(t + 1 < total)) {
-                e = entry(t + 1);
-                fetch(e);
-            }
-        } else {
-            fetch(ecur);
-            put();
-            if (__any(t + 1 < total)) e = entry(t + 1);
-        }
-        wave_sync();
+    auto step = [&](uint32_t t, uint32_t e, uint32_t enext) {
+        Fetch p = plan(t + 1, enext);
+#pragma unroll
+        for (uint32_t i = 0; i < CH; ++i) asm volatile("" : "+v"(p.at[i]));  // before the wait, not after it
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         union {
-            uint4 v[S::CH];
+            uint4 v[CH];
             Rec r;
         } o;
 #pragma unroll
-        for (uint32_t c = 0; c < S::CH; ++c) o.v[c] = stage[lane * S::STRIDE + c];
-        if (act) f(o.r, ecur);
+        for (uint32_t c = 0; c < CH; ++c) o.v[c] = stage[lane * CH + (c ^ S::swizzle(lane))];
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // read before the next records overwrite it
+        if (t >= listed) e = uint32_t(k);
+        const auto first = early(o.r, e);
+        asm volatile("" ::: "memory");
+        issue(p);
+        if (t < listed) f(o.r, e, first);
+    };
+    uint4 q = row(0);
+    issue(plan(0, q.x));
+    for (uint32_t t = 0;; t += 4) {
+        const uint4 nq = row((t >> 2) + 1);
+        step(t, q.x, q.y);
+        if (t + 1 >= most) break;
+        step(t + 1, q.y, q.z);
+        if (t + 2 >= most) break;
+        step(t + 2, q.z, q.w);
+        if (t + 3 >= most) break;
+        step(t + 3, q.w, nq.x);
+        if (t + 4 >= most) break;
+        q = nq;
     }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing may still write into the stage
 }
 
 // ---- a group of lanes per particle -------------------------------------------------------------------
@@ -1142,25 +1104,25 @@ struct PairAcc64 {
     double ax = 0.0, ay = 0.0, az = 0.0, du = 0.0, divv = 0.0;
     double g[6] = { 0.0, 0.0, 0.0, 0.0, 0.0, 0.0 };
     __device__ __forceinline__ void factors(double, double) {}
-    __device__ __forceinline__ void divergence(double mjr, double v) { divv += mjr * v; }
+    __device__ __forceinline__ void divergence(double mjr, double v) { divv = fma(mjr, v, divv); }
     __device__ __forceinline__ void pressure(double mj, double vx, double vy, double vz) {
-        ax -= mj * vx;
-        ay -= mj * vy;
-        az -= mj * vz;
+        ax = fma(mj, -vx, ax);
+        ay = fma(mj, -vy, ay);
+        az = fma(mj, -vz, az);
     }
     __device__ __forceinline__ void gradient(double mjr, const double v[6]) {
-        for (int c = 0; c < 6; ++c) g[c] += mjr * v[c];
+        for (int c = 0; c < 6; ++c) g[c] = fma(mjr, v[c], g[c]);
     }
     __device__ __forceinline__ void stresses(double mj, double vx, double vy, double vz) {
-        ax += mj * vx;
-        ay += mj * vy;
-        az += mj * vz;
+        ax = fma(mj, vx, ax);
+        ay = fma(mj, vy, ay);
+        az = fma(mj, vz, az);
     }
     __device__ __forceinline__ void viscosity(double mj, double vx, double vy, double vz, double heat) {
-        ax -= mj * vx;
-        ay -= mj * vy;
-        az -= mj * vz;
-        du += mj * heat;
+        ax = fma(mj, -vx, ax);
+        ay = fma(mj, -vy, ay);
+        az = fma(mj, -vz, az);
+        du = fma(mj, heat, du);
     }
 };
 
@@ -1315,38 +1277,56 @@ __device__ __forceinline__ void pairs_fp64_body(size_t t, DevState s, const Para
     uint32_t cnt = valid ? count[k] : 0u;
     const uint32_t listed = cnt < kmax ? cnt : kmax;
     const bool solid = prm.solid_stress != 0;
-    auto term = [&](const PairRec& o, uint32_t k2, auto& sum) {
-        const double rx = me.x - o.x, ry = me.y - o.y, rz = me.z - o.z;
-        const double hbar = 0.5 * (me.h + o.h);
-        const double hInv = 1.0 / hbar;
-        const double hInv2 = hInv * hInv;
-        const double d2 = rx * rx + ry * ry + rz * rz;
-        const double gk = lut_grad(lut, d2 * hInv2);
+    struct Early {
+        double rx, ry, rz, hbar, hInv, hInv2, d2;
+        LutPair lut;
+        uint32_t group;
+    };
+    // the fused multiply-adds are written out: which products fuse must not depend on the instance, as the sums
+    // are the same bits with one lane and with a group
+    auto early = [&](const PairRec& o, uint32_t k2) {
+#pragma clang fp contract(off)
+        Early a;
+        a.rx = me.x - o.x, a.ry = me.y - o.y, a.rz = me.z - o.z;
+        a.hbar = 0.5 * (me.h + o.h);
+        a.hInv = 1.0 / a.hbar;
+        a.hInv2 = a.hInv * a.hInv;
+        a.d2 = fma(a.rz, a.rz, fma(a.rx, a.rx, a.ry * a.ry));
+        a.lut = lut_fetch(lut, a.d2 * a.hInv2);
+        a.group = solid ? group[k2] : 0u;
+        return a;
+    };
+    auto term = [&](const PairRec& o, const Early& a, auto& sum) {
+#pragma clang fp contract(off)
+        const double rx = a.rx, ry = a.ry, rz = a.rz, hbar = a.hbar, hInv = a.hInv, hInv2 = a.hInv2, d2 = a.d2;
+        const double gk = a.lut.value();
         const double h5g = (hInv2 * hInv2) * hInv * gk;
         const double gx = rx * h5g, gy = ry * h5g, gz = rz * h5g;
         const double wx = o.vx - me.vx, wy = o.vy - me.vy, wz = o.vz - me.vz;  // v_j - v_i
         const double mj = o.m;
         const double mjr = mj * rhoInv;
         sum.factors(mj, mjr);
-        sum.divergence(mjr, wx * gx + wy * gy + wz * gz);
+        const double wg = fma(wz, gz, fma(wx, gx, wy * gy));
+        sum.divergence(mjr, wg);
         const double coef = me.pr + o.pr;
         sum.pressure(mj, coef * gx, coef * gy, coef * gz);
-        if (solid && gi == group[k2] && gi != NO_GROUP) {
-            const double gv[6] = { wx * gx, wy * gy, wz * gz, 0.5 * (wx * gy + wy * gx), 0.5 * (wx * gz + wz * gx),
-                                   0.5 * (wy * gz + wz * gy) };
+        if (solid && gi == a.group && gi != NO_GROUP) {
+            const double gv[6] = { wx * gx, wy * gy, wz * gz, 0.5 * fma(wx, gy, wy * gx), 0.5 * fma(wx, gz, wz * gx),
+                                   0.5 * fma(wy, gz, wz * gy) };
             sum.gradient(mjr, gv);
             const double xx = me.sxx + o.sxx, yy = me.syy + o.syy, xy = me.sxy + o.sxy;
             const double xz = me.sxz + o.sxz, yz = me.syz + o.syz;
-            sum.stresses(mj, xx * gx + xy * gy + xz * gz, xy * gx + yy * gy + yz * gz, xz * gx + yz * gy + (-xx - yy) * gz);
+            sum.stresses(mj, fma(xz, gz, fma(xx, gx, xy * gy)), fma(yz, gz, fma(yy, gy, xy * gx)),
+                         fma(-xx - yy, gz, fma(xz, gx, yz * gy)));
         }
         // artificial viscosity, only in convergent flow
-        const double dvdr = -(wx * rx + wy * ry + wz * rz);  // (v_i - v_j) . (r_i - r_j)
+        const double dvdr = -fma(wz, rz, fma(wx, rx, wy * ry));  // (v_i - v_j) . (r_i - r_j)
         if (dvdr < 0.0) {
             const double rhobar = 0.5 * (me.rho + o.rho);
             const double csbar = 0.5 * (me.cs + o.cs);
-            const double mu = hbar * dvdr / (d2 + 1.e-2 * (hbar * hbar));
-            const double av = (-prm.av_alpha * csbar * mu + prm.av_beta * (mu * mu)) / rhobar;
-            sum.viscosity(mj, av * gx, av * gy, av * gz, 0.5 * av * -(wx * gx + wy * gy + wz * gz));
+            const double mu = hbar * dvdr / fma(1.e-2, hbar * hbar, d2);
+            const double av = fma(prm.av_beta, mu * mu, -(prm.av_alpha * csbar * mu)) / rhobar;
+            sum.viscosity(mj, av * gx, av * gy, av * gz, 0.5 * av * -wg);
         }
     };
     PairAcc64 ps;
@@ -1354,17 +1334,18 @@ __device__ __forceinline__ void pairs_fp64_body(size_t t, DevState s, const Para
         __shared__ PairTerms64 rows[BLOCK];
         __shared__ double all[BLOCK / LANES][PAIR_SUMS];
         double acc[GROUP_SUMS<LANES>] = {};
-        sum_shared<LANES>(rec, list, k, kmax >> 2, listed, sub, rows + threadIdx.x / LANES * LANES, acc, term);
+        sum_shared<LANES>(rec, list, k, kmax >> 2, listed, sub, rows + threadIdx.x / LANES * LANES, acc,
+                          [&](const PairRec& o, uint32_t k2, auto& sum) { term(o, early(o, k2), sum); });
         collect_shared<LANES>(acc, sub, all, ps);
         // from here on thread p of the block goes on with its particle p
         k = (t - threadIdx.x) / LANES + threadIdx.x;
         valid = threadIdx.x < blockDim.x / LANES && k < n;
         if (valid) cnt = count[k];
     } else {
-        __shared__ uint4 stage[PAIRS64_STAGE ? (BLOCK / 64) * StageOf<PairRec>::WORDS : 1];
-        uint4* my_stage = PAIRS64_STAGE ? stage + (threadIdx.x >> 6) * StageOf<PairRec>::WORDS : stage;
-        for_each_neighbor<PAIRS64_STAGE>(rec, list, k, kmax >> 2, listed, my_stage,
-                                         [&](const PairRec& o, uint32_t k2) { term(o, k2, ps); });
+        __shared__ uint4 stage[(BLOCK / 64) * StageOf<PairRec>::WORDS];
+        uint4* my_stage = stage + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * StageOf<PairRec>::WORDS;
+        for_each_neighbor(rec, list, k, kmax >> 2, listed, my_stage,
+                          early, [&](const PairRec& o, uint32_t, const Early& a) { term(o, a, ps); });
     }
     pairs_finish<FUSED>(s, prm, order, k, valid, cnt, ps, fa);
 }
@@ -1547,12 +1528,11 @@ __device__ __forceinline__ void pairs_mixed_body(size_t t, DevState s, const Par
         valid = threadIdx.x < blockDim.x / LANES && k < n;
         if (valid) cnt = count[k];
     } else {
-        // the LDS stage exists whenever the gather mode uses it (one uint4 otherwise)
-        constexpr bool STAGE = PAIRSMX_STAGE == 1 || PAIRSMX_STAGE == 2;
-        __shared__ uint4 stage[STAGE ? (BLOCK / 64) * StageOf<PairRecF>::WORDS : 1];
-        uint4* my_stage = STAGE ? stage + (threadIdx.x >> 6) * StageOf<PairRecF>::WORDS : stage;
-        for_each_neighbor<PAIRSMX_STAGE>(rec, list, k, kmax >> 2, listed, my_stage,
-                                         [&](const PairRecF& o, uint32_t e) { term(o, e, ps); });
+        __shared__ uint4 stage[(BLOCK / 64) * StageOf<PairRecF>::WORDS];
+        uint4* my_stage = stage + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * StageOf<PairRecF>::WORDS;
+        for_each_neighbor(rec, list, k, kmax >> 2, listed, my_stage,
+                          [](const PairRecF&, uint32_t) { return 0; },
+                          [&](const PairRecF& o, uint32_t e, int) { term(o, e, ps); });
     }
     pairs_finish<FUSED>(s, prm, order, k, valid, cnt, ps, fa);
 }
