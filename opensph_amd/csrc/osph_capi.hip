@@ -43,24 +43,20 @@ struct BatchPlan {
     BatchMember* host = nullptr;
     unsigned long long* small = nullptr;
     Mailbox box;  // host mirror of small
-    uint64_t *keys = nullptr, *keys_sorted = nullptr;
-    uint32_t *vals = nullptr, *vals_sorted = nullptr;
-    void* sort_temp = nullptr;
-    size_t sort_temp_bytes = 0;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
-    int graph_bits = -1, graph_screened = -1, graph_plain = -1;
+    int graph_screened = -1, graph_plain = -1;
 
     void drop_graph() {
         if (exec) (void)hipGraphExecDestroy(exec);
         if (graph) (void)hipGraphDestroy(graph);
         exec = nullptr;
         graph = nullptr;
-        graph_bits = graph_screened = graph_plain = -1;
+        graph_screened = graph_plain = -1;
     }
     ~BatchPlan() {
         drop_graph();
-        void* dp[] = { tables, dev, small, keys, keys_sorted, vals, vals_sorted, sort_temp };
+        void* dp[] = { tables, dev, small };
         for (void* p : dp) (void)hipFree(p);
         if (host) (void)hipHostFree(host);
         mailbox_destroy(box);
@@ -90,14 +86,12 @@ struct osph_ctx {
     int since_reorder = 0;
 
     // neighbour structures (all sized for cap particles)
-    uint32_t *keys_sorted = nullptr, *order = nullptr;  // keys_sorted: batched steps
+    uint32_t* order = nullptr;
     uint2 *where = nullptr, *bucket = nullptr;          // rows of the particles, and their buckets (launch_cell_sort)
     const char* failed_launch = nullptr;  // name of the first timed launch that left a HIP error
     uint32_t *row_count = nullptr, *row_start = nullptr;  // [slot_cap] counts (zero between searches) and their sums
     size_t slot_cap = 0;
     uint32_t* cell_first = nullptr;  // [cells + 1]: first sorted position of each cell (valid rows only)
-    uint32_t* row_range = nullptr;   // [2 rows]: sorted range of each row of cells (batched steps)
-    size_t row_cap = 0;
     size_t cell_cap = 0;
     PairRec* rec = nullptr;
     PairRecF* recf = nullptr;
@@ -220,7 +214,6 @@ void free_state(osph_ctx* c) {
     c->dblock2 = nullptr;
     c->ublock2 = nullptr;
     c->perm = c->perm2 = c->slot_of = nullptr;
-    (void)hipFree(c->keys_sorted);
     (void)hipFree(c->where);
     (void)hipFree(c->bucket);
     (void)hipFree(c->order);
@@ -232,7 +225,7 @@ void free_state(osph_ctx* c) {
     (void)hipFree(c->count);
     c->dblock = nullptr;
     c->ublock = nullptr;
-    c->keys_sorted = c->order = nullptr;
+    c->order = nullptr;
     c->where = c->bucket = nullptr;
     c->rec = nullptr;
     c->recf = nullptr;
@@ -263,16 +256,6 @@ int ensure_list(osph_ctx* c, size_t entries) {
     c->list_cap = 0;
     HIPCHK(c, hipMalloc(&c->list, entries * sizeof(uint32_t)));
     c->list_cap = entries;
-    return OSPH_OK;
-}
-
-int ensure_rows(osph_ctx* c, size_t rows) {
-    if (rows <= c->row_cap) return OSPH_OK;
-    (void)hipFree(c->row_range);
-    c->row_range = nullptr;
-    c->row_cap = 0;
-    HIPCHK(c, hipMalloc(&c->row_range, 2 * rows * sizeof(uint32_t)));
-    c->row_cap = rows;
     return OSPH_OK;
 }
 
@@ -603,15 +586,12 @@ int plan_search(osph_ctx* c, const unsigned long long* sh, size_t* rows_out) {
         base += uint32_t(rows_end);
         g.slots += uint32_t(rows_end >> bits);
     }
-    g.key_bits = 1;
-    while (g.key_bits < 32 && (uint64_t(1) << g.key_bits) < uint64_t(base)) ++g.key_bits;
     c->grid = g;
     if (int e = ensure_cells(c, size_t(base))) return e;
     size_t rows = 0;
     for (int cl = 0; cl < g.nclass; ++cl) {
         if (!g.c[cl].empty) rows += size_t(g.c[cl].dim[1]) * size_t(g.c[cl].dim[2]);
     }
-    if (int e = ensure_rows(c, rows)) return e;
     *rows_out = rows;
     if (c->cfg.precision == OSPH_PRECISION_MIXED) {
         // fixed-point frames: the smallest power-of-two steps with the position and velocity boxes within
@@ -1010,7 +990,6 @@ void osph_destroy(osph_ctx* c) {
     if (c->grav_done) (void)hipEventDestroy(c->grav_done);
     free_state(c);
     (void)hipFree(c->cell_first);
-    (void)hipFree(c->row_range);
     (void)hipFree(c->row_count);
     (void)hipFree(c->row_start);
     (void)hipFree(c->list);
@@ -1048,7 +1027,6 @@ int osph_resize(osph_ctx* c, size_t n) {
         HIPCHK(c, hipMalloc(&c->perm, sizeof(uint32_t) * cap));
         HIPCHK(c, hipMalloc(&c->perm2, sizeof(uint32_t) * cap));
         HIPCHK(c, hipMalloc(&c->slot_of, sizeof(uint32_t) * cap));
-        HIPCHK(c, hipMalloc(&c->keys_sorted, sizeof(uint32_t) * cap));
         HIPCHK(c, hipMalloc(&c->where, sizeof(uint2) * cap));
         HIPCHK(c, hipMalloc(&c->bucket, sizeof(uint2) * cap));
         HIPCHK(c, hipMalloc(&c->order, sizeof(uint32_t) * cap));
@@ -1392,13 +1370,6 @@ int make_plan(const std::vector<osph_ctx*>& ms, BatchPlan*& out) {
         P->total += c->n;
     }
     if (P->total >= (size_t(1) << 32)) return lead->fail(OSPH_ERR_ARG, "a batch must hold fewer than 2^32 particles");
-    HIPCHK(lead, hipMalloc(&P->keys, P->total * sizeof(uint64_t)));
-    HIPCHK(lead, hipMalloc(&P->keys_sorted, P->total * sizeof(uint64_t)));
-    HIPCHK(lead, hipMalloc(&P->vals, P->total * sizeof(uint32_t)));
-    HIPCHK(lead, hipMalloc(&P->vals_sorted, P->total * sizeof(uint32_t)));
-    // sized once for the widest key, so that the captured graph's arguments stay valid
-    P->sort_temp_bytes = std::max<size_t>(sort_pairs64_temp_bytes(P->total, 64), 256);
-    HIPCHK(lead, hipMalloc(&P->sort_temp, P->sort_temp_bytes));
     out = P;
     return OSPH_OK;
 }
@@ -1450,32 +1421,29 @@ int batch_step(const std::vector<osph_ctx*>& ms, const std::vector<double>& dts,
     mailbox_post(st, P->box, 0, P->small, count * SMALL_WORDS);
     if (int e = wait_box(lead, P->box)) return e;
     // each member's grid, screen and fixed-point frames, planned as its own search plans them
-    int key_bits = 1;
     bool screened = false, plain = false;
-    uint32_t off = 0;
     for (size_t k = 0; k < count; ++k) {
         osph_ctx* c = ms[k];
         BatchMember& b = P->host[k];
         size_t rows = 0;
         if (int e = plan_search(c, P->box.host + SMALL_WORDS * k, &rows)) return e;
         if (int e = ensure_list(c, list_entries(c->n, c->kmax))) return e;
-        int xslots = 1;
-        for (int cl = 0; cl < c->grid.nclass; ++cl) {
-            if (!c->grid.c[cl].empty) xslots = std::max(xslots, c->grid.c[cl].dim[0] + 1);
-        }
+        const size_t slots_before = c->slot_cap;
+        if (int e = ensure_slots(c, c->grid.slots)) return e;
+        // new counts are cleared on the member's stream, the batch runs on the lead's
+        if (c->slot_cap != slots_before) HIPCHK(c, hipStreamSynchronize(c->stream));
         b.grid = c->grid;
         b.screen = c->screen;
         b.fx = c->fixed;
         b.kmax = c->kmax;
         b.rows = uint32_t(rows);
-        b.xslots = xslots;
         b.reorder = reorder_due(c) ? 1 : 0;
         b.s2 = b.reorder ? other_state(c) : c->s;
-        b.key_off = off;
-        off += uint32_t(c->n);
-        b.keys_sorted = c->keys_sorted;
         b.order = c->order;
-        b.row_range = c->row_range;
+        b.row_count = c->row_count;
+        b.row_start = c->row_start;
+        b.where = c->where;
+        b.bucket = c->bucket;
         b.cell_first = c->cell_first;
         b.perm = c->perm;
         b.perm2 = c->perm2;
@@ -1486,21 +1454,14 @@ int batch_step(const std::vector<osph_ctx*>& ms, const std::vector<double>& dts,
         b.group = c->group;
         b.list = c->list;
         b.count = c->count;
-        key_bits = std::max(key_bits, c->grid.key_bits);
         (b.screen.on ? screened : plain) = true;
     }
-    int member_bits = 0;
-    while ((size_t(1) << member_bits) < count) ++member_bits;
     HIPCHK(lead, hipMemcpyAsync(P->dev, P->host, count * sizeof(BatchMember), hipMemcpyHostToDevice, st));
-    batch_cell_keys(l, P->dev, P->pb, key_bits, P->keys, P->vals);
-    HIPCHK(lead, sort_pairs64(l, P->sort_temp, P->sort_temp_bytes, P->keys, P->keys_sorted, P->vals, P->vals_sorted,
-                              P->total, key_bits + member_bits));
     const bool fuse = P->tune.fuse_finalize == 1 || (P->tune.fuse_finalize == -1 && !P->mixed);
-    // the stages after the sort: their launch shapes and arguments are fixed for the plan (the per-step
+    // the stages from the sort on: their launch shapes and arguments are fixed for the plan (the per-step
     // values are in the member table), so they are captured once and replayed
     auto rest = [&]() {
-        batch_split(l, P->dev, P->pb, key_bits, P->keys_sorted, P->vals_sorted);
-        batch_cells(l, P->dev, P->pb);
+        batch_sort(l, P->dev, int(count), P->pb);
         batch_permute(l, P->dev, P->pb);
         batch_pack(l, P->dev, P->pb, P->mixed);
         batch_lists(l, P->dev, P->lb, screened, plain);
@@ -1508,14 +1469,12 @@ int batch_step(const std::vector<osph_ctx*>& ms, const std::vector<double>& dts,
         if (!fuse) batch_finalize_correct(l, P->dev, P->pb);
     };
     if (P->tune.batch_graph) {
-        if (!P->exec || P->graph_bits != key_bits || P->graph_screened != int(screened) ||
-            P->graph_plain != int(plain)) {
+        if (!P->exec || P->graph_screened != int(screened) || P->graph_plain != int(plain)) {
             P->drop_graph();
             HIPCHK(lead, hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
             rest();
             HIPCHK(lead, hipStreamEndCapture(st, &P->graph));
             HIPCHK(lead, hipGraphInstantiate(&P->exec, P->graph, nullptr, nullptr, 0));
-            P->graph_bits = key_bits;
             P->graph_screened = int(screened);
             P->graph_plain = int(plain);
         }

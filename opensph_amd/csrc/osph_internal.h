@@ -90,17 +90,15 @@ struct GridClass {
     double cell, inv_cell;
     int dim[3];
     int bits;             // 2^bits > every dim: x slots per row, and the width of y and z in the row key
-    uint32_t base;        // offset of the class's cells in the cell tables and in the sort keys
+    uint32_t base;        // offset of the class's cells in the cell tables
     uint32_t slot0;       // offset of the class's rows (by the Morton code of y, z) in the row arrays
     int empty;
 };
 
-// The sort key of a particle is its cell index: base(class) + row_key(x, y, z), the classes' key ranges
-// packed back to back (each as long as its largest row key + 1), so the keys are dense and as short
-// as the cell count allows (fewer radix-sort passes).
+// A particle's cell index is base(class) + row_key(x, y, z), the classes' ranges packed back to back (each as long as its
+// largest row key + 1).
 struct Grid {
     int nclass;
-    int key_bits;  // bits of the sort key that can be nonzero
     uint32_t slots;  // rows of all classes, by their Morton codes
     double hmin;
     GridClass c[MAX_CLASSES];
@@ -340,12 +338,11 @@ struct BatchMember {
     Fixed fx;
     uint32_t n, kmax;
     uint32_t rows;    // rows of the member's grid (all classes)
-    int xslots;       // largest dim_x + 1 over its classes
     int reorder;      // this step moves the state into cell order (s -> s2)
-    uint32_t key_off; // first position of the member in the batch's sort arrays
     unsigned long long* small;  // accumulators (SMALL_* layout)
     unsigned long long* part;   // per-block partial bounds
-    uint32_t *keys_sorted, *order, *row_range, *cell_first;
+    uint32_t *order, *cell_first, *row_count, *row_start;
+    uint2 *where, *bucket;
     uint32_t *perm, *perm2, *slot_of;
     void* rec;        // PairRec (FP64) or PairRecF (mixed precision)
     double4* pos;
@@ -370,11 +367,7 @@ inline uint32_t batch_blocks_for(size_t n, int block) {
 // Stage launchers over all `count` members (M in device memory).  `pb`: blocks of BLOCK threads per
 // particle; `lb`: blocks of the list kernel's size; `qb`: blocks of the pair kernel's size and lanes.
 void batch_advance(const Launch& l, const BatchMember* M, int count, BatchBlocks pb, bool vel);
-void batch_cell_keys(const Launch& l, const BatchMember* M, BatchBlocks pb, int key_bits, uint64_t* keys,
-                     uint32_t* vals);
-void batch_split(const Launch& l, const BatchMember* M, BatchBlocks pb, int key_bits, const uint64_t* keys,
-                 const uint32_t* vals);
-void batch_cells(const Launch& l, const BatchMember* M, BatchBlocks pb);
+void batch_sort(const Launch& l, const BatchMember* M, int count, BatchBlocks pb);
 void batch_permute(const Launch& l, const BatchMember* M, BatchBlocks pb);
 void batch_pack(const Launch& l, const BatchMember* M, BatchBlocks pb, bool mixed);
 void batch_lists(const Launch& l, const BatchMember* M, BatchBlocks lb, bool screened, bool plain);
@@ -382,9 +375,6 @@ void batch_lists(const Launch& l, const BatchMember* M, BatchBlocks lb, bool scr
 void batch_pairs(const Launch& l, const BatchMember* M, BatchBlocks qb, bool mixed, bool fuse, int lanes,
                  const double* lut);
 void batch_finalize_correct(const Launch& l, const BatchMember* M, BatchBlocks pb);
-size_t sort_pairs64_temp_bytes(size_t n, int key_bits);
-hipError_t sort_pairs64(const Launch& l, void* temp, size_t temp_bytes, const uint64_t* keys_in, uint64_t* keys_out,
-                        const uint32_t* vals_in, uint32_t* vals_out, size_t n, int key_bits);
 
 // Grady-Kipp flaws of one body on the device (osph_set_flaws): flaw p (1-based) hits particle
 // flaw_target(seed, p, nb); the first pass records first[i] = min p (first initialised to ~0), cover

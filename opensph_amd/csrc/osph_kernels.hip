@@ -8,7 +8,6 @@
 #include "osph_device.h"
 #include "osph_internal.h"
 
-#include <rocprim/device/device_radix_sort.hpp>
 
 namespace osph {
 
@@ -249,34 +248,10 @@ __device__ __forceinline__ void cell_of(const GridClass& g, double x, double y, 
     }
 }
 
-__device__ __forceinline__ uint32_t cell_key_of(const DevState& s, const Grid& g, size_t i) {
-    const int cls = h_class(s.d[H][i], g.hmin, g.nclass);
-    int c[3];
-    cell_of(g.c[cls], s.d[X][i], s.d[Y][i], s.d[Z][i], c);
-    return g.c[cls].base + row_key(uint32_t(c[0]), uint32_t(c[1]), uint32_t(c[2]), g.c[cls].bits);
-}
-
 __global__ void __launch_bounds__(BLOCK) k_fill_u32(uint32_t* p, size_t count, uint32_t value) {
     for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < count; i += size_t(gridDim.x) * blockDim.x) {
         p[i] = value;
     }
-}
-
-// Cell index of a sort key (the key itself: keys are dense cell indices, monotonic in sorted order).
-__device__ __forceinline__ uint32_t cell_index(const Grid&, uint32_t key) { return key; }
-
-// First sorted position in [lo, hi) whose cell index is >= c (hi when none is).
-__device__ __forceinline__ uint32_t first_at_least(const uint32_t* __restrict__ keys, const Grid& g, uint32_t c,
-                                                   uint32_t lo, uint32_t hi) {
-    while (lo < hi) {
-        const uint32_t mid = lo + ((hi - lo) >> 1);
-        if (cell_index(g, keys[mid]) < c) {
-            lo = mid + 1;
-        } else {
-            hi = mid;
-        }
-    }
-    return lo;
 }
 
 // Row q of the grid (rows of all non-empty classes numbered in turn): its class, y and z.
@@ -296,17 +271,6 @@ __device__ __forceinline__ bool row_of(const Grid& g, size_t q, int& cls, uint32
     return false;
 }
 
-__device__ __forceinline__ void row_range_at(const uint32_t* __restrict__ keys, const Grid& g,
-                                             uint32_t* __restrict__ range, size_t q, uint32_t n) {
-    int cls;
-    uint32_t cy, cz;
-    if (!row_of(g, q, cls, cy, cz)) return;
-    const GridClass& G = g.c[cls];
-    const uint32_t row = G.base + row_key(0u, cy, cz, G.bits);
-    range[2 * q] = first_at_least(keys, g, row, 0u, n);
-    range[2 * q + 1] = first_at_least(keys, g, row + (1u << G.bits), 0u, n);
-}
-
 // ---- sort by cell and cell table ------------------------------------------------------------------------
 // The order of the particles by cell and the cell table, by rows of cells: a row (slot0(class) + Morton(y, z), the
 // sort key without x) is a bucket, and a row's particles are ordered by (x, particle) on their own.  Four launches
@@ -317,9 +281,8 @@ __device__ __forceinline__ void row_range_at(const uint32_t* __restrict__ keys, 
 // The buckets are filled with atomics, in any order; the order within a row does not depend on it.
 
 // Counts the particles of every row: where[i] = (row << 8 | x, rank in the row).  One atomic per row and wavefront.
-__global__ void __launch_bounds__(BLOCK) k_row_count(DevState s, Grid g, uint32_t* __restrict__ row_count,
-                                                     uint2* __restrict__ where, size_t n) {
-    const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void row_count_at(const DevState& s, const Grid& g, uint32_t* __restrict__ row_count,
+                                             uint2* __restrict__ where, size_t i, size_t n) {
     const bool valid = i < n;
     const uint32_t lane = threadIdx.x & 63u;
     uint32_t row = 0xffffffffu, x = 0;
@@ -348,17 +311,22 @@ __global__ void __launch_bounds__(BLOCK) k_row_count(DevState s, Grid g, uint32_
     if (valid) where[i] = make_uint2((row << 8) | x, base + before);
 }
 
+__global__ void __launch_bounds__(BLOCK) k_row_count(DevState s, Grid g, uint32_t* __restrict__ row_count,
+                                                     uint2* __restrict__ where, size_t n) {
+    row_count_at(s, g, row_count, where, size_t(blockIdx.x) * blockDim.x + threadIdx.x, n);
+}
+
 // row_start = exclusive prefix sums of the counts (slots + 1 entries).  Block b sums the counts before its tile of
 // SCAN_TILE itself, and scans its tile: no second pass and no waiting for other blocks (53k slots at the 1M impact:
 // 14 blocks, the last reading 230 KB; one block stepping through all of them took 25 us).
 constexpr uint32_t SCAN_BLOCK = 1024, SCAN_TILE = 4 * SCAN_BLOCK;
-__global__ void __launch_bounds__(SCAN_BLOCK) k_row_scan(const uint32_t* __restrict__ row_count,
-                                                         uint32_t* __restrict__ row_start) {
+__device__ __forceinline__ void row_scan_tile(const uint32_t* __restrict__ row_count, uint32_t* __restrict__ row_start,
+                                              uint32_t block) {
     __shared__ uint32_t wave_sum[2][SCAN_BLOCK / 64];
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     // the arrays hold whole tiles, the entries past the last row zero
     const uint4* in = reinterpret_cast<const uint4*>(row_count);
-    const uint32_t tile = blockIdx.x * SCAN_BLOCK;  // in quads
+    const uint32_t tile = block * SCAN_BLOCK;  // in quads
     uint32_t prior = 0;
     for (uint32_t t = threadIdx.x; t < tile; t += SCAN_BLOCK) {
         const uint4 q = in[t];
@@ -387,17 +355,28 @@ __global__ void __launch_bounds__(SCAN_BLOCK) k_row_scan(const uint32_t* __restr
     reinterpret_cast<uint4*>(row_start)[tile + threadIdx.x] = o;
 }
 
+__global__ void __launch_bounds__(SCAN_BLOCK) k_row_scan(const uint32_t* __restrict__ row_count,
+                                                         uint32_t* __restrict__ row_start) {
+    row_scan_tile(row_count, row_start, blockIdx.x);
+}
+
 // bucket[row_start + rank] = (particle, x): x in the high word, so that the 64-bit values order by (x, particle).
 // The counts go back to zero for the next search.
+__device__ __forceinline__ void row_scatter_at(const uint2* __restrict__ where, const uint32_t* __restrict__ row_start,
+                                               uint32_t* __restrict__ row_count, uint32_t slots,
+                                               uint2* __restrict__ bucket, size_t i, size_t threads, size_t n) {
+    for (size_t t = i; t < slots; t += threads) row_count[t] = 0u;
+    if (i >= n) return;
+    const uint2 w = where[i];
+    bucket[row_start[w.x >> 8] + w.y] = make_uint2(uint32_t(i), w.x & 255u);
+}
+
 __global__ void __launch_bounds__(BLOCK) k_row_scatter(const uint2* __restrict__ where,
                                                        const uint32_t* __restrict__ row_start,
                                                        uint32_t* __restrict__ row_count, uint32_t slots,
                                                        uint2* __restrict__ bucket, size_t n) {
-    const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    for (size_t t = i; t < slots; t += size_t(gridDim.x) * blockDim.x) row_count[t] = 0u;
-    if (i >= n) return;
-    const uint2 w = where[i];
-    bucket[row_start[w.x >> 8] + w.y] = make_uint2(uint32_t(i), w.x & 255u);
+    row_scatter_at(where, row_start, row_count, slots, bucket, size_t(blockIdx.x) * blockDim.x + threadIdx.x,
+                   size_t(gridDim.x) * blockDim.x, n);
 }
 
 // Ascending sort of v[0..m) by the block: bitonic with every comparator directed upwards (the first step of each
@@ -432,9 +411,9 @@ struct RowStage {
     uint32_t start[256];      // counts by x, then their exclusive prefix sums
     uint32_t idx[ROW_WAVE];   // particles placed by cell
 };
-__global__ void __launch_bounds__(BLOCK) k_row_order(Grid g, const uint32_t* __restrict__ row_start,
-                                                     uint2* __restrict__ bucket, uint32_t* __restrict__ order,
-                                                     uint32_t* __restrict__ first, size_t rows) {
+__device__ __forceinline__ void row_order_block(const Grid& g, const uint32_t* __restrict__ row_start,
+                                                uint2* __restrict__ bucket, uint32_t* __restrict__ order,
+                                                uint32_t* __restrict__ first, size_t rows, size_t block) {
     constexpr int WAVES = BLOCK / 64;
     union Lds {
         RowStage stage[WAVES];
@@ -443,7 +422,7 @@ __global__ void __launch_bounds__(BLOCK) k_row_order(Grid g, const uint32_t* __r
     __shared__ Lds lds;
     __shared__ uint32_t long_row[WAVES][4];  // first position, particles, cell base and dim_x of a long row
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63u;
-    const size_t q = size_t(blockIdx.x) * WAVES + wave;
+    const size_t q = block * WAVES + wave;
     int cls = 0;
     uint32_t cy = 0, cz = 0;
     const bool valid = q < rows && row_of(g, q, cls, cy, cz);
@@ -539,20 +518,10 @@ __global__ void __launch_bounds__(BLOCK) k_row_order(Grid g, const uint32_t* __r
     }
 }
 
-// One thread per cell x in [0, dim_x] of a row: the binary search runs inside the row's own range.
-__device__ __forceinline__ void cell_first_at(const uint32_t* __restrict__ keys, const Grid& g,
-                                              const uint32_t* __restrict__ range, uint32_t* __restrict__ first,
-                                              size_t t, size_t rows, int xslots) {
-    const size_t q = t / size_t(xslots);
-    const uint32_t x = uint32_t(t % size_t(xslots));
-    if (q >= rows) return;
-    int cls;
-    uint32_t cy, cz;
-    if (!row_of(g, q, cls, cy, cz)) return;
-    const GridClass& G = g.c[cls];
-    if (x > uint32_t(G.dim[0])) return;
-    const uint32_t cell = G.base + row_key(x, cy, cz, G.bits);
-    first[cell] = first_at_least(keys, g, cell, range[2 * q], range[2 * q + 1]);
+__global__ void __launch_bounds__(BLOCK) k_row_order(Grid g, const uint32_t* __restrict__ row_start,
+                                                     uint2* __restrict__ bucket, uint32_t* __restrict__ order,
+                                                     uint32_t* __restrict__ first, size_t rows) {
+    row_order_block(g, row_start, bucket, order, first, rows, blockIdx.x);
 }
 
 // Pack the neighbour-side data of particle order[k] into rec[k].
@@ -2373,45 +2342,36 @@ __global__ void __launch_bounds__(BLOCK) kb_bounds_final(const BatchMember* __re
     bounds_final_at(vi, a.part, pb.first[m + 1] - pb.first[m], a.small + SMALL_CLASSES, a.small + SMALL_VEL);
 }
 
-// The sort key of a batch holds the member above the member's own cell key, so that one sort groups the
-// particles by member and, within a member, orders them as the member's own sort does (stable, by slot).
-__global__ void __launch_bounds__(BLOCK) kb_cell_keys(const BatchMember* __restrict__ M, BatchBlocks pb, int key_bits,
-                                                      uint64_t* __restrict__ keys, uint32_t* __restrict__ vals) {
+// The four launches of a member's own sort, on each member's rows: 16 members of 5k to 212k particles 190 -> 45 us,
+// against one radix sort of all members' keys and two kernels for the tables, 24 launches.
+__global__ void __launch_bounds__(BLOCK) kb_row_count(const BatchMember* __restrict__ M, BatchBlocks pb) {
     uint32_t m, bid, nb;
     const BatchMember& a = batch_block(M, pb, m, bid, nb);
-    const size_t i = size_t(bid) * BLOCK + threadIdx.x;
-    if (i >= a.n) return;
-    const uint32_t at = a.key_off + uint32_t(i);
-    keys[at] = (uint64_t(m) << key_bits) | uint64_t(cell_key_of(a.s, a.grid, i));
-    vals[at] = at;
+    row_count_at(a.s, a.grid, a.row_count, a.where, size_t(bid) * BLOCK + threadIdx.x, a.n);
 }
 
-// The member's part of the sorted arrays: its cell keys and its slot order.
-__global__ void __launch_bounds__(BLOCK) kb_split(const BatchMember* __restrict__ M, BatchBlocks pb, int key_bits,
-                                                  const uint64_t* __restrict__ keys, const uint32_t* __restrict__ vals) {
-    uint32_t m, bid, nb;
-    const BatchMember& a = batch_block(M, pb, m, bid, nb);
-    const size_t j = size_t(bid) * BLOCK + threadIdx.x;
-    if (j >= a.n) return;
-    const uint32_t at = a.key_off + uint32_t(j);
-    a.keys_sorted[j] = uint32_t(keys[at] & ((uint64_t(1) << key_bits) - 1));
-    a.order[j] = vals[at] - a.key_off;
-}
-
-__global__ void __launch_bounds__(BLOCK) kb_row_range(const BatchMember* __restrict__ M, BatchBlocks pb) {
-    uint32_t m, bid, nb;
-    const BatchMember& a = batch_block(M, pb, m, bid, nb);
-    for (size_t q = size_t(bid) * BLOCK + threadIdx.x; q < a.rows; q += size_t(nb) * BLOCK) {
-        row_range_at(a.keys_sorted, a.grid, a.row_range, q, a.n);
+constexpr unsigned SCAN_BLOCKS = 8;  // per member, over its tiles
+__global__ void __launch_bounds__(SCAN_BLOCK) kb_row_scan(const BatchMember* __restrict__ M) {
+    const BatchMember& a = M[blockIdx.y];
+    for (uint32_t t = blockIdx.x; t < a.grid.slots / SCAN_TILE + 1u; t += SCAN_BLOCKS) {
+        row_scan_tile(a.row_count, a.row_start, t);
+        __syncthreads();
     }
 }
 
-__global__ void __launch_bounds__(BLOCK) kb_cell_first(const BatchMember* __restrict__ M, BatchBlocks pb) {
+__global__ void __launch_bounds__(BLOCK) kb_row_scatter(const BatchMember* __restrict__ M, BatchBlocks pb) {
     uint32_t m, bid, nb;
     const BatchMember& a = batch_block(M, pb, m, bid, nb);
-    const size_t total = size_t(a.rows) * size_t(a.xslots);
-    for (size_t t = size_t(bid) * BLOCK + threadIdx.x; t < total; t += size_t(nb) * BLOCK) {
-        cell_first_at(a.keys_sorted, a.grid, a.row_range, a.cell_first, t, a.rows, a.xslots);
+    row_scatter_at(a.where, a.row_start, a.row_count, a.grid.slots, a.bucket, size_t(bid) * BLOCK + threadIdx.x,
+                   size_t(nb) * BLOCK, a.n);
+}
+
+__global__ void __launch_bounds__(BLOCK) kb_row_order(const BatchMember* __restrict__ M, BatchBlocks pb) {
+    uint32_t m, bid, nb;
+    const BatchMember& a = batch_block(M, pb, m, bid, nb);
+    for (size_t b = bid; b * (BLOCK / 64) < a.rows; b += nb) {
+        row_order_block(a.grid, a.row_start, a.bucket, a.order, a.cell_first, a.rows, b);
+        __syncthreads();
     }
 }
 
@@ -2487,19 +2447,11 @@ void batch_advance(const Launch& l, const BatchMember* M, int count, BatchBlocks
     kb_bounds_final<<<unsigned(count) * unsigned(nv), BLOCK, 0, l.stream>>>(M, pb, nv);
 }
 
-void batch_cell_keys(const Launch& l, const BatchMember* M, BatchBlocks pb, int key_bits, uint64_t* keys,
-                     uint32_t* vals) {
-    kb_cell_keys<<<pb.total, BLOCK, 0, l.stream>>>(M, pb, key_bits, keys, vals);
-}
-
-void batch_split(const Launch& l, const BatchMember* M, BatchBlocks pb, int key_bits, const uint64_t* keys,
-                 const uint32_t* vals) {
-    kb_split<<<pb.total, BLOCK, 0, l.stream>>>(M, pb, key_bits, keys, vals);
-}
-
-void batch_cells(const Launch& l, const BatchMember* M, BatchBlocks pb) {
-    kb_row_range<<<pb.total, BLOCK, 0, l.stream>>>(M, pb);
-    kb_cell_first<<<pb.total, BLOCK, 0, l.stream>>>(M, pb);
+void batch_sort(const Launch& l, const BatchMember* M, int count, BatchBlocks pb) {
+    kb_row_count<<<pb.total, BLOCK, 0, l.stream>>>(M, pb);
+    kb_row_scan<<<dim3(SCAN_BLOCKS, unsigned(count)), SCAN_BLOCK, 0, l.stream>>>(M);
+    kb_row_scatter<<<pb.total, BLOCK, 0, l.stream>>>(M, pb);
+    kb_row_order<<<pb.total, BLOCK, 0, l.stream>>>(M, pb);
 }
 
 void batch_permute(const Launch& l, const BatchMember* M, BatchBlocks pb) {
@@ -2543,21 +2495,6 @@ void batch_pairs(const Launch& l, const BatchMember* M, BatchBlocks qb, bool mix
 
 void batch_finalize_correct(const Launch& l, const BatchMember* M, BatchBlocks pb) {
     kb_finalize_correct<<<pb.total, BLOCK, 0, l.stream>>>(M, pb);
-}
-
-// 64-bit keys (member above cell) of the batched sort, rocPRIM's default configuration.
-size_t sort_pairs64_temp_bytes(size_t n, int key_bits) {
-    size_t bytes = 0;
-    (void)rocprim::radix_sort_pairs(nullptr, bytes, (const uint64_t*)nullptr, (uint64_t*)nullptr,
-                                    (const uint32_t*)nullptr, (uint32_t*)nullptr, n, 0u, unsigned(key_bits));
-    return bytes;
-}
-
-hipError_t sort_pairs64(const Launch& l, void* temp, size_t temp_bytes, const uint64_t* keys_in, uint64_t* keys_out,
-                        const uint32_t* vals_in, uint32_t* vals_out, size_t n, int key_bits) {
-    if (!n) return hipSuccess;
-    return rocprim::radix_sort_pairs(temp, temp_bytes, keys_in, keys_out, vals_in, vals_out, n, 0u,
-                                     unsigned(key_bits), l.stream);
 }
 
 }  // namespace osph
