@@ -190,11 +190,15 @@ struct Tuning {
 // gathers of a single wavefront per SIMD (also when the tuner asks for more than one).  Fused pair kernel in us with
 // 16 / 4 / 1 lanes, gas (one class) and impact: 2k particles FP64 24 / 50 / 98 and 33 / 66 / 149, mixed 15 / 31 / 48;
 // 21k FP64 57 / 60 / 98 and 74 / 90 / 181, mixed 30 / 31 / 48; 43k FP64 103 / 78 / 100 and 138 / 110 / 183, mixed
-// 47 / 36 / 49; 85k FP64 190 / 145 / 118 and 247 / 170 / 201, mixed 87 / 65 / 59.
-constexpr size_t PAIRS_BELOW_16 = 24576, PAIRS_BELOW_4 = 65536;
-inline int pair_lanes(const Tuning& t, size_t n) {
+// 47 / 36 / 49.  From four lanes to one, with the single lanes' records fetched together: gas 48k FP64 79 / 75, mixed
+// 37 / 48, 68k 130 / 93 and 63 / 55.  Where several smoothing-length classes meet the lists differ in length (66 on
+// average, up to 287 at an impact) and a wavefront of single lanes takes the longest: impact 68k FP64 156 / 193, mixed
+// 76 / 130, 96k 163 / 178 and 84 / 121, 117k 220 / 205 and 114 / 142, 159k 288 / 181 and 130 / 118 (two gas bodies of two
+// classes, whose lists are alike, lose 12 us a step between the lines).
+constexpr size_t PAIRS_BELOW_16 = 24576, PAIRS_BELOW_4 = 65536, PAIRS_BELOW_4_CLASSES = 98304;
+inline int pair_lanes(const Tuning& t, size_t n, int nclass) {
     if (n < PAIRS_BELOW_16) return 16;
-    return t.pairs_lanes > 1 || n < PAIRS_BELOW_4 ? 4 : 1;
+    return t.pairs_lanes > 1 || n < (nclass > 1 ? PAIRS_BELOW_4_CLASSES : PAIRS_BELOW_4) ? 4 : 1;
 }
 
 // Particles below which the list kernel gives each a group of lanes: one lane per particle takes about 80 us
@@ -294,11 +298,11 @@ struct FuseArgs {
 };
 void launch_pairs_fp64(const Launch& l, DevState s, Params prm, const PairRec* rec, const uint32_t* group,
                        const uint32_t* order, const uint32_t* list, const uint32_t* count, const double* lut_grads,
-                       uint32_t kmax, size_t n, const FuseArgs* fuse = nullptr);
+                       uint32_t kmax, int nclass, size_t n, const FuseArgs* fuse = nullptr);
 void launch_pack_mixed(const Launch& l, DevState s, Params prm, Fixed fx, const uint32_t* order, PairRecF* rec,
                        double4* pos, float4* posf, Screen sc, uint32_t* group, size_t n);
 void launch_pairs_mixed(const Launch& l, DevState s, Params prm, Fixed fx, const PairRecF* rec, const uint32_t* group,
-                        const uint32_t* order, const uint32_t* list, const uint32_t* count, uint32_t kmax, size_t n,
+                        const uint32_t* order, const uint32_t* list, const uint32_t* count, uint32_t kmax, int nclass, size_t n,
                         const FuseArgs* fuse = nullptr);
 void launch_finalize(const Launch& l, DevState s, const osph_material* mats, Params prm, size_t n);
 void launch_zero_derivatives(const Launch& l, DevState s, size_t n);

@@ -1937,8 +1937,9 @@ __global__ void __launch_bounds__(BLOCK) k_criteria(DevState s, const osph_mater
     reduce_criteria(v, mins);
 }
 
-// Statistics of the neighbour counts (SymmetricSolver.cpp:172-179): a bounded grid, so that few blocks meet in the
-// three words.
+// Statistics of the neighbour counts (SymmetricSolver.cpp:172-179): a bounded grid and one set of atomics per block, as
+// those on the same three words take their turns (559k counts 13 us; with a set per wavefront, 128 blocks 27
+// and 512 blocks 76).
 constexpr unsigned STATS_BLOCKS = 128;
 __global__ void __launch_bounds__(BLOCK) k_count_stats(const uint32_t* __restrict__ counts,
                                                        unsigned long long* __restrict__ stats, size_t n) {
@@ -1953,7 +1954,20 @@ __global__ void __launch_bounds__(BLOCK) k_count_stats(const uint32_t* __restric
     inv = wave_max(inv);
     mx = wave_max(mx);
     for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
+    __shared__ unsigned long long red[BLOCK / 64][3];
     if ((threadIdx.x & 63u) == 0) {
+        unsigned long long* r = red[threadIdx.x >> 6];
+        r[0] = inv;
+        r[1] = mx;
+        r[2] = sum;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < BLOCK / 64; ++w) {
+            inv = red[w][0] > inv ? red[w][0] : inv;
+            mx = red[w][1] > mx ? red[w][1] : mx;
+            sum += red[w][2];
+        }
         atomicMax(&stats[0], inv);
         atomicMax(&stats[1], mx);
         atomicAdd(&stats[2], sum);
@@ -2191,10 +2205,10 @@ void launch_neighbor_lists(const Launch& l, const double4* pos, const float4* po
 
 void launch_pairs_fp64(const Launch& l, DevState s, Params prm, const PairRec* rec, const uint32_t* group,
                        const uint32_t* order, const uint32_t* list, const uint32_t* count, const double* lut_grads,
-                       uint32_t kmax, size_t n, const FuseArgs* fuse) {
+                       uint32_t kmax, int nclass, size_t n, const FuseArgs* fuse) {
     if (!n) return;
     const int b = l.tune.pairs_block;
-    const int lanes = pair_lanes(l.tune, n);
+    const int lanes = pair_lanes(l.tune, n, nclass);
     const unsigned grid = grid_for(n * size_t(lanes), b);
     const size_t lds = size_t(l.tune.pairs_lds);
     const FuseArgs fa = fuse ? *fuse : FuseArgs{};
@@ -2217,11 +2231,11 @@ void launch_pack_mixed(const Launch& l, DevState s, Params prm, Fixed fx, const 
 }
 
 void launch_pairs_mixed(const Launch& l, DevState s, Params prm, Fixed fx, const PairRecF* rec, const uint32_t* group,
-                        const uint32_t* order, const uint32_t* list, const uint32_t* count, uint32_t kmax, size_t n,
+                        const uint32_t* order, const uint32_t* list, const uint32_t* count, uint32_t kmax, int nclass, size_t n,
                         const FuseArgs* fuse) {
     if (!n) return;
     const int b = l.tune.pairs_block;
-    const int lanes = pair_lanes(l.tune, n);
+    const int lanes = pair_lanes(l.tune, n, nclass);
     const unsigned grid = grid_for(n * size_t(lanes), b);
     const size_t lds = size_t(l.tune.pairs_lds);
     const FuseArgs fa = fuse ? *fuse : FuseArgs{};
