@@ -37,8 +37,8 @@ FLOP_PER_QUADRUPOLE = 61.0
 # HBM bytes per launch of the pair kernel at the default workload and tuning, after contact, from two
 # rocprofv3 --pmc passes over this bench (FETCH_SIZE scaled by 2.000, WRITE_SIZE by 1.000: the factors the
 # 1 GiB device copy of --calibrate reads).  None where not measured.
-MEASURED_TRAFFIC_BYTES = {"pairs_mixed_finalize_correct": (2 * 420926 + 312715) * 1024.0,
-                          "pairs_fp64_finalize_correct": (2 * 557645 + 315804) * 1024.0}
+MEASURED_TRAFFIC_BYTES = {"pairs_mixed_finalize_correct": (2 * 434427 + 314342) * 1024.0,
+                          "pairs_fp64_finalize_correct": (2 * 601184 + 317939) * 1024.0}
 # Algorithmic HBM bytes of one pair-kernel launch per particle: each particle's own neighbour record
 # (64 B mixed, 128 B FP64), its order, count and group entries and the 92 B it writes (acceleration,
 # du, divergence, velocity gradient: 11 doubles, and the neighbour count); plus 4 B per listed neighbour.
@@ -55,12 +55,12 @@ PAIR_BYTES_PER_NEIGHBOR = 4.0
 # the issue-rate roof counts instructions, not flops.  A CU issues one
 # wave64 VALU instruction per cycle (four SIMDs, four cycles each), so the chip's roof is
 # 256 CUs x 2.4 GHz = 6.14e11 wave-instructions/s (x 64 lanes x 2 = the 78.6 TFLOP/s FMA peak).
-VALU_INSTR_PER_64_PAIR_EVALS = {"pairs_mixed_finalize_correct": 1.833e8 / (2 * 35218390 / 64),
-                                "pairs_fp64_finalize_correct": 1.970e8 / (2 * 35218390 / 64)}
+VALU_INSTR_PER_64_PAIR_EVALS = {"pairs_mixed_finalize_correct": 1.605e8 / (2 * 35218390 / 64),
+                                "pairs_fp64_finalize_correct": 1.526e8 / (2 * 35218390 / 64)}
 VALU_ISSUE_PEAK = 256 * 2.4e9
 # The same for the Barnes-Hut evaluation of the 8,000,000-particle N-body sphere (FETCH_SIZE x 2 +
-# WRITE_SIZE, KiB per dispatch, averaged over the 2 dispatches with the state in Morton order).
-NBODY_TRAFFIC_BYTES = {"eval_mixed": (2 * 2045976 + 245187) * 1024.0, "eval": (2 * 1957327 + 248606) * 1024.0}
+# WRITE_SIZE, KiB per dispatch, averaged over the 3 dispatches with the state in Morton order).
+NBODY_TRAFFIC_BYTES = {"eval_mixed": (2 * 1428153 + 250832) * 1024.0, "eval": (2 * 1292650 + 241718) * 1024.0}
 
 
 def log(*a):
