@@ -407,7 +407,7 @@ __device__ __forceinline__ void block_sort(unsigned long long* v, uint32_t m) {
 // impact).  The block sorts longer rows together, in LDS up to ROW_BLOCK particles (rows of 1M particles' cells
 // hold ~64; far outliers that stretch the grid to its 250 cells make them longer).
 constexpr uint32_t ROW_WAVE = 512, ROW_BLOCK = 2048;
-struct RowStage {
+struct alignas(16) RowStage {  // start is read 16 bytes at a time
     uint32_t start[256];      // counts by x, then their exclusive prefix sums
     uint32_t idx[ROW_WAVE];   // particles placed by cell
 };
@@ -419,6 +419,7 @@ __device__ __forceinline__ void row_order_block(const Grid& g, const uint32_t* _
         RowStage stage[WAVES];
         unsigned long long key[ROW_BLOCK];
     };
+    static_assert(alignof(Lds) >= 16, "RowStage::start is read 16 bytes at a time");
     __shared__ Lds lds;
     __shared__ uint32_t long_row[WAVES][4];  // first position, particles, cell base and dim_x of a long row
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63u;
