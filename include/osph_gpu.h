@@ -252,8 +252,10 @@ int osph_adjoint_clear(osph_ctx* ctx);
  * "pairs_lanes" (1, the default: one lane per particle in the pair kernels, or a group of lanes when the particles are
  * too few to fill the GPU; 2 or 4: a group of lanes; the sums are the same, bit for bit),
  * "cell_divisor" (1 to 4: neighbour-grid cells of 2 h_max / divisor, default 3), "lists_screen" (1: FP32-screened
- * neighbour test, 0: FP64 only, -1: screened in mixed precision only), "reorder_period" (the resident state
- * is moved into cell order every this many neighbour searches; 0 never; default 40), "fuse_finalize" (1: the
+ * neighbour test, 0: FP64 only, -1: screened in mixed precision only), "sort_cells" (the buckets of the sort by
+ * cell: 1 cells, 0 rows of cells, -1, the default: cells where rows may be long; the order is the same),
+ * "reorder_period" (the resident state is moved into cell order every this many neighbour searches; 0 never;
+ * default 40), "fuse_finalize" (1: the
  * PC step's finalize, corrector and criteria run in the pair kernel, the default, 0: as a separate pass,
  * -1: fused for FP64 only). */
 int osph_tune(osph_ctx* ctx, const char* key, long long value);

@@ -45,14 +45,14 @@ struct BatchPlan {
     Mailbox box;  // host mirror of small
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
-    int graph_screened = -1, graph_plain = -1;
+    int graph_screened = -1, graph_plain = -1, graph_cells = -1;
 
     void drop_graph() {
         if (exec) (void)hipGraphExecDestroy(exec);
         if (graph) (void)hipGraphDestroy(graph);
         exec = nullptr;
         graph = nullptr;
-        graph_screened = graph_plain = -1;
+        graph_screened = graph_plain = graph_cells = -1;
     }
     ~BatchPlan() {
         drop_graph();
@@ -585,7 +585,10 @@ int plan_search(osph_ctx* c, const unsigned long long* sh, size_t* rows_out) {
         if (uint64_t(base) + rows_end > (uint64_t(1) << 32) - 2) return c->fail(OSPH_ERR_STATE, "cell count exceeds 32 bits");
         base += uint32_t(rows_end);
         g.slots += uint32_t(rows_end >> bits);
+        if (sort_by_cells(G, size_t(ccount[cl]))) g.by_cells = 1;
     }
+    g.cells = base;
+    if (c->tune.sort_cells >= 0) g.by_cells = c->tune.sort_cells;
     c->grid = g;
     if (int e = ensure_cells(c, size_t(base))) return e;
     size_t rows = 0;
@@ -1427,7 +1430,7 @@ int batch_step(const std::vector<osph_ctx*>& ms, const std::vector<double>& dts,
     mailbox_post(st, P->box, 0, P->small, count * SMALL_WORDS);
     if (int e = wait_box(lead, P->box)) return e;
     // each member's grid, screen and fixed-point frames, planned as its own search plans them
-    bool screened = false, plain = false;
+    bool screened = false, plain = false, cells = false;
     for (size_t k = 0; k < count; ++k) {
         osph_ctx* c = ms[k];
         BatchMember& b = P->host[k];
@@ -1461,13 +1464,14 @@ int batch_step(const std::vector<osph_ctx*>& ms, const std::vector<double>& dts,
         b.list = c->list;
         b.count = c->count;
         (b.screen.on ? screened : plain) = true;
+        cells = cells || c->grid.by_cells;
     }
     HIPCHK(lead, hipMemcpyAsync(P->dev, P->host, count * sizeof(BatchMember), hipMemcpyHostToDevice, st));
     const bool fuse = P->tune.fuse_finalize == 1 || (P->tune.fuse_finalize == -1 && !P->mixed);
     // the stages from the sort on: their launch shapes and arguments are fixed for the plan (the per-step
     // values are in the member table), so they are captured once and replayed
     auto rest = [&]() {
-        batch_sort(l, P->dev, int(count), P->pb);
+        batch_sort(l, P->dev, int(count), P->pb, cells);
         batch_permute(l, P->dev, P->pb);
         batch_pack(l, P->dev, P->pb, P->mixed);
         batch_lists(l, P->dev, P->lb, screened, plain);
@@ -1475,7 +1479,8 @@ int batch_step(const std::vector<osph_ctx*>& ms, const std::vector<double>& dts,
         if (!fuse) batch_finalize_correct(l, P->dev, P->pb);
     };
     if (P->tune.batch_graph) {
-        if (!P->exec || P->graph_screened != int(screened) || P->graph_plain != int(plain)) {
+        if (!P->exec || P->graph_screened != int(screened) || P->graph_plain != int(plain) ||
+            P->graph_cells != int(cells)) {
             P->drop_graph();
             HIPCHK(lead, hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
             rest();
@@ -1483,6 +1488,7 @@ int batch_step(const std::vector<osph_ctx*>& ms, const std::vector<double>& dts,
             HIPCHK(lead, hipGraphInstantiate(&P->exec, P->graph, nullptr, nullptr, 0));
             P->graph_screened = int(screened);
             P->graph_plain = int(plain);
+            P->graph_cells = int(cells);
         }
         HIPCHK(lead, hipGraphLaunch(P->exec, st));
     } else {
@@ -1857,6 +1863,8 @@ int osph_tune(osph_ctx* c, const char* key, long long value) {
         c->tune.cell_divisor = int(value);
     } else if (k == "lists_screen" && (value == -1 || value == 0 || value == 1)) {
         c->tune.lists_screen = int(value);
+    } else if (k == "sort_cells" && (value == -1 || value == 0 || value == 1)) {
+        c->tune.sort_cells = int(value);
     } else if (k == "reorder_period" && value >= 0 && value <= 1000000) {
         c->tune.reorder_period = int(value);
     } else if (k == "fuse_finalize" && (value == -1 || value == 0 || value == 1)) {

@@ -3,6 +3,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <cmath>
 #include <cstddef>
 #include <cstdint>
 
@@ -100,6 +102,8 @@ struct GridClass {
 struct Grid {
     int nclass;
     uint32_t slots;  // rows of all classes, by their Morton codes
+    uint32_t cells;  // entries of the cell table
+    int by_cells;    // the sort's buckets: cells, or rows of cells (sort_by_cells)
     double hmin;
     GridClass c[MAX_CLASSES];
 };
@@ -177,6 +181,7 @@ struct Tuning {
     int lists_block = 256;
     int lists_lds = 0;
     int cell_divisor = 3;  // cells of 2 h_max(class) / divisor
+    int sort_cells = -1;   // buckets of the sort by cell: 1 cells, 0 rows of cells, -1 by sort_by_cells
     int lists_screen = -1; // FP32 screen in the list kernel: 1 on, 0 off, -1 on for mixed precision only
     int reorder_period = 40;  // move the state into cell order every this many searches (0: never); at the
                               // 1M impact 10 / 20 / 40 / 80 measured 1.738 / 1.724 / 1.723 / 1.736 ms per
@@ -209,6 +214,21 @@ inline int pair_lanes(const Tuning& t, size_t n, int nclass) {
 constexpr size_t LISTS_SHARED_BELOW = 131072, LISTS_SHARED_BELOW_CLASSES = 262144;
 inline bool lists_shared(const Grid& g, size_t n) {
     return n < (g.nclass > 1 ? LISTS_SHARED_BELOW_CLASSES : LISTS_SHARED_BELOW);
+}
+
+// Whether a class's rows of cells may be too long to be ordered a row at a time (the sort's buckets, see
+// osph_kernels.hip): by the mean over its rows, and by the rows of a compact body of n particles at their usual distance
+// of h / 1.3 (w of them along a cell's edge: n^(1/3) / w cells of w^3 in a row), which is what outliers that stretch
+// the cells leave.  Sort in us by rows / cells, one body with a particle so many diameters away: 1M in touch 31 / 157 (n^(1/3)
+// w^2 = 75), 5 away 51 / 64 (400), 10 away 279 / 69 (1600), 20 away 5621 / 172; 300k 5 away 27 / 44 (123), 10 away 58 / 41
+// (490), 50 away 37294 / 199; 125k 10 away 30 / 32 (200), 20 away 112 / 39 (800); 50k 20 away 44 / 33 (333); 10k 50 away
+// 98 / 33 (380); 2k up to 50 away 20 / 30 (80).  Sheets of 125k / 300k / 1M particles, mean 500 / 1200 / 4000: 29 / 48,
+// 44 / 50, 163 / 58; lines of 2k / 10k / 50k: 27 / 27, 174 / 34, 3153 / 45.
+constexpr double ROWS_BODY = 320.0, ROWS_MEAN = 1000.0;
+inline bool sort_by_cells(const GridClass& g, size_t n) {
+    const double w = 1.3 * g.cell / g.hmax, count = double(n);
+    const double body = std::min(count, std::cbrt(count) * w * w), mean = count / (double(g.dim[1]) * double(g.dim[2]));
+    return body > ROWS_BODY || mean > ROWS_MEAN;
 }
 
 struct Launch {
@@ -277,7 +297,8 @@ void launch_gather_planes(const Launch& l, double* dst, int nc, double* const* p
 void launch_clear_u32(const Launch& l, uint32_t* p, size_t count, uint32_t value);
 // The particles ordered by cell (order[], ties by slot), and first[cell] = the first sorted position whose cell
 // index is >= cell, for every cell (x, y, z) of a row (y < dim_y, z < dim_z) with x in [0, dim_x].  row_count and
-// row_start: row_slots(g.slots) words, the counts zero (and zero again afterwards); where, bucket: n entries.
+// row_start: row_slots(g.slots) words, the counts zero (and zero again afterwards); where, bucket: n entries;
+// first: g.cells entries.
 size_t row_slots(uint32_t slots);
 void launch_cell_sort(const Launch& l, DevState s, Grid g, uint32_t* row_count, uint32_t* row_start, uint2* where,
                       uint2* bucket, uint32_t* order, uint32_t* first, size_t rows, size_t n);
@@ -371,7 +392,8 @@ inline uint32_t batch_blocks_for(size_t n, int block) {
 // Stage launchers over all `count` members (M in device memory).  `pb`: blocks of BLOCK threads per
 // particle; `lb`: blocks of the list kernel's size; `qb`: blocks of the pair kernel's size and lanes.
 void batch_advance(const Launch& l, const BatchMember* M, int count, BatchBlocks pb, bool vel);
-void batch_sort(const Launch& l, const BatchMember* M, int count, BatchBlocks pb);
+// cells: some member's grid is sorted by cells.
+void batch_sort(const Launch& l, const BatchMember* M, int count, BatchBlocks pb, bool cells);
 void batch_permute(const Launch& l, const BatchMember* M, BatchBlocks pb);
 void batch_pack(const Launch& l, const BatchMember* M, BatchBlocks pb, bool mixed);
 void batch_lists(const Launch& l, const BatchMember* M, BatchBlocks lb, bool screened, bool plain);

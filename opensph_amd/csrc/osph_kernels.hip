@@ -272,32 +272,44 @@ __device__ __forceinline__ bool row_of(const Grid& g, size_t q, int& cls, uint32
 }
 
 // ---- sort by cell and cell table ------------------------------------------------------------------------
-// The order of the particles by cell and the cell table, by rows of cells: a row (slot0(class) + Morton(y, z), the
-// sort key without x) is a bucket, and a row's particles are ordered by (x, particle) on their own.  Four launches
-// -- count, scan, scatter, order -- whatever the particle count, where a radix sort of the keys took 3 passes over
-// them (onesweep, 84 us at 1M particles) or about ten merge launches (below 1M: 120 us at 559k, 40 us at 43k),
-// and two more kernels built the table (30 us at 1M).  Measured here: 12 + 8 + 6 + 14 us at 1M, 20 us in all up to
-// 170k particles (launch latency).
-// The buckets are filled with atomics, in any order; the order within a row does not depend on it.
+// The order of the particles by (cell, particle), and the cell table, in one of two ways (sort_by_cells).
+//
+// By rows of cells: a row (slot0(class) + Morton(y, z), the cell index without x) is a bucket, and a row's particles
+// are ordered by (x, particle) on their own.  Four launches -- count, scan, scatter, order -- whatever the particle
+// count, where a radix sort of the keys took 3 passes over them (onesweep, 84 us at 1M particles) or about ten merge
+// launches (below 1M: 120 us at 559k, 40 us at 43k), and two more kernels built the table (30 us at 1M).  Measured
+// here: 12 + 8 + 6 + 14 us at 1M, 20 us in all up to 170k particles (launch latency).
+//
+// By cells, where rows are long: far outliers stretch the cells to 1/250 of the extent, and a compact body then fills a
+// few rows of thousands of particles, too much for a wavefront or block each.  The cells themselves are the buckets
+// and the cell table holds their counts; a particle's place in its cell is the number of lower particles there, counted
+// by a thread each.  That costs a fraction of what the list kernel does with the same cell (it tests the cell's
+// particles, and those of the cells around it, for the same particle), and no row or cell has to fit anywhere.
+//
+// The buckets are filled with atomics, in any order; the order within them does not depend on it.
 
-// Counts the particles of every row: where[i] = (row << 8 | x, rank in the row).  One atomic per row and wavefront.
+// Counts the particles of every row: where[i] = (row << 8 | x, rank in the row), or by CELLS of every cell (in `first`)
+// and row: where[i] = (cell, rank in the cell).  One atomic per row or cell and wavefront.
+template <bool CELLS>
 __device__ __forceinline__ void row_count_at(const DevState& s, const Grid& g, uint32_t* __restrict__ row_count,
-                                             uint2* __restrict__ where, size_t i, size_t n) {
+                                             uint32_t* __restrict__ first, uint2* __restrict__ where, size_t i, size_t n) {
     const bool valid = i < n;
     const uint32_t lane = threadIdx.x & 63u;
-    uint32_t row = 0xffffffffu, x = 0;
+    uint32_t row = 0, key = 0xffffffffu;
     if (valid) {
         const int cls = h_class(s.d[H][i], g.hmin, g.nclass);
         int c[3];
         cell_of(g.c[cls], s.d[X][i], s.d[Y][i], s.d[Z][i], c);
-        row = g.c[cls].slot0 + (spread2(uint32_t(c[1])) | (spread2(uint32_t(c[2])) << 1));
-        x = uint32_t(c[0]);
+        const uint32_t mor = row_key(0u, uint32_t(c[1]), uint32_t(c[2]), 0);
+        row = g.c[cls].slot0 + mor;
+        key = CELLS ? g.c[cls].base + (mor << g.c[cls].bits) + uint32_t(c[0]) : (row << 8) | uint32_t(c[0]);
     }
-    // the lanes of one row: its first lane adds their number, each gets its rank among them
+    // the lanes of one bucket: its first lane adds their number, each gets its rank among them
+    const uint32_t bucket = CELLS ? key : row;
     uint32_t leader = lane, before = 0, total = 0;
     for (unsigned long long open = __ballot(valid); open != 0ull;) {
         const int l = __builtin_ctzll(open);
-        const unsigned long long same = __ballot(row == uint32_t(__builtin_amdgcn_readlane(row, l))) & open;
+        const unsigned long long same = __ballot(bucket == uint32_t(__builtin_amdgcn_readlane(bucket, l))) & open;
         if ((same >> lane) & 1ull) {
             leader = uint32_t(l);
             before = uint32_t(__popcll(same & ((1ull << lane) - 1ull)));
@@ -306,14 +318,18 @@ __device__ __forceinline__ void row_count_at(const DevState& s, const Grid& g, u
         open &= ~same;
     }
     uint32_t base = 0;
-    if (valid && leader == lane) base = atomicAdd(&row_count[row], total);
+    if (valid && leader == lane) {
+        base = atomicAdd(CELLS ? &first[key] : &row_count[row], total);
+        if (CELLS) atomicAdd(&row_count[row], total);
+    }
     base = uint32_t(__shfl(int(base), int(leader), 64));
-    if (valid) where[i] = make_uint2((row << 8) | x, base + before);
+    if (valid) where[i] = make_uint2(key, base + before);
 }
 
+template <bool CELLS>
 __global__ void __launch_bounds__(BLOCK) k_row_count(DevState s, Grid g, uint32_t* __restrict__ row_count,
-                                                     uint2* __restrict__ where, size_t n) {
-    row_count_at(s, g, row_count, where, size_t(blockIdx.x) * blockDim.x + threadIdx.x, n);
+                                                     uint32_t* __restrict__ first, uint2* __restrict__ where, size_t n) {
+    row_count_at<CELLS>(s, g, row_count, first, where, size_t(blockIdx.x) * blockDim.x + threadIdx.x, n);
 }
 
 // row_start = exclusive prefix sums of the counts (slots + 1 entries).  Block b sums the counts before its tile of
@@ -360,64 +376,155 @@ __global__ void __launch_bounds__(SCAN_BLOCK) k_row_scan(const uint32_t* __restr
     row_scan_tile(row_count, row_start, blockIdx.x);
 }
 
-// bucket[row_start + rank] = (particle, x): x in the high word, so that the 64-bit values order by (x, particle).
-// The counts go back to zero for the next search.
+// bucket[row_start + rank] = (particle, x), or by CELLS the particle alone at its cell's first position + rank.  The row
+// counts go back to zero for the next search.
+template <bool CELLS>
 __device__ __forceinline__ void row_scatter_at(const uint2* __restrict__ where, const uint32_t* __restrict__ row_start,
-                                               uint32_t* __restrict__ row_count, uint32_t slots,
-                                               uint2* __restrict__ bucket, size_t i, size_t threads, size_t n) {
+                                               const uint32_t* __restrict__ first, uint32_t* __restrict__ row_count,
+                                               uint32_t slots, uint2* __restrict__ bucket, size_t i, size_t threads,
+                                               size_t n) {
     for (size_t t = i; t < slots; t += threads) row_count[t] = 0u;
     if (i >= n) return;
     const uint2 w = where[i];
-    bucket[row_start[w.x >> 8] + w.y] = make_uint2(uint32_t(i), w.x & 255u);
+    if constexpr (CELLS) {
+        reinterpret_cast<uint32_t*>(bucket)[first[w.x] + w.y] = uint32_t(i);
+    } else {
+        bucket[row_start[w.x >> 8] + w.y] = make_uint2(uint32_t(i), w.x & 255u);
+    }
 }
 
+template <bool CELLS>
 __global__ void __launch_bounds__(BLOCK) k_row_scatter(const uint2* __restrict__ where,
                                                        const uint32_t* __restrict__ row_start,
+                                                       const uint32_t* __restrict__ first,
                                                        uint32_t* __restrict__ row_count, uint32_t slots,
                                                        uint2* __restrict__ bucket, size_t n) {
-    row_scatter_at(where, row_start, row_count, slots, bucket, size_t(blockIdx.x) * blockDim.x + threadIdx.x,
-                   size_t(gridDim.x) * blockDim.x, n);
+    row_scatter_at<CELLS>(where, row_start, first, row_count, slots, bucket, size_t(blockIdx.x) * blockDim.x + threadIdx.x,
+                          size_t(gridDim.x) * blockDim.x, n);
 }
 
-// Ascending sort of v[0..m) by the block: bitonic with every comparator directed upwards (the first step of each
-// merge mirrors), so that the missing partners past m act as largest values.
-__device__ __forceinline__ void block_sort(unsigned long long* v, uint32_t m) {
-    for (uint32_t size = 2; size < 2 * m; size <<= 1) {
-        for (uint32_t step = size; step > 1; step >>= 1) {
-            __syncthreads();
-            const uint32_t half = step >> 1;
-            for (uint32_t p = threadIdx.x; p < m; p += blockDim.x) {
-                const uint32_t q = step == size ? p ^ (size - 1u) : p ^ half;
-                if (q > p && q < m) {
-                    const unsigned long long a = v[p], b = v[q];
-                    if (b < a) {
-                        v[p] = b;
-                        v[q] = a;
-                    }
-                }
-            }
+// One wavefront per row: the counts of its cells in `first` become first sorted positions, with that of the row's end in
+// the slot past its last cell.  The cells of rows without particles keep their zeros, equal entries, so that every x-run
+// of them reads as empty.
+__device__ __forceinline__ void cell_starts_at(const Grid& g, const uint32_t* __restrict__ row_start,
+                                               uint32_t* __restrict__ first, size_t rows, size_t q) {
+    int cls = 0;
+    uint32_t cy = 0, cz = 0;
+    if (q >= rows || !row_of(g, q, cls, cy, cz)) return;  // uniform over the wavefront
+    const GridClass& G = g.c[cls];
+    const uint32_t lane = threadIdx.x & 63u, mor = row_key(0u, cy, cz, 0);
+    uint32_t run = row_start[G.slot0 + mor];
+    if (row_start[G.slot0 + mor + 1u] == run) return;
+    uint32_t* cell = first + G.base + (mor << G.bits);
+    for (uint32_t x0 = 0; x0 <= uint32_t(G.dim[0]); x0 += 64u) {
+        const uint32_t x = x0 + lane;
+        const uint32_t c = x < uint32_t(G.dim[0]) ? cell[x] : 0u;
+        uint32_t incl = c;
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t u = uint32_t(__shfl_up(int(incl), o, 64));
+            if (lane >= uint32_t(o)) incl += u;
         }
+        if (x <= uint32_t(G.dim[0])) cell[x] = run + incl - c;
+        run += uint32_t(__shfl(int(incl), 63, 64));
     }
-    __syncthreads();
+}
+
+__global__ void __launch_bounds__(BLOCK) k_cell_starts(Grid g, const uint32_t* __restrict__ row_start,
+                                                       uint32_t* __restrict__ first, size_t rows) {
+    cell_starts_at(g, row_start, first, rows, size_t(blockIdx.x) * (BLOCK / 64) + (threadIdx.x >> 6));
+}
+
+// order[] by CELLS: particle i goes behind the lower particles of its cell.
+__device__ __forceinline__ void cell_order_at(const uint2* __restrict__ where, const uint32_t* __restrict__ first,
+                                              const uint32_t* __restrict__ placed, uint32_t* __restrict__ order, size_t i,
+                                              size_t n) {
+    if (i >= n) return;
+    const uint32_t cell = where[i].x;
+    const uint32_t a = first[cell], b = first[cell + 1u];
+    uint32_t r = a;
+#pragma unroll 4
+    for (uint32_t j = a; j < b; ++j) r += placed[j] < uint32_t(i) ? 1u : 0u;
+    order[r] = uint32_t(i);
+}
+
+__global__ void __launch_bounds__(BLOCK) k_cell_order(const uint2* __restrict__ where, const uint32_t* __restrict__ first,
+                                                      const uint32_t* __restrict__ placed, uint32_t* __restrict__ order,
+                                                      size_t n) {
+    cell_order_at(where, first, placed, order, size_t(blockIdx.x) * blockDim.x + threadIdx.x, n);
 }
 
 // One wavefront per row (y < dim_y, z < dim_z of every class): its particles ordered by (x, particle) into order[],
 // and first[cell] = the first sorted position whose cell is >= cell, for x in [0, dim_x].  Up to ROW_WAVE
 // particles in LDS: counted by x, placed, and each ranked among those of its own cell (0.6 per cell at the
-// impact).  The block sorts longer rows together, in LDS up to ROW_BLOCK particles (rows of 1M particles' cells
-// hold ~64; far outliers that stretch the grid to its 250 cells make them longer).
+// impact).  Longer rows (rare here, see sort_by_cells) take the block together, one after the other, the same way, and
+// beyond ROW_BLOCK particles through the row's part of scratch[] (the particles' rows, used up by the scatter).
 constexpr uint32_t ROW_WAVE = 512, ROW_BLOCK = 2048;
 struct alignas(16) RowStage {  // start is read 16 bytes at a time
     uint32_t start[256];      // counts by x, then their exclusive prefix sums
     uint32_t idx[ROW_WAVE];   // particles placed by cell
 };
+struct alignas(16) LongRowStage {
+    uint32_t start[256];
+    uint32_t next[256];       // the next free place of each cell
+    uint2 placed[ROW_BLOCK];
+};
+
+// start[0..256) from counts to exclusive prefix sums, by one wavefront.
+__device__ __forceinline__ void scan_cells(uint32_t* start) {
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint4 c = reinterpret_cast<const uint4*>(start)[lane];
+    const uint32_t sum = c.x + c.y + c.z + c.w;
+    uint32_t incl = sum;
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t u = uint32_t(__shfl_up(int(incl), o, 64));
+        if (lane >= uint32_t(o)) incl += u;
+    }
+    uint4 st;
+    st.x = incl - sum;
+    st.y = st.x + c.x;
+    st.z = st.y + c.y;
+    st.w = st.z + c.z;
+    reinterpret_cast<uint4*>(start)[lane] = st;
+}
+
+// The block's order of one long row of m particles from sorted position f on.
+__device__ __forceinline__ void order_long_row(LongRowStage& S, const uint2* __restrict__ row, uint2* placed,
+                                               uint32_t* __restrict__ order, uint32_t* __restrict__ cell, uint32_t dimx,
+                                               uint32_t f, uint32_t m) {
+    for (uint32_t x = threadIdx.x; x < 256u; x += BLOCK) S.start[x] = 0u;
+    __syncthreads();
+    for (uint32_t p = threadIdx.x; p < m; p += BLOCK) atomicAdd(&S.start[row[p].y], 1u);
+    __syncthreads();
+    if (threadIdx.x < 64u) scan_cells(S.start);
+    __syncthreads();
+    for (uint32_t x = threadIdx.x; x < 256u; x += BLOCK) {
+        S.next[x] = S.start[x];
+        if (x <= dimx) cell[x] = f + S.start[x];
+    }
+    __syncthreads();
+    for (uint32_t p = threadIdx.x; p < m; p += BLOCK) {
+        const uint2 e = row[p];
+        placed[atomicAdd(&S.next[e.y], 1u)] = e;
+    }
+    __syncthreads();
+    for (uint32_t p = threadIdx.x; p < m; p += BLOCK) {
+        const uint2 e = placed[p];
+        const uint32_t a = S.start[e.y], b = S.start[e.y + 1u];  // x <= 250: x + 1 is an entry
+        uint32_t r = a;
+        for (uint32_t j = a; j < b; ++j) r += placed[j].x < e.x ? 1u : 0u;
+        order[f + r] = e.x;
+    }
+    __syncthreads();
+}
+
 __device__ __forceinline__ void row_order_block(const Grid& g, const uint32_t* __restrict__ row_start,
-                                                uint2* __restrict__ bucket, uint32_t* __restrict__ order,
-                                                uint32_t* __restrict__ first, size_t rows, size_t block) {
+                                                const uint2* __restrict__ bucket, uint2* __restrict__ scratch,
+                                                uint32_t* __restrict__ order, uint32_t* __restrict__ first, size_t rows,
+                                                size_t block) {
     constexpr int WAVES = BLOCK / 64;
     union Lds {
         RowStage stage[WAVES];
-        unsigned long long key[ROW_BLOCK];
+        LongRowStage row;
     };
     static_assert(alignof(Lds) >= 16, "RowStage::start is read 16 bytes at a time");
     __shared__ Lds lds;
@@ -428,7 +535,7 @@ __device__ __forceinline__ void row_order_block(const Grid& g, const uint32_t* _
     uint32_t cy = 0, cz = 0;
     const bool valid = q < rows && row_of(g, q, cls, cy, cz);
     const GridClass& G = g.c[cls];
-    const uint32_t mor = spread2(cy) | (spread2(cz) << 1);
+    const uint32_t mor = row_key(0u, cy, cz, 0);
     const uint32_t dimx = uint32_t(G.dim[0]), cell0 = G.base + (mor << G.bits);
     uint32_t s0 = 0, cnt = 0;
     if (valid) {
@@ -455,19 +562,7 @@ __device__ __forceinline__ void row_order_block(const Grid& g, const uint32_t* _
             }
         }
         wave_sync();
-        const uint4 c = reinterpret_cast<const uint4*>(S.start)[lane];
-        const uint32_t sum = c.x + c.y + c.z + c.w;
-        uint32_t incl = sum;
-        for (int o = 1; o < 64; o <<= 1) {
-            const uint32_t u = uint32_t(__shfl_up(int(incl), o, 64));
-            if (lane >= uint32_t(o)) incl += u;
-        }
-        uint4 st;
-        st.x = incl - sum;
-        st.y = st.x + c.x;
-        st.z = st.y + c.y;
-        st.w = st.z + c.z;
-        reinterpret_cast<uint4*>(S.start)[lane] = st;
+        scan_cells(S.start);
         wave_sync();
         for (uint32_t x = lane; x <= dimx; x += 64u) first[cell0 + x] = s0 + S.start[x];
 #pragma unroll
@@ -496,33 +591,16 @@ __device__ __forceinline__ void row_order_block(const Grid& g, const uint32_t* _
     for (int w = 0; w < WAVES; ++w) {
         const uint32_t f = long_row[w][0], m = long_row[w][1];
         if (m == 0) continue;
-        unsigned long long* v = reinterpret_cast<unsigned long long*>(bucket + f);
-        if (m <= ROW_BLOCK) {
-            for (uint32_t p = threadIdx.x; p < m; p += BLOCK) lds.key[p] = v[p];
-            v = lds.key;
-        }
-        block_sort(v, m);
-        for (uint32_t p = threadIdx.x; p < m; p += BLOCK) order[f + p] = uint32_t(v[p]);
-        for (uint32_t x = threadIdx.x; x <= long_row[w][3]; x += BLOCK) {
-            uint32_t lo = 0, hi = m;
-            while (lo < hi) {
-                const uint32_t mid = lo + ((hi - lo) >> 1);
-                if (uint32_t(v[mid] >> 32) < x) {
-                    lo = mid + 1;
-                } else {
-                    hi = mid;
-                }
-            }
-            first[long_row[w][2] + x] = f + lo;
-        }
-        __syncthreads();
+        order_long_row(lds.row, bucket + f, m <= ROW_BLOCK ? lds.row.placed : scratch + f, order, first + long_row[w][2],
+                       long_row[w][3], f, m);
     }
 }
 
 __global__ void __launch_bounds__(BLOCK) k_row_order(Grid g, const uint32_t* __restrict__ row_start,
-                                                     uint2* __restrict__ bucket, uint32_t* __restrict__ order,
-                                                     uint32_t* __restrict__ first, size_t rows) {
-    row_order_block(g, row_start, bucket, order, first, rows, blockIdx.x);
+                                                     const uint2* __restrict__ bucket, uint2* __restrict__ scratch,
+                                                     uint32_t* __restrict__ order, uint32_t* __restrict__ first,
+                                                     size_t rows) {
+    row_order_block(g, row_start, bucket, scratch, order, first, rows, blockIdx.x);
 }
 
 // Pack the neighbour-side data of particle order[k] into rec[k].
@@ -2139,10 +2217,20 @@ void launch_cell_sort(const Launch& l, DevState s, Grid g, uint32_t* row_count, 
                       uint2* bucket, uint32_t* order, uint32_t* first, size_t rows, size_t n) {
     // without particles nothing reads the table
     if (!rows || !n) return;
-    k_row_count<<<grid_for(n), BLOCK, 0, l.stream>>>(s, g, row_count, where, n);
-    k_row_scan<<<unsigned(row_slots(g.slots) / SCAN_TILE), SCAN_BLOCK, 0, l.stream>>>(row_count, row_start);
-    k_row_scatter<<<grid_for(n), BLOCK, 0, l.stream>>>(where, row_start, row_count, g.slots, bucket, n);
-    k_row_order<<<grid_for(rows, BLOCK / 64), BLOCK, 0, l.stream>>>(g, row_start, bucket, order, first, rows);
+    const unsigned blocks = grid_for(n), scans = unsigned(row_slots(g.slots) / SCAN_TILE), waves = grid_for(rows, BLOCK / 64);
+    if (g.by_cells) {
+        launch_clear_u32(l, first, g.cells, 0u);
+        k_row_count<true><<<blocks, BLOCK, 0, l.stream>>>(s, g, row_count, first, where, n);
+        k_row_scan<<<scans, SCAN_BLOCK, 0, l.stream>>>(row_count, row_start);
+        k_cell_starts<<<waves, BLOCK, 0, l.stream>>>(g, row_start, first, rows);
+        k_row_scatter<true><<<blocks, BLOCK, 0, l.stream>>>(where, row_start, first, row_count, g.slots, bucket, n);
+        k_cell_order<<<blocks, BLOCK, 0, l.stream>>>(where, first, reinterpret_cast<const uint32_t*>(bucket), order, n);
+    } else {
+        k_row_count<false><<<blocks, BLOCK, 0, l.stream>>>(s, g, row_count, first, where, n);
+        k_row_scan<<<scans, SCAN_BLOCK, 0, l.stream>>>(row_count, row_start);
+        k_row_scatter<false><<<blocks, BLOCK, 0, l.stream>>>(where, row_start, first, row_count, g.slots, bucket, n);
+        k_row_order<<<waves, BLOCK, 0, l.stream>>>(g, row_start, bucket, where, order, first, rows);
+    }
 }
 
 void launch_clear_u32(const Launch& l, uint32_t* p, size_t count, uint32_t value) {
@@ -2357,12 +2445,24 @@ __global__ void __launch_bounds__(BLOCK) kb_bounds_final(const BatchMember* __re
     bounds_final_at(vi, a.part, pb.first[m + 1] - pb.first[m], a.small + SMALL_CLASSES, a.small + SMALL_VEL);
 }
 
-// The four launches of a member's own sort, on each member's rows: 16 members of 5k to 212k particles 190 -> 45 us,
+// The launches of a member's own sort, on each member's rows: 16 members of 5k to 212k particles 190 -> 45 us,
 // against one radix sort of all members' keys and two kernels for the tables, 24 launches.
+__global__ void __launch_bounds__(BLOCK) kb_cell_clear(const BatchMember* __restrict__ M, BatchBlocks pb) {
+    uint32_t m, bid, nb;
+    const BatchMember& a = batch_block(M, pb, m, bid, nb);
+    if (!a.grid.by_cells) return;
+    for (size_t t = size_t(bid) * BLOCK + threadIdx.x; t < a.grid.cells; t += size_t(nb) * BLOCK) a.cell_first[t] = 0u;
+}
+
 __global__ void __launch_bounds__(BLOCK) kb_row_count(const BatchMember* __restrict__ M, BatchBlocks pb) {
     uint32_t m, bid, nb;
     const BatchMember& a = batch_block(M, pb, m, bid, nb);
-    row_count_at(a.s, a.grid, a.row_count, a.where, size_t(bid) * BLOCK + threadIdx.x, a.n);
+    const size_t i = size_t(bid) * BLOCK + threadIdx.x;
+    if (a.grid.by_cells) {
+        row_count_at<true>(a.s, a.grid, a.row_count, a.cell_first, a.where, i, a.n);
+    } else {
+        row_count_at<false>(a.s, a.grid, a.row_count, a.cell_first, a.where, i, a.n);
+    }
 }
 
 constexpr unsigned SCAN_BLOCKS = 8;  // per member, over its tiles
@@ -2374,18 +2474,36 @@ __global__ void __launch_bounds__(SCAN_BLOCK) kb_row_scan(const BatchMember* __r
     }
 }
 
+__global__ void __launch_bounds__(BLOCK) kb_cell_starts(const BatchMember* __restrict__ M, BatchBlocks pb) {
+    uint32_t m, bid, nb;
+    const BatchMember& a = batch_block(M, pb, m, bid, nb);
+    if (!a.grid.by_cells) return;
+    for (size_t b = bid; b * (BLOCK / 64) < a.rows; b += nb) {
+        cell_starts_at(a.grid, a.row_start, a.cell_first, a.rows, b * (BLOCK / 64) + (threadIdx.x >> 6));
+    }
+}
+
 __global__ void __launch_bounds__(BLOCK) kb_row_scatter(const BatchMember* __restrict__ M, BatchBlocks pb) {
     uint32_t m, bid, nb;
     const BatchMember& a = batch_block(M, pb, m, bid, nb);
-    row_scatter_at(a.where, a.row_start, a.row_count, a.grid.slots, a.bucket, size_t(bid) * BLOCK + threadIdx.x,
-                   size_t(nb) * BLOCK, a.n);
+    const size_t i = size_t(bid) * BLOCK + threadIdx.x, threads = size_t(nb) * BLOCK;
+    if (a.grid.by_cells) {
+        row_scatter_at<true>(a.where, a.row_start, a.cell_first, a.row_count, a.grid.slots, a.bucket, i, threads, a.n);
+    } else {
+        row_scatter_at<false>(a.where, a.row_start, a.cell_first, a.row_count, a.grid.slots, a.bucket, i, threads, a.n);
+    }
 }
 
 __global__ void __launch_bounds__(BLOCK) kb_row_order(const BatchMember* __restrict__ M, BatchBlocks pb) {
     uint32_t m, bid, nb;
     const BatchMember& a = batch_block(M, pb, m, bid, nb);
+    if (a.grid.by_cells) {
+        cell_order_at(a.where, a.cell_first, reinterpret_cast<const uint32_t*>(a.bucket), a.order,
+                      size_t(bid) * BLOCK + threadIdx.x, a.n);
+        return;
+    }
     for (size_t b = bid; b * (BLOCK / 64) < a.rows; b += nb) {
-        row_order_block(a.grid, a.row_start, a.bucket, a.order, a.cell_first, a.rows, b);
+        row_order_block(a.grid, a.row_start, a.bucket, a.where, a.order, a.cell_first, a.rows, b);
         __syncthreads();
     }
 }
@@ -2462,9 +2580,11 @@ void batch_advance(const Launch& l, const BatchMember* M, int count, BatchBlocks
     kb_bounds_final<<<unsigned(count) * unsigned(nv), BLOCK, 0, l.stream>>>(M, pb, nv);
 }
 
-void batch_sort(const Launch& l, const BatchMember* M, int count, BatchBlocks pb) {
+void batch_sort(const Launch& l, const BatchMember* M, int count, BatchBlocks pb, bool cells) {
+    if (cells) kb_cell_clear<<<pb.total, BLOCK, 0, l.stream>>>(M, pb);
     kb_row_count<<<pb.total, BLOCK, 0, l.stream>>>(M, pb);
     kb_row_scan<<<dim3(SCAN_BLOCKS, unsigned(count)), SCAN_BLOCK, 0, l.stream>>>(M);
+    if (cells) kb_cell_starts<<<pb.total, BLOCK, 0, l.stream>>>(M, pb);
     kb_row_scatter<<<pb.total, BLOCK, 0, l.stream>>>(M, pb);
     kb_row_order<<<pb.total, BLOCK, 0, l.stream>>>(M, pb);
 }

@@ -1,0 +1,139 @@
+"""The sort by cell where rows of cells are long -- bodies whose outliers stretch the grid, sheets, lines, dense bodies: the
+same bits with cells and with rows as the buckets, alone and in a batch, and a time that the particles' places do not
+decide."""
+import numpy as np
+import pytest
+
+from opensph_amd import gpu
+from opensph_amd.state import ParticleState, RunConfig, basalt
+from oracle.bridge import Oracle
+
+pytestmark = pytest.mark.gpu
+
+
+def particles(x, h):
+    st = ParticleState(len(x), [basalt()])
+    st["r"][:, :3] = x
+    st["r"][:, 3] = h
+    st["v"][:, :3] = np.random.default_rng(len(x)).normal(0.0, 1.0, size=(len(x), 3))
+    st["m"], st["rho"], st["reduce"] = 1.0, 2700.0, 1.0
+    return st
+
+
+def ball(n, seed=1):
+    k = int(np.ceil((2.0 * n) ** (1.0 / 3.0)))
+    x = np.stack(np.meshgrid(*[np.arange(k) - 0.5 * k] * 3, indexing="ij"), -1).reshape(-1, 3)
+    x = x[np.argsort(np.einsum("ij,ij->i", x, x), kind="stable")[:n]]
+    return np.random.default_rng(seed).permutation(x) + np.random.default_rng(seed).normal(0.0, 0.05, size=(n, 3))
+
+
+def box(n, size, seed):
+    return np.random.default_rng(seed).uniform(0.0, 1.0, size=(n, 3)) * np.asarray(size)
+
+
+CASES = {
+    # rows of 513 and more, and of more than 2048 particles, in a grid of 250 rows each way
+    "rows of a wavefront": lambda: (np.vstack([box(512, (140, .1, .1), 1), box(513, (140, .1, .1), 2) + [0, 5, 0]]), 1.0),
+    "rows of a block": lambda: (np.vstack([box(2048, (150, .1, .1), 3), box(2049, (150, .1, .1), 4) + [0, 5, 0],
+                                           box(700, (150, .1, .1), 5) + [0, 9, 0], [[0, 160, 0], [0, 0, 160]]]), 1.0),
+    "long rows, side by side": lambda: (np.vstack([box(2500 + 300 * k, (150, .1, .1), k) + [0, 0.667 * k, 0]
+                                                   for k in range(5)] + [[[0, 160, 0], [0, 0, 160]]]), 0.5),
+    "outliers": lambda: (np.vstack([ball(12000), [[0, 0, 900], [700, 0, 0], [0, -4000, 0]]]), 1.3),
+    "one cell": lambda: (np.vstack([box(1500, (3, 3, 3), 6), [[5e5, 0, 0]]]), 0.4),
+    "classes": lambda: (np.vstack([ball(6000), box(2000, (6, 6, 6), 7) + [20, 0, 0], [[1500, 0, 0]]]),
+                        np.r_[np.full(6000, 1.3), np.full(2000, 0.35), [1.3]]),
+    "one": lambda: (np.zeros((1, 3)), 1.0),
+}
+
+
+def stepped(st, precision, batch, **tuning):
+    cfg = RunConfig(criteria=1, initial_dt=1e-4, max_dt=1e-4)
+    other = particles(ball(300), 1.3)
+    members = [gpu.GpuSolver(s, cfg, precision=precision) for s in ([other, st] if batch else [st])]
+    for g in members:
+        g.tune(reorder_period=2, **tuning)
+    for _ in range(3):
+        for g in members:
+            g.dt = 1e-4
+        if batch:
+            gpu.step_batch(members)
+        else:
+            members[0].step()
+    out = members[-1].download(st)
+    for g in members:
+        g.close()
+    return out
+
+
+@pytest.mark.parametrize("name", list(CASES))
+def test_rows_and_cells_give_one_order(name):
+    x, h = CASES[name]()
+    st = particles(x, h)
+    print(f"[case] long rows, {name}, n={st.n}", flush=True)
+    want = np.stack(Oracle().pairs(st["r"]), axis=1)
+    want = want[np.lexsort((want[:, 1], want[:, 0]))]
+    for cells in (0, 1):
+        g = gpu.GpuSolver(st, RunConfig(criteria=1, initial_dt=1e-6))
+        g.tune(sort_cells=cells)
+        assert np.array_equal(np.stack(g.pairs(), axis=1), want)
+        g.close()
+    for precision in ("fp64", "mixed"):
+        rows = stepped(st, precision, False, sort_cells=0)
+        for batch, tuning in ((False, dict(sort_cells=1)), (False, {}), (True, dict(sort_cells=0)), (True, dict(sort_cells=1))):
+            got = stepped(st, precision, batch, **tuning)
+            for k in rows.a:
+                assert np.array_equal(rows[k], got[k]), (precision, batch, tuning, k)
+
+
+def test_a_batch_of_rows_and_cells():
+    """Members of both kinds, from one step to the next: the captured stages follow."""
+    cfg = RunConfig(criteria=1, initial_dt=1e-3, max_dt=1e-3)
+    st = particles(ball(9000), 1.3)
+    st["v"][0, 0] = 3e6  # leaves, so that this member's rows get long
+    states = [particles(ball(500), 1.3), st, particles(CASES["outliers"]()[0], 1.3)]
+    print("[case] batch of rows and cells", flush=True)
+    alone = [gpu.GpuSolver(s, cfg) for s in states]
+    batch = [gpu.GpuSolver(s, cfg) for s in states]
+    for _ in range(4):
+        for g in alone + batch:
+            g.dt = 1e-3
+        for g in alone:
+            g.step()
+        gpu.step_batch(batch)
+    for s, a, b in zip(states, alone, batch):
+        x, y = a.download(s), b.download(s)
+        for k in x.a:
+            assert np.array_equal(x[k], y[k]), k
+    for g in alone + batch:
+        g.close()
+
+
+def sort_us(x, h):
+    g = gpu.GpuSolver(particles(x, h), RunConfig(criteria=1, initial_dt=1e-6))
+    g.integrate()
+    g.profile(True)
+    for _ in range(5):
+        g.integrate()
+    ms, launches = g.profile_read()["cell_sort"]
+    g.close()
+    return 1e3 * ms / launches
+
+
+@pytest.mark.parametrize("name", ["outliers", "sheet", "line"])
+def test_time_does_not_depend_on_the_places(name):
+    """300k particles in a compact body take 20 to 27 us, far outliers 117, one line 150; the bound is twenty
+    times the compact body's (a sort in place by one block: 4200 us and more than 100 ms)."""
+    n = 300000
+    body = ball(n)
+    compact = sort_us(body, 1.3)
+    if name == "outliers":
+        half = body[:, 0] > 0
+        x = body + 2400.0 * np.c_[half, np.zeros(n), np.zeros(n)]
+    elif name == "sheet":
+        x = np.c_[np.arange(n) % 150, np.arange(n) // 150, np.zeros(n)] * [0.3, 1.0, 1.0]
+    else:
+        x = np.c_[np.arange(n), np.zeros(n), np.zeros(n)]
+    print(f"[case] sort time, {name}", flush=True)
+    t = sort_us(x, 1.3)
+    print(f"compact {compact:.0f} us, {name} {t:.0f} us", flush=True)
+    assert t < 20.0 * compact
