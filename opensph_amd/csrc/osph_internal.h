@@ -206,14 +206,32 @@ inline int pair_lanes(const Tuning& t, size_t n, int nclass) {
     return t.pairs_lanes > 1 || n < (nclass > 1 ? PAIRS_BELOW_4_CLASSES : PAIRS_BELOW_4) ? 4 : 1;
 }
 
+// Rows of cells a particle's lists walk, over all classes (49 in cells of 2h/3; a grid stretched by outliers, or flat, has
+// fewer and longer ones).
+inline double walked_rows(const Grid& g) {
+    double rows = 0.0;
+    for (int cl = 0; cl < g.nclass; ++cl) {
+        const GridClass& c = g.c[cl];
+        if (c.empty) continue;
+        const double across = 4.0 * c.hmax / c.cell + 1.0;
+        rows += std::min(double(c.dim[1]), across) * std::min(double(c.dim[2]), across);
+    }
+    return rows;
+}
+
 // Particles below which the list kernel gives each a group of lanes: one lane per particle takes about 80 us
 // however few they are, and 170 us where two smoothing-length classes meet (a lane there walks ~1000 candidates).
 // Measured, groups against single lanes: one class, 85k particles 47 against 80 us (mixed) and 61 against 82 us
 // (FP64), 169k 84 against 84 and 114 against 90; two classes, 170k 85 against 168 and 113 against 171, 340k 162
-// against 177 and 212 against 188.
+// against 177 and 212 against 188.  A group's lanes take a row each, so few long rows leave most of them idle: 12 rows, 125k
+// 166 against 186 us (FP64); 9.5 rows, 200k 333 against 219; 9 rows, 30k 67 against 133; 6.6 rows, 60k 256 against 216; 5.3
+// rows, 30k 207 against 217, 90k 35 against 22 (a sheet); 4 rows, 60k 537 against 227; 3 rows, 125k 2127 against 498; one row
+// (a line), 300 8 against 7, 30k 133 against 48.
 constexpr size_t LISTS_SHARED_BELOW = 131072, LISTS_SHARED_BELOW_CLASSES = 262144;
+constexpr double LISTS_SHARED_PER_ROW = 9000.0;  // for every row but one
 inline bool lists_shared(const Grid& g, size_t n) {
-    return n < (g.nclass > 1 ? LISTS_SHARED_BELOW_CLASSES : LISTS_SHARED_BELOW);
+    return n < (g.nclass > 1 ? LISTS_SHARED_BELOW_CLASSES : LISTS_SHARED_BELOW) &&
+           double(n) < LISTS_SHARED_PER_ROW * (walked_rows(g) - 1.0);
 }
 
 // Whether a class's rows of cells may be too long to be ordered a row at a time (the sort's buckets, see

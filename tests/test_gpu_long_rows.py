@@ -108,13 +108,13 @@ def test_a_batch_of_rows_and_cells():
         g.close()
 
 
-def sort_us(x, h):
+def kernel_us(x, h, name):
     g = gpu.GpuSolver(particles(x, h), RunConfig(criteria=1, initial_dt=1e-6))
     g.integrate()
     g.profile(True)
     for _ in range(5):
         g.integrate()
-    ms, launches = g.profile_read()["cell_sort"]
+    ms, launches = g.profile_read()[name]
     g.close()
     return 1e3 * ms / launches
 
@@ -125,7 +125,7 @@ def test_time_does_not_depend_on_the_places(name):
     times the compact body's (a sort in place by one block: 4200 us and more than 100 ms)."""
     n = 300000
     body = ball(n)
-    compact = sort_us(body, 1.3)
+    compact = kernel_us(body, 1.3, "cell_sort")
     if name == "outliers":
         half = body[:, 0] > 0
         x = body + 2400.0 * np.c_[half, np.zeros(n), np.zeros(n)]
@@ -134,6 +134,24 @@ def test_time_does_not_depend_on_the_places(name):
     else:
         x = np.c_[np.arange(n), np.zeros(n), np.zeros(n)]
     print(f"[case] sort time, {name}", flush=True)
-    t = sort_us(x, 1.3)
+    t = kernel_us(x, 1.3, "cell_sort")
     print(f"compact {compact:.0f} us, {name} {t:.0f} us", flush=True)
     assert t < 20.0 * compact
+
+
+@pytest.mark.parametrize("shape", ["bodies far apart", "sheet", "line"])
+def test_lists_of_few_long_rows(shape):
+    """Below 131072 particles a group of lanes makes a particle's list, above a single one; where the particle walks few
+    rows, the smaller number must not take longer for it (with groups: 4.3, 2.0 and more than 2.5 times)."""
+    def places(n):
+        if shape == "sheet":
+            return np.c_[np.arange(n) % 354, np.arange(n) // 354, np.zeros(n)]
+        if shape == "line":
+            return np.c_[np.arange(n), np.zeros(n), np.zeros(n)]
+        x = ball(n)
+        return x + 1550.0 * np.c_[x[:, 0] > 0, np.zeros(n), np.zeros(n)]
+
+    print(f"[case] lists, {shape}", flush=True)
+    few, many = (min(kernel_us(places(n), 1.3, "neighbor_lists") for _ in range(2)) for n in (125000, 135000))
+    print(f"125k {few:.0f} us, 135k {many:.0f} us", flush=True)
+    assert few < 1.5 * many
