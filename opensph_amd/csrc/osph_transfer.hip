@@ -1,4 +1,4 @@
-// Device results into the caller's (pageable) host memory.
+// Device results into the caller's host memory, pageable as a rule.
 //
 // hipMemcpyAsync into pageable memory goes through the runtime's staging buffer, 1 MB at a time: each megabyte is
 // copied by the device (20 us), then by one host thread, about 12 GB/s in all.  Here the pieces go through pinned
@@ -113,6 +113,15 @@ hipError_t copy_range(hipStream_t stream, PinnedBuffer& b, unsigned char* host, 
     return err;
 }
 
+// Whether the runtime knows the memory (allocated or registered through it), so that the device can copy to it itself.
+bool known_memory(const void* p) {
+    const hipError_t before = hipPeekAtLastError();
+    hipPointerAttribute_t at{};
+    if (hipPointerGetAttributes(&at, p) == hipSuccess) return at.type != hipMemoryTypeUnregistered;
+    if (before == hipSuccess) (void)hipGetLastError();  // an earlier error stays
+    return false;
+}
+
 __global__ void __launch_bounds__(256) k_post(const unsigned long long* __restrict__ src, size_t count,
                                               unsigned long long* __restrict__ host, unsigned long long* __restrict__ posts,
                                               unsigned long long value) {
@@ -186,15 +195,19 @@ hipError_t copy_to_host(hipStream_t stream, void* host, const void* dev, size_t 
     if (!bytes) return hipSuccess;
     int device = 0;
     if (hipError_t e = hipGetDevice(&device)) return e;
+    auto direct = [&]() -> hipError_t {
+        if (hipError_t e = hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, stream)) return e;
+        return hipStreamSynchronize(stream);
+    };
+    // into the caller's pinned memory the device copies at the link's rate: 70k x 32 B 64 us, 1M x 32 B 617 us, where the
+    // pieces below take 148 and 927 us
+    if (known_memory(host)) return direct();
     const size_t hw = std::max<size_t>(std::thread::hardware_concurrency(), 1);
     const size_t want = std::min({ size_t(COPY_THREADS), hw, bytes / THREAD_BYTES + 1 });
     PinnedBuffer buf[COPY_THREADS];
     size_t parts = 0;
     while (parts < want && take_buffer(device, buf[parts])) ++parts;
-    if (parts == 0) {
-        if (hipError_t e = hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, stream)) return e;
-        return hipStreamSynchronize(stream);
-    }
+    if (parts == 0) return direct();
     // whole pieces per part
     const size_t share = ((bytes + parts - 1) / parts + PIECE - 1) / PIECE * PIECE;
     hipError_t errs[COPY_THREADS];

@@ -1,0 +1,26 @@
+"""copy_to_host on a runtime without a device: where results go directly, the pinned buffers and what it does when something
+is not to be had."""
+import pytest
+
+import host_stub
+
+pytestmark = pytest.mark.skipif(not host_stub.available(), reason="needs the built library and g++")
+
+
+@pytest.fixture(scope="module")
+def stub(tmp_path_factory):
+    return host_stub.build_stub(tmp_path_factory.mktemp("stub"))
+
+
+@pytest.mark.parametrize("n", [3, 2000, 300000])
+def test_pinned_destination_is_copied_to_directly(stub, n):
+    """A buffer that the runtime knows takes the device's copy itself: one copy of all bytes, no pinned buffer."""
+    host_stub.run(stub, f"""
+        s = solver({n})
+        p = C.c_void_p()
+        assert stub.hipHostMalloc(C.byref(p), C.c_size_t(32 * {n}), 0) == 0
+        stub.stub_reset()
+        assert get(s, p.value) == 0
+        assert stub.stub_counter(1) == 1 and stub.stub_counter(3) == 32 * {n}, [stub.stub_counter(k) for k in range(4)]
+        assert stub.stub_counter(0) == 0 and stub.stub_counter(2) == 0
+    """)
