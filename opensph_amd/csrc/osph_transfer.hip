@@ -44,34 +44,44 @@ PinnedPool& pool() {
     return p;
 }
 
-void destroy_buffer(PinnedBuffer& b) {
-    for (hipEvent_t e : b.done) {
+void destroy_events(PinnedBuffer& b) {
+    for (hipEvent_t& e : b.done) {
         if (e) (void)hipEventDestroy(e);
+        e = nullptr;
     }
+}
+
+void destroy_buffer(PinnedBuffer& b) {
+    destroy_events(b);
     if (b.mem) (void)hipHostFree(b.mem);
     b = PinnedBuffer{};
 }
 
-// A buffer whose events belong to `device`; false when the pool is at its limit or the allocation fails (the caller
-// then copies without one).
+// A buffer whose events belong to `device`: an idle one of that device, a new one, or at the limit an idle one of another
+// device (the memory serves all, the events are made anew).  False when all are in use or something cannot be
+// allocated (the caller then copies without one).
 bool take_buffer(int device, PinnedBuffer& out) {
     PinnedPool& p = pool();
+    PinnedBuffer b;
     {
         std::lock_guard<std::mutex> g(p.lock);
-        for (size_t k = 0; k < p.idle.size(); ++k) {
-            if (p.idle[k].device != device) continue;
-            out = p.idle[k];
+        size_t k = 0;
+        while (k < p.idle.size() && p.idle[k].device != device) ++k;
+        if (k == p.idle.size() && p.made < MAX_BUFFERS) {
+            ++p.made;
+        } else if (!p.idle.empty()) {
+            k = std::min(k, p.idle.size() - 1);
+            b = p.idle[k];
             p.idle.erase(p.idle.begin() + long(k));
-            return true;
+        } else {
+            return false;
         }
-        if (p.made >= MAX_BUFFERS) return false;
-        ++p.made;
     }
-    PinnedBuffer b;
+    if (b.device != device) destroy_events(b);
     b.device = device;
-    if (hipHostMalloc(reinterpret_cast<void**>(&b.mem), 2 * PIECE, hipHostMallocPortable) == hipSuccess &&
-        hipEventCreateWithFlags(&b.done[0], hipEventDisableTiming) == hipSuccess &&
-        hipEventCreateWithFlags(&b.done[1], hipEventDisableTiming) == hipSuccess) {
+    bool made = b.mem || hipHostMalloc(reinterpret_cast<void**>(&b.mem), 2 * PIECE, hipHostMallocPortable) == hipSuccess;
+    for (hipEvent_t& e : b.done) made = made && (e || hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess);
+    if (made) {
         out = b;
         return true;
     }

@@ -24,3 +24,20 @@ def test_pinned_destination_is_copied_to_directly(stub, n):
         assert stub.stub_counter(1) == 1 and stub.stub_counter(3) == 32 * {n}, [stub.stub_counter(k) for k in range(4)]
         assert stub.stub_counter(0) == 0 and stub.stub_counter(2) == 0
     """)
+
+
+def test_idle_buffers_pass_from_one_device_to_another(stub):
+    """Two devices have four pinned buffers each, which is all there may be; a third one gets idle ones, with events of its
+    own."""
+    host_stub.run(stub, """
+        out = np.zeros((300000, 4))
+        for device in (0, 1, 2, 0, 2):
+            stub.hipSetDevice(device)
+            s = solver(300000)
+            stub.stub_reset()
+            assert get(s, out) == 0
+            assert stub.stub_counter(0) == 0, (device, "pageable copies")
+            assert stub.stub_counter(6) == 0, (device, "another device's events")
+            if device == 0:
+                first = s  # the pool goes with the last context
+    """)
