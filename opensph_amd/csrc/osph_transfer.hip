@@ -12,8 +12,8 @@
 #include <algorithm>
 #include <chrono>
 #include <cstring>
+#include <exception>
 #include <mutex>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -236,8 +236,8 @@ hipError_t copy_to_host(hipStream_t stream, void* host, const void* dev, size_t 
                 errs[k] = hipSetDevice(device);
                 if (errs[k] == hipSuccess) part(k);
             });
-        } catch (const std::system_error&) {
-            break;  // no further thread to be had: this one does the rest
+        } catch (const std::exception&) {
+            break;  // no further thread, or no memory for one: this one does the rest
         }
     }
     part(0);

@@ -41,3 +41,17 @@ def test_idle_buffers_pass_from_one_device_to_another(stub):
             if device == 0:
                 first = s  # the pool goes with the last context
     """)
+
+
+def test_no_memory_for_a_thread(stub):
+    """A further copy thread whose state cannot be allocated: the calling thread does the rest."""
+    host_stub.run(stub, """
+        s = solver(300000)
+        out = np.zeros((300000, 4))
+        assert get(s, out) == 0
+        stub.stub_reset()
+        stub.stub_fail_new(1)
+        rc = get(s, out)
+        stub.stub_fail_new(0)
+        assert rc == 0 and stub.stub_counter(1) == 5, (rc, stub.stub_counter(1))
+    """)
