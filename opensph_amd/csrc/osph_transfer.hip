@@ -77,6 +77,7 @@ bool take_buffer(int device, PinnedBuffer& out) {
             return false;
         }
     }
+    const hipError_t before = hipPeekAtLastError();
     if (b.device != device) destroy_events(b);
     b.device = device;
     bool made = b.mem || hipHostMalloc(reinterpret_cast<void**>(&b.mem), 2 * PIECE, hipHostMallocPortable) == hipSuccess;
@@ -85,7 +86,7 @@ bool take_buffer(int device, PinnedBuffer& out) {
         out = b;
         return true;
     }
-    (void)hipGetLastError();
+    if (before == hipSuccess) (void)hipGetLastError();  // an earlier error stays
     destroy_buffer(b);
     std::lock_guard<std::mutex> g(p.lock);
     --p.made;

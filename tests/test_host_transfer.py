@@ -55,3 +55,16 @@ def test_no_memory_for_a_thread(stub):
         stub.stub_fail_new(0)
         assert rc == 0 and stub.stub_counter(1) == 5, (rc, stub.stub_counter(1))
     """)
+
+
+def test_an_earlier_launch_error_is_reported(stub):
+    """The kernel that gathers the result did not start, and no pinned buffer is to be had: the call fails all the same."""
+    host_stub.run(stub, """
+        s = solver(2000)
+        out = np.zeros((2000, 4))
+        stub.stub_fail_host_malloc(1)
+        assert get(s, out) == 0  # without pinned memory
+        stub.stub_fail_kernel(b"k_planes_to_stage", 1)
+        assert get(s, out) != 0
+        assert get(s, out) == 0  # the error was reported once
+    """)
