@@ -91,6 +91,7 @@ struct osph_ctx {
     const char* failed_launch = nullptr;  // name of the first timed launch that left a HIP error
     uint32_t *row_count = nullptr, *row_start = nullptr;  // [slot_cap] counts (zero between searches) and their sums
     size_t slot_cap = 0;
+    bool slots_clean = false;  // the counts are zero
     uint32_t* cell_first = nullptr;  // [cells + 1]: first sorted position of each cell (valid rows only)
     size_t cell_cap = 0;
     PairRec* rec = nullptr;
@@ -259,19 +260,30 @@ int ensure_list(osph_ctx* c, size_t entries) {
     return OSPH_OK;
 }
 
-// The row counts and sums; new counts start at zero, and every search leaves them so.
-int ensure_slots(osph_ctx* c, uint32_t slots) {
+int sync_check(osph_ctx* c);
+
+// The row counts and sums for a search, the counts at zero: every search that runs to its end leaves them so, new
+// ones and those of a search whose launches failed are cleared here.  *cleared: whether they were, on this
+// context's stream.  slots_clean is false from here until the sort's launches have succeeded.
+int ensure_slots(osph_ctx* c, uint32_t slots, bool* cleared = nullptr) {
     const size_t need = row_slots(slots);
-    if (need <= c->slot_cap) return OSPH_OK;
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    (void)hipFree(c->row_count);
-    (void)hipFree(c->row_start);
-    c->row_count = c->row_start = nullptr;
-    c->slot_cap = 0;
-    HIPCHK(c, hipMalloc(&c->row_count, need * sizeof(uint32_t)));
-    HIPCHK(c, hipMalloc(&c->row_start, need * sizeof(uint32_t)));
-    launch_clear_u32(Launch{ c->stream }, c->row_count, need, 0u);
-    c->slot_cap = need;
+    if (need > c->slot_cap) {
+        HIPCHK(c, hipStreamSynchronize(c->stream));
+        (void)hipFree(c->row_count);
+        (void)hipFree(c->row_start);
+        c->row_count = c->row_start = nullptr;
+        c->slot_cap = 0;
+        c->slots_clean = false;
+        HIPCHK(c, hipMalloc(&c->row_count, need * sizeof(uint32_t)));
+        HIPCHK(c, hipMalloc(&c->row_start, need * sizeof(uint32_t)));
+        c->slot_cap = need;
+    }
+    if (cleared) *cleared = !c->slots_clean;
+    if (!c->slots_clean) {
+        launch_clear_u32(Launch{ c->stream }, c->row_count, c->slot_cap, 0u);
+        if (hipPeekAtLastError() != hipSuccess) return sync_check(c);
+    }
+    c->slots_clean = false;
     return OSPH_OK;
 }
 
@@ -668,6 +680,9 @@ int search_finish(osph_ctx* c) {
     timed(c, "cell_sort", [&] {
         launch_cell_sort(l, c->s, g, c->row_count, c->row_start, c->where, c->bucket, c->order, c->cell_first, rows, n);
     });
+    // nothing may be launched on an order that was not written
+    if (hipPeekAtLastError() != hipSuccess) return sync_check(c);
+    c->slots_clean = true;
     if (reorder_due(c)) {
         // move the state into this search's cell order: the record gather and the pair kernels' writes
         // then run over (nearly) consecutive slots until the next reorder
@@ -1437,10 +1452,10 @@ int batch_step(const std::vector<osph_ctx*>& ms, const std::vector<double>& dts,
         size_t rows = 0;
         if (int e = plan_search(c, P->box.host + SMALL_WORDS * k, &rows)) return e;
         if (int e = ensure_list(c, list_entries(c->n, c->kmax))) return e;
-        const size_t slots_before = c->slot_cap;
-        if (int e = ensure_slots(c, c->grid.slots)) return e;
-        // new counts are cleared on the member's stream, the batch runs on the lead's
-        if (c->slot_cap != slots_before) HIPCHK(c, hipStreamSynchronize(c->stream));
+        bool cleared = false;
+        if (int e = ensure_slots(c, c->grid.slots, &cleared)) return e;
+        // the counts are cleared on the member's stream, the batch runs on the lead's
+        if (cleared) HIPCHK(c, hipStreamSynchronize(c->stream));
         b.grid = c->grid;
         b.screen = c->screen;
         b.fx = c->fixed;
@@ -1472,6 +1487,7 @@ int batch_step(const std::vector<osph_ctx*>& ms, const std::vector<double>& dts,
     // values are in the member table), so they are captured once and replayed
     auto rest = [&]() {
         batch_sort(l, P->dev, int(count), P->pb, cells);
+        if (hipPeekAtLastError() != hipSuccess) return;  // nothing on orders that were not written
         batch_permute(l, P->dev, P->pb);
         batch_pack(l, P->dev, P->pb, P->mixed);
         batch_lists(l, P->dev, P->lb, screened, plain);
@@ -1484,7 +1500,12 @@ int batch_step(const std::vector<osph_ctx*>& ms, const std::vector<double>& dts,
             P->drop_graph();
             HIPCHK(lead, hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
             rest();
+            const bool whole = hipPeekAtLastError() == hipSuccess;
             HIPCHK(lead, hipStreamEndCapture(st, &P->graph));
+            if (!whole) {
+                P->drop_graph();
+                return sync_check(lead);
+            }
             HIPCHK(lead, hipGraphInstantiate(&P->exec, P->graph, nullptr, nullptr, 0));
             P->graph_screened = int(screened);
             P->graph_plain = int(plain);
@@ -1494,6 +1515,8 @@ int batch_step(const std::vector<osph_ctx*>& ms, const std::vector<double>& dts,
     } else {
         rest();
     }
+    if (hipPeekAtLastError() != hipSuccess) return sync_check(lead);
+    for (osph_ctx* c : ms) c->slots_clean = true;
     mailbox_post(st, P->box, 0, P->small, count * SMALL_WORDS);
     if (int e = wait_box(lead, P->box)) return e;
     for (size_t k = 0; k < count; ++k) {

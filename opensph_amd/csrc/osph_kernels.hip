@@ -2218,17 +2218,24 @@ void launch_cell_sort(const Launch& l, DevState s, Grid g, uint32_t* row_count, 
     // without particles nothing reads the table
     if (!rows || !n) return;
     const unsigned blocks = grid_for(n), scans = unsigned(row_slots(g.slots) / SCAN_TILE), waves = grid_for(rows, BLOCK / 64);
-    if (g.by_cells) {
-        launch_clear_u32(l, first, g.cells, 0u);
-        k_row_count<true><<<blocks, BLOCK, 0, l.stream>>>(s, g, row_count, first, where, n);
-        k_row_scan<<<scans, SCAN_BLOCK, 0, l.stream>>>(row_count, row_start);
-        k_cell_starts<<<waves, BLOCK, 0, l.stream>>>(g, row_start, first, rows);
-        k_row_scatter<true><<<blocks, BLOCK, 0, l.stream>>>(where, row_start, first, row_count, g.slots, bucket, n);
+    const bool cells = g.by_cells != 0;
+    // a kernel that does not start leaves the next one values of an older grid as indexes: the chain ends there
+    auto failed = [] { return hipPeekAtLastError() != hipSuccess; };
+    if (cells) launch_clear_u32(l, first, g.cells, 0u);
+    if (failed()) return;
+    const auto count = cells ? k_row_count<true> : k_row_count<false>;
+    count<<<blocks, BLOCK, 0, l.stream>>>(s, g, row_count, first, where, n);
+    if (failed()) return;
+    k_row_scan<<<scans, SCAN_BLOCK, 0, l.stream>>>(row_count, row_start);
+    if (failed()) return;
+    if (cells) k_cell_starts<<<waves, BLOCK, 0, l.stream>>>(g, row_start, first, rows);
+    if (failed()) return;
+    const auto scatter = cells ? k_row_scatter<true> : k_row_scatter<false>;
+    scatter<<<blocks, BLOCK, 0, l.stream>>>(where, row_start, first, row_count, g.slots, bucket, n);
+    if (failed()) return;
+    if (cells) {
         k_cell_order<<<blocks, BLOCK, 0, l.stream>>>(where, first, reinterpret_cast<const uint32_t*>(bucket), order, n);
     } else {
-        k_row_count<false><<<blocks, BLOCK, 0, l.stream>>>(s, g, row_count, first, where, n);
-        k_row_scan<<<scans, SCAN_BLOCK, 0, l.stream>>>(row_count, row_start);
-        k_row_scatter<false><<<blocks, BLOCK, 0, l.stream>>>(where, row_start, first, row_count, g.slots, bucket, n);
         k_row_order<<<waves, BLOCK, 0, l.stream>>>(g, row_start, bucket, where, order, first, rows);
     }
 }
@@ -2581,11 +2588,17 @@ void batch_advance(const Launch& l, const BatchMember* M, int count, BatchBlocks
 }
 
 void batch_sort(const Launch& l, const BatchMember* M, int count, BatchBlocks pb, bool cells) {
+    auto failed = [] { return hipPeekAtLastError() != hipSuccess; };  // as in launch_cell_sort
     if (cells) kb_cell_clear<<<pb.total, BLOCK, 0, l.stream>>>(M, pb);
+    if (failed()) return;
     kb_row_count<<<pb.total, BLOCK, 0, l.stream>>>(M, pb);
+    if (failed()) return;
     kb_row_scan<<<dim3(SCAN_BLOCKS, unsigned(count)), SCAN_BLOCK, 0, l.stream>>>(M);
+    if (failed()) return;
     if (cells) kb_cell_starts<<<pb.total, BLOCK, 0, l.stream>>>(M, pb);
+    if (failed()) return;
     kb_row_scatter<<<pb.total, BLOCK, 0, l.stream>>>(M, pb);
+    if (failed()) return;
     kb_row_order<<<pb.total, BLOCK, 0, l.stream>>>(M, pb);
 }
 

@@ -23,7 +23,7 @@ std::string failing;            // launches of a kernel whose name holds this fa
 int failures = 0;               // ... this many times
 bool host_malloc_fails = false;
 std::atomic<bool> new_fails{ false };
-long long counters[8];          // see stub_counter
+long long counters[9];          // see stub_counter
 thread_local int device = 0, last_error = SUCCESS;
 thread_local size_t launch_config[4];
 
@@ -83,17 +83,18 @@ void run(const std::string& name, void** args) {
     } else if (is("8k_boundsE")) {
         write_bounds(arg<uint64_t*>(args, 1));
     } else if (is("14k_bounds_finalE")) {
-        auto* acc = arg<uint64_t*>(args, 2);  // the classes' bounds
-        std::memset(acc, 0, 8 * 40);
-        write_bounds(acc);
-        acc[8] = 64;
+        auto* small = arg<uint64_t*>(args, 2);  // the step's accumulators, the first class's bounds from word 16 on
+        std::memset(small, 0, 8 * 64);
+        write_bounds(small + 16);
+        small[16 + 8] = 64;
+        for (int k = 56; k < 62; ++k) small[k] = ordered(0.0);  // velocities
+    } else if (is("13k_row_scatter")) {  // (where, row_start, first, row_count, slots, ...)
+        std::memset(arg<uint32_t*>(args, 3), 0, 4 * size_t(arg<uint32_t>(args, 4)));
+        ++counters[5];
     } else if (is("11k_row_count")) {  // (DevState, Grid, row_count, ...): the counts have to start at zero
         auto* counts = arg<uint32_t*>(args, 2);
         for (int k = 0; k < 4096; ++k) counters[4] += counts[k] != 0;
         counts[0] += 64;
-    } else if (is("13k_row_scatter")) {  // (where, row_start, first, row_count, slots, ...)
-        std::memset(arg<uint32_t*>(args, 3), 0, 4 * size_t(arg<uint32_t>(args, 4)));
-        ++counters[5];
     }
 }
 
@@ -112,7 +113,7 @@ extern "C" {
 // ---- the test's side ------------------------------------------------------------------------------------------
 // 0 copies to unregistered host memory, 1 to pinned host memory, 2 pinned allocations, 3 bytes of the largest copy to
 // the host, 4 row counts found non-zero, 5 scatters, 6 events recorded on another device than their own, 7 the largest
-// y or z extent of a launch
+// y or z extent of a launch, 8 launches of a search's kernels with an error pending
 long long stub_counter(int k) { return counters[k]; }
 void stub_reset() { std::memset(counters, 0, sizeof(counters)); }
 void stub_fail_kernel(const char* name, int times) { failing = name, failures = times; }
@@ -250,6 +251,9 @@ int hipLaunchKernel(const void* host, Dim3 grid, Dim3, void** args, size_t, void
     const std::string& name = kernels[host];
     if (counters[7] < (long long)grid.y) counters[7] = grid.y;
     if (counters[7] < (long long)grid.z) counters[7] = grid.z;
+    for (const char* k : { "k_row_", "k_cell_", "kb_row_", "kb_cell_", "k_pack", "k_permute", "k_neighbor_lists" }) {
+        if (last_error != SUCCESS && name.find(k) != std::string::npos) ++counters[8];
+    }
     if (failures > 0 && name.find(failing) != std::string::npos) {
         --failures;
         return fail(OUT_OF_MEMORY);

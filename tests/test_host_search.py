@@ -1,0 +1,52 @@
+"""A neighbour search whose launches fail, on a runtime without a device: the calls after it start from clean row counts, and
+nothing is launched on what the failed kernel did not write."""
+import pytest
+
+import host_stub
+
+pytestmark = pytest.mark.skipif(not host_stub.available(), reason="needs the built library and g++")
+
+BODY = """
+    s = solver(64, {precision!r})
+    def call():
+        nd, crit, dt = C.c_double(), C.c_int(), 1e-6
+        if {batch}:
+            two = (C.c_void_p * 2)(s.ctx, other.ctx)
+            return s.L.osph_step_pc_batch(two, 2, (C.c_double * 2)(dt, dt), (C.c_double * 2)(), (C.c_int * 2)())
+        return s.L.osph_step_pc(s.ctx, dt, C.byref(nd), C.byref(crit))
+    other = solver(64, {precision!r})
+    for g in (s, other):
+        g.tune(sort_cells={cells}, batch_graph=0)
+    stub.stub_box(30.0)
+    assert call() == 0
+    stub.stub_reset()
+    assert call() == 0 and stub.stub_counter(5) == {scatters}
+    stub.stub_fail_kernel({kernel!r}, 1)
+    assert call() != 0
+    assert stub.stub_counter(8) == 0, "launches after the failed one"
+    stub.stub_reset()
+    for _ in range(2):
+        assert call() == 0
+    assert stub.stub_counter(4) == 0, "row counts that do not start at zero"
+"""
+
+
+@pytest.fixture(scope="module")
+def stub(tmp_path_factory):
+    return host_stub.build_stub(tmp_path_factory.mktemp("stub"))
+
+
+@pytest.mark.parametrize("kernel", ["k_row_count", "k_row_scan", "k_row_scatter", "k_row_order"])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_a_failed_launch_of_the_sort(stub, kernel, precision):
+    host_stub.run(stub, BODY.format(precision=precision, batch=False, cells=0, scatters=1, kernel=kernel.encode()))
+
+
+@pytest.mark.parametrize("kernel", ["k_fill_u32", "k_row_count", "k_row_scan", "k_cell_starts", "k_row_scatter", "k_cell_order"])
+def test_a_failed_launch_of_the_sort_by_cells(stub, kernel):
+    host_stub.run(stub, BODY.format(precision="fp64", batch=False, cells=1, scatters=1, kernel=kernel.encode()))
+
+
+@pytest.mark.parametrize("cells,kernel", [(0, "kb_row_scatter"), (1, "kb_cell_clear"), (1, "kb_cell_starts"), (0, "kb_row_order")])
+def test_a_failed_launch_in_a_batch(stub, cells, kernel):
+    host_stub.run(stub, BODY.format(precision="fp64", batch=True, cells=cells, scatters=0, kernel=kernel.encode()))
