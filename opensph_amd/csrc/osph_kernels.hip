@@ -2474,8 +2474,8 @@ __global__ void __launch_bounds__(BLOCK) kb_row_count(const BatchMember* __restr
 
 constexpr unsigned SCAN_BLOCKS = 8;  // per member, over its tiles
 __global__ void __launch_bounds__(SCAN_BLOCK) kb_row_scan(const BatchMember* __restrict__ M) {
-    const BatchMember& a = M[blockIdx.y];
-    for (uint32_t t = blockIdx.x; t < a.grid.slots / SCAN_TILE + 1u; t += SCAN_BLOCKS) {
+    const BatchMember& a = M[blockIdx.x / SCAN_BLOCKS];
+    for (uint32_t t = blockIdx.x % SCAN_BLOCKS; t < a.grid.slots / SCAN_TILE + 1u; t += SCAN_BLOCKS) {
         row_scan_tile(a.row_count, a.row_start, t);
         __syncthreads();
     }
@@ -2593,7 +2593,7 @@ void batch_sort(const Launch& l, const BatchMember* M, int count, BatchBlocks pb
     if (failed()) return;
     kb_row_count<<<pb.total, BLOCK, 0, l.stream>>>(M, pb);
     if (failed()) return;
-    kb_row_scan<<<dim3(SCAN_BLOCKS, unsigned(count)), SCAN_BLOCK, 0, l.stream>>>(M);
+    kb_row_scan<<<SCAN_BLOCKS * unsigned(count), SCAN_BLOCK, 0, l.stream>>>(M);
     if (failed()) return;
     if (cells) kb_cell_starts<<<pb.total, BLOCK, 0, l.stream>>>(M, pb);
     if (failed()) return;

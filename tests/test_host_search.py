@@ -50,3 +50,16 @@ def test_a_failed_launch_of_the_sort_by_cells(stub, kernel):
 @pytest.mark.parametrize("cells,kernel", [(0, "kb_row_scatter"), (1, "kb_cell_clear"), (1, "kb_cell_starts"), (0, "kb_row_order")])
 def test_a_failed_launch_in_a_batch(stub, cells, kernel):
     host_stub.run(stub, BODY.format(precision="fp64", batch=True, cells=cells, scatters=0, kernel=kernel.encode()))
+
+
+def test_a_batch_has_no_limit_of_the_grid(stub):
+    """The members lie along x, whose extent is 2^31 - 1 blocks; y and z end at 65535."""
+    host_stub.run(stub, """
+        members = [solver(64) for _ in range(5)]
+        for g in members:
+            g.tune(batch_graph=0)
+        stub.stub_reset()
+        ctxs = (C.c_void_p * 5)(*[g.ctx for g in members])
+        assert members[0].L.osph_step_pc_batch(ctxs, 5, (C.c_double * 5)(*[1e-6] * 5), (C.c_double * 5)(), (C.c_int * 5)()) == 0
+        assert stub.stub_counter(7) == 1, stub.stub_counter(7)
+    """)
