@@ -719,8 +719,13 @@ __device__ __forceinline__ void add_multipole(const NodeMom& q, double drx, doub
     a[2] += az;
 }
 
-// 1 / sqrt(x) for x > 0: the hardware estimate and one third-order step, y (1 + e/2 + 3 e^2 / 8) with e = 1 - x y^2.
+// 1 / sqrt(x) for x > 0: the hardware estimate and one third-order step, y (1 + e/2 + 3 e^2 / 8) with e = 1 - x y^2, the
+// binomial series of (1 - e)^(-1/2) to second order (Householder 1970, The Numerical Treatment of a Single Nonlinear
+// Equation, for the family).  WIDE: an infinite x, a squared distance past the largest number, is taken as that
+// number, as its estimate would be 0 and the step 0 * infinity.
+template <bool WIDE>
 __device__ __forceinline__ double rsqrt_step(double x) {
+    if (WIDE) x = __builtin_fmin(x, 1.79769313486231570815e308);
     const double y = __builtin_amdgcn_rsq(x);
     const double e = fma(-(x * y), y, 1.0);
     return fma(y * e, fma(e, 0.375, 0.5), y);
@@ -766,10 +771,10 @@ __device__ __forceinline__ void octupole_dd(const NodeRow<double, 3>& r, double 
 //   octupole   7.5 il^7 (q3:dd) - 17.5 il^9 (q3:ddd) d
 // The terms along d share one factor and the tensors carry theirs (-3, 7.5) from the staging: 40 FP64
 // instructions for a quadrupole, against about 65 in the order the reference writes them.
-template <int ORDER>
+template <int ORDER, bool WIDE>
 __device__ __forceinline__ void expand(const NodeRow<double, ORDER>& r, double x, double y, double z, double a[3]) {
     const double dx = r.v[0] - x, dy = r.v[1] - y, dz = r.v[2] - z;
-    const double il = rsqrt_step(dx * dx + dy * dy + dz * dz);
+    const double il = rsqrt_step<WIDE>(dx * dx + dy * dy + dz * dz);
     const double inv = il * il, i3 = inv * il;
     double s = i3 * r.v[3];
     if constexpr (ORDER >= 2) {
@@ -1161,7 +1166,9 @@ __device__ __forceinline__ void add_shared(const Planes& s, const uint32_t* __re
 // lanes of 9 x 7, against 51 of 17 x 3).  A batch is B = S floor(64 / S) entries, so that each of the S splits of
 // the wavefront takes the same number.  One comparison against the batch's largest softening radius sends a pair
 // to the branch that handles softening and the particle itself; the others are Newtonian.
-template <int ORDER>
+// WIDE: the tree's box is so wide that squared distances can overflow; the others save the test of it (2 % of the N-body
+// step of 1M particles).
+template <int ORDER, bool WIDE>
 __global__ void __launch_bounds__(BLOCK) k_eval(Tree t, Planes s, const uint32_t* __restrict__ order,
                                                 const uint32_t* __restrict__ targets, uint32_t ntargets, WalkLists wl,
                                                 uint32_t split, EvalCounts counts, const double* __restrict__ grads) {
@@ -1234,8 +1241,8 @@ __global__ void __launch_bounds__(BLOCK) k_eval(Tree t, Planes s, const uint32_t
                 wave_sync();
                 for (uint32_t j = j0; j < cnt; j += S) {
                     const NodeRow<double, ORDER> r = S_.row[j];
-                    expand<ORDER>(r, me0.x, me0.y, me0.z, a0);
-                    expand<ORDER>(r, me1.x, me1.y, me1.z, a1);
+                    expand<ORDER, WIDE>(r, me0.x, me0.y, me0.z, a0);
+                    expand<ORDER, WIDE>(r, me1.x, me1.y, me1.z, a1);
                 }
                 wave_sync();
             }
@@ -1268,7 +1275,7 @@ __global__ void __launch_bounds__(BLOCK) k_eval(Tree t, Planes s, const uint32_t
                     if (d2 <= far) {
                         if (S_.idx[j] != k) add_pair<false>(grads, rx, ry, rz, 0.5 * (S_.h[j] + me.w), o.m, a);
                     } else {
-                        const double il = rsqrt_step(d2);
+                        const double il = rsqrt_step<WIDE>(d2);
                         const double f = (o.m * il) * (il * il);
                         a[0] += rx * f;
                         a[1] += ry * f;
@@ -1931,6 +1938,7 @@ struct osph_gravity {
     WalkNodeF* wnf = nullptr;
     bool skip_ready = false;  // the skip links of this tree are built (by the first evaluation at points)
     double ctr[3] = { 0.0, 0.0, 0.0 }, invL = 1.0;
+    bool wide = false;  // squared distances within the root box may overflow
     int walk_screen = -1;  // 1, -1: FP32-screened opening tests, 0: FP64 tests (the same lists)
     uint32_t *leaf_at = nullptr, *targets = nullptr, *ntargets_dev = nullptr;
     void* select_temp = nullptr;
@@ -2243,6 +2251,7 @@ int build_tree(osph_gravity* g, bool reorder = false) {
     int e = 0;
     if (ext > 0.0) (void)std::frexp(ext, &e);
     g->invL = std::ldexp(1.0, -e);
+    g->wide = !(ext < std::ldexp(1.0, 510));  // every distance lies within the root box
     g->skip_ready = false;
     Tree t = tree_of(g);
     timed(g, "morton", [&] { k_morton<<<grid_for(n), BLOCK, 0, st>>>(g->s, lo[0], lo[1], lo[2], scale, g->keys, g->iota, n); });
@@ -2304,7 +2313,8 @@ void launch_eval(osph_gravity* g, const Tree& t, const WalkLists& wl, const Eval
     if (g->precision == OSPH_PRECISION_MIXED) {
         k_eval_mixed<ORDER><<<blocks, BLOCK, 0, g->stream>>>(t, g->s, g->order, g->targets, nt, wl, split, counts, grads);
     } else {
-        k_eval<ORDER><<<blocks, BLOCK, 0, g->stream>>>(t, g->s, g->order, g->targets, nt, wl, split, counts, grads);
+        const auto kernel = g->wide ? k_eval<ORDER, true> : k_eval<ORDER, false>;
+        kernel<<<blocks, BLOCK, 0, g->stream>>>(t, g->s, g->order, g->targets, nt, wl, split, counts, grads);
     }
 }
 
