@@ -25,10 +25,6 @@ constexpr int COPY_THREADS = 4;
 constexpr size_t MAX_BUFFERS = 8;          // pinned buffers of the process (32 MB)
 constexpr size_t THREAD_BYTES = size_t(2) << 20;  // a further thread for every so many bytes
 
-// Between these the runtime's own copy is the faster one; us of the runtime's copy / of the pieces, median of 200 reads: 16 kB
-// 31 / 18, 64 kB 49 / 33, 128 kB 30 / 35, 512 kB 45 / 53, 1 MB 68 / 75, 2 MB 142 / 143, 4 MB 268 / 211.
-constexpr size_t DIRECT_FROM = 100000, DIRECT_BELOW = size_t(2) << 20;
-
 struct PinnedBuffer {
     unsigned char* mem = nullptr;  // two pieces
     hipEvent_t done[2] = { nullptr, nullptr };
@@ -216,7 +212,7 @@ hipError_t copy_to_host(hipStream_t stream, void* host, const void* dev, size_t 
     };
     // into the caller's pinned memory the device copies at the link's rate: 70k x 32 B 64 us, 1M x 32 B 617 us, where the
     // pieces below take 148 and 927 us
-    if (known_memory(host) || (bytes >= DIRECT_FROM && bytes < DIRECT_BELOW)) return direct();
+    if (known_memory(host)) return direct();
     const size_t hw = std::max<size_t>(std::thread::hardware_concurrency(), 1);
     const size_t want = std::min({ size_t(COPY_THREADS), hw, bytes / THREAD_BYTES + 1 });
     PinnedBuffer buf[COPY_THREADS];

@@ -68,16 +68,3 @@ def test_an_earlier_launch_error_is_reported(stub):
         assert get(s, out) != 0
         assert get(s, out) == 0  # the error was reported once
     """)
-
-
-@pytest.mark.parametrize("n,pieces", [(3, 1), (2047, 1), (3200, 0), (32768, 0), (65535, 0), (65536, 1), (200000, 4)])
-def test_sizes_that_take_the_pinned_pieces(stub, n, pieces):
-    """Below 100 kB and from 2 MB on, in pieces of 2 MB; the runtime's own copy is the faster one between."""
-    host_stub.run(stub, f"""
-        s = solver({n})
-        out = np.zeros(({n}, 4))
-        stub.stub_reset()
-        assert get(s, out) == 0
-        assert (stub.stub_counter(0), stub.stub_counter(1)) == ({1 if pieces == 0 else 0}, {pieces}), \\
-            (stub.stub_counter(0), stub.stub_counter(1))
-    """)
