@@ -1553,8 +1553,7 @@ int osph_step_pc_batch(osph_ctx** ctxs, int count, const double* dt, double* nex
             if (ctxs[j] == ctxs[k]) return ctxs[k]->fail(OSPH_ERR_ARG, "a context appears twice in the batch");
         }
     }
-    // one launch per stage when the members with particles share the precision and the lanes per particle
-    // (which fix the order of the pair sums) and none has self-gravity attached
+    // one launch per stage when the members with particles share the precision and none has self-gravity attached
     std::vector<osph_ctx*> ms;
     std::vector<double> dts;
     std::vector<int> at;
@@ -1563,9 +1562,7 @@ int osph_step_pc_batch(osph_ctx** ctxs, int count, const double* dt, double* nex
         osph_ctx* c = ctxs[k];
         if (!(dt[k] > 0.0) || !std::isfinite(dt[k])) return c->fail(OSPH_ERR_ARG, "time step must be positive");
         if (!c->n) continue;
-        if (!ms.empty() && (c->cfg.precision != ms[0]->cfg.precision || c->tune.pairs_lanes != ms[0]->tune.pairs_lanes)) {
-            batched = false;
-        }
+        if (!ms.empty() && c->cfg.precision != ms[0]->cfg.precision) batched = false;
         if (c->grav) batched = false;
         ms.push_back(c);
         dts.push_back(dt[k]);

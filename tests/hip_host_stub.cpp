@@ -23,7 +23,7 @@ std::string failing;            // launches of a kernel whose name holds this fa
 int failures = 0;               // ... this many times
 bool host_malloc_fails = false;
 std::atomic<bool> new_fails{ false };
-long long counters[9];          // see stub_counter
+long long counters[10];          // see stub_counter
 thread_local int device = 0, last_error = SUCCESS;
 thread_local size_t launch_config[4];
 
@@ -113,7 +113,8 @@ extern "C" {
 // ---- the test's side ------------------------------------------------------------------------------------------
 // 0 copies to unregistered host memory, 1 to pinned host memory, 2 pinned allocations, 3 bytes of the largest copy to
 // the host, 4 row counts found non-zero, 5 scatters, 6 events recorded on another device than their own, 7 the largest
-// y or z extent of a launch, 8 launches of a search's kernels with an error pending
+// y or z extent of a launch, 8 launches of a search's kernels with an error pending,
+// 9 launches for all members of a batch
 long long stub_counter(int k) { return counters[k]; }
 void stub_reset() { std::memset(counters, 0, sizeof(counters)); }
 void stub_fail_kernel(const char* name, int times) { failing = name, failures = times; }
@@ -251,6 +252,7 @@ int hipLaunchKernel(const void* host, Dim3 grid, Dim3, void** args, size_t, void
     const std::string& name = kernels[host];
     if (counters[7] < (long long)grid.y) counters[7] = grid.y;
     if (counters[7] < (long long)grid.z) counters[7] = grid.z;
+    if (name.find("kb_") != std::string::npos) ++counters[9];
     for (const char* k : { "k_row_", "k_cell_", "kb_row_", "kb_cell_", "k_pack", "k_permute", "k_neighbor_lists" }) {
         if (last_error != SUCCESS && name.find(k) != std::string::npos) ++counters[8];
     }

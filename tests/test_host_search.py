@@ -63,3 +63,17 @@ def test_a_batch_has_no_limit_of_the_grid(stub):
         assert members[0].L.osph_step_pc_batch(ctxs, 5, (C.c_double * 5)(*[1e-6] * 5), (C.c_double * 5)(), (C.c_int * 5)()) == 0
         assert stub.stub_counter(7) == 1, stub.stub_counter(7)
     """)
+
+
+@pytest.mark.parametrize("lanes", [(1, 1), (1, 2), (4, 1), (2, 4)])
+def test_members_with_other_lanes_are_batched(stub, lanes):
+    """The sums are the same bits whatever the lanes per particle, so these do not keep members apart."""
+    host_stub.run(stub, f"""
+        members = [solver(64) for _ in range(2)]
+        for g, lanes in zip(members, {lanes}):
+            g.tune(pairs_lanes=lanes)
+        stub.stub_reset()
+        ctxs = (C.c_void_p * 2)(*[g.ctx for g in members])
+        assert members[0].L.osph_step_pc_batch(ctxs, 2, (C.c_double * 2)(1e-6, 1e-6), (C.c_double * 2)(), (C.c_int * 2)()) == 0
+        assert stub.stub_counter(9) > 0
+    """)
