@@ -261,7 +261,7 @@ int osph_adjoint_clear(osph_ctx* ctx);
 int osph_tune(osph_ctx* ctx, const char* key, long long value);
 /* Launch-shape autotuner (no reference counterpart): coordinate descent over osph_tune keys.  keys[k] takes
  * the n_values[k] candidates values[sum(n_values[<k]) ...], the first of them the starting value (keys = NULL:
- * pairs_lanes 1/2/4, cell_divisor 3/2/4, lists_block 256/128, pairs_block 256/128, fuse_finalize 1/0/-1).
+ * pairs_lanes 1/4, cell_divisor 3/2/4, lists_block 256/128, pairs_block 256/128, fuse_finalize 1/0/-1).
  * Each candidate is timed over `steps` osph_step_pc calls with time step dt (after one untimed step) on the
  * resident state, which is restored on the device after every candidate: the tuning leaves the run where it
  * was.  One key at a time, in order, the fastest value is kept.  The chosen values are applied and written

@@ -77,3 +77,19 @@ def test_members_with_other_lanes_are_batched(stub, lanes):
         assert members[0].L.osph_step_pc_batch(ctxs, 2, (C.c_double * 2)(1e-6, 1e-6), (C.c_double * 2)(), (C.c_int * 2)()) == 0
         assert stub.stub_counter(9) > 0
     """)
+
+
+def test_the_tuner_times_every_launch_shape_once(stub):
+    """The default space, in the library and in Python: no two candidates that are the same launch at every size."""
+    host_stub.run(stub, """
+        from opensph_amd import autotune
+        s = solver(64)
+        trials = C.c_int()
+        chosen = (C.c_longlong * 5)()
+        best = C.c_double()
+        assert s.L.osph_step_pc(s.ctx, 1e-6, None, None) == 0
+        assert s.L.osph_autotune(s.ctx, 1e-6, 1, None, None, None, 0, chosen, C.byref(best), None, 0, C.byref(trials)) == 0
+        assert trials.value == 1 + sum(len(v) - 1 for _, v in autotune.DEFAULT_SPACE)
+        lanes = dict(autotune.DEFAULT_SPACE)["pairs_lanes"]
+        assert len(lanes) == len({4 if v > 1 else 1 for v in lanes})  # 2 and 4 are one launch
+    """)
