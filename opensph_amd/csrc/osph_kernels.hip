@@ -1100,16 +1100,16 @@ constexpr int PAIR_SUMS = 11;  // ax, ay, az, du, div v, grad v (xx, yy, zz, xy,
 enum PairSum : int { SUM_A = 0, SUM_DU = 3, SUM_DIV = 4, SUM_G = 5 };
 
 // FP64: a component gets up to three products factor * x per neighbour, each one fused multiply-add as on a single
-// lane (pressure, stress and viscosity for the accelerations; one product for the others).
+// lane (pressure, stress and viscosity for the accelerations; one product for the others).  A product that the pair does not
+// have is 0 * -0, which leaves every sum as it is, also where the mass is infinite or not a number.
 struct alignas(16) PairTerms64 {
-    double m, mr;       // factors: mass for the accelerations and du, m / rho_i for the velocity gradients
-    double x[11];       // first product of each component
+    double m, ms, mv, mr, mg;  // factors: the mass (pressure; stress; viscosity and du), m / rho_i (divergence; gradients)
+    double x[11];              // first product of each component
     double stress[3], visc[3];
-    double pad;
     __device__ __forceinline__ void clear() {
-        m = mr = 0.0;
-        for (int c = 0; c < 11; ++c) x[c] = 0.0;
-        for (int c = 0; c < 3; ++c) stress[c] = visc[c] = 0.0;
+        m = ms = mv = mr = mg = 0.0;
+        for (int c = 0; c < 11; ++c) x[c] = -0.0;
+        for (int c = 0; c < 3; ++c) stress[c] = visc[c] = -0.0;
     }
     __device__ __forceinline__ void factors(double mj, double mjr) {
         m = mj;
@@ -1121,31 +1121,33 @@ struct alignas(16) PairTerms64 {
         x[1] = -vy;
         x[2] = -vz;
     }
-    __device__ __forceinline__ void gradient(double, const double v[6]) {
+    __device__ __forceinline__ void gradient(double mjr, const double v[6]) {
+        mg = mjr;
         for (int c = 0; c < 6; ++c) x[SUM_G + c] = v[c];
     }
-    __device__ __forceinline__ void stresses(double, double vx, double vy, double vz) {
+    __device__ __forceinline__ void stresses(double mj, double vx, double vy, double vz) {
+        ms = mj;
         stress[0] = vx;
         stress[1] = vy;
         stress[2] = vz;
     }
-    __device__ __forceinline__ void viscosity(double, double vx, double vy, double vz, double heat) {
+    __device__ __forceinline__ void viscosity(double mj, double vx, double vy, double vz, double heat) {
+        mv = mj;
         visc[0] = -vx;
         visc[1] = -vy;
         visc[2] = -vz;
         x[SUM_DU] = heat;
     }
     __device__ __forceinline__ double add_to(double acc, int c) const {
-        const double f = c < SUM_DIV ? m : mr;
-        acc = fma(f, x[c], acc);
+        acc = fma(c < SUM_DU ? m : c == SUM_DU ? mv : c == SUM_DIV ? mr : mg, x[c], acc);
         if (c < 3) {
-            acc = fma(f, stress[c], acc);
-            acc = fma(f, visc[c], acc);
+            acc = fma(ms, stress[c], acc);
+            acc = fma(mv, visc[c], acc);
         }
         return acc;
     }
 };
-static_assert(sizeof(PairTerms64) == 160, "PairTerms64 is 160 bytes");
+static_assert(sizeof(PairTerms64) == 176, "PairTerms64 is 176 bytes");
 
 // The sums of one lane's particle in FP64, the same products accumulated in place.
 struct PairAcc64 {
