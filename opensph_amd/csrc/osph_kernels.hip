@@ -8,6 +8,9 @@
 #include "osph_device.h"
 #include "osph_internal.h"
 
+#include <algorithm>
+#include <type_traits>
+
 
 namespace osph {
 
@@ -1218,6 +1221,7 @@ struct alignas(16) PairTermsF {
         x[1] = vy;
         x[2] = vz;
     }
+    __device__ __forceinline__ void finish() {}
     __device__ __forceinline__ double add_to(double acc, int c) const { return acc + double(x[c]); }
 };
 
@@ -1253,7 +1257,10 @@ __device__ __forceinline__ void sum_shared(const Rec* __restrict__ rec, const ui
         const Rec on = rec[en];
         Terms v;
         v.clear();
-        if (t0 + sub < listed) f(o, e, v);
+        if (t0 + sub < listed) {
+            f(o, e, v);
+            v.finish();
+        }
         rows[sub] = v;
         wave_sync();
         const uint32_t cnt = t0 < listed ? min(listed - t0, uint32_t(LANES)) : 0u;
@@ -2252,6 +2259,21 @@ void launch_bounds_reduce(const Launch& l, DevState s, unsigned long long* acc, 
     k_bounds<<<g, BLOCK, 0, l.stream>>>(s, acc, n);
 }
 
+namespace {
+
+unsigned fill_blocks(size_t count) { return std::min(grid_for(count), 4096u); }
+
+// Starts a kernel; false if it did not start (the error also stays as the runtime's last one).  The runtime is asked once
+// for both, where <<<>>> and a look at the last error take two more calls.
+template <typename... P>
+bool started(const Launch& l, void (*kernel)(P...), unsigned blocks, unsigned threads,
+             typename std::common_type<P>::type... args) {
+    void* at[] = { &args... };
+    return hipLaunchKernel(reinterpret_cast<const void*>(kernel), dim3(blocks), dim3(threads), at, 0, l.stream) == hipSuccess;
+}
+
+}  // namespace
+
 // Whole scan tiles with an entry past the last row.
 size_t row_slots(uint32_t slots) { return (size_t(slots) / SCAN_TILE + 1) * SCAN_TILE; }
 
@@ -2260,33 +2282,27 @@ void launch_cell_sort(const Launch& l, DevState s, Grid g, uint32_t* row_count, 
     // without particles nothing reads the table
     if (!rows || !n) return;
     const unsigned blocks = grid_for(n), scans = unsigned(row_slots(g.slots) / SCAN_TILE), waves = grid_for(rows, BLOCK / 64);
-    const bool cells = g.by_cells != 0;
+    const auto* placed = reinterpret_cast<const uint32_t*>(bucket);
     // a kernel that does not start leaves the next one values of an older grid as indexes: the chain ends there
-    auto failed = [] { return hipPeekAtLastError() != hipSuccess; };
-    if (cells) launch_clear_u32(l, first, g.cells, 0u);
-    if (failed()) return;
-    const auto count = cells ? k_row_count<true> : k_row_count<false>;
-    count<<<blocks, BLOCK, 0, l.stream>>>(s, g, row_count, first, where, n);
-    if (failed()) return;
-    k_row_scan<<<scans, SCAN_BLOCK, 0, l.stream>>>(row_count, row_start);
-    if (failed()) return;
-    if (cells) k_cell_starts<<<waves, BLOCK, 0, l.stream>>>(g, row_start, first, rows);
-    if (failed()) return;
-    const auto scatter = cells ? k_row_scatter<true> : k_row_scatter<false>;
-    scatter<<<blocks, BLOCK, 0, l.stream>>>(where, row_start, first, row_count, g.slots, bucket, n);
-    if (failed()) return;
-    if (cells) {
-        k_cell_order<<<blocks, BLOCK, 0, l.stream>>>(where, first, reinterpret_cast<const uint32_t*>(bucket), order, n);
+    if (g.by_cells) {
+        const size_t cells = g.cells;
+        (void)(started(l, k_fill_u32, fill_blocks(cells), BLOCK, first, cells, 0u) &&
+               started(l, k_row_count<true>, blocks, BLOCK, s, g, row_count, first, where, n) &&
+               started(l, k_row_scan, scans, SCAN_BLOCK, row_count, row_start) &&
+               started(l, k_cell_starts, waves, BLOCK, g, row_start, first, rows) &&
+               started(l, k_row_scatter<true>, blocks, BLOCK, where, row_start, first, row_count, g.slots, bucket, n) &&
+               started(l, k_cell_order, blocks, BLOCK, where, first, placed, order, n));
     } else {
-        k_row_order<<<waves, BLOCK, 0, l.stream>>>(g, row_start, bucket, where, order, first, rows);
+        (void)(started(l, k_row_count<false>, blocks, BLOCK, s, g, row_count, first, where, n) &&
+               started(l, k_row_scan, scans, SCAN_BLOCK, row_count, row_start) &&
+               started(l, k_row_scatter<false>, blocks, BLOCK, where, row_start, first, row_count, g.slots, bucket, n) &&
+               started(l, k_row_order, waves, BLOCK, g, row_start, bucket, where, order, first, rows));
     }
 }
 
 void launch_clear_u32(const Launch& l, uint32_t* p, size_t count, uint32_t value) {
     if (!count) return;
-    unsigned g = grid_for(count);
-    g = g > 4096 ? 4096 : g;
-    k_fill_u32<<<g, BLOCK, 0, l.stream>>>(p, count, value);
+    k_fill_u32<<<fill_blocks(count), BLOCK, 0, l.stream>>>(p, count, value);
 }
 
 size_t bounds_partials(size_t n) { return size_t(grid_for(n)) * BOUND_VALUES; }
@@ -2630,18 +2646,11 @@ void batch_advance(const Launch& l, const BatchMember* M, int count, BatchBlocks
 }
 
 void batch_sort(const Launch& l, const BatchMember* M, int count, BatchBlocks pb, bool cells) {
-    auto failed = [] { return hipPeekAtLastError() != hipSuccess; };  // as in launch_cell_sort
-    if (cells) kb_cell_clear<<<pb.total, BLOCK, 0, l.stream>>>(M, pb);
-    if (failed()) return;
-    kb_row_count<<<pb.total, BLOCK, 0, l.stream>>>(M, pb);
-    if (failed()) return;
-    kb_row_scan<<<SCAN_BLOCKS * unsigned(count), SCAN_BLOCK, 0, l.stream>>>(M);
-    if (failed()) return;
-    if (cells) kb_cell_starts<<<pb.total, BLOCK, 0, l.stream>>>(M, pb);
-    if (failed()) return;
-    kb_row_scatter<<<pb.total, BLOCK, 0, l.stream>>>(M, pb);
-    if (failed()) return;
-    kb_row_order<<<pb.total, BLOCK, 0, l.stream>>>(M, pb);
+    // as in launch_cell_sort
+    (void)((!cells || started(l, kb_cell_clear, pb.total, BLOCK, M, pb)) && started(l, kb_row_count, pb.total, BLOCK, M, pb) &&
+           started(l, kb_row_scan, SCAN_BLOCKS * unsigned(count), SCAN_BLOCK, M) &&
+           (!cells || started(l, kb_cell_starts, pb.total, BLOCK, M, pb)) &&
+           started(l, kb_row_scatter, pb.total, BLOCK, M, pb) && started(l, kb_row_order, pb.total, BLOCK, M, pb));
 }
 
 void batch_permute(const Launch& l, const BatchMember* M, BatchBlocks pb) {
