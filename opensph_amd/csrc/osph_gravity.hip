@@ -1613,7 +1613,9 @@ __device__ __forceinline__ bool far_term(double rx, double ry, double rz, double
 // term; few targets per block keep the last wave of blocks short.  n targets and sources, M4, before -> now:
 // 500 174 -> 13 us, 3000 1039 -> 51, 12345 4245 -> 534, 30000 10355 -> 2472 (364 G terms/s).  32 targets per block:
 // 17, 81, 539, 2413 us; 64: 26, 131, 547, 2508; 8 sources a wavefront per chunk: 735 us at 12345; sources gathered from
-// the planes instead of LDS: 656; the general form for every pair: 612.
+// the planes instead of LDS: 656; the general form for every pair: 612.  These are random places: on a lattice many
+// separations have a component that is exactly 0, which far_term leaves to the general form, and wavefronts run both:
+// a close-packed sphere of 3182 / 13788 / 31925 takes 85 / 970 / 3933 us, 1.5 times as long for its pairs.
 constexpr int DIRECT_TARGETS = 16, DIRECT_WAVES = 8, DIRECT_SUB = 2;
 
 template <bool M4>
@@ -2293,7 +2295,9 @@ int build_tree(osph_gravity* g, bool reorder = false) {
 }
 
 // Targets below which a block of four wavefronts shares each target: with a wavefront per target, 6000 of them
-// are about six per SIMD; fewer leave SIMDs without the wavefronts that hide the loads.
+// are about six per SIMD; fewer leave SIMDs without the wavefronts that hide the loads.  One wavefront / four in us, quadrupole
+// FP64, octupole FP64, quadrupole mixed: 1200 targets 187 / 98, 202 / 114, 199 / 92; 3720 264 / 221, 317 / 273, 210 / 189; 5817
+// (100k particles) 423 / 391, 503 / 472, 304 / 312; 7351 445 / 447, 552 / 568, 352 / 365; 11521 699 / 757, 896 / 921, 489 / 563.
 constexpr uint32_t EVAL_SHARED_TARGETS = 6000;
 
 // Targets per walk group: the largest group shares the most work, but it takes about four wavefronts per SIMD

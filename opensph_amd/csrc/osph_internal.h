@@ -188,7 +188,7 @@ struct Tuning {
                               // FP64 step and 1.243 / 1.223 / 1.216 / 1.222 ms per mixed step (fused)
     int fuse_finalize = 1;    // PC step: finalize, corrector and criteria in the pair kernel: 1 always, 0 never,
                               // -1 for FP64 only (the mixed step measured 1.246 ms unfused, 1.234 ms fused)
-    int batch_graph = 1;      // batched steps replay their stages after the sort as a captured HIP graph
+    int batch_graph = 1;      // batched steps replay their stages from the sort on as a captured HIP graph
 };
 
 // Lanes per particle in the pair kernels: a group of 16 or of 4 while one lane each leaves the chip waiting for the

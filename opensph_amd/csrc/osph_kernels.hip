@@ -832,7 +832,8 @@ __device__ __forceinline__ void neighbor_list_at(const double4* __restrict__ pos
 // row of cells at a time and counts its hits, a prefix sum over the group places them.  One lane per particle
 // walks its ~37 rows one after the other, each row two dependent loads (80 us whatever the particle count, until
 // the particles fill the chip); here the group's rows are in flight together.  The rows are numbered over the
-// rectangle of planes and rows around the particle; those of its corners yield no candidates.
+// rectangle of planes and rows around the particle; those of its corners yield no candidates.  Measured against single
+// lanes (lists_shared); other group sizes were not.
 constexpr uint32_t LIST_LANES = 16;
 template <bool SCREEN>
 __device__ __forceinline__ void neighbor_list_shared_at(const double4* __restrict__ pos,
@@ -894,7 +895,7 @@ __device__ __forceinline__ void neighbor_list_shared_at(const double4* __restric
                     const int x0 = max(0, int(floorf(pcx - w)));
                     const int x1 = min(G.dim[0] - 1, int(floorf(pcx + w)));
                     if (x0 <= x1) {
-                        const uint32_t row = G.base + ((spread2(uint32_t(cy)) | (spread2(uint32_t(cz)) << 1)) << G.bits);
+                        const uint32_t row = G.base + row_key(0u, uint32_t(cy), uint32_t(cz), G.bits);
                         b = first[row + uint32_t(x0)];
                         e = first[row + uint32_t(x1) + 1u];
                     }
@@ -2598,6 +2599,8 @@ __global__ void __launch_bounds__(BLOCK) kb_pack(const BatchMember* __restrict__
     }
 }
 
+// (Single lanes whatever the members' sizes: the members' grids, which the choice of groups goes by, are planned in every
+// step, and the launch is captured once.)
 template <bool SCREEN>
 __global__ void __launch_bounds__(BLOCK) kb_lists(const BatchMember* __restrict__ M, BatchBlocks lb) {
     uint32_t m, bid, nb;
