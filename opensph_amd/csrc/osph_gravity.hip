@@ -2194,6 +2194,7 @@ int build_moments(osph_gravity* g, const Tree& t) {
         k_fill_u32g<<<1, BLOCK, 0, st>>>(per_level, MAX_DEPTH + 1, 0u);
         k_depth<<<std::min<unsigned>(grid_for(n - 1), LEVEL_BLOCKS), BLOCK, 0, st>>>(t, g->flag, per_level);
     });
+    if (hipPeekAtLastError() != hipSuccess) return sync(g);  // the moments index by what the launches so far have written
     timed(g, "moments", [&] {
         k_levels<<<1, BLOCK, 0, st>>>(per_level, cursor, g->ntargets_dev, t.error, mailbox_next(g->box));
         k_leaf_moments<<<grid_for(n * size_t(LEAF_LANES)), BLOCK, 0, st>>>(t, g->targets, g->ntargets_dev);
@@ -2257,10 +2258,16 @@ int build_tree(osph_gravity* g, bool reorder = false) {
     g->skip_ready = false;
     Tree t = tree_of(g);
     timed(g, "morton", [&] { k_morton<<<grid_for(n), BLOCK, 0, st>>>(g->s, lo[0], lo[1], lo[2], scale, g->keys, g->iota, n); });
+    // (the library's calls take the last error with them)
+    hipError_t err = hipPeekAtLastError();
     timed(g, "sort", [&] {
-        (void)hipcub::DeviceRadixSort::SortPairs(g->sort_temp, g->sort_temp_bytes, g->keys, g->keys_sorted, g->iota,
-                                                 g->order, int(n), 0, 63, st);
+        if (err == hipSuccess) {
+            err = hipcub::DeviceRadixSort::SortPairs(g->sort_temp, g->sort_temp_bytes, g->keys, g->keys_sorted, g->iota,
+                                                     g->order, int(n), 0, 63, st);
+        }
     });
+    if (err != hipSuccess) (void)hipGetLastError();
+    GCHK(g, err);
     if (reorder && g->reorder_period > 0 && ++g->since_reorder >= g->reorder_period) {
         g->since_reorder = 0;
         Planes dst{};
@@ -2282,9 +2289,14 @@ int build_tree(osph_gravity* g, bool reorder = false) {
     timed(g, "leaves", [&] {
         k_fill_u32g<<<std::min<unsigned>(grid_for(n), 4096), BLOCK, 0, st>>>(g->leaf_at, n, END);
         k_mark_leaves<<<grid_for(2 * n - 1), BLOCK, 0, st>>>(t, g->leaf_at);
-        (void)hipcub::DeviceSelect::If(g->select_temp, g->select_temp_bytes, g->leaf_at, g->targets, g->ntargets_dev,
-                                       int(n), NotEnd(), st);
+        err = hipPeekAtLastError();
+        if (err == hipSuccess) {
+            err = hipcub::DeviceSelect::If(g->select_temp, g->select_temp_bytes, g->leaf_at, g->targets, g->ntargets_dev,
+                                           int(n), NotEnd(), st);
+        }
     });
+    if (err != hipSuccess) (void)hipGetLastError();
+    GCHK(g, err);
     g->ntargets = 1;  // a single particle is the tree's one leaf
     if (n > 1) {
         if (int e = build_moments(g, t)) return e;

@@ -82,6 +82,13 @@ void run(const std::string& name, void** args) {
         for (size_t k = 0; k < arg<size_t>(args, 1); ++k) arg<uint32_t*>(args, 0)[k] = arg<uint32_t>(args, 2);
     } else if (is("8k_boundsE")) {
         write_bounds(arg<uint64_t*>(args, 1));
+    } else if (is("9k_bounds3E")) {
+        write_bounds(arg<uint64_t*>(args, 1));
+    } else if (is("8k_levelsE")) {  // the host's words come by value: (host, posts, value)
+        struct Post { uint64_t *host, *posts, value; };
+        const Post post = arg<Post>(args, 4);
+        post.host[7] = 1;
+        *post.posts = post.value;
     } else if (is("14k_bounds_finalE")) {
         auto* small = arg<uint64_t*>(args, 2);  // the step's accumulators, the first class's bounds from word 16 on
         std::memset(small, 0, 8 * 64);
@@ -113,7 +120,7 @@ extern "C" {
 // ---- the test's side ------------------------------------------------------------------------------------------
 // 0 copies to unregistered host memory, 1 to pinned host memory, 2 pinned allocations, 3 bytes of the largest copy to
 // the host, 4 row counts found non-zero, 5 scatters, 6 events recorded on another device than their own, 7 the largest
-// y or z extent of a launch, 8 launches of a search's kernels with an error pending,
+// y or z extent of a launch, 8 launches of a search's, the pair sums' and gravity's kernels with an error pending,
 // 9 launches for all members of a batch
 long long stub_counter(int k) { return counters[k]; }
 void stub_reset() { std::memset(counters, 0, sizeof(counters)); }
@@ -253,7 +260,8 @@ int hipLaunchKernel(const void* host, Dim3 grid, Dim3, void** args, size_t, void
     if (counters[7] < (long long)grid.y) counters[7] = grid.y;
     if (counters[7] < (long long)grid.z) counters[7] = grid.z;
     if (name.find("kb_") != std::string::npos) ++counters[9];
-    for (const char* k : { "k_row_", "k_cell_", "kb_row_", "kb_cell_", "k_pack", "k_permute", "k_neighbor_lists" }) {
+    for (const char* k : { "k_row_", "k_cell_", "kb_row_", "kb_cell_", "k_pack", "k_permute", "k_neighbor_lists", "k_pairs",
+                           "k_levels", "k_leaf_moments", "k_bucket", "k_moments_", "k_walk", "k_eval" }) {
         if (last_error != SUCCESS && name.find(k) != std::string::npos) ++counters[8];
     }
     if (failures > 0 && name.find(failing) != std::string::npos) {

@@ -93,3 +93,18 @@ def test_the_tuner_times_every_launch_shape_once(stub):
         lanes = dict(autotune.DEFAULT_SPACE)["pairs_lanes"]
         assert len(lanes) == len({4 if v > 1 else 1 for v in lanes})  # 2 and 4 are one launch
     """)
+
+
+@pytest.mark.parametrize("kernel", ["k_morton", "k_radix_tree", "k_mark_leaves", "k_depth"])
+def test_a_failed_launch_of_the_tree(stub, kernel):
+    """The moments index by depths and children."""
+    host_stub.run(stub, f"""
+        from opensph_amd.gravity import GpuGravity
+        g = GpuGravity(np.arange(256.0).reshape(64, 4), np.ones(64))
+        assert g.L.osph_gravity_build(g.ctx) == 0
+        stub.stub_reset()
+        stub.stub_fail_kernel({kernel.encode()!r}, 1)
+        assert g.L.osph_gravity_build(g.ctx) != 0
+        assert stub.stub_counter(8) == 0, stub.stub_counter(8)
+        assert g.L.osph_gravity_build(g.ctx) == 0
+    """)
