@@ -714,11 +714,12 @@ uint32_t* overflow_flag(osph_ctx* c) { return reinterpret_cast<uint32_t*>(c->sma
 
 int launch_lists(osph_ctx* c) {
     if (int e = ensure_list(c, list_entries(c->n, c->kmax))) return e;
+    bool written = false;
     timed(c, "neighbor_lists", [&] {
-        launch_neighbor_lists(L(c), c->pos, c->posf, c->screen, c->grid, c->cell_first, c->list, c->count, c->kmax,
-                              overflow_flag(c), c->n);
+        written = launch_neighbor_lists(L(c), c->pos, c->posf, c->screen, c->grid, c->cell_first, c->list, c->count, c->kmax,
+                                        overflow_flag(c), c->n);
     });
-    return OSPH_OK;
+    return written ? OSPH_OK : sync_check(c);  // nothing may be launched on lists that were not written
 }
 
 // After an overflow of the lists (a particle with more than kmax neighbours): grow kmax to fit the

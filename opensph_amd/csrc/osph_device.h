@@ -5,6 +5,7 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <type_traits>
 
 namespace osph {
 
@@ -13,6 +14,15 @@ constexpr int BLOCK = 256;
 inline unsigned grid_for(size_t n, int block = BLOCK) {
     size_t g = (n + block - 1) / block;
     return unsigned(g > 0 ? g : 1);
+}
+
+// Starts a kernel; false if it did not start (the error also stays as the runtime's last one).  The runtime is asked once
+// for both, where <<<>>> and a look at the last error take two more calls.
+template <typename... P>
+bool started(hipStream_t stream, void (*kernel)(P...), unsigned blocks, unsigned threads, size_t lds,
+             typename std::common_type<P>::type... args) {
+    void* at[] = { &args... };
+    return hipLaunchKernel(reinterpret_cast<const void*>(kernel), dim3(blocks), dim3(threads), at, lds, stream) == hipSuccess;
 }
 
 // Workgroups are dealt round-robin to the 8 XCDs (each with its own L2).  Renumber them so that XCD x

@@ -323,7 +323,7 @@ void launch_cell_sort(const Launch& l, DevState s, Grid g, uint32_t* row_count, 
 void launch_pack(const Launch& l, DevState s, Params prm, const uint32_t* order, PairRec* rec, double4* pos,
                  float4* posf, Screen sc, uint32_t* group, size_t n);
 // Neighbour lists are row-major: list[k * kmax + c], kmax a multiple of 4.
-void launch_neighbor_lists(const Launch& l, const double4* pos, const float4* posf, Screen sc, Grid g,
+bool launch_neighbor_lists(const Launch& l, const double4* pos, const float4* posf, Screen sc, Grid g,
                            const uint32_t* first, uint32_t* list, uint32_t* count, uint32_t kmax, uint32_t* overflow,
                            size_t n);
 // With fuse set, the pair kernels go on, per particle, with what k_finalize_correct does (the finalize

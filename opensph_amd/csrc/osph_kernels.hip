@@ -2264,15 +2264,6 @@ namespace {
 
 unsigned fill_blocks(size_t count) { return std::min(grid_for(count), 4096u); }
 
-// Starts a kernel; false if it did not start (the error also stays as the runtime's last one).  The runtime is asked once
-// for both, where <<<>>> and a look at the last error take two more calls.
-template <typename... P>
-bool started(const Launch& l, void (*kernel)(P...), unsigned blocks, unsigned threads,
-             typename std::common_type<P>::type... args) {
-    void* at[] = { &args... };
-    return hipLaunchKernel(reinterpret_cast<const void*>(kernel), dim3(blocks), dim3(threads), at, 0, l.stream) == hipSuccess;
-}
-
 }  // namespace
 
 // Whole scan tiles with an entry past the last row.
@@ -2287,17 +2278,17 @@ void launch_cell_sort(const Launch& l, DevState s, Grid g, uint32_t* row_count, 
     // a kernel that does not start leaves the next one values of an older grid as indexes: the chain ends there
     if (g.by_cells) {
         const size_t cells = g.cells;
-        (void)(started(l, k_fill_u32, fill_blocks(cells), BLOCK, first, cells, 0u) &&
-               started(l, k_row_count<true>, blocks, BLOCK, s, g, row_count, first, where, n) &&
-               started(l, k_row_scan, scans, SCAN_BLOCK, row_count, row_start) &&
-               started(l, k_cell_starts, waves, BLOCK, g, row_start, first, rows) &&
-               started(l, k_row_scatter<true>, blocks, BLOCK, where, row_start, first, row_count, g.slots, bucket, n) &&
-               started(l, k_cell_order, blocks, BLOCK, where, first, placed, order, n));
+        (void)(started(l.stream, k_fill_u32, fill_blocks(cells), BLOCK, 0, first, cells, 0u) &&
+               started(l.stream, k_row_count<true>, blocks, BLOCK, 0, s, g, row_count, first, where, n) &&
+               started(l.stream, k_row_scan, scans, SCAN_BLOCK, 0, row_count, row_start) &&
+               started(l.stream, k_cell_starts, waves, BLOCK, 0, g, row_start, first, rows) &&
+               started(l.stream, k_row_scatter<true>, blocks, BLOCK, 0, where, row_start, first, row_count, g.slots, bucket, n) &&
+               started(l.stream, k_cell_order, blocks, BLOCK, 0, where, first, placed, order, n));
     } else {
-        (void)(started(l, k_row_count<false>, blocks, BLOCK, s, g, row_count, first, where, n) &&
-               started(l, k_row_scan, scans, SCAN_BLOCK, row_count, row_start) &&
-               started(l, k_row_scatter<false>, blocks, BLOCK, where, row_start, first, row_count, g.slots, bucket, n) &&
-               started(l, k_row_order, waves, BLOCK, g, row_start, bucket, where, order, first, rows));
+        (void)(started(l.stream, k_row_count<false>, blocks, BLOCK, 0, s, g, row_count, first, where, n) &&
+               started(l.stream, k_row_scan, scans, SCAN_BLOCK, 0, row_count, row_start) &&
+               started(l.stream, k_row_scatter<false>, blocks, BLOCK, 0, where, row_start, first, row_count, g.slots, bucket, n) &&
+               started(l.stream, k_row_order, waves, BLOCK, 0, g, row_start, bucket, where, order, first, rows));
     }
 }
 
@@ -2333,29 +2324,19 @@ void launch_pack(const Launch& l, DevState s, Params prm, const uint32_t* order,
     k_pack<<<grid_for(n), BLOCK, 0, l.stream>>>(s, prm, order, rec, pos, posf, sc, group, n);
 }
 
-void launch_neighbor_lists(const Launch& l, const double4* pos, const float4* posf, Screen sc, Grid g,
+bool launch_neighbor_lists(const Launch& l, const double4* pos, const float4* posf, Screen sc, Grid g,
                            const uint32_t* first, uint32_t* list, uint32_t* count, uint32_t kmax, uint32_t* overflow,
                            size_t n) {
-    if (!n) return;
+    if (!n) return true;
     const int b = l.tune.lists_block;
+    const size_t lds = size_t(l.tune.lists_lds);
     if (lists_shared(g, n)) {
-        const unsigned grid = grid_for(n * LIST_LANES, b);
-        if (sc.on) {
-            k_neighbor_lists_shared<true><<<grid, b, size_t(l.tune.lists_lds), l.stream>>>(
-                pos, posf, sc, g, first, list, count, kmax, overflow, n);
-        } else {
-            k_neighbor_lists_shared<false><<<grid, b, size_t(l.tune.lists_lds), l.stream>>>(
-                pos, posf, sc, g, first, list, count, kmax, overflow, n);
-        }
-        return;
+        const auto kernel = sc.on ? k_neighbor_lists_shared<true> : k_neighbor_lists_shared<false>;
+        return started(l.stream, kernel, grid_for(n * LIST_LANES, b), unsigned(b), lds, pos, posf, sc, g, first, list, count,
+                       kmax, overflow, n);
     }
-    if (sc.on) {
-        k_neighbor_lists<true><<<grid_for(n, b), b, size_t(l.tune.lists_lds), l.stream>>>(
-            pos, posf, sc, g, first, list, count, kmax, overflow, n);
-    } else {
-        k_neighbor_lists<false><<<grid_for(n, b), b, size_t(l.tune.lists_lds), l.stream>>>(
-            pos, posf, sc, g, first, list, count, kmax, overflow, n);
-    }
+    const auto kernel = sc.on ? k_neighbor_lists<true> : k_neighbor_lists<false>;
+    return started(l.stream, kernel, grid_for(n, b), unsigned(b), lds, pos, posf, sc, g, first, list, count, kmax, overflow, n);
 }
 
 void launch_pairs_fp64(const Launch& l, DevState s, Params prm, const PairRec* rec, const uint32_t* group,
@@ -2650,10 +2631,10 @@ void batch_advance(const Launch& l, const BatchMember* M, int count, BatchBlocks
 
 void batch_sort(const Launch& l, const BatchMember* M, int count, BatchBlocks pb, bool cells) {
     // as in launch_cell_sort
-    (void)((!cells || started(l, kb_cell_clear, pb.total, BLOCK, M, pb)) && started(l, kb_row_count, pb.total, BLOCK, M, pb) &&
-           started(l, kb_row_scan, SCAN_BLOCKS * unsigned(count), SCAN_BLOCK, M) &&
-           (!cells || started(l, kb_cell_starts, pb.total, BLOCK, M, pb)) &&
-           started(l, kb_row_scatter, pb.total, BLOCK, M, pb) && started(l, kb_row_order, pb.total, BLOCK, M, pb));
+    (void)((!cells || started(l.stream, kb_cell_clear, pb.total, BLOCK, 0, M, pb)) && started(l.stream, kb_row_count, pb.total, BLOCK, 0, M, pb) &&
+           started(l.stream, kb_row_scan, SCAN_BLOCKS * unsigned(count), SCAN_BLOCK, 0, M) &&
+           (!cells || started(l.stream, kb_cell_starts, pb.total, BLOCK, 0, M, pb)) &&
+           started(l.stream, kb_row_scatter, pb.total, BLOCK, 0, M, pb) && started(l.stream, kb_row_order, pb.total, BLOCK, 0, M, pb));
 }
 
 void batch_permute(const Launch& l, const BatchMember* M, BatchBlocks pb) {

@@ -95,6 +95,20 @@ def test_the_tuner_times_every_launch_shape_once(stub):
     """)
 
 
+@pytest.mark.parametrize("call", ["osph_integrate(s.ctx, None)", "osph_step_pc(s.ctx, 1e-6, None, None)", "osph_build_neighbors(s.ctx)"])
+def test_a_failed_launch_of_the_lists(stub, call):
+    """The pair sums would follow entries that nobody wrote."""
+    host_stub.run(stub, f"""
+        s = solver(64)
+        assert s.L.{call} == 0
+        stub.stub_reset()
+        stub.stub_fail_kernel(b"k_neighbor_lists", 1)
+        assert s.L.{call} != 0
+        assert stub.stub_counter(8) == 0, stub.stub_counter(8)
+        assert s.L.{call} == 0
+    """)
+
+
 @pytest.mark.parametrize("kernel", ["k_morton", "k_radix_tree", "k_mark_leaves", "k_depth"])
 def test_a_failed_launch_of_the_tree(stub, kernel):
     """The moments index by depths and children."""
