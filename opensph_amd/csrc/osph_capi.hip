@@ -1494,6 +1494,7 @@ int batch_step(const std::vector<osph_ctx*>& ms, const std::vector<double>& dts,
         batch_permute(l, P->dev, P->pb);
         batch_pack(l, P->dev, P->pb, P->mixed);
         batch_lists(l, P->dev, P->lb, screened, plain);
+        if (hipPeekAtLastError() != hipSuccess) return;  // nor on lists
         batch_pairs(l, P->dev, P->qb, P->mixed, fuse, P->lanes, lead->lut);
         if (!fuse) batch_finalize_correct(l, P->dev, P->pb);
     };

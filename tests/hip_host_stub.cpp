@@ -260,7 +260,8 @@ int hipLaunchKernel(const void* host, Dim3 grid, Dim3, void** args, size_t, void
     if (counters[7] < (long long)grid.y) counters[7] = grid.y;
     if (counters[7] < (long long)grid.z) counters[7] = grid.z;
     if (name.find("kb_") != std::string::npos) ++counters[9];
-    for (const char* k : { "k_row_", "k_cell_", "kb_row_", "kb_cell_", "k_pack", "k_permute", "k_neighbor_lists", "k_pairs",
+    for (const char* k : { "k_row_", "k_cell_", "kb_row_", "kb_cell_", "k_pack", "k_permute", "k_neighbor_lists", "k_pairs", "kb_pack",
+                           "kb_permute", "kb_pairs", "kb_finalize",
                            "k_levels", "k_leaf_moments", "k_bucket", "k_moments_", "k_walk", "k_eval" }) {
         if (last_error != SUCCESS && name.find(k) != std::string::npos) ++counters[8];
     }

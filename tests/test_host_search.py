@@ -47,7 +47,7 @@ def test_a_failed_launch_of_the_sort_by_cells(stub, kernel):
     host_stub.run(stub, BODY.format(precision="fp64", batch=False, cells=1, scatters=1, kernel=kernel.encode()))
 
 
-@pytest.mark.parametrize("cells,kernel", [(0, "kb_row_scatter"), (1, "kb_cell_clear"), (1, "kb_cell_starts"), (0, "kb_row_order")])
+@pytest.mark.parametrize("cells,kernel", [(0, "kb_row_scatter"), (1, "kb_cell_clear"), (1, "kb_cell_starts"), (0, "kb_row_order"), (0, "kb_lists")])
 def test_a_failed_launch_in_a_batch(stub, cells, kernel):
     host_stub.run(stub, BODY.format(precision="fp64", batch=True, cells=cells, scatters=0, kernel=kernel.encode()))
 
