@@ -237,11 +237,11 @@ inline bool lists_shared(const Grid& g, size_t n) {
 // Whether a class's rows of cells may be too long to be ordered a row at a time (the sort's buckets, see
 // osph_kernels.hip): by the mean over its rows, and by the rows of a compact body of n particles at their usual distance
 // of h / 1.3 (w of them along a cell's edge: n^(1/3) / w cells of w^3 in a row), which is what outliers that stretch
-// the cells leave.  Sort in us by rows / cells, one body with a particle so many diameters away: 1M in touch 31 / 157 (n^(1/3)
-// w^2 = 75), 5 away 51 / 64 (400), 10 away 279 / 69 (1600), 20 away 5621 / 172; 300k 5 away 27 / 44 (123), 10 away 58 / 41
-// (490), 50 away 37294 / 199; 125k 10 away 30 / 32 (200), 20 away 112 / 39 (800); 50k 20 away 44 / 33 (333); 10k 50 away
-// 98 / 33 (380); 2k up to 50 away 20 / 30 (80).  Sheets of 125k / 300k / 1M particles, mean 500 / 1200 / 4000: 29 / 48,
-// 44 / 50, 163 / 58; lines of 2k / 10k / 50k: 27 / 27, 174 / 34, 3153 / 45.
+// the cells leave.  Sort in us by rows / cells, one body with a particle so many diameters away: 1M in touch 30 / 185 (n^(1/3)
+// w^2 = 75), 5 away 53 / 68 (400), 10 away 278 / 63 (1600), 20 away 5639 / 86; 300k 5 away 26 / 49 (123), 10 away 55 / 36
+// (490), 50 away 37213 / 76; 125k 10 away 32 / 34 (200), 20 away 115 / 34 (800); 50k 20 away 49 / 29 (333); 10k 50 away
+// 98 / 33 (380); 2k up to 50 away 20 / 30 (80).  Sheets of 125k / 300k / 1M particles, mean 500 / 1200 / 4000: 33 / 48,
+// 48 / 53, 161 / 63; lines of 2k / 10k / 50k: 29 / 27, 173 / 30, 3151 / 34.
 constexpr double ROWS_BODY = 320.0, ROWS_MEAN = 1000.0;
 inline bool sort_by_cells(const GridClass& g, size_t n) {
     const double w = 1.3 * g.cell / g.hmax, count = double(n);

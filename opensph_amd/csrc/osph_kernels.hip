@@ -286,10 +286,31 @@ __device__ __forceinline__ bool row_of(const Grid& g, size_t q, int& cls, uint32
 // By cells, where rows are long: far outliers stretch the cells to 1/250 of the extent, and a compact body then fills a
 // few rows of thousands of particles, too much for a wavefront or block each.  The cells themselves are the buckets
 // and the cell table holds their counts; a particle's place in its cell is the number of lower particles there, counted
-// by a thread each.  That costs a fraction of what the list kernel does with the same cell (it tests the cell's
-// particles, and those of the cells around it, for the same particle), and no row or cell has to fit anywhere.
+// by a thread each.  A wavefront puts its particles of a cell next to one another, so the count goes by such runs: 64 particles
+// each where a cell holds most of them, or where the state is nearly in cell order, down to one each in a random order, and then
+// still a fraction of what the list kernel does with the same cell.  No row or cell has to fit anywhere.
 //
 // The buckets are filled with atomics, in any order; the order within them does not depend on it.
+
+// The valid lanes of the wavefront with this lane's bucket: the first of them, how many lie before this one, and all.
+struct WaveRun {
+    uint32_t leader, before, total;
+};
+__device__ __forceinline__ WaveRun wave_run(uint32_t bucket, bool valid) {
+    const uint32_t lane = threadIdx.x & 63u;
+    WaveRun run{ lane, 0u, 0u };
+    for (unsigned long long open = __ballot(valid); open != 0ull;) {
+        const int l = __builtin_ctzll(open);
+        const unsigned long long same = __ballot(bucket == uint32_t(__builtin_amdgcn_readlane(bucket, l))) & open;
+        if ((same >> lane) & 1ull) {
+            run.leader = uint32_t(l);
+            run.before = uint32_t(__popcll(same & ((1ull << lane) - 1ull)));
+            run.total = uint32_t(__popcll(same));
+        }
+        open &= ~same;
+    }
+    return run;
+}
 
 // Counts the particles of every row: where[i] = (row << 8 | x, rank in the row), or by CELLS of every cell (in `first`)
 // and row: where[i] = (cell, rank in the cell).  One atomic per row or cell and wavefront.
@@ -297,7 +318,6 @@ template <bool CELLS>
 __device__ __forceinline__ void row_count_at(const DevState& s, const Grid& g, uint32_t* __restrict__ row_count,
                                              uint32_t* __restrict__ first, uint2* __restrict__ where, size_t i, size_t n) {
     const bool valid = i < n;
-    const uint32_t lane = threadIdx.x & 63u;
     uint32_t row = 0, key = 0xffffffffu;
     if (valid) {
         const int cls = h_class(s.d[H][i], g.hmin, g.nclass);
@@ -308,25 +328,14 @@ __device__ __forceinline__ void row_count_at(const DevState& s, const Grid& g, u
         key = CELLS ? g.c[cls].base + (mor << g.c[cls].bits) + uint32_t(c[0]) : (row << 8) | uint32_t(c[0]);
     }
     // the lanes of one bucket: its first lane adds their number, each gets its rank among them
-    const uint32_t bucket = CELLS ? key : row;
-    uint32_t leader = lane, before = 0, total = 0;
-    for (unsigned long long open = __ballot(valid); open != 0ull;) {
-        const int l = __builtin_ctzll(open);
-        const unsigned long long same = __ballot(bucket == uint32_t(__builtin_amdgcn_readlane(bucket, l))) & open;
-        if ((same >> lane) & 1ull) {
-            leader = uint32_t(l);
-            before = uint32_t(__popcll(same & ((1ull << lane) - 1ull)));
-            total = uint32_t(__popcll(same));
-        }
-        open &= ~same;
-    }
+    const WaveRun run = wave_run(CELLS ? key : row, valid);
     uint32_t base = 0;
-    if (valid && leader == lane) {
-        base = atomicAdd(CELLS ? &first[key] : &row_count[row], total);
-        if (CELLS) atomicAdd(&row_count[row], total);
+    if (valid && run.leader == (threadIdx.x & 63u)) {
+        base = atomicAdd(CELLS ? &first[key] : &row_count[row], run.total);
+        if (CELLS) atomicAdd(&row_count[row], run.total);
     }
-    base = uint32_t(__shfl(int(base), int(leader), 64));
-    if (valid) where[i] = make_uint2(key, base + before);
+    base = uint32_t(__shfl(int(base), int(run.leader), 64));
+    if (valid) where[i] = make_uint2(key, base + run.before);
 }
 
 template <bool CELLS>
@@ -379,19 +388,20 @@ __global__ void __launch_bounds__(SCAN_BLOCK) k_row_scan(const uint32_t* __restr
     row_scan_tile(row_count, row_start, blockIdx.x);
 }
 
-// bucket[row_start + rank] = (particle, x), or by CELLS the particle alone at its cell's first position + rank.  The row
-// counts go back to zero for the next search.
+// bucket[row_start + rank] = (particle, x), or by CELLS (particle, particles of its wavefront's run) at its cell's first
+// position + rank.  The row counts go back to zero for the next search.
 template <bool CELLS>
 __device__ __forceinline__ void row_scatter_at(const uint2* __restrict__ where, const uint32_t* __restrict__ row_start,
                                                const uint32_t* __restrict__ first, uint32_t* __restrict__ row_count,
                                                uint32_t slots, uint2* __restrict__ bucket, size_t i, size_t threads,
                                                size_t n) {
     for (size_t t = i; t < slots; t += threads) row_count[t] = 0u;
-    if (i >= n) return;
-    const uint2 w = where[i];
+    const bool valid = i < n;
+    const uint2 w = valid ? where[i] : make_uint2(0u, 0u);
     if constexpr (CELLS) {
-        reinterpret_cast<uint32_t*>(bucket)[first[w.x] + w.y] = uint32_t(i);
-    } else {
+        const uint32_t total = wave_run(w.x, valid).total;
+        if (valid) bucket[first[w.x] + w.y] = make_uint2(uint32_t(i), total);
+    } else if (valid) {
         bucket[row_start[w.x >> 8] + w.y] = make_uint2(uint32_t(i), w.x & 255u);
     }
 }
@@ -437,23 +447,27 @@ __global__ void __launch_bounds__(BLOCK) k_cell_starts(Grid g, const uint32_t* _
     cell_starts_at(g, row_start, first, rows, size_t(blockIdx.x) * (BLOCK / 64) + (threadIdx.x >> 6));
 }
 
-// order[] by CELLS: particle i goes behind the lower particles of its cell.
+// order[] by CELLS: particle i goes behind the lower particles of its cell, those of lower wavefronts a run at a time.
 __device__ __forceinline__ void cell_order_at(const uint2* __restrict__ where, const uint32_t* __restrict__ first,
-                                              const uint32_t* __restrict__ placed, uint32_t* __restrict__ order, size_t i,
+                                              const uint2* __restrict__ bucket, uint32_t* __restrict__ order, size_t i,
                                               size_t n) {
     if (i >= n) return;
-    const uint32_t cell = where[i].x;
-    const uint32_t a = first[cell], b = first[cell + 1u];
+    const uint2 w = where[i];
+    const uint32_t a = first[w.x], b = first[w.x + 1u], wave = uint32_t(i >> 6);
     uint32_t r = a;
-#pragma unroll 4
-    for (uint32_t j = a; j < b; ++j) r += placed[j] < uint32_t(i) ? 1u : 0u;
+    for (uint32_t j = a; j < b;) {
+        const uint2 run = bucket[j];
+        if ((run.x >> 6) < wave) r += run.y;
+        if ((run.x >> 6) == wave) r += a + w.y - j;  // its own run: those before it
+        j += max(run.y, 1u);
+    }
     order[r] = uint32_t(i);
 }
 
 __global__ void __launch_bounds__(BLOCK) k_cell_order(const uint2* __restrict__ where, const uint32_t* __restrict__ first,
-                                                      const uint32_t* __restrict__ placed, uint32_t* __restrict__ order,
+                                                      const uint2* __restrict__ bucket, uint32_t* __restrict__ order,
                                                       size_t n) {
-    cell_order_at(where, first, placed, order, size_t(blockIdx.x) * blockDim.x + threadIdx.x, n);
+    cell_order_at(where, first, bucket, order, size_t(blockIdx.x) * blockDim.x + threadIdx.x, n);
 }
 
 // One wavefront per row (y < dim_y, z < dim_z of every class): its particles ordered by (x, particle) into order[],
@@ -2274,7 +2288,6 @@ void launch_cell_sort(const Launch& l, DevState s, Grid g, uint32_t* row_count, 
     // without particles nothing reads the table
     if (!rows || !n) return;
     const unsigned blocks = grid_for(n), scans = unsigned(row_slots(g.slots) / SCAN_TILE), waves = grid_for(rows, BLOCK / 64);
-    const auto* placed = reinterpret_cast<const uint32_t*>(bucket);
     // a kernel that does not start leaves the next one values of an older grid as indexes: the chain ends there
     if (g.by_cells) {
         const size_t cells = g.cells;
@@ -2283,7 +2296,7 @@ void launch_cell_sort(const Launch& l, DevState s, Grid g, uint32_t* row_count, 
                started(l.stream, k_row_scan, scans, SCAN_BLOCK, 0, row_count, row_start) &&
                started(l.stream, k_cell_starts, waves, BLOCK, 0, g, row_start, first, rows) &&
                started(l.stream, k_row_scatter<true>, blocks, BLOCK, 0, where, row_start, first, row_count, g.slots, bucket, n) &&
-               started(l.stream, k_cell_order, blocks, BLOCK, 0, where, first, placed, order, n));
+               started(l.stream, k_cell_order, blocks, BLOCK, 0, where, first, bucket, order, n));
     } else {
         (void)(started(l.stream, k_row_count<false>, blocks, BLOCK, 0, s, g, row_count, first, where, n) &&
                started(l.stream, k_row_scan, scans, SCAN_BLOCK, 0, row_count, row_start) &&
@@ -2494,11 +2507,14 @@ __global__ void __launch_bounds__(BLOCK) kb_bounds_final(const BatchMember* __re
 
 // The launches of a member's own sort, on each member's rows: 16 members of 5k to 212k particles 190 -> 45 us,
 // against one radix sort of all members' keys and two kernels for the tables, 24 launches.
-__global__ void __launch_bounds__(BLOCK) kb_cell_clear(const BatchMember* __restrict__ M, BatchBlocks pb) {
-    uint32_t m, bid, nb;
-    const BatchMember& a = batch_block(M, pb, m, bid, nb);
+// (A stretched grid has up to 16.7M cells however few particles the member has, so these two take blocks of their own.)
+constexpr unsigned CELL_BLOCKS = 256;  // per member
+__global__ void __launch_bounds__(BLOCK) kb_cell_clear(const BatchMember* __restrict__ M) {
+    const BatchMember& a = M[blockIdx.x / CELL_BLOCKS];
     if (!a.grid.by_cells) return;
-    for (size_t t = size_t(bid) * BLOCK + threadIdx.x; t < a.grid.cells; t += size_t(nb) * BLOCK) a.cell_first[t] = 0u;
+    for (uint32_t t = blockIdx.x % CELL_BLOCKS * BLOCK + threadIdx.x; t < a.grid.cells; t += CELL_BLOCKS * BLOCK) {
+        a.cell_first[t] = 0u;
+    }
 }
 
 __global__ void __launch_bounds__(BLOCK) kb_row_count(const BatchMember* __restrict__ M, BatchBlocks pb) {
@@ -2521,12 +2537,12 @@ __global__ void __launch_bounds__(SCAN_BLOCK) kb_row_scan(const BatchMember* __r
     }
 }
 
-__global__ void __launch_bounds__(BLOCK) kb_cell_starts(const BatchMember* __restrict__ M, BatchBlocks pb) {
-    uint32_t m, bid, nb;
-    const BatchMember& a = batch_block(M, pb, m, bid, nb);
+__global__ void __launch_bounds__(BLOCK) kb_cell_starts(const BatchMember* __restrict__ M) {
+    const BatchMember& a = M[blockIdx.x / CELL_BLOCKS];
     if (!a.grid.by_cells) return;
-    for (size_t b = bid; b * (BLOCK / 64) < a.rows; b += nb) {
-        cell_starts_at(a.grid, a.row_start, a.cell_first, a.rows, b * (BLOCK / 64) + (threadIdx.x >> 6));
+    constexpr uint32_t WAVES = BLOCK / 64;
+    for (uint32_t q = blockIdx.x % CELL_BLOCKS * WAVES + (threadIdx.x >> 6); q < a.rows; q += CELL_BLOCKS * WAVES) {
+        cell_starts_at(a.grid, a.row_start, a.cell_first, a.rows, q);
     }
 }
 
@@ -2545,8 +2561,7 @@ __global__ void __launch_bounds__(BLOCK) kb_row_order(const BatchMember* __restr
     uint32_t m, bid, nb;
     const BatchMember& a = batch_block(M, pb, m, bid, nb);
     if (a.grid.by_cells) {
-        cell_order_at(a.where, a.cell_first, reinterpret_cast<const uint32_t*>(a.bucket), a.order,
-                      size_t(bid) * BLOCK + threadIdx.x, a.n);
+        cell_order_at(a.where, a.cell_first, a.bucket, a.order, size_t(bid) * BLOCK + threadIdx.x, a.n);
         return;
     }
     for (size_t b = bid; b * (BLOCK / 64) < a.rows; b += nb) {
@@ -2631,9 +2646,9 @@ void batch_advance(const Launch& l, const BatchMember* M, int count, BatchBlocks
 
 void batch_sort(const Launch& l, const BatchMember* M, int count, BatchBlocks pb, bool cells) {
     // as in launch_cell_sort
-    (void)((!cells || started(l.stream, kb_cell_clear, pb.total, BLOCK, 0, M, pb)) && started(l.stream, kb_row_count, pb.total, BLOCK, 0, M, pb) &&
+    (void)((!cells || started(l.stream, kb_cell_clear, CELL_BLOCKS * unsigned(count), BLOCK, 0, M)) && started(l.stream, kb_row_count, pb.total, BLOCK, 0, M, pb) &&
            started(l.stream, kb_row_scan, SCAN_BLOCKS * unsigned(count), SCAN_BLOCK, 0, M) &&
-           (!cells || started(l.stream, kb_cell_starts, pb.total, BLOCK, 0, M, pb)) &&
+           (!cells || started(l.stream, kb_cell_starts, CELL_BLOCKS * unsigned(count), BLOCK, 0, M)) &&
            started(l.stream, kb_row_scatter, pb.total, BLOCK, 0, M, pb) && started(l.stream, kb_row_order, pb.total, BLOCK, 0, M, pb));
 }
 

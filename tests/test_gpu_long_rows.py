@@ -121,7 +121,7 @@ def kernel_us(x, h, name):
 
 @pytest.mark.parametrize("name", ["outliers", "sheet", "line"])
 def test_time_does_not_depend_on_the_places(name):
-    """300k particles in a compact body take 20 to 27 us, far outliers 117, one line 150; the bound is twenty
+    """300k particles in a compact body take 20 to 27 us, far outliers 82, one line 62; the bound is twenty
     times the compact body's (a sort in place by one block: 4200 us and more than 100 ms)."""
     n = 300000
     body = ball(n)
